@@ -84,10 +84,9 @@ YKA_API const char* yka_build_info(void);
  * key 10: tokens per prefill slice (passes wider than 64 rows), 0 = 1024; 128 .. 4096;
  * key 11: 16-bit row type at the boundary: 0 = fp16 (default), 1 = bf16, the type of the reference's activations
  *        (q35_kernels.cu:1048,1062: Q, gate and attention outputs are bf16 there).  With 1, d_q16 / d_k16 / d_v16 of every
- *        entry point are bf16 and are converted to fp16 by one extra launch per call (round to nearest; exact for
+ *        entry point are bf16 and are converted to fp16 by the kernels that read them (round to nearest; exact for
  *        magnitudes between 2^-14 and 65504, i.e. for normalised activations), attention outputs are rounded once from
- *        their fp32 value to bf16, and yka_attn_post writes q16 / gate16 as bf16.  Setting it to 1 the first time reserves
- *        the staging rows (max_rows of Q, K and V): do that before capturing passes; the call is not on the launch path. */
+ *        their fp32 value to bf16, and yka_attn_post writes q16 / gate16 as bf16. */
 YKA_API int yka_set_opt(yka_kv* kv, int key, int value);
 
 /* Paged mode: logical page p of `layer` (-1 = every layer) lives in physical page h_table[p]; n_pages = max_ctx/256

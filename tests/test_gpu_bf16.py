@@ -88,3 +88,38 @@ def test_post_step_writes_gate_rows(native, oracle, head_dim, bf):
         assert np.array_equal(q.view(np.uint16), q_plain.view(np.uint16))
     for a, b in zip(rows, rows_plain):             # the cache rows do not depend on the row type or on the gate rows
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("form,M", [("128", 2), ("128", 3), ("128", 10), ("128", 11), ("128", 65), ("128 streams", 5), ("256", 2), ("256", 3), ("256 streams", 5),
+                                    ("kv5", 1), ("kv5", 3), ("kv4", 2), ("kv4", 64), ("kv5 streams", 3)])
+def test_bf16_rows_are_read_as_their_fp16_rounding(native, form, M):
+    """Every kernel that reads 16-bit rows (one case per kernel and at the row counts where the dispatch changes): bf16 rows
+    give what their values rounded to fp16 give - the cache bit for bit, fp16 subnormals and roundings included - and the
+    same fp32 outputs rounded to bf16 instead of fp16."""
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(9200 + M)
+    D, streams = (128 if form[:3] == "128" else 256), form.endswith("streams")
+    ctx = 290
+    size = lambda *s: rng.standard_normal(s) * 2.0 ** rng.integers(-18, 4, s)           # down to fp16 subnormals
+    qb, kb, vb = (native.bf16_bits(size(ctx + M, h, D).astype(np.float32)) for h in (24, 4, 4))
+    as16 = lambda b: native.bf16_to_f32(b).astype(np.float16)
+    got = {}
+    for bf in (0, 1):
+        rows = (lambda b: b) if bf else as16
+        with native.KvCache(n_layers=M if streams else 1, max_ctx=512, max_rows=512, head_dim=D) as kv:
+            if form[:2] == "kv":
+                kv.set_profile(kvqp.synthetic(layers=M if streams else 1, kk=int(form[2]), seed=3))
+            kv.set_opt(11, bf)
+            for layer in range(M if streams else 1):
+                kv.append_host(layer, rows(kb[:ctx]), rows(vb[:ctx]), 0)
+            q, k, v = rows(qb[ctx:]), rows(kb[ctx:]), rows(vb[ctx:])
+            if streams:
+                out = kv.ms_call(q, k, v, [ctx - 7 * t for t in range(M)], list(range(M)))
+            else:
+                out = kv.layer_call(0, q, k, v, ctx)
+            got[bf] = [out.view(np.uint16)] + [a for layer in range(M if streams else 1) for a in kv.export_rows(layer, 0, ctx + (1 if streams else M))]
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert np.array_equal(a, b)
+    f16, bf = got[0][0].view(np.float16).astype(np.float32), native.bf16_to_f32(got[1][0])
+    # one fp32 value rounded to fp16 (11 significant bits: 2^-11 of it; 2^-25 below the normal range) and to bf16 (8: 2^-8)
+    assert np.max(np.abs(bf - f16) - (2.0 ** -8 + 2.0 ** -11) * 1.01 * np.abs(f16)) <= 2.0 ** -24

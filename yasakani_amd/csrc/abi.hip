@@ -37,7 +37,6 @@ struct yka_kv {
   int opt_splits_narrow = 0, opt_splits_wide = 0, opt_force_narrow = 0, opt_unrot = 0, opt_ctx_hint = 0, opt_profile_layer = 0, opt_merge_in_launch = 0;
   int opt_chunk_slice = 0;                     // tokens per prefill slice (0: kChunkSlice)
   int opt_io_bf16 = 0;                         // 16-bit rows at the boundary (Q, new K / V, gate, outputs) are bf16, not fp16
-  uint16_t *stage_q = nullptr, *stage_k = nullptr, *stage_v = nullptr;   // fp16 images of bf16 inputs (allocated when option key 11 is set)
   int opt_mid_rows = 10, opt_splits_mid = 0;   // widest window the mid kernel takes (0: none; measured faster than the wide kernel up to 10 rows), its split count (0: automatic)
   // trellis-coded rows (set by yka_kv_set_profile; head_dim 256 only): rows as the reference lays them out, per layer
   // [K payload n_kv * max_ctx * stride][V payload][K scales n_kv * max_ctx fp32][V scales]
@@ -178,7 +177,7 @@ void tb_append(yka_kv* kv, int layer, const float* k32, const float* v32, const 
   for (int t0 = 0; t0 < M; t0 += kTbTileTok) {
     TbEncArgs A{};
     A.blob = T.blob; A.nm = T.nm; A.has_trellis = 1; A.desc = T.desc; A.ngrp = T.ngrp; A.mult_off = T.mult_off;
-    A.k32 = k32; A.v32 = v32; A.k16 = k16; A.v16 = v16; A.d_pos = d_pos; A.layer = layer; A.tok0 = t0; A.n_kv = kv->cfg.n_kv_heads;
+    A.k32 = k32; A.v32 = v32; A.k16 = k16; A.v16 = v16; A.in_bf16 = kv->opt_io_bf16; A.d_pos = d_pos; A.layer = layer; A.tok0 = t0; A.n_kv = kv->cfg.n_kv_heads;
     A.max_ctx = kv->cfg.max_ctx; A.rot = rot; A.pos_limit = pos_limit;
     A.nrow = std::min(kTbTileTok, M - t0) * 2 * kv->cfg.n_kv_heads;
     A.scr = T.scr; A.scr_w_ofs = T.scr_w_ofs;
@@ -203,22 +202,13 @@ void no_trellis(const yka_kv* kv) {
   if (kv->tb) throw std::runtime_error("this entry point does not work on trellis-coded rows");
 }
 
-// bf16 rows at the boundary: one launch turns the pass's Q / new K / new V rows into the fp16 rows the kernels read
-// (either group may be absent); outputs are written as bf16 by the combiners themselves.
-void rows_to_f16(yka_kv* kv, const uint16_t*& q16, const uint16_t*& k16, const uint16_t*& v16, int M, hipStream_t st) {
-  if (!kv->opt_io_bf16) return;
-  if (M < 1 || M > kv->cfg.max_rows) throw std::runtime_error("bf16 rows: the staging rows hold max_rows rows per pass");
-  const size_t nq = (size_t)M * kv->cfg.n_heads * kv->D(), nk = (size_t)M * kv->cfg.n_kv_heads * kv->D();
-  launch_bf16_to_f16(q16, kv->stage_q, q16 ? nq : 0, k16, kv->stage_k, v16, kv->stage_v, nk, st);
-  if (q16) q16 = kv->stage_q;
-  if (k16) { k16 = kv->stage_k; v16 = kv->stage_v; }
-}
-
 void do_append(yka_kv* kv, int layer, const uint16_t* k16, const uint16_t* v16, int M, const int* d_pos, hipStream_t st) {
-  { const uint16_t* none = nullptr; rows_to_f16(kv, none, k16, v16, M, st); }
   if (kv->tb) tb_append(kv, layer, nullptr, nullptr, k16, v16, M, d_pos, 0, st);
-  else if (kv->r256()) launch_append256(AppendArgs{kv->view(layer), k16, v16, d_pos, M}, st);
-  else launch_append(AppendArgs{kv->view(layer), k16, v16, d_pos, M}, st);
+  else {
+    AppendArgs A{kv->view(layer), k16, v16, d_pos, M};
+    A.in_bf16 = kv->opt_io_bf16;
+    if (kv->r256()) launch_append256(A, st); else launch_append(A, st);
+  }
 }
 void need_128(const yka_kv* kv) {
   if (kv->r256()) throw std::runtime_error("this entry point exists for head_dim 128 only");
@@ -231,10 +221,7 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
                hipStream_t st, int mode = 0, const uint16_t* k16 = nullptr, const uint16_t* v16 = nullptr, const Workspace* ws = nullptr) {
   const int NH = kv->cfg.n_heads;
   const Workspace W = ws ? *ws : Workspace{kv->pm, kv->pl, kv->pacc16, kWsPairs, kv->tickets};
-  rows_to_f16(kv, q16, k16, v16, M, st);
-  const int io_was = kv->opt_io_bf16;
-  struct Restore { yka_kv* kv; int v; ~Restore() { kv->opt_io_bf16 = v; } } restore{kv, io_was};
-  kv->opt_io_bf16 = 0;                             // the rows are fp16 from here on (nested do_append calls must not convert again)
+  const int bf16 = kv->opt_io_bf16;                // type of the 16-bit rows that come in and of the outputs
   if (kv->tb) {
     // trellis-coded rows: the encoder runs first (two launches); rows of at most 2 tokens (or option key 3) run on row
     // tiles of 2 tokens x 6 heads, wider slices on 128-row workgroups that decode every tile once into LDS
@@ -250,9 +237,9 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
       S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
       const TbAttnArgs A{T.kpay(layer), T.vpay(layer), T.kscl(layer), T.vscl(layer), kv->cfg.max_ctx, kv->cfg.n_kv_heads, T.stride,
                          T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, layer, q16 + (size_t)s0 * NH * 256, d_pos, depth, Ms, s0, NH, S,
-                         kv->pm, kv->pl, kv->pacc16};
+                         kv->pm, kv->pl, kv->pacc16, RowMap{}, bf16};
       if (narrow) launch_attend_tb(A, T.kb, st); else launch_attend_tb_wide(A, T.kb, st);
-      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, io_was}, st);
+      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
     }
     return;
   }
@@ -271,8 +258,9 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
       S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
       AttnArgs A{kv->view(layer), q16 + (size_t)s0 * NH * 256, d_pos, depth, Ms, s0, NH, S, 0, kv->pm, kv->pl, kv->pacc16,
                  fuse256 ? k16 : nullptr, fuse256 ? v16 : nullptr};
+      A.in_bf16 = bf16;
       if (narrow) launch_attend256(A, st); else launch_attend256_wide(A, st);
-      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, io_was}, st);
+      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
     }
     return;
   }
@@ -294,16 +282,17 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     const int S = narrow ? narrow_splits(kv, Ms, W.pairs) : mid ? mid_splits(kv, Ms, W.pairs) : (chunk ? chunk_splits(kv, Ms, W.pairs) : wide_splits(kv, Ms, W.pairs));
     AttnArgs A{kv->view(layer), q16 + (size_t)s0 * NH * kD, d_pos, depth, Ms, s0, NH, S, wide_rows_per_block(Ms), W.pm, W.pl, W.pacc16,
                fuse_append ? k16 : nullptr, fuse_append ? v16 : nullptr};
+    A.in_bf16 = bf16;
     // option key 7, rows of at most 2 tokens: the last workgroup of each column merges the splits inside the attention launch
     const bool one_launch = narrow && mode == 0 && !kv->opt_unrot && kv->opt_merge_in_launch;
     if (one_launch) {
       // the counters are put back to zero by a fill kernel in front of every such launch: a launch that ended half way
       // (or anything else that left one non-zero) cannot make a later call skip its merge
       launch_zero_ints(W.tickets, kv->cfg.n_kv_heads * kMaxSlice, st);
-      A.tickets = W.tickets; A.out16 = out16 + (size_t)s0 * NH * kD; A.out_bf16 = io_was;
+      A.tickets = W.tickets; A.out16 = out16 + (size_t)s0 * NH * kD; A.out_bf16 = bf16;
     }
     if (narrow) launch_attend_narrow(A, st); else if (mid) launch_attend_mid(A, st); else launch_attend_wide(A, st);
-    if (mode != 2 && !one_launch) launch_combine(CombineArgs{W.pm, W.pl, W.pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * kD, kv->opt_unrot, io_was}, st);
+    if (mode != 2 && !one_launch) launch_combine(CombineArgs{W.pm, W.pl, W.pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * kD, kv->opt_unrot, bf16}, st);
   }
 }
 
@@ -313,8 +302,7 @@ void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const ui
                   const int* row_slot, uint16_t* out16, hipStream_t st) {
   const int NH = kv->cfg.n_heads, D = kv->D();
   const bool r256 = kv->r256();
-  rows_to_f16(kv, q16, k16, v16, M, st);
-  const int io_was = kv->opt_io_bf16;
+  const int bf16 = kv->opt_io_bf16;
   if (kv->tb) {
     // trellis-coded rows: every container is a stream of the layer option key 6 names; its groups code and decode the rows
     const yka_kv::Tb& T = *kv->tb;
@@ -329,25 +317,26 @@ void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const ui
       RowMap Rs = R; Rs.pos += s0; Rs.slot += s0;
       const TbAttnArgs A{T.kpay(0), T.vpay(0), T.kscl(0), T.vscl(0), kv->cfg.max_ctx, kv->cfg.n_kv_heads, T.stride,
                          T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, pl, q16 + (size_t)s0 * NH * 256, nullptr, nullptr, Ms, s0, NH, S,
-                         kv->pm, kv->pl, kv->pacc16, Rs};
+                         kv->pm, kv->pl, kv->pacc16, Rs, bf16};
       launch_attend_tb(A, T.kb, st);
-      launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, io_was}, st);
+      launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
     }
     return;
   }
   const RowMap R{row_pos, row_slot, kv->cfg.n_layers, kv->layer_bytes, kv->n_pages};
-  if (k16) { const AppendArgs P{kv->view(0), k16, v16, nullptr, M, R}; if (r256) launch_append256(P, st); else launch_append(P, st); }
+  if (k16) { AppendArgs P{kv->view(0), k16, v16, nullptr, M, R}; P.in_bf16 = bf16; if (r256) launch_append256(P, st); else launch_append(P, st); }
   for (int s0 = 0; s0 < M; s0 += kMaxSlice) {
     const int Ms = std::min(kMaxSlice, M - s0);
     int S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : (r256 ? 512 : 1024) / (kv->cfg.n_kv_heads * Ms);   // 2 / 4 waves per SIMD
     S = std::min(std::max(2, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
     RowMap Rs = R; Rs.pos += s0; Rs.slot += s0;
     AttnArgs A{kv->view(0), q16 + (size_t)s0 * NH * D, nullptr, nullptr, Ms, s0, NH, S, 128, kv->pm, kv->pl, kv->pacc16, nullptr, nullptr, Rs};
-    const CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * D, kv->opt_unrot, io_was};
+    A.in_bf16 = bf16;
+    const CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * D, kv->opt_unrot, bf16};
     if (r256) { launch_attend256(A, st); launch_combine256(C, st); }
     else if (!kv->opt_unrot && kv->opt_merge_in_launch) {
       launch_zero_ints(kv->tickets, kv->cfg.n_kv_heads * kMaxSlice, st);
-      A.tickets = kv->tickets; A.out16 = C.out16; A.out_bf16 = io_was; launch_attend_narrow(A, st);
+      A.tickets = kv->tickets; A.out16 = C.out16; A.out_bf16 = bf16; launch_attend_narrow(A, st);
     }
     else { launch_attend_narrow(A, st); launch_combine(C, st); }
   }
@@ -437,7 +426,6 @@ void yka_kv_close(yka_kv* kv) {
     (void)hipFree(kv->tb->scr); (void)hipFree(kv->tb->stage);
     delete kv->tb;
   }
-  (void)hipFree(kv->stage_q); (void)hipFree(kv->stage_k); (void)hipFree(kv->stage_v);
   (void)hipFree(kv->pool); (void)hipFree(kv->tables); (void)hipFree(kv->pm); (void)hipFree(kv->pl); (void)hipFree(kv->pacc16); (void)hipFree(kv->d_pos); (void)hipFree(kv->tickets);
   delete kv;
 }
@@ -455,18 +443,7 @@ int yka_set_opt(yka_kv* kv, int key, int value) {
     case 7: kv->opt_merge_in_launch = value != 0; break;
     case 8: if (value < 0 || value > kMaxSlice) throw std::runtime_error("widest window of the mid kernel must be in [0, 64]"); kv->opt_mid_rows = value; break;
     case 9: if (value < 0 || value > kMaxSplits) throw std::runtime_error("splits must be in [0, 256]"); kv->opt_splits_mid = value; break;
-    case 11: {
-      if (value != 0 && value != 1) throw std::runtime_error("row type must be 0 (fp16) or 1 (bf16)");
-      if (value && !kv->stage_q) {                 // not on the launch path: the staging rows are reserved here, once
-        HIPCHK(hipSetDevice(kv->cfg.device));
-        const size_t nq = (size_t)kv->cfg.max_rows * kv->cfg.n_heads * kv->D(), nk = (size_t)kv->cfg.max_rows * kv->cfg.n_kv_heads * kv->D();
-        HIPCHK(hipMalloc((void**)&kv->stage_q, nq * 2));
-        HIPCHK(hipMalloc((void**)&kv->stage_k, nk * 2));
-        HIPCHK(hipMalloc((void**)&kv->stage_v, nk * 2));
-      }
-      kv->opt_io_bf16 = value;
-      break;
-    }
+    case 11: if (value != 0 && value != 1) throw std::runtime_error("row type must be 0 (fp16) or 1 (bf16)"); kv->opt_io_bf16 = value; break;
     case 10: if (value != 0 && (value < 128 || value > 4096)) throw std::runtime_error("prefill slice must be 0 or in [128, 4096] tokens"); kv->opt_chunk_slice = value; break;
     default: throw std::runtime_error("unknown option key");
   }

@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(256) append256_kernel(AppendArgs A) {
     if (pos < 0 || pos >= A.kv.max_ctx) return;
   }
   const size_t e = ((size_t)tok * A.kv.n_kv + kvh) * kD2 + d;
-  float x = A.k32 ? (isv ? A.v32 : A.k32)[e] : __half2float(__ushort_as_half((isv ? A.v16 : A.k16)[e]));
+  float x = A.k32 ? (isv ? A.v32 : A.k32)[e] : row16_value((isv ? A.v16 : A.k16)[e], A.in_bf16);
   if (A.rot) x = rotate256(x, buf, false);
   quant_store_row256(A.kv, kvh, pos, isv, x, d, red, fld);
 }
@@ -267,8 +267,8 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
       if (r < 0 || r >= A.kv.max_ctx || !(held || unseen)) continue;
       mine = true;
       const size_t e = ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD2 + threadIdx.x;
-      quant_store_row256(A.kv, kvh, r, false, __half2float(__ushort_as_half(A.k16[e])), threadIdx.x, a_red, a_fld);
-      quant_store_row256(A.kv, kvh, r, true, __half2float(__ushort_as_half(A.v16[e])), threadIdx.x, a_red, a_fld);
+      quant_store_row256(A.kv, kvh, r, false, row16_value(A.k16[e], A.in_bf16), threadIdx.x, a_red, a_fld);
+      quant_store_row256(A.kv, kvh, r, true, row16_value(A.v16[e], A.in_bf16), threadIdx.x, a_red, a_fld);
     }
     if (mine) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -281,10 +281,13 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   h8 qf[8];
   {
     const uint16_t* qrow = A.q16 + ((size_t)tl * A.n_heads + head) * kD2 + 64 * g;
+    uint4 u[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) u[t] = vrow ? *reinterpret_cast<const uint4*>(qrow + 8 * t) : make_uint4(0, 0, 0, 0);
+    rows16_to_f16(u, A.in_bf16);
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      uint4 u = vrow ? *reinterpret_cast<const uint4*>(qrow + 8 * t) : make_uint4(0, 0, 0, 0);
-      const h8 c = __builtin_bit_cast(h8, u);
+      const h8 c = __builtin_bit_cast(h8, u[t]);
       qf[t] = h8{c[7], c[3], c[6], c[2], c[5], c[1], c[4], c[0]};
     }
   }

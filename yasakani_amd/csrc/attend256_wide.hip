@@ -152,7 +152,8 @@ __device__ __forceinline__ void quant_store_word256(const KvView& kv, int kvh, i
 
 }  // namespace
 
-// grid (S, n_kv, ceil(6M / 128)), block 512; wave w owns rows [16 w, 16 (w+1)) of the block
+// grid (S, n_kv, ceil(6M / 128)), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 rows come in
+template <bool BF>
 __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   __shared__ __align__(16) uint8_t lds[2][kLdsBuf];
   const int split = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
@@ -170,15 +171,21 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   if (vrow) { const int tg = A.tok0 + tl; len = min(pos + (A.depth ? (int)A.depth[tg] : tg) + 1, A.kv.max_ctx); }
   // Q fragments: k-step t of 8, lane (row i, group g), element e <-> channel 8 (4t + g) + [7,3,6,2,5,1,4,0][e]
   h8 qf[8];
+  uint4 qraw[8];                               // as loaded; bf16 rows become qf behind the wait for the first tile
   {
     const uint16_t* qrow = A.q16 + ((size_t)tl * A.n_heads + head) * kD2 + 8 * g;
 #pragma unroll
+    for (int t = 0; t < 8; ++t) qraw[t] = vrow ? *reinterpret_cast<const uint4*>(qrow + 32 * t) : make_uint4(0, 0, 0, 0);
+  }
+  auto q_ready = [&]() __attribute__((always_inline)) {
+    if constexpr (BF) rows16_to_f16(qraw);
+#pragma unroll
     for (int t = 0; t < 8; ++t) {
-      uint4 u = vrow ? *reinterpret_cast<const uint4*>(qrow + 32 * t) : make_uint4(0, 0, 0, 0);
-      const h8 c = __builtin_bit_cast(h8, u);
+      const h8 c = __builtin_bit_cast(h8, qraw[t]);
       qf[t] = h8{c[7], c[3], c[6], c[2], c[5], c[1], c[4], c[0]};
     }
-  }
+  };
+  if constexpr (!BF) q_ready();
   const bool has_rows = row0 < nrows;                       // wave uniform
 
   // key range of the workgroup: its splits cut [0, maxlen) of the block's longest row into 32-key tiles
@@ -211,6 +218,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
         const uint16_t* src = ((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD2 + 8 * c;
         rawv[it] = mine[it] ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
       }
+      if constexpr (BF) rows16_to_f16(rawv);
 #pragma unroll
       for (int it = 0; it < 8; ++it) {
         const int hh = it * 16 + slot;
@@ -237,6 +245,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   if (tile0 < tile1) {
     load_tile_raw(tile0, raw0);
     wait_raw<0>(raw0);
+    if constexpr (BF) q_ready();               // every load has been answered: the query costs no trip to memory of its own
     dequant_to_lds(lds[0], tid, raw0, magic);
     load_tile_raw(min(tile0 + 1, tile1 - 1), raw1);
     load_tile_raw(min(tile0 + 2, tile1 - 1), raw0);
@@ -356,7 +365,9 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
 
 void launch_attend256_wide(const AttnArgs& A, hipStream_t st) {
   const int rows = kG * A.M, rb = (rows + 127) / 128;
-  hipLaunchKernelGGL(attend256_wide_kernel, dim3(A.S, A.kv.n_kv, rb), dim3(NT), 0, st, A);
+  const dim3 grid(A.S, A.kv.n_kv, rb);
+  if (A.in_bf16) hipLaunchKernelGGL(attend256_wide_kernel<true>, grid, dim3(NT), 0, st, A);
+  else hipLaunchKernelGGL(attend256_wide_kernel<false>, grid, dim3(NT), 0, st, A);
 }
 
 }  // namespace yka

@@ -128,6 +128,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
     dep[rt] = v ? (A.depth ? (int)A.depth[tg] : tg) : -1;
   }
   const int pos = *A.d_pos;
+  rows16_to_f16(qraw, A.in_bf16);
 #pragma unroll
   for (int rt = 0; rt < NRT; ++rt) {
     const h8 c = __builtin_bit_cast(h8, qraw[rt]);
@@ -183,6 +184,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
           const uint16_t* src = ((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD + 8 * c;
           rawv[it] = t < nst ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
         }
+        rows16_to_f16(rawv, A.in_bf16);
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
           const int hh = h0 + it * 16 + slot, t = hh >> 1, r = pos + A.tok0 + t;

@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
       mine = true;
       const bool isv = threadIdx.x >= 128;
       const uint16_t* src = (isv ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD;
-      quant_store_row(A.kv, kvh, r, isv, src, threadIdx.x & 127);
+      quant_store_row(A.kv, kvh, r, isv, src, threadIdx.x & 127, A.in_bf16);
     }
     if (mine) {                      // uniform over the workgroup
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -284,9 +284,13 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
     // kinds of products are 4 q n and neither factor costs fp16 range at one end only (a plain 1/16 on the odd channels
     // pushes queries below 1e-3 into the subnormals); the 4 leaves with the softmax scale
     const _Float16 se = (_Float16)4.f, so = (_Float16)0.25f;
+    uint4 qw[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) qw[m] = __builtin_bit_cast(uint4, vrow ? (qraw[m] | u32x4{z, z, z, z}) : u32x4{0u, 0u, 0u, 0u});
+    rows16_to_f16(qw, A.in_bf16);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      const h8 c = __builtin_bit_cast(h8, vrow ? (qraw[m] | u32x4{z, z, z, z}) : u32x4{0u, 0u, 0u, 0u});
+      const h8 c = __builtin_bit_cast(h8, qw[m]);
       qf[m] = h8{c[0] * se, c[4] * se, c[1] * so, c[5] * so, c[2] * se, c[6] * se, c[3] * so, c[7] * so};
       // -8 * 2^-24 * (sum of the row's 32 query channels of group m): the lane's 8 channels, then its 3 sister lanes
       float qs = 0.f;

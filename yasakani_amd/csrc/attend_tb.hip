@@ -115,10 +115,11 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
   const int tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
 
   h8 qf[8];                                          // k-step t: channels 64 g + 8 t .. + 7 of row i
+  uint4 qraw[8];
   {
     const uint16_t* qrow = A.q16 + ((size_t)tl * A.n_heads + head) * kD2 + 64 * g;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, vrow ? *reinterpret_cast<const uint4*>(qrow + 8 * t) : make_uint4(0, 0, 0, 0));
+    for (int t = 0; t < 8; ++t) qraw[t] = vrow ? *reinterpret_cast<const uint4*>(qrow + 8 * t) : make_uint4(0, 0, 0, 0);
   }
   const float sc_log2 = kLog2e * 0.0625f * A.gfac[gK];      // log2(e) / sqrt(256) x gain / 256 of the K table
   const size_t row0 = (size_t)kvh * A.max_ctx;
@@ -167,6 +168,9 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
     }
   };
   if (tile0 + wave < tile1) load_k(tile0 + wave);
+  rows16_to_f16(qraw, A.in_bf16);                    // behind the first tile's requests: a bf16 query does not hold them up
+#pragma unroll
+  for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, qraw[t]);
   for (int T = tile0 + wave; T < tile1; T += 4) {
     const int t0 = T << 5;
     f4 vsc[2];

@@ -135,8 +135,8 @@ __device__ __forceinline__ void decode_to_lds(uint8_t* buf, int tid, const Raw& 
   reinterpret_cast<uint32_t*>(buf + kLdsS)[tid & 63] = R.sc;      // waves repeat each other (no divergent branch)
 }
 
-// grid (S, n_kv, ceil(6M / 128)), block 512; wave w owns rows [16 w, 16 (w+1)) of the block
-template <int KB>
+// grid (S, n_kv, ceil(6M / 128)), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 queries
+template <int KB, bool BF>
 __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   constexpr int kTabBytes = 4 << (8 + KB);
   __shared__ __align__(16) uint8_t lds[2][kLdsBuf];
@@ -166,11 +166,18 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   if (vrow) { const int tg = A.tok0 + tl; len = min(pos + (A.depth ? (int)A.depth[tg] : tg) + 1, A.max_ctx); }
   // Q fragments: k-step t of 8, lane (row i, group g), element e <-> channel 8 (4t + g) + e
   h8 qf[8];
+  uint4 qraw[8];                               // as loaded; bf16 rows become qf behind the wait for the first tile
   {
     const uint16_t* qrow = A.q16 + ((size_t)tl * A.n_heads + head) * kD2 + 8 * g;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, vrow ? *reinterpret_cast<const uint4*>(qrow + 32 * t) : make_uint4(0, 0, 0, 0));
+    for (int t = 0; t < 8; ++t) qraw[t] = vrow ? *reinterpret_cast<const uint4*>(qrow + 32 * t) : make_uint4(0, 0, 0, 0);
   }
+  auto q_ready = [&]() __attribute__((always_inline)) {
+    if constexpr (BF) rows16_to_f16(qraw);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, qraw[t]);
+  };
+  if constexpr (!BF) q_ready();
   const bool has_rows = row0 < nrows;                       // wave uniform
 
   // key range of the workgroup: its splits cut [0, maxlen) of the block's longest row into 32-key tiles
@@ -198,6 +205,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   if (tile0 < tile1) {
     load_tile_raw(tile0, raw);
     wait_raw(raw);
+    if constexpr (BF) q_ready();               // every load has been answered: the query costs no trip to memory of its own
     decode_to_lds<KB>(lds[0], tid, raw, offs, tabK, tabV);
     load_tile_raw(min(tile0 + 1, tile1 - 1), raw);
   }
@@ -321,8 +329,10 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
 void launch_attend_tb_wide(const TbAttnArgs& A, int kb, hipStream_t st) {
   const int rows = kG * A.M, rb = (rows + 127) / 128;
   const dim3 grid(A.S, A.n_kv, rb);
-  if (kb == 4) hipLaunchKernelGGL(attend_tb_wide_kernel<4>, grid, dim3(NT), 0, st, A);
-  else hipLaunchKernelGGL(attend_tb_wide_kernel<5>, grid, dim3(NT), 0, st, A);
+  if (kb == 4 && A.in_bf16) hipLaunchKernelGGL((attend_tb_wide_kernel<4, true>), grid, dim3(NT), 0, st, A);
+  else if (kb == 4) hipLaunchKernelGGL((attend_tb_wide_kernel<4, false>), grid, dim3(NT), 0, st, A);
+  else if (A.in_bf16) hipLaunchKernelGGL((attend_tb_wide_kernel<5, true>), grid, dim3(NT), 0, st, A);
+  else hipLaunchKernelGGL((attend_tb_wide_kernel<5, false>), grid, dim3(NT), 0, st, A);
 }
 
 }  // namespace yka

@@ -165,6 +165,9 @@ __device__ __forceinline__ void dequant_to_lds(uint8_t* buf, int tid, const Raw&
 // blocks of F whole pairs (the k-th is row block k mod n_rb of pair x + 8 (k / n_rb)): all row blocks of such a pair run
 // on one XCD at about the same time and each tile leaves HBM once.  The workgroups left over on every XCD take the
 // remaining pairs in order.
+// BF: Q / new K / new V are bf16 rows; a kernel of its own, because a branch around the conversion in this one costs the fp16
+// rows 1.5 % (755 against 767 us for 16 layers of 64 rows at 32,768 tokens)
+template <bool BF>
 __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   __shared__ __align__(16) uint8_t lds[2][2][kLdsBuf];               // [group][buffer]
   const int n_rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block;
@@ -196,18 +199,24 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   const size_t pidx = ((size_t)tl * A.S + split) * A.n_heads + head;
   // B operand of S^T = K Q^T, k-step ks: lane (row j, half h) holds chunk 2ks+h = (group ks/2, sub-chunk 2(ks&1)+h)
   h8 qf[8];
+  uint4 qraw[8];                               // as loaded; bf16 rows become qf behind the wait for the first tile
   {
     const uint16_t* qrow = A.q16 + ((size_t)tl * A.n_heads + head) * kD;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qraw[ks] = vrow ? *reinterpret_cast<const uint4*>(qrow + 32 * (ks >> 1) + 8 * (2 * (ks & 1) + h)) : make_uint4(0, 0, 0, 0);
+  }
+  auto q_ready = [&]() __attribute__((always_inline)) {
+    if constexpr (BF) rows16_to_f16(qraw);
     // the odd nibble of a byte is 16 (n - 8) in the K image: its query channels carry 1/4 and the others 4 (products 4 q n
     // either way; a plain 1/16 would push small queries into the fp16 subnormals), the 4 leaves with the softmax scale
     const _Float16 se = (_Float16)4.f, so = (_Float16)0.25f;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      uint4 u = vrow ? *reinterpret_cast<const uint4*>(qrow + 32 * (ks >> 1) + 8 * (2 * (ks & 1) + h)) : make_uint4(0, 0, 0, 0);
-      const h8 c = __builtin_bit_cast(h8, u);
+      const h8 c = __builtin_bit_cast(h8, qraw[ks]);
       qf[ks] = h8{c[0] * se, c[4] * se, c[1] * so, c[5] * so, c[2] * se, c[6] * se, c[3] * so, c[7] * so};
     }
-  }
+  };
+  if constexpr (!BF) q_ready();
   const bool has_rows = row0 < min(nrows, (rb + 1) * RPB);             // wave uniform
 
   // key range of the workgroup: its splits cut [0, maxlen) of the block's longest row into 32-key tiles
@@ -251,6 +260,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
         const uint16_t* src = ((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD + 8 * c;
         rawv[it] = t < tok_hi ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
       }
+      if constexpr (BF) rows16_to_f16(rawv);
 #pragma unroll
       for (int it = 0; it < 8; ++it) {
         const int hh = it * 16 + slot, t = hh >> 1, r = pos + A.tok0 + t;
@@ -285,6 +295,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   if (nu > 0) {
     load_tile_raw(tile_of(0), raw0);
     wait_raw<0>(raw0);
+    if constexpr (BF) q_ready();               // every load has been answered: the query costs no trip to memory of its own
     dequant_to_lds(lds[grp][0], gt, raw0, magic, sc_log2);
     load_tile_raw(tile_of(1), raw1);
     load_tile_raw(tile_of(2), raw0);
@@ -486,7 +497,9 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
 
 void launch_attend_wide(const AttnArgs& A, hipStream_t st) {
   const int rows = kG * A.M, rb = (rows + A.rows_per_block - 1) / A.rows_per_block;
-  hipLaunchKernelGGL(attend_wide_kernel, dim3(A.S * A.kv.n_kv * rb), dim3(NT), 0, st, A);
+  const dim3 grid(A.S * A.kv.n_kv * rb);
+  if (A.in_bf16) hipLaunchKernelGGL(attend_wide_kernel<true>, grid, dim3(NT), 0, st, A);
+  else hipLaunchKernelGGL(attend_wide_kernel<false>, grid, dim3(NT), 0, st, A);
 }
 
 }  // namespace yka

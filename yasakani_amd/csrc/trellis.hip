@@ -108,6 +108,7 @@ struct RowRef {
   bool valid;          // multi-stream pass: false if the row names no container
 };
 // Probe form: rows with their own group and position.  Cache form: row r of the launch = (token r / (2 n_kv), K | V, kv head)
+template <bool BF>
 __device__ __forceinline__ RowRef locate_row(const TbEncArgs& A, int r, float* rot_buf) {
   const int d = threadIdx.x;
   RowRef R{};
@@ -129,7 +130,7 @@ __device__ __forceinline__ RowRef locate_row(const TbEncArgs& A, int r, float* r
     }
     R.group = (A.layer * A.n_kv + kvh) * 2 + R.is_v;
     const size_t src = ((size_t)tok * A.n_kv + kvh) * 256 + d;
-    R.x = A.k32 ? (R.is_v ? A.v32 : A.k32)[src] : __half2float(__ushort_as_half((R.is_v ? A.v16 : A.k16)[src]));
+    R.x = A.k32 ? (R.is_v ? A.v32 : A.k32)[src] : row16_value((R.is_v ? A.v16 : A.k16)[src], BF);
     R.index = (size_t)kvh * A.max_ctx + (size_t)max(0, min(R.pos, A.max_ctx - 1));
   }
   if (A.rot) R.x = rotate256(R.x, rot_buf, false);
@@ -421,6 +422,7 @@ __device__ __forceinline__ void wave_chunk3(const int* xi, const int (&ci4)[4], 
 
 // grid rows * nm, block 256: block = (row, multiplier); wave c = chunk c.  Writes the 256 states of the row under this
 // multiplier and the 8 partial error sums to scratch.
+template <bool BF>
 __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) {
   __shared__ float part8[8];
   __shared__ float rot_buf[256];
@@ -431,7 +433,7 @@ __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) {
   const int d = threadIdx.x, wave = d >> 6, lane = d & 63;
   const int row = blockIdx.x / A.nm, mult = blockIdx.x % A.nm;
   const Profile P{A.blob, A.desc, A.ngrp, A.mult_off};
-  const RowRef R = locate_row(A, row, rot_buf);
+  const RowRef R = locate_row<BF>(A, row, rot_buf);
   const GroupRec G = read_group(P, R.group);
   if (!G.present || R.pos < G.guard || G.mode != 0) return;                // uniform over the block: nothing to search
   // everything the search needs from memory is requested before the residual's block reductions
@@ -525,6 +527,7 @@ __device__ __forceinline__ Coded code_trellis(const TbEncArgs& A, const Profile&
 
 // grid rows, block 256: codes the row (best multiplier of the search, or the flat quantizer), rebuilds what it decodes to,
 // packs the fields, stores payload / scale / projection coefficients
+template <bool BF>
 __global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
   __shared__ float part8[8];
   __shared__ float rot_buf[256];
@@ -532,7 +535,7 @@ __global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
   __shared__ float totals[kMaxMult], mults[kMaxMult];
   const int d = threadIdx.x, row = blockIdx.x;
   const Profile P{A.blob, A.desc, A.ngrp, A.mult_off};
-  const RowRef R = locate_row(A, row, rot_buf);
+  const RowRef R = locate_row<BF>(A, row, rot_buf);
   const GroupRec G = read_group(P, R.group);
   Coded C{0, 4, 1.f, R.x, false};
   float rebuilt = R.x;                                   // rows that stay uncoded come back as they are
@@ -614,8 +617,13 @@ __global__ void __launch_bounds__(256) tb_unpack_kernel(const uint8_t* blob, con
 
 void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
   if (A.nrow <= 0) return;
-  if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
-  hipLaunchKernelGGL(tb_select_kernel, dim3(A.nrow), dim3(256), 0, st, A);
+  if (A.in_bf16) {                       // BF: k16 / v16 are bf16 rows
+    if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<true>, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
+    hipLaunchKernelGGL(tb_select_kernel<true>, dim3(A.nrow), dim3(256), 0, st, A);
+    return;
+  }
+  if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<false>, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
+  hipLaunchKernelGGL(tb_select_kernel<false>, dim3(A.nrow), dim3(256), 0, st, A);
 }
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t st) {

@@ -47,7 +47,8 @@ __device__ __forceinline__ KvView slot_view(KvView v, const RowMap& R, int slot)
 // k32 / v32 / rot: 256-channel rows only (attend256.hip) - fp32 source rows instead of fp16 ones, and the signed Hadamard
 // rotation applied to every row before it is quantized (src/q35_kernels.cu:1036,1060 + launch_tb_requant)
 struct AppendArgs { KvView kv; const uint16_t* k16; const uint16_t* v16; const int* d_pos; int M; RowMap rows;
-                    const float* k32 = nullptr; const float* v32 = nullptr; int rot = 0; };
+                    const float* k32 = nullptr; const float* v32 = nullptr; int rot = 0;
+                    int in_bf16 = 0; };   // k16 / v16 are bf16 rows
 
 // partial results of the split-KV kernels (same roles as pm/pl/pacc of the reference, args.hpp:10):
 //   pm, pl [rows_tok][S][n_heads] fp32; pacc16 [rows_tok][S][n_heads][128] fp16 = acc / l (normalised, so that fp16
@@ -70,6 +71,7 @@ struct AttnArgs {
   // tile) column takes a ticket from tickets[kv head * gridDim.z + row tile] once its partials are out, and the one that
   // draws the last ticket merges the column's partials into out16 and puts the counter back to zero
   int* tickets = nullptr; uint16_t* out16 = nullptr; int out_bf16 = 0;
+  int in_bf16 = 0;   // q16 / k16 / v16 are bf16 rows (rows16_to_f16)
 };
 // unrot != 0: the output row gets the inverse signed Hadamard rotation (7 butterfly stages, x 1/16, signs) before it is
 // rounded to fp16 - the counterpart of rotating V rows on their way into the cache (src/q35_kernels.cu:1421)
@@ -109,6 +111,7 @@ struct TbEncArgs {
   uint8_t* pay0; uint8_t* pay1; float* scl0; float* scl1; int stride;
   int pos_limit;                      // cache form: rows at positions >= pos_limit are not stored (0: no limit besides max_ctx)
   RowMap rows;                        // cache form, multi-stream pass: token t sits at rows.pos[t] of container rows.slot[t] (pay / scl = container 0)
+  int in_bf16;                        // cache form: k16 / v16 are bf16 rows
 };
 // attention over trellis-coded rows (attend_tb.hip).  pairs [groups][2^(8 + kb)]: entry i = the table's integers, as two
 // fp16 values, of the states (i >> kb) & 255 and i & 255 (two consecutive elements from 8 + kb stream bits); gfac [groups]:
@@ -119,6 +122,7 @@ struct TbAttnArgs {
   const uint16_t* q16; const int* d_pos; const uint8_t* depth; int M, tok0, n_heads, S;
   float* pm; float* pl; uint16_t* pacc16;
   RowMap rows;  // narrow kernel only: multi-stream pass (one token per workgroup column; kpay .. vscl = container 0, `layer` = the profile's layer)
+  int in_bf16 = 0;   // q16 is bf16 rows
 };
 void launch_attend_tb(const TbAttnArgs&, int kb, hipStream_t);        // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend_tb_wide(const TbAttnArgs&, int kb, hipStream_t);   // 3..64 rows: 128 query rows per workgroup, tiles decoded once into LDS
@@ -149,8 +153,6 @@ void launch_dequant_rows(const KvView&, int pos0, int n, float* k, float* v, hip
 void launch_codec_probe(const uint16_t* x16, int rows, uint8_t* codes, uint16_t* scales, float* y, hipStream_t);
 void launch_set_int(int* p, int v, hipStream_t);
 void launch_zero_ints(int* p, int n, hipStream_t);   // a fill kernel (safe inside a captured graph, unlike a memset node)
-// bf16 rows -> fp16 rows (round to nearest even; exact for magnitudes fp16 holds), n values each; any pointer pair may be null
-void launch_bf16_to_f16(const uint16_t* a, uint16_t* a16, size_t na, const uint16_t* b, uint16_t* b16, const uint16_t* c, uint16_t* c16, size_t nbc, hipStream_t);
 // the reference's own 256-channel row format (row256.hip): mode 0 = int8 rows, 1 = flat int4 (32 MSB-first words per row)
 void launch_row256_encode(const float* x, int rows, int mode, int rot, int8_t* q8, uint32_t* words, float* scales, hipStream_t);
 void launch_row256_decode(int rows, int mode, int rot, const int8_t* q8, const uint32_t* words, const float* scales, float* y, hipStream_t);
@@ -170,6 +172,29 @@ __device__ __forceinline__ uint16_t f2bf_bits(float x) {
   return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 __device__ __forceinline__ float bf_bits2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
+// Rows a caller hands over in bf16 (option key 11) become fp16 where they are read: every kernel that takes 16-bit rows
+// calls these on the registers it has loaded.  The fp32 value of a bf16 is rounded to fp16 (nearest even; exact for
+// magnitudes between 2^-14 and 65504).  The flag is a kernel argument, i.e. a scalar.  One branch serves all
+// registers of a thread (a branch per register makes every load wait for the one before it: 4 us of the 36 us of a
+// 1,024-row prefill slice); kernels whose fp16 form a branch would slow down have a form of their own for bf16 rows.
+// A launch of its own that converted the rows first cost 1.5 .. 4 us of every call (a third of a decode call at 1,000
+// tokens: 9.8 us with it, 7.0 without).
+__device__ __forceinline__ uint32_t bf_pair_to_f16(uint32_t w) {
+  const uint16_t lo = __half_as_ushort(__float2half_rn(__uint_as_float(w << 16))), hi = __half_as_ushort(__float2half_rn(__uint_as_float(w & 0xffff0000u)));
+  return (uint32_t)lo | ((uint32_t)hi << 16);
+}
+template <int N>
+__device__ __forceinline__ void rows16_to_f16(uint4 (&r)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) { r[k].x = bf_pair_to_f16(r[k].x); r[k].y = bf_pair_to_f16(r[k].y); r[k].z = bf_pair_to_f16(r[k].z); r[k].w = bf_pair_to_f16(r[k].w); }
+}
+template <int N>
+__device__ __forceinline__ void rows16_to_f16(uint4 (&r)[N], int bf16) { if (bf16) rows16_to_f16(r); }
+// one value: both readings and a select, no branch
+__device__ __forceinline__ float row16_value(uint16_t b, int bf16) {
+  const float as_f16 = __half2float(__ushort_as_half(b)), as_bf16 = __half2float(__float2half_rn(bf_bits2f(b)));
+  return bf16 ? as_bf16 : as_f16;
+}
 // 8 fp32 results -> 16 bytes of fp16 or bf16
 __device__ __forceinline__ uint4 pack_out8(const float* y, int bf16) {
   uint32_t w[4];
