@@ -1,0 +1,63 @@
+"""Prefill chunks (more than 64 rows): the number of splits is chosen on the device from the position, and a slice that uses
+one writes its output without a combiner.  Against the oracle, and against the decode kernel forced on the same rows."""
+import numpy as np
+import pytest
+
+from tests.tolerances import assert_attn_close
+
+pytestmark = pytest.mark.gpu
+
+
+# rows around a row block (21 1/3 tokens), a slice (2,048) and its tail; contexts on both sides of one split
+@pytest.mark.parametrize("M,ctx,max_ctx,paged", [
+    (65, 0, 4096, False), (65, 3000, 32768, True), (85, 31, 512, False), (129, 700, 8192, True), (683, 0, 8192, False),
+    (300, 5000, 32768, False), (1100, 33, 1280, True),
+])
+def test_against_the_oracle(native, oracle, M, ctx, max_ctx, paged):
+    q, k, v, kn, vn, _ = oracle.make_inputs(M, ctx, M)
+    oc = oracle.Cache(max_ctx)
+    with native.KvCache(max_ctx=max_ctx, max_rows=M, paged=paged) as kv:
+        if paged:
+            kv.set_page_table(np.random.default_rng(M).permutation(max_ctx // 256).astype(np.int32))
+        if ctx:
+            oc.append(k, v, 0)
+            kv.import_rows(0, 0, oc.kc[:, :ctx], oc.ks[:, :ctx], oc.vc[:, :ctx], oc.vs[:, :ctx])
+        kv.poison_workspace()
+        out = kv.layer_call(0, q, kn, vn, ctx)
+        got = kv.export_rows(0, ctx, M)
+    oc.append(kn, vn, ctx)
+    for a, b in zip(got, (oc.kc, oc.ks, oc.vc, oc.vs)):
+        assert (a == b[:, ctx:ctx + M]).all(), "appended rows differ"
+    # rows of a handful of keys: two fp16 spacings on values in [2, 4] (tolerances.py)
+    assert_attn_close(out, oc.attend_f32(q, ctx, None, threads=8, want_f32=True)[1], f"M={M} ctx={ctx}", two_spacings=ctx < 64)
+
+
+# 2,049 and 2,100 rows: a second slice of 1 and 52 rows.  Option 4 (inverse rotation) and forced split counts keep the combiner.
+# Both sides round V and P to fp16 and sum in fp32 in another order: 1e-3 between them, two bf16 roundings (2^-8 each) on top.
+@pytest.mark.parametrize("M,ctx,opts", [(2049, 0, []), (2100, 4000, []), (1500, 0, [(4, 1)]), (1500, 2000, [(4, 1)]), (700, 9000, [(2, 5)]),
+                                        (333, 0, [(11, 1)]), (1500, 7000, [(11, 1)]), (90, 12000, [(10, 128)])])
+def test_against_the_decode_kernel(native, M, ctx, opts):
+    rng = np.random.default_rng(M + ctx)
+    bf16 = (11, 1) in opts
+
+    def rows(n, heads):
+        x = rng.standard_normal((n, heads, 128)).astype(np.float32)
+        return (x.view(np.uint32) >> 16).astype(np.uint16).view(np.float16) if bf16 else x.astype(np.float16)
+
+    with native.KvCache(max_ctx=16384, max_rows=max(M, 2048)) as kv:
+        for key, val in opts:
+            kv.set_opt(key, val)
+        for p in range(0, ctx, 2048):
+            n = min(2048, ctx - p)
+            kv.append_host(0, rows(n, 4), rows(n, 4), p)
+        q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
+        kv.poison_workspace()
+        out = kv.layer_call(0, q, k, v, ctx)
+        kv.set_opt(3, 1)
+        ref = kv.layer_call(0, q, k, v, ctx)
+    wide = (lambda x: (x.view(np.uint16).astype(np.uint32) << 16).view(np.float32)) if bf16 else (lambda x: x.astype(np.float32))
+    out, ref = wide(out), wide(ref)
+    assert np.isfinite(out).all()
+    assert np.linalg.norm(out - ref) <= (1e-3 + (2 * 2.0 ** -8 if bf16 else 0)) * np.linalg.norm(ref)
+    per_row = np.linalg.norm(out - ref, axis=2) / np.linalg.norm(ref, axis=2)
+    assert per_row.max() <= (4e-3 if not bf16 else 1.2e-2)

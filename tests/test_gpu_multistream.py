@@ -166,3 +166,37 @@ def test_rows_of_one_stream_and_bad_rows_256(native, oracle):
         for t, s in enumerate(slots):
             if LENS[s] + (3 if s == 0 else 1 if s == 2 else 0) > pos[t]:
                 assert_attn_close(out[t:t + 1], refs[s].attend_f32(q[t:t + 1], int(pos[t])), f"attend-only row {t}")
+
+
+# The workgroups of a pass are shared out by the streams' lengths: one long stream beside many short ones, every number of
+# rows a slice can have (1, 2, a full slice of 64, a second slice), rows that name nothing between them.  The reference is
+# one-row passes over the same containers.
+@pytest.mark.parametrize("M", [1, 2, 3, 33, 64, 65])
+@pytest.mark.parametrize("dim", [128, 256])
+def test_streams_of_very_different_lengths(native, dim, M):
+    rng = np.random.default_rng(M + dim)
+    ctx = 9216
+    lens = [9000] + [int(x) for x in rng.integers(1, 200, M - 1)] if M % 2 else [int(x) for x in rng.integers(1, 700, M)]
+
+    def rows(n, heads):
+        return rng.standard_normal((n, heads, dim)).astype(np.float16)
+
+    with native.KvCache(n_layers=M, head_dim=dim, max_ctx=ctx, max_rows=max(M, 1024)) as kv:
+        for s, n in enumerate(lens):
+            for p in range(0, n, 1024):
+                kv.append_host(s, rows(min(1024, n - p), 4), rows(min(1024, n - p), 4), p)
+        slots = rng.permutation(M).astype(np.int32)
+        pos = np.array([lens[s] for s in slots], np.int32)
+        bad = [t for t in range(M) if M > 3 and t % 11 == 5]
+        pos[bad] = ctx
+        q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
+        kv.poison_workspace()
+        out = kv.ms_call(q, k, v, pos, slots)
+        for t in range(M):
+            if t in bad:
+                assert not (out[t].view(np.uint16) & 0x7fff).any()
+                continue
+            ref = kv.layer_call(int(slots[t]), q[t:t + 1], k[t:t + 1], v[t:t + 1], int(pos[t])).astype(np.float32)[0]
+            # the same kernel arithmetic with another split count: fp16 partials and outputs, 2^-11 each, summed in fp32
+            assert np.linalg.norm(out[t].astype(np.float32) - ref) <= 1e-3 * np.linalg.norm(ref), f"row {t}: stream of {pos[t]} tokens"
+        assert [kv.export_rows(int(slots[t]), int(pos[t]), 1)[0].any() for t in range(M) if t not in bad].count(False) == 0

@@ -105,6 +105,8 @@ void on_device(const yka_kv* kv) {
 
 constexpr int kMaxSplits = 256;
 constexpr size_t kWsPairs = 4096;  // (token, split) pairs the partial workspace holds: 4096 * 24 * (256 + 8) bytes = 26 MB
+constexpr size_t kChunkPairs = 12288;   // where a handle takes prefill chunks (max_rows > 64): 2,048 rows x 6 splits, 78 MB
+size_t ws_pairs_of(const yka_kv* kv) { return kv->cfg.max_rows > kMaxSlice ? kChunkPairs : kWsPairs; }
 
 // splits for the narrow kernel: one workgroup per CU (256 of them) while a workgroup then walks at most 48 tiles - its
 // waves keep the next tile in flight, and half as many partial rows make the combiner cheaper (measured: 12.2 against
@@ -145,16 +147,24 @@ int mid_splits(const yka_kv* kv, int M, size_t ws_pairs = kWsPairs) {
   return std::min(S, std::max(1, (int)(ws_pairs / (size_t)M)));
 }
 
-// Prefill chunks: slices of up to 1024 tokens (48 row blocks of 128 rows per kv head), splits = the fewest that put three
-// workgroups on every CU (all of them walk nearly the same number of tiles, so the grid drains evenly), each at least
-// eight tiles long and within the partial workspace.
-constexpr int kChunkSlice = 1024;
-int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs = kWsPairs) {
+// Prefill chunks: slices of up to 2048 tokens, 128 rows per workgroup.  How many splits a slice uses is decided on the
+// device (chunk_splits_used: a chunk early in its context needs none); the grid provides the number between 1 and
+// kChunkMaxSplits that fills the rounds of 256 workgroups best on a long context - each split at least eight tiles of the
+// expected context, at most 2,048 workgroups and the partial workspace.
+constexpr int kChunkSlice = 2048;
+int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
   if (kv->opt_splits_wide > 0) return std::max(1, std::min(kv->opt_splits_wide, (int)(ws_pairs / (size_t)Ms)));
   const int rb = (kG * Ms + 127) / 128, base = kv->cfg.n_kv_heads * rb;
   const int ctx = kv->opt_ctx_hint > 0 ? std::min(kv->opt_ctx_hint, kv->cfg.max_ctx) : kv->cfg.max_ctx;
-  int S = std::min((768 + base - 1) / base, ((ctx + 31) / 32) / 8);
-  return std::max(1, std::min(std::min(kMaxSplits, S), (int)(ws_pairs / (size_t)Ms)));
+  const int top = std::min({kChunkMaxSplits, (int)(ws_pairs / (size_t)Ms), ((ctx + 31) / 32) / 8, 2048 / base});
+  int best = 1;
+  double best_fill = 0;
+  for (int s = 1; s <= top; ++s) {
+    const int n = base * s, rounds = (n + 255) / 256;
+    const double fill = n / (256.0 * rounds) - 0.005 * s;
+    if (fill > best_fill) { best_fill = fill; best = s; }
+  }
+  return best;
 }
 
 void check_layer(const yka_kv* kv, int layer) {
@@ -268,9 +278,9 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
   // kernel for every 64-row slice (each slice stores its own rows); only a wide pass forced through the narrow kernel
   // launches the append kernel first
   // A pass of more than 64 rows is a prefill chunk (the reference cuts it into 64-row slices, engine35.cpp:935-947, one
-  // attention launch each).  Here its rows are appended by one launch, then slices of up to 1024 tokens go through the
-  // wide kernel - 128 rows per workgroup whatever the slice, the key range cut evenly into as many splits as give every
-  // CU three workgroups - and one combiner launch per slice merges them.
+  // attention launch each).  Here its rows are appended by one launch, then slices of up to 2048 tokens go through the
+  // wide kernel - 128 rows per workgroup whatever the slice, the key range cut evenly into as many splits as the length
+  // found on the device justifies - and one combiner launch per slice merges them.
   const bool chunk = M > kMaxSlice && !kv->opt_force_narrow && !ws;
   const bool fuse_append = k16 && !chunk && (M <= 2 || !kv->opt_force_narrow);
   if (k16 && !fuse_append) do_append(kv, layer, k16, v16, M, d_pos, st);
@@ -279,10 +289,15 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     const int Ms = std::min(slice, M - s0);
     const bool narrow = !chunk && (Ms <= 2 || kv->opt_force_narrow);
     const bool mid = !chunk && !narrow && Ms <= kv->opt_mid_rows;
-    const int S = narrow ? narrow_splits(kv, Ms, W.pairs) : mid ? mid_splits(kv, Ms, W.pairs) : (chunk ? chunk_splits(kv, Ms, W.pairs) : wide_splits(kv, Ms, W.pairs));
+    const int S = narrow ? narrow_splits(kv, Ms, W.pairs) : mid ? mid_splits(kv, Ms, W.pairs) : (chunk ? chunk_splits(kv, Ms, kv->ws_rows) : wide_splits(kv, Ms, W.pairs));
     AttnArgs A{kv->view(layer), q16 + (size_t)s0 * NH * kD, d_pos, depth, Ms, s0, NH, S, wide_rows_per_block(Ms), W.pm, W.pl, W.pacc16,
                fuse_append ? k16 : nullptr, fuse_append ? v16 : nullptr};
     A.in_bf16 = bf16;
+    CombineArgs C{W.pm, W.pl, W.pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * kD, kv->opt_unrot, bf16};
+    if (chunk && !kv->opt_splits_wide) {
+      A.adapt = C.adapt = 1; C.d_pos = d_pos; C.tok0 = s0; C.n_kv = kv->cfg.n_kv_heads; C.max_ctx = kv->cfg.max_ctx;
+      if (!kv->opt_unrot && mode != 2) { A.out16 = C.out16; C.direct = 1; }
+    }
     // option key 7, rows of at most 2 tokens: the last workgroup of each column merges the splits inside the attention launch
     const bool one_launch = narrow && mode == 0 && !kv->opt_unrot && kv->opt_merge_in_launch;
     if (one_launch) {
@@ -291,16 +306,17 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
       launch_zero_ints(W.tickets, kv->cfg.n_kv_heads * kMaxSlice, st);
       A.tickets = W.tickets; A.out16 = out16 + (size_t)s0 * NH * kD; A.out_bf16 = bf16;
     }
-    if (narrow) launch_attend_narrow(A, st); else if (mid) launch_attend_mid(A, st); else launch_attend_wide(A, st);
-    if (mode != 2 && !one_launch) launch_combine(CombineArgs{W.pm, W.pl, W.pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * kD, kv->opt_unrot, bf16}, st);
+    if (narrow) launch_attend_narrow(A, st); else if (mid) launch_attend_mid(A, st); else if (chunk) launch_attend_chunk(A, st); else launch_attend_wide(A, st);
+    if (mode != 2 && !one_launch && !(C.direct && S == 1)) launch_combine(C, st);
   }
 }
 
-// Multi-stream pass: rows are appended first (several rows of one stream may follow each other and read each other's
-// keys), then every row attends to keys [0, pos[t]] of its own container.  One token per workgroup column.
+// Multi-stream pass: rows are appended (several rows of one stream may follow each other and read each other's keys) by the
+// attention launch or, beyond 64 rows and with a split count set by the caller, by a launch in front of it; every row attends to keys [0, pos[t]] of its own container.  One token per workgroup column.
 void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const uint16_t* v16, int M, const int* row_pos,
                   const int* row_slot, uint16_t* out16, hipStream_t st) {
   const int NH = kv->cfg.n_heads, D = kv->D();
+  const int share = !kv->opt_splits_narrow;        // the splits follow the streams' lengths (ms_share) unless the caller set their number
   const bool r256 = kv->r256();
   const int bf16 = kv->opt_io_bf16;
   if (kv->tb) {
@@ -317,24 +333,33 @@ void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const ui
       RowMap Rs = R; Rs.pos += s0; Rs.slot += s0;
       const TbAttnArgs A{T.kpay(0), T.vpay(0), T.kscl(0), T.vscl(0), kv->cfg.max_ctx, kv->cfg.n_kv_heads, T.stride,
                          T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, pl, q16 + (size_t)s0 * NH * 256, nullptr, nullptr, Ms, s0, NH, S,
-                         kv->pm, kv->pl, kv->pacc16, Rs, bf16};
+                         kv->pm, kv->pl, kv->pacc16, Rs, bf16, share};
       launch_attend_tb(A, T.kb, st);
-      launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
+      CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
+      C.max_ctx = kv->cfg.max_ctx;
+      if (share) C.rows = Rs;
+      launch_combine256(C, st);
     }
     return;
   }
   const RowMap R{row_pos, row_slot, kv->cfg.n_layers, kv->layer_bytes, kv->n_pages};
-  if (k16) { AppendArgs P{kv->view(0), k16, v16, nullptr, M, R}; P.in_bf16 = bf16; if (r256) launch_append256(P, st); else launch_append(P, st); }
+  // passes of at most 64 rows store their rows inside the attention launch (ms_new_rows)
+  const bool one_launch = !r256 && !kv->opt_unrot && kv->opt_merge_in_launch;
+  const bool fuse = k16 && share && !one_launch && M <= kMaxSlice;
+  if (k16 && !fuse) { AppendArgs P{kv->view(0), k16, v16, nullptr, M, R}; P.in_bf16 = bf16; if (r256) launch_append256(P, st); else launch_append(P, st); }
   for (int s0 = 0; s0 < M; s0 += kMaxSlice) {
     const int Ms = std::min(kMaxSlice, M - s0);
-    int S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : (r256 ? 512 : 1024) / (kv->cfg.n_kv_heads * Ms);   // 2 / 4 waves per SIMD
+    int S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : 512 / (kv->cfg.n_kv_heads * Ms);   // two workgroups per CU: one round
     S = std::min(std::max(2, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
     RowMap Rs = R; Rs.pos += s0; Rs.slot += s0;
     AttnArgs A{kv->view(0), q16 + (size_t)s0 * NH * D, nullptr, nullptr, Ms, s0, NH, S, 128, kv->pm, kv->pl, kv->pacc16, nullptr, nullptr, Rs};
     A.in_bf16 = bf16;
-    const CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * D, kv->opt_unrot, bf16};
+    CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * D, kv->opt_unrot, bf16};
+    C.max_ctx = kv->cfg.max_ctx;
+    if (share && !one_launch) { A.adapt = 1; C.rows = Rs; }
+    if (fuse) { A.k16 = k16; A.v16 = v16; }
     if (r256) { launch_attend256(A, st); launch_combine256(C, st); }
-    else if (!kv->opt_unrot && kv->opt_merge_in_launch) {
+    else if (one_launch) {
       launch_zero_ints(kv->tickets, kv->cfg.n_kv_heads * kMaxSlice, st);
       A.tickets = kv->tickets; A.out16 = C.out16; A.out_bf16 = bf16; launch_attend_narrow(A, st);
     }
@@ -397,7 +422,7 @@ yka_kv* yka_kv_open(const yka_kv_config* cfg) {
       HIPCHK(hipMalloc((void**)&kv->tables, ident.size() * 4));
       HIPCHK(hipMemcpy(kv->tables, ident.data(), ident.size() * 4, hipMemcpyHostToDevice));
     }
-    kv->ws_rows = kWsPairs;
+    kv->ws_rows = ws_pairs_of(kv);
     const size_t np = kv->ws_rows * cfg->n_heads;
     HIPCHK(hipMalloc((void**)&kv->pm, np * 4));
     HIPCHK(hipMalloc((void**)&kv->pl, np * 4));
@@ -517,7 +542,7 @@ int yka_kv_poison_workspace(yka_kv* kv) {
   YKA_TRY
   on_device(kv);
   HIPCHK(hipDeviceSynchronize());
-  const size_t rows = kWsPairs * (size_t)kv->cfg.n_heads;
+  const size_t rows = kv->ws_rows * (size_t)kv->cfg.n_heads;
   HIPCHK(hipMemset(kv->pm, 0xff, rows * 4));
   HIPCHK(hipMemset(kv->pl, 0xff, rows * 4));
   HIPCHK(hipMemset(kv->pacc16, 0xff, rows * (size_t)kv->D() * 2));

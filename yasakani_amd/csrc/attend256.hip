@@ -212,13 +212,20 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   __shared__ float s_m[4][16], s_l[4][16];
   __shared__ __align__(16) float s_wn[16][4];
   __shared__ float s_acc[4][16][kD2 + 4];
-  const int split = blockIdx.x, kvh = blockIdx.y, rt = blockIdx.z;
+  int split = blockIdx.x, rt = blockIdx.z;
+  const int kvh = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  int pos; bool row_ok = true;
+  int pos, slot = 0; bool row_ok = true;
+  MsShare share{};
   if (MS) {
+    if (A.adapt) {
+      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, split + A.S * rt);
+      if (share.row < 0) return;
+      split = share.split; rt = share.row;
+    }
     pos = A.rows.pos[rt];
-    const int slot = A.rows.slot[rt];
+    slot = A.rows.slot[rt];
     row_ok = pos >= 0 && pos < A.kv.max_ctx && slot >= 0 && slot < A.rows.n_slots;   // a bad row reads nothing and yields zeros
     A.kv = slot_view(A.kv, A.rows, row_ok ? slot : 0);
   } else {
@@ -240,11 +247,13 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   // as many of the launched splits as the length found on the device justifies (two 32-key tiles per workgroup at
   // least); the others leave the "no keys" marker, whose rows the combiner does not read
   const int ntiles = (maxlen + 31) >> 5;
-  const int s_used = min(A.S, max(1, ntiles >> 1));
+  const int s_used = MS && A.adapt ? share.n : min(A.S, max(1, ntiles >> 1));
+  // partials of (token tj, split) start at pair * n_heads
+  auto pair_of = [&](int tj) __attribute__((always_inline)) { return MS && A.adapt ? share.base + split : (size_t)tj * A.S + split; };
   if (split >= s_used) {
     const int j = threadIdx.x, tj = TPT * rt + j / kG;
     if (j < TPT * kG && tj < A.M) {
-      const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
       A.pm[p] = -1e30f; A.pl[p] = 0.f;
     }
     return;
@@ -255,6 +264,23 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   // ---- fused quantize-on-append (rows of at most 2 tokens, one row tile): a row of this pass is written by the one
   //      workgroup whose tile range holds it - the only workgroup of this kv head that reads it in this launch; writer
   //      and readers are waves of one CU and one write-through L1, so workgroup-scope fences order the stores ----
+  if (MS && A.k16 && row_ok) {
+    __shared__ float a_red[4];
+    __shared__ uint8_t a_fld[256];
+    int lane_pos;
+    uint64_t todo = ms_new_rows(A.rows, A.M, slot, pos, tile0, tile1, lane_pos);
+    if (todo) {                        // uniform over the workgroup
+      for (; todo; todo &= todo - 1) {
+        const int t = __builtin_ctzll(todo), r = __builtin_amdgcn_readlane(lane_pos, t);
+        const size_t e = ((size_t)t * A.kv.n_kv + kvh) * kD2 + threadIdx.x;
+        quant_store_row256(A.kv, kvh, r, false, row16_value(A.k16[e], A.in_bf16), threadIdx.x, a_red, a_fld);
+        quant_store_row256(A.kv, kvh, r, true, row16_value(A.v16[e], A.in_bf16), threadIdx.x, a_red, a_fld);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __syncthreads();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+  }
   if (!MS && A.k16) {
     __shared__ float a_red[4];
     __shared__ uint8_t a_fld[256];
@@ -394,7 +420,7 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
     s_wn[j][w] = L > 0.f ? ww / L : 0.f;
     const int tj = TPT * rt + j / kG;
     if (w == 0 && j < TPT * kG && tj < A.M) {
-      const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
       A.pm[p] = M2; A.pl[p] = L;
     }
   }
@@ -404,7 +430,7 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
     const int tj = TPT * rt + j / kG;
     if (tj >= A.M) continue;
     const f4 w4 = *reinterpret_cast<const f4*>(s_wn[j]);
-    const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+    const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
     const float y = w4[0] * s_acc[0][j][d] + w4[1] * s_acc[1][j][d] + w4[2] * s_acc[2][j][d] + w4[3] * s_acc[3][j][d];
     A.pacc16[p * kD2 + d] = __half_as_ushort(__float2half_rn(y));
   }
@@ -420,7 +446,13 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
   __shared__ float s_o[8][kD2 + 4];
   __shared__ float s_wsum[8];
   const int head = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x;
-  const size_t p0 = (size_t)tok * A.S * A.n_heads + head;
+  size_t pair0 = (size_t)tok * A.S;
+  if (A.rows.pos) {
+    const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
+    A.S = __builtin_amdgcn_readlane(P.mine, tok);
+    pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
+  }
+  const size_t p0 = pair0 * A.n_heads + head;
   // 8 split lanes; each takes splits sl, sl + 8, ... (at most kInFlight of them: the launcher picks kInFlight so that
   // 8 * kInFlight >= S).  Their partial rows are requested first, together with the (m, l) pairs the weights come from:
   // one memory round trip instead of two.  A row of weight 0 may be one that no workgroup wrote: it is zeroed before use.
@@ -428,11 +460,14 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
   const uint16_t* src = A.pacc16 + p0 * kD2 + c8;
   const size_t stride = (size_t)A.n_heads * kD2;
   uint4 u[kInFlight];
+  auto request = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < kInFlight; ++k) {
-    const int sp = sl + 8 * k;
-    u[k] = sp < A.S ? *reinterpret_cast<const uint4*>(src + (size_t)sp * stride) : make_uint4(0, 0, 0, 0);
-  }
+    for (int k = 0; k < kInFlight; ++k) {
+      const int sp = s0 + sl + 8 * k;
+      u[k] = sp < A.S ? *reinterpret_cast<const uint4*>(src + (size_t)sp * stride) : make_uint4(0, 0, 0, 0);
+    }
+  };
+  request(0);
   float pmv = -1e30f, plv = 0.f;
   if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
   float M2 = pmv;
@@ -446,15 +481,20 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
   __syncthreads();
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float wsum = 0.f;
+  for (int s0 = 0;;) {                             // one batch, except for a stream with more than 8 * kInFlight splits
 #pragma unroll
-  for (int k = 0; k < kInFlight; ++k) {
-    const int sp = sl + 8 * k;
-    const float w = sp < A.S ? s_w[sp] : 0.f;
-    const uint4 r = w != 0.f ? u[k] : make_uint4(0, 0, 0, 0);
-    const h8 v = __builtin_bit_cast(h8, r);
+    for (int k = 0; k < kInFlight; ++k) {
+      const int sp = s0 + sl + 8 * k;
+      const float w = sp < A.S ? s_w[sp] : 0.f;
+      const uint4 r = w != 0.f ? u[k] : make_uint4(0, 0, 0, 0);
+      const h8 v = __builtin_bit_cast(h8, r);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
-    wsum += w;
+      for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
+      wsum += w;
+    }
+    s0 += 8 * kInFlight;
+    if (s0 >= A.S) break;
+    request(s0);
   }
 #pragma unroll
   for (int c = 0; c < 8; ++c) s_o[sl][c8 + c] = acc[c];
@@ -482,6 +522,11 @@ void launch_attend256(const AttnArgs& A, hipStream_t st) {
   else hipLaunchKernelGGL(attend256_kernel<false>, dim3(A.S, A.kv.n_kv, (A.M + 1) / 2), dim3(256), 0, st, A);
 }
 void launch_combine256(const CombineArgs& A, hipStream_t st) {
+  if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most): half of them with 2 streams
+    if (A.M < 8) hipLaunchKernelGGL(combine256_kernel<16>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    else hipLaunchKernelGGL(combine256_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    return;
+  }
   // 8 split lanes x kInFlight rows each must cover the S <= 256 splits
   if (A.S > 128) hipLaunchKernelGGL(combine256_kernel<32>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
   else if (A.S > 32) hipLaunchKernelGGL(combine256_kernel<16>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);

@@ -189,13 +189,20 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
   __shared__ int s_ticket;
   constexpr int TPT = MS ? 1 : 2;
   const bool fused = A.tickets != nullptr;                 // uniform over the grid
-  const int split = blockIdx.x, kvh = blockIdx.y, rt = blockIdx.z;
+  int split = blockIdx.x, rt = blockIdx.z;
+  const int kvh = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // a scalar: tile indices and page pointers are wave uniform
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  int pos; bool row_ok = true;
+  int pos, slot = 0; bool row_ok = true;
+  MsShare share{};
   if (MS) {
+    if (A.adapt) {
+      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, split + A.S * rt);
+      if (share.row < 0) return;
+      split = share.split; rt = share.row;
+    }
     pos = A.rows.pos[rt];
-    const int slot = A.rows.slot[rt];
+    slot = A.rows.slot[rt];
     row_ok = pos >= 0 && pos < A.kv.max_ctx && slot >= 0 && slot < A.rows.n_slots;   // a bad row reads nothing and yields zeros
     A.kv = slot_view(A.kv, A.rows, row_ok ? slot : 0);
   } else {
@@ -220,11 +227,13 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
   // device: at least two 32-key tiles per workgroup.  The other workgroups leave the "no keys" marker and exit, and
   // the combiner does not read their rows.
   const int ntiles = (maxlen + 31) >> 5;
-  const int s_used = min(A.S, max(1, ntiles >> 1));
+  const int s_used = MS && A.adapt ? share.n : min(A.S, max(1, ntiles >> 1));
+  // partials of (token tj, split) start at pair * n_heads
+  auto pair_of = [&](int tj) __attribute__((always_inline)) { return MS && A.adapt ? share.base + split : (size_t)tj * A.S + split; };
   if (split >= s_used) {
     const int j = threadIdx.x, tj = TPT * rt + j / kG;
     if (j < TPT * kG && tj < A.M) {
-      const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
       if (fused) { st_agent(A.pm + p, -1e30f); st_agent(A.pl + p, 0.f); }
       else { A.pm[p] = -1e30f; A.pl[p] = 0.f; }
     }
@@ -240,6 +249,20 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
   //      whose tile range holds it - the only workgroup of this kv head that will read it in this launch.  Writer and
   //      readers are waves of one workgroup, i.e. of one CU and one (write-through) L1, so workgroup-scope fences
   //      around the barrier order the stores before the loads without any cache maintenance. ----
+  if (MS && A.k16 && row_ok) {
+    int lane_pos;
+    uint64_t todo = ms_new_rows(A.rows, A.M, slot, pos, tile0, tile1, lane_pos);
+    if (todo) {                        // uniform over the workgroup
+      for (; todo; todo &= todo - 1) {
+        const int t = __builtin_ctzll(todo);
+        const bool isv = threadIdx.x >= 128;
+        quant_store_row(A.kv, kvh, __builtin_amdgcn_readlane(lane_pos, t), isv, (isv ? A.v16 : A.k16) + ((size_t)t * A.kv.n_kv + kvh) * kD, threadIdx.x & 127, A.in_bf16);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __syncthreads();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+  }
   if (!MS && A.k16) {
     bool mine = false;
     for (int t = 0; t < A.M; ++t) {
@@ -448,7 +471,7 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
       const float m0 = s_m[0][j], m1 = s_m[1][j], m2 = s_m[2][j], m3 = s_m[3][j];
       const float M2 = fmaxf(fmaxf(m0, m1), fmaxf(m2, m3));
       const float w[4] = {exp2f(m0 - M2), exp2f(m1 - M2), exp2f(m2 - M2), exp2f(m3 - M2)};
-      const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
       const float L = w[0] * s_l[0][j] + w[1] * s_l[1][j] + w[2] * s_l[2][j] + w[3] * s_l[3][j];
       float4 a0[4], a1[4];                                    // all eight reads first: one LDS round trip, not eight
 #pragma unroll
@@ -495,7 +518,17 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   __shared__ float s_o[16][kD + 4];
   __shared__ float s_wsum[16];
   const int head = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x;
-  const size_t p0 = (size_t)tok * A.S * A.n_heads + head;      // split s lives at p0 + s * n_heads
+  if (A.adapt) {
+    A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S);
+    if (A.S == 1 && A.direct) return;
+  }
+  size_t pair0 = (size_t)tok * A.S;
+  if (A.rows.pos) {
+    const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
+    A.S = __builtin_amdgcn_readlane(P.mine, tok);
+    pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
+  }
+  const size_t p0 = pair0 * A.n_heads + head;                  // split s lives at p0 + s * n_heads
   // 16 split lanes; each takes splits sl, sl+16, ... (at most kInFlight of them: the launcher picks kInFlight so that
   // 16 * kInFlight >= S).  Their partial rows are requested first, together with the (m, l) pairs the weights come
   // from: one memory round trip instead of two.  A row of weight 0 may be one that no workgroup wrote: it is zeroed
@@ -504,11 +537,14 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   const uint16_t* src = A.pacc16 + p0 * kD + c8;
   const size_t stride = (size_t)A.n_heads * kD;
   uint4 u[kInFlight];
+  auto request = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < kInFlight; ++k) {
-    const int sp = sl + 16 * k;
-    u[k] = sp < A.S ? *reinterpret_cast<const uint4*>(src + (size_t)sp * stride) : make_uint4(0, 0, 0, 0);
-  }
+    for (int k = 0; k < kInFlight; ++k) {
+      const int sp = s0 + sl + 16 * k;
+      u[k] = sp < A.S ? *reinterpret_cast<const uint4*>(src + (size_t)sp * stride) : make_uint4(0, 0, 0, 0);
+    }
+  };
+  request(0);
   // weights: every thread looks at one split
   float pmv = -1e30f, plv = 0.f;
   if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
@@ -522,15 +558,20 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   __syncthreads();
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float wsum = 0.f;
+  for (int s0 = 0;;) {                             // one batch, except for a stream with more than 16 * kInFlight splits
 #pragma unroll
-  for (int k = 0; k < kInFlight; ++k) {
-    const int sp = sl + 16 * k;
-    const float w = sp < A.S ? s_w[sp] : 0.f;
-    const uint4 r = w != 0.f ? u[k] : make_uint4(0, 0, 0, 0);
-    const h8 v = __builtin_bit_cast(h8, r);
+    for (int k = 0; k < kInFlight; ++k) {
+      const int sp = s0 + sl + 16 * k;
+      const float w = sp < A.S ? s_w[sp] : 0.f;
+      const uint4 r = w != 0.f ? u[k] : make_uint4(0, 0, 0, 0);
+      const h8 v = __builtin_bit_cast(h8, r);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
-    wsum += w;
+      for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
+      wsum += w;
+    }
+    s0 += 16 * kInFlight;
+    if (s0 >= A.S) break;
+    request(s0);
   }
 #pragma unroll
   for (int c = 0; c < 8; ++c) s_o[sl][c8 + c] = acc[c];
@@ -565,9 +606,15 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
 // waves per workgroup, no LDS and no barrier.  Lane = (split lane 0..3, 8 channels); a split lane takes splits sl, sl + 4,
 // ... (at most 8), requests their rows together with the (m, l) pairs, and the four split lanes are summed by two
 // cross-lane exchanges.  Same arithmetic as combine_kernel up to the order of the sums.
+// ADAPT: rows of a prefill slice; as many workgroups as the chip holds at once (8 per CU), each walks its share - most slices on
+// short contexts find nothing to do here and should not pay for dispatching thousands of workgroups to find out.
+template <bool ADAPT>
 __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);               // row = tok * n_heads + head
-  if (row >= A.M * A.n_heads) return;
+  if constexpr (ADAPT) {
+    A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S);
+    if (A.S == 1 && A.direct) return;
+  }
+  for (int row = blockIdx.x * 4 + (threadIdx.x >> 6); row < A.M * A.n_heads; row += ADAPT ? 4 * (int)gridDim.x : A.M * A.n_heads) {   // row = tok * n_heads + head
   const int tok = row / A.n_heads, head = row % A.n_heads, lane = threadIdx.x & 63, sl = lane >> 4, c8 = (lane & 15) * 8;
   const size_t p0 = (size_t)tok * A.S * A.n_heads + head;
   const size_t stride = (size_t)A.n_heads * kD;
@@ -605,10 +652,19 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) yv[c] = acc[c] * inv;
     *reinterpret_cast<uint4*>(A.out16 + (size_t)row * kD + c8) = pack_out8(yv, A.out_bf16);
-  }
+  }  }
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
-  if (A.S <= 32 && !A.unrot && A.M >= 8) { hipLaunchKernelGGL(combine_rows_kernel, dim3((A.M * A.n_heads + 3) / 4), dim3(256), 0, st, A); return; }
+  if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most)
+    hipLaunchKernelGGL(combine_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    return;
+  }
+  if (A.S <= 32 && !A.unrot && A.M >= 8) {
+    const int wgs = (A.M * A.n_heads + 3) / 4;
+    if (A.adapt) hipLaunchKernelGGL(combine_rows_kernel<true>, dim3(min(wgs, 2048)), dim3(256), 0, st, A);
+    else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, A);
+    return;
+  }
   if (A.S > 128) hipLaunchKernelGGL(combine_kernel<16>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);   // S <= 256
   else if (A.S > 64) hipLaunchKernelGGL(combine_kernel<8>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
   else hipLaunchKernelGGL(combine_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);

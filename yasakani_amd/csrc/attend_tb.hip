@@ -64,12 +64,19 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
   float (*s_acc)[16][kD2 + 4] = reinterpret_cast<float (*)[16][kD2 + 4]>(s_buf);
   const uint8_t* const s_tabK = s_buf;
   const uint8_t* const s_tabV = s_buf + kTabBytes;
-  const int split = blockIdx.x, kvh = blockIdx.y, rt = blockIdx.z;
+  int split = blockIdx.x, rt = blockIdx.z;
+  const int kvh = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int gK = (A.layer * A.n_kv + kvh) * 2, gV = gK + 1;
   int pos; bool row_ok = true;
+  MsShare share{};
   if (MS) {
+    if (A.adapt) {
+      share = ms_share(A.rows, A.M, A.max_ctx, A.S * A.M, split + A.S * rt);
+      if (share.row < 0) return;
+      split = share.split; rt = share.row;
+    }
     pos = A.rows.pos[rt];
     const int slot = A.rows.slot[rt];
     row_ok = pos >= 0 && pos < A.max_ctx && slot >= 0 && slot < A.rows.n_slots;   // a bad row reads nothing and yields zeros
@@ -94,11 +101,13 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
   for (int o = 1; o < 16; o <<= 1) { maxlen = max(maxlen, __shfl_xor(maxlen, o, 64)); minlen = min(minlen, __shfl_xor(minlen, o, 64)); }
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
   const int ntiles = (maxlen + 31) >> 5;
-  const int s_used = min(A.S, max(1, ntiles >> 1));
+  const int s_used = MS && A.adapt ? share.n : min(A.S, max(1, ntiles >> 1));
+  // partials of (token tj, split) start at pair * n_heads
+  auto pair_of = [&](int tj) __attribute__((always_inline)) { return MS && A.adapt ? share.base + split : (size_t)tj * A.S + split; };
   if (split >= s_used) {                             // the "no keys" marker; the combiner does not read such rows
     const int j = threadIdx.x, tj = TPT * rt + j / kG;
     if (j < TPT * kG && tj < A.M) {
-      const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
       A.pm[p] = -1e30f; A.pl[p] = 0.f;
     }
     return;
@@ -309,7 +318,7 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
     s_wn[j][w] = L > 0.f ? ww * A.gfac[gV] / L : 0.f;
     const int tj = TPT * rt + j / kG;
     if (w == 0 && j < TPT * kG && tj < A.M) {
-      const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
       A.pm[p] = M2; A.pl[p] = L;
     }
   }
@@ -319,7 +328,7 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
     const int tj = TPT * rt + j / kG;
     if (tj >= A.M) continue;
     const f4 w4 = *reinterpret_cast<const f4*>(s_wn[j]);
-    const size_t p = ((size_t)tj * A.S + split) * A.n_heads + kvh * kG + j % kG;
+    const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
     float y = w4[0] * s_acc[0][j][d] + w4[1] * s_acc[1][j][d] + w4[2] * s_acc[2][j][d] + w4[3] * s_acc[3][j][d];
     if (A.mu && w4[0] + w4[1] + w4[2] + w4[3] > 0.f) y += A.mu[(size_t)gV * 256 + d];
     A.pacc16[p * kD2 + d] = __half_as_ushort(__float2half_rn(y));

@@ -1,5 +1,5 @@
 // Split-KV attention for windows of 3..64 query tokens (verify windows) and for prefill chunks cut into slices of up to
-// 1024 tokens (one launch per slice, every workgroup 128 rows of it).  gfx950.
+// 2048 tokens (one launch per slice, every workgroup 128 rows of it).  gfx950.
 //
 // Same mathematics as the narrow kernel (reference: src/q35_atxpk4.cuh:71-499 for the window shape, row geometry
 // src/q35_atxpk.cu:391-411): every row t of the window runs an online softmax over the keys [0, len(t)) of its
@@ -167,13 +167,24 @@ __device__ __forceinline__ void dequant_to_lds(uint8_t* buf, int tid, const Raw&
 // remaining pairs in order.
 // BF: Q / new K / new V are bf16 rows; a kernel of its own, because a branch around the conversion in this one costs the fp16
 // rows 1.5 % (755 against 767 us for 16 layers of 64 rows at 32,768 tokens)
-template <bool BF>
+// CHUNK: slice of a prefill chunk, whose rows an append launch has stored: no rows to quantize, the key range cut evenly
+// into the number of splits the length found on the device justifies (chunk_splits_used), the other workgroups exit.  A
+// slice that uses one split writes its output rows instead of partials.  While the keys of all kv heads fit one XCD's L2
+// the longest row blocks start first, spread over the XCDs (on a short context a block's length is its place in the slice).
+template <bool BF, bool CHUNK>
 __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   __shared__ __align__(16) uint8_t lds[2][2][kLdsBuf];               // [group][buffer]
   const int n_rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block;
+  const int pos = *A.d_pos;
+  if constexpr (CHUNK) { if (A.adapt) A.S = chunk_splits_used(pos, A.tok0, A.M, A.kv.n_kv, A.kv.max_ctx, A.S); }
+  const int total = CHUNK ? A.S * A.kv.n_kv * n_rb : (int)gridDim.x;
+  if (CHUNK && (int)blockIdx.x >= total) return;
   int pair, rb;
-  {
-    const int total = gridDim.x, x = blockIdx.x & 7, k = blockIdx.x >> 3, F = (total >> 3) / n_rb;
+  if (CHUNK && A.adapt && (min(pos + A.tok0 + A.M, A.kv.max_ctx) + 31) / 32 * 4608 * A.kv.n_kv <= (4 << 20)) {
+    const int pairs = A.S * A.kv.n_kv;
+    rb = n_rb - 1 - (int)blockIdx.x / pairs; pair = (int)blockIdx.x % pairs;
+  } else {
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, F = (total >> 3) / n_rb;
     if (k < F * n_rb) { pair = x + 8 * (k / n_rb); rb = k % n_rb; }
     else {
       const int base_e = (total >> 3) - F * n_rb;                     // leftover workgroups of an XCD, +1 on the first total mod 8
@@ -185,7 +196,6 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   const int tid = threadIdx.x, gt = tid & (NTG - 1);                  // gt: thread index inside the group
   const int grp = __builtin_amdgcn_readfirstlane(tid >> 8);           // wave uniform
   const int wave = __builtin_amdgcn_readfirstlane(gt >> 6), lane = tid & 63, j = lane & 31, h = lane >> 5;
-  const int pos = *A.d_pos;
   const int nrows = kG * A.M;
 
   // row of this lane: R = rb*rows_per_block + wave*32 + j  ->  token R/6 of the slice, head kvh*6 + R%6
@@ -233,21 +243,19 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   // does first (measured: about the time of 7 tiles for 64 rows): every workgroup of the launch then finishes at about
   // the same time (with the window tiles alone, 12 of the 252 workgroups of a 64-row pass were idle after two tiles and
   // the others walked 51 tiles instead of 49).
-  const int kWindowCost = A.k16 ? 1 + A.M / 10 : 0;
+  const int kWindowCost = !CHUNK && A.k16 ? 1 + A.M / 10 : 0;
   const int Tnew = min(ntiles, max(0, pos + A.tok0) >> 5);            // first tile that holds a row of this slice
   const int Tw = A.S > 1 ? min(Tnew, (A.S - 1) * ((ntiles + kWindowCost + A.S - 1) / A.S)) : Tnew;
-  // A pass wider than one slice (a prefill chunk: its rows were appended by a launch of their own) has no window split:
-  // its key range is cut evenly.
   int tile0, tile1;
   if (A.S == 1) { tile0 = 0; tile1 = ntiles; }
-  else if (A.M > kMaxSlice) { const int tps = (ntiles + A.S - 1) / A.S; tile0 = min(ntiles, split * tps); tile1 = min(ntiles, tile0 + tps); }
+  else if (CHUNK) { const int tps = (ntiles + A.S - 1) / A.S; tile0 = min(ntiles, split * tps); tile1 = min(ntiles, tile0 + tps); }
   else if (split == A.S - 1) { tile0 = Tw; tile1 = ntiles; }
   else { const int tps = (Tw + A.S - 2) / (A.S - 1); tile0 = split * tps; tile1 = min(Tw, tile0 + tps); }
   // ---- fused quantize-on-append: every workgroup of the window split stores the slice's rows up to its own last
   //      token (the row blocks of one kv head write identical bytes: each row is the same sequence of IEEE operations
   //      on the same inputs whoever computes it) and reads them back after a workgroup barrier: writer and readers
   //      are waves of one CU and one write-through L1.  Group 0 quantizes; the barrier is the workgroup's. ----
-  if (A.k16 && split == A.S - 1) {
+  if (!CHUNK && A.k16 && split == A.S - 1) {
     // 16 lanes per 128-channel row, 16 rows (K and V of 8 tokens) per step; all loads of the slice (at most 64 tokens)
     // are requested before the first row is quantized
     static_assert(kMaxSlice <= 64, "8 steps of 16 rows cover K and V of a slice");
@@ -470,7 +478,8 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   uint8_t* stage = &lds[0][0][0] + wave * (64 * 64 * 4);     // 4 waves x 8704 bytes, 16384 bytes apart
   float l = l_run;
   l += __shfl_xor(l, 32, 64);
-  if (vrow && h == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
+  const bool direct = CHUNK && A.S == 1 && A.out16;          // uniform over the grid
+  if (!direct && vrow && h == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int a0 = 0; a0 < 2; ++a0)
@@ -479,7 +488,14 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
       h8 v;
 #pragma unroll
       for (int c = 0; c < 8; ++c) v[c] = (_Float16)(o[c & 3][4 * (2 * (c >> 2) + a0) + b] * inv);
-      *reinterpret_cast<uint4*>(stage + j * kOPitch + (64 * a0 + 32 * h + 8 * b) * 2) = __builtin_bit_cast(uint4, v);
+      uint4 packed = __builtin_bit_cast(uint4, v);
+      if (CHUNK && BF && direct) {
+        float y[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) y[c] = o[c & 3][4 * (2 * (c >> 2) + a0) + b] * inv;
+        packed = pack_out8(y, 1);
+      }
+      *reinterpret_cast<uint4*>(stage + j * kOPitch + (64 * a0 + 32 * h + 8 * b) * 2) = packed;
     }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");     // the wave reads back what its own lanes wrote
   const int chunk = lane & 15;
@@ -488,18 +504,21 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
     const int jr = 4 * k + (lane >> 4);
     const int Rr = row0 + jr;
     if (Rr < nrows && Rr < (rb + 1) * RPB) {
-      const size_t p = ((size_t)(Rr / kG) * A.S + split) * A.n_heads + kvh * kG + Rr % kG;
+      const size_t p = ((size_t)(Rr / kG) * A.S + split) * A.n_heads + kvh * kG + Rr % kG;   // S == 1: also the output row
       const uint4 v = *reinterpret_cast<const uint4*>(stage + jr * kOPitch + chunk * 16);
-      *reinterpret_cast<uint4*>(A.pacc16 + p * kD + chunk * 8) = v;
+      *reinterpret_cast<uint4*>((direct ? A.out16 : A.pacc16) + p * kD + chunk * 8) = v;
     }
   }
 }
 
-void launch_attend_wide(const AttnArgs& A, hipStream_t st) {
+template <bool CHUNK>
+static void launch_wide(const AttnArgs& A, hipStream_t st) {
   const int rows = kG * A.M, rb = (rows + A.rows_per_block - 1) / A.rows_per_block;
   const dim3 grid(A.S * A.kv.n_kv * rb);
-  if (A.in_bf16) hipLaunchKernelGGL(attend_wide_kernel<true>, grid, dim3(NT), 0, st, A);
-  else hipLaunchKernelGGL(attend_wide_kernel<false>, grid, dim3(NT), 0, st, A);
+  if (A.in_bf16) hipLaunchKernelGGL((attend_wide_kernel<true, CHUNK>), grid, dim3(NT), 0, st, A);
+  else hipLaunchKernelGGL((attend_wide_kernel<false, CHUNK>), grid, dim3(NT), 0, st, A);
 }
+void launch_attend_wide(const AttnArgs& A, hipStream_t st) { launch_wide<false>(A, st); }
+void launch_attend_chunk(const AttnArgs& A, hipStream_t st) { launch_wide<true>(A, st); }
 
 }  // namespace yka

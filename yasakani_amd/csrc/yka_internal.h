@@ -66,17 +66,25 @@ struct AttnArgs {
   // before reading them.  Narrow kernel (M <= 2): rows [0, M) of the pass; wide kernel: k16/v16 point at row 0 of the
   // pass and the slice stores its own rows tok0 .. tok0 + M - 1.
   const uint16_t* k16; const uint16_t* v16;
-  RowMap rows;  // narrow kernel only: multi-stream pass, one token per workgroup column, no depth table, no fused append
+  RowMap rows;  // narrow kernel only: multi-stream pass, one token per workgroup column, no depth table; k16 / v16 with at most 64 rows
   // narrow kernel only: tickets != nullptr folds the split combine into the launch - every workgroup of a (kv head, row
   // tile) column takes a ticket from tickets[kv head * gridDim.z + row tile] once its partials are out, and the one that
   // draws the last ticket merges the column's partials into out16 and puts the counter back to zero
   int* tickets = nullptr; uint16_t* out16 = nullptr; int out_bf16 = 0;
   int in_bf16 = 0;   // q16 / k16 / v16 are bf16 rows (rows16_to_f16)
+  // wide kernel, slice of a prefill chunk (launch_attend_chunk): adapt != 0 lets the device choose how many of the S launched
+  // splits the slice uses (chunk_splits_used); out16 != nullptr: a slice that uses one writes its output rows itself
+  // multi-stream pass: adapt != 0 shares the S * M workgroups of a kv head out by the streams' lengths (ms_share)
+  int adapt = 0;
 };
 // unrot != 0: the output row gets the inverse signed Hadamard rotation (7 butterfly stages, x 1/16, signs) before it is
 // rounded to fp16 - the counterpart of rotating V rows on their way into the cache (src/q35_kernels.cu:1421)
 struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; int S; int M; int n_heads; uint16_t* out16; int unrot;
-                     int out_bf16 = 0; };   // outputs leave as bf16 (rounded once from the fp32 result) instead of fp16
+                     int out_bf16 = 0;      // outputs leave as bf16 (rounded once from the fp32 result) instead of fp16
+  // adapt != 0: partials of launch_attend_chunk - the splits in use follow from *d_pos as they did there, and with direct != 0 a
+  // slice that used one split has written its output already
+  int adapt = 0; int direct = 0; const int* d_pos = nullptr; int tok0 = 0; int n_kv = 0; int max_ctx = 0;
+  RowMap rows; };        // rows.pos != nullptr: partials of a multi-stream pass shared out by ms_share
 // projection outputs xq [M][n_heads][128], xk / xv [M][n_kv][128] fp32 -> q16 and the cache rows at *d_pos + t
 struct PostArgs {
   KvView kv; const float* xq; const float* xk; const float* xv; int M; int n_heads; const int* d_pos;
@@ -123,6 +131,7 @@ struct TbAttnArgs {
   float* pm; float* pl; uint16_t* pacc16;
   RowMap rows;  // narrow kernel only: multi-stream pass (one token per workgroup column; kpay .. vscl = container 0, `layer` = the profile's layer)
   int in_bf16 = 0;   // q16 is bf16 rows
+  int adapt = 0;     // multi-stream pass: workgroups shared out by ms_share
 };
 void launch_attend_tb(const TbAttnArgs&, int kb, hipStream_t);        // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend_tb_wide(const TbAttnArgs&, int kb, hipStream_t);   // 3..64 rows: 128 query rows per workgroup, tiles decoded once into LDS
@@ -134,6 +143,7 @@ void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const
 void launch_append(const AppendArgs&, hipStream_t);
 void launch_attend_narrow(const AttnArgs&, hipStream_t);   // 16-row tiles: 2 tokens x 6 heads per workgroup column
 void launch_attend_wide(const AttnArgs&, hipStream_t);     // 3..64 tokens, and prefill slices
+void launch_attend_chunk(const AttnArgs&, hipStream_t);    // slices of a prefill chunk (rows already in the cache) on the wide kernel
 void launch_attend_mid(const AttnArgs&, hipStream_t);      // 3..16 tokens: a wave owns whole tiles, row tiles of 16 rows (wider: blocks of 16 tokens)
 void launch_combine(const CombineArgs&, hipStream_t);
 void launch_attn_post(const PostArgs&, hipStream_t);
@@ -205,6 +215,85 @@ __device__ __forceinline__ uint4 pack_out8(const float* y, int bf16) {
     w[k] = (uint32_t)lo | ((uint32_t)hi << 16);
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Splits a slice of a prefill chunk uses, of the `S` its launch provides for.  The host sizes the grid without knowing the
+// position, so the choice is made on the device, by every wave of the attention launch and again by the combiner: lane s - 1
+// prices s splits, the cheapest wins (ties: the fewest).  Whole numbers only, so that two compilations cannot disagree.
+// Times are in sixteenths of the time a workgroup takes for one 32-key tile (0.56 us): a workgroup costs kChunkOverhead
+// tiles before and after its loop (about 10 us: launch, query, first tile, merge, stores), one workgroup runs per CU, the
+// longest start first, and more than one split costs a combiner pass over M * s partial rows.
+// 1,500 rows on an empty cache in containers of 8,192 tokens, us per layer call: 105 with slices of 1,024 tokens in 4 and 8
+// splits (39 + 39 in the attention, 23 in the combiners), 48 with one split (44 in the attention, which then waits for its
+// longest workgroup: 47 tiles).  2,048 rows behind 131,072: the same with 2 splits of one slice as with 4 of two.
+constexpr int kChunkOverhead = 18, kChunkMaxSplits = 64;
+__device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n_kv, int max_ctx, int S) {
+  const int base = n_kv * ((kG * M + 127) / 128), s = (int)(threadIdx.x & 63) + 1;
+  const int first = max(0, min(pos + tok0 + min(M, 128 / kG + 1), max_ctx)), last = max(0, min(pos + tok0 + M, max_ctx));
+  const int lo = ((first + 31) >> 5) * 16 / s + 16 * kChunkOverhead, hi = ((last + 31) >> 5) * 16 / s + 16 * kChunkOverhead;
+  const int n = base * s, idle = (256 - (n & 255)) & 255;            // workgroups, and CUs without one in the last round
+  int t = max(hi, (n >> 1) * (lo + hi) / 256 + lo * idle / 256);
+  if (s > 1) t += 96 + M * s / 13;
+  int best = s <= S ? t : 0x7fffffff, at = s;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int bt = __shfl_xor(best, o, 64), ba = __shfl_xor(at, o, 64);
+    if (bt < best || (bt == best && ba < at)) { best = bt; at = ba; }
+  }
+  return __builtin_amdgcn_readfirstlane(at);
+}
+
+// Multi-stream pass: how the W workgroups of one kv head are shared out over the pass's M <= 64 rows.  Streams differ in
+// length, and with the same number of splits for each the workgroups of the longest set the pace: every split is given
+// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 2 and no row more than 256.  c =
+// (tiles of all rows) / (W - M) always fits, since every row may round up by one; four halvings look for a smaller one.
+// 16 streams of 2,000 to 32,000 tokens: 36.7 us a pass with 16 splits each (the longest stream's workgroups walk 62 tiles,
+// the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.  Row t's splits are
+// workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by every wave from the
+// row map (lane t looks at row t), again by the combiner: whole numbers, so that both agree.
+struct MsShare { int row, split, n; size_t base; };
+__device__ __forceinline__ int ms_row_tiles(const RowMap& R, int t, int max_ctx) {      // 0: a row that names no container or position
+  const int pos = R.pos[t], slot = R.slot[t];
+  return pos >= 0 && pos < max_ctx && slot >= 0 && slot < R.n_slots ? (pos + 32) >> 5 : 0;
+}
+struct MsPlan { int mine, incl; };                 // of row `lane`: its splits, and the splits up to and including it
+__device__ __forceinline__ MsPlan ms_plan(const RowMap& R, int M, int max_ctx, int W) {
+  const int lane = threadIdx.x & 63, tiles = lane < M ? ms_row_tiles(R, lane, max_ctx) : 0;
+  int total = tiles, most = tiles;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) { total += __shfl_xor(total, o, 64); most = max(most, __shfl_xor(most, o, 64)); }
+  int lo = max(2, max((most + 255) >> 8, (total + W - 1) / W)), c = max(lo, (total + W - M - 1) / (W - M));
+  int mine = (tiles + c - 1) / c;
+  for (int it = 0; it < 4 && lo < c; ++it) {       // c always fits; a smaller one may
+    const int mid = (lo + c) >> 1, want = (tiles + mid - 1) / mid;
+    int sum = want;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    if (__builtin_amdgcn_readfirstlane(sum) <= W) { c = mid; mine = want; } else lo = mid + 1;
+  }
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) { const int up = __shfl_up(incl, o, 64); incl += lane >= o ? up : 0; }
+  return {mine, incl};
+}
+// workgroup b of the kv head; row = -1: nothing left for it
+__device__ __forceinline__ MsShare ms_share(const RowMap& R, int M, int max_ctx, int W, int b) {
+  const MsPlan P = ms_plan(R, M, max_ctx, W);
+  const int row = __popcll(__ballot(P.incl <= b));
+  if (row >= M) return {-1, 0, 0, 0};
+  const int n = __builtin_amdgcn_readlane(P.mine, row), base = __builtin_amdgcn_readlane(P.incl, row) - n;
+  return {row, b - base, n, (size_t)base};
+}
+
+// Multi-stream pass of at most 64 rows whose attention launch stores the new rows itself: the rows of the pass (bit t = row
+// t) that a workgroup of a row at `pos` in container `slot` has to store before it reads tiles [tile0, tile1) - rows of the
+// same stream it can see.  Rows of one stream that follow each other are stored by every workgroup that reads them, the same
+// bytes each time, so that no workgroup depends on another.
+__device__ __forceinline__ uint64_t ms_new_rows(const RowMap& R, int M, int slot, int pos, int tile0, int tile1, int& lane_pos) {
+  const int lane = threadIdx.x & 63;
+  lane_pos = lane < M ? R.pos[lane] : -1;
+  const bool mine = lane < M && R.slot[lane] == slot && lane_pos >= 0 && lane_pos <= pos && (lane_pos >> 5) >= tile0 && (lane_pos >> 5) < tile1;
+  return __ballot(mine);
 }
 
 // start of the (page, kv head) block that holds token t
