@@ -61,3 +61,31 @@ def test_against_the_decode_kernel(native, M, ctx, opts):
     assert np.linalg.norm(out - ref) <= (1e-3 + (2 * 2.0 ** -8 if bf16 else 0)) * np.linalg.norm(ref)
     per_row = np.linalg.norm(out - ref, axis=2) / np.linalg.norm(ref, axis=2)
     assert per_row.max() <= (4e-3 if not bf16 else 1.2e-2)
+
+
+# the 256-channel formats: slices of 1,024 tokens on the wide kernels, row blocks of equal height; the same comparison
+@pytest.mark.parametrize("kk", [0, 4, 5])
+@pytest.mark.parametrize("M,ctx,opts", [(65, 0, []), (22, 500, []), (43, 100, []), (1025, 0, []), (1100, 700, [(4, 1)]), (200, 3000, [(2, 3)])])
+def test_256_channel_rows(native, kk, M, ctx, opts):
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(M + ctx + kk)
+
+    def rows(n, heads):
+        return rng.standard_normal((n, heads, 256)).astype(np.float16)
+
+    with native.KvCache(max_ctx=8192, head_dim=256, max_rows=max(M, 1024)) as kv:
+        if kk:
+            kv.set_profile(kvqp.synthetic(layers=1, kk=kk, seed=5))
+        for key, val in opts:
+            kv.set_opt(key, val)
+        for p in range(0, ctx, 1024):
+            n = min(1024, ctx - p)
+            kv.append_host(0, rows(n, 4), rows(n, 4), p)
+        q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
+        kv.poison_workspace()
+        out = kv.layer_call(0, q, k, v, ctx).astype(np.float32)
+        kv.set_opt(3, 1)
+        ref = kv.layer_call(0, q, k, v, ctx).astype(np.float32)
+    assert np.isfinite(out).all()
+    assert np.linalg.norm(out - ref) <= 1e-3 * np.linalg.norm(ref)
+    assert (np.linalg.norm(out - ref, axis=2) / np.linalg.norm(ref, axis=2)).max() <= 4e-3

@@ -167,6 +167,36 @@ int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
   return best;
 }
 
+// 256-channel rows, both formats: how a pass is cut.  Passes of more than 64 rows (prompt chunks) go through the wide kernels
+// in slices of up to 1,024 tokens: in slices of 64 a chunk on a short context is mostly launches (1,500 first rows, int4: 533 us per layer call in 24 slices, 146 in two).
+// Row blocks of one slice get the same number of rows, in whole waves: the fragment reads of the waves that have rows set
+// the pace of a tile, so 144 rows are 80 + 64 and not 128 + 16 (24 rows at 9,001 tokens: 25.0 us per
+// layer call against 26.1).
+// Splits: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
+// rounds of 256 workgroups best.
+struct Part256 { int Ms, S, rows_per_block; bool narrow; };
+int slice256(const yka_kv* kv, int M) { return M > kMaxSlice && !kv->opt_force_narrow ? 1024 : kMaxSlice; }
+Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
+  const int ctx = kv->opt_ctx_hint > 0 ? std::min(kv->opt_ctx_hint, kv->cfg.max_ctx) : kv->cfg.max_ctx, ctx_tiles = (ctx + 31) / 32;
+  const int Ms = std::min(slice, M - s0), rows = kG * Ms, rb = (rows + 127) / 128, base = kv->cfg.n_kv_heads * rb;
+  const bool narrow = Ms <= 2 || kv->opt_force_narrow;
+  int S;
+  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min(512 / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
+  else if (kv->opt_splits_wide > 0) S = kv->opt_splits_wide;
+  else if (Ms <= kMaxSlice) S = std::min(256 / base, ctx_tiles / (2 * rb));
+  else {
+    S = 1;
+    double best = 0;
+    for (int s = 1; s <= std::min(1024 / base, ctx_tiles / 8); ++s) {
+      const double fill = base * s / (256.0 * ((base * s + 255) / 256)) - 0.01 * s;
+      if (fill > best) { best = fill; S = s; }
+    }
+  }
+  const size_t pairs = Ms > kMaxSlice ? kv->ws_rows : kWsPairs;
+  S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(pairs / (size_t)Ms));
+  return {Ms, S, ((rows + rb - 1) / rb + 15) / 16 * 16, narrow};
+}
+
 void check_layer(const yka_kv* kv, int layer) {
   if (layer < 0 || layer >= kv->cfg.n_layers) throw std::runtime_error("layer out of range");
 }
@@ -238,39 +268,32 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     const yka_kv::Tb& T = *kv->tb;
     check_tb_layer(kv, layer);
     if (k16) do_append(kv, layer, k16, v16, M, d_pos, st);
-    const int ctx = kv->opt_ctx_hint > 0 ? std::min(kv->opt_ctx_hint, kv->cfg.max_ctx) : kv->cfg.max_ctx;
-    for (int s0 = 0; s0 < M; s0 += kMaxSlice) {
-      const int Ms = std::min(kMaxSlice, M - s0), tiles = (Ms + 1) / 2, rb = (kG * Ms + 127) / 128;
-      const bool narrow = Ms <= 2 || kv->opt_force_narrow;
-      int S = narrow ? (kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::min(512 / (kv->cfg.n_kv_heads * tiles), ((ctx + 31) / 32) / 2))
-                     : (kv->opt_splits_wide > 0 ? kv->opt_splits_wide : std::min(256 / (kv->cfg.n_kv_heads * rb), ((ctx + 31) / 32) / (2 * rb)));
-      S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
-      const TbAttnArgs A{T.kpay(layer), T.vpay(layer), T.kscl(layer), T.vscl(layer), kv->cfg.max_ctx, kv->cfg.n_kv_heads, T.stride,
-                         T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, layer, q16 + (size_t)s0 * NH * 256, d_pos, depth, Ms, s0, NH, S,
-                         kv->pm, kv->pl, kv->pacc16, RowMap{}, bf16};
-      if (narrow) launch_attend_tb(A, T.kb, st); else launch_attend_tb_wide(A, T.kb, st);
-      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
+    const int slice = slice256(kv, M);
+    for (int s0 = 0; s0 < M; s0 += slice) {
+      const Part256 P = part256(kv, M, s0, slice);
+      TbAttnArgs A{T.kpay(layer), T.vpay(layer), T.kscl(layer), T.vscl(layer), kv->cfg.max_ctx, kv->cfg.n_kv_heads, T.stride,
+                   T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, layer, q16 + (size_t)s0 * NH * 256, d_pos, depth, P.Ms, s0, NH, P.S,
+                   kv->pm, kv->pl, kv->pacc16, RowMap{}, bf16};
+      A.rows_per_block = P.rows_per_block;
+      if (P.narrow) launch_attend_tb(A, T.kb, st); else launch_attend_tb_wide(A, T.kb, st);
+      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
     }
     return;
   }
   if (kv->r256()) {
     // 256-channel rows: rows of at most 2 tokens (or option key 3) run on row tiles of 2 tokens x 6 heads, two workgroups
-    // per CU; wider slices on 128-row workgroups of 8 waves, one per CU.  Both kernels store the rows of a pass of one
-    // slice themselves; a wide pass forced through the decode kernel and a pass of several slices launch the append first.
+    // per CU; wider slices on workgroups of 8 waves and up to 128 rows, one per CU.  Both kernels store the rows of a pass of
+    // one slice themselves; a wide pass forced through the decode kernel and a pass of several slices launch the append first.
     const bool fuse256 = k16 && (M <= 2 || (M <= kMaxSlice && !kv->opt_force_narrow));
     if (k16 && !fuse256) do_append(kv, layer, k16, v16, M, d_pos, st);
-    const int ctx = kv->opt_ctx_hint > 0 ? std::min(kv->opt_ctx_hint, kv->cfg.max_ctx) : kv->cfg.max_ctx;
-    for (int s0 = 0; s0 < M; s0 += kMaxSlice) {
-      const int Ms = std::min(kMaxSlice, M - s0), tiles = (Ms + 1) / 2, rb = (kG * Ms + 127) / 128;
-      const bool narrow = Ms <= 2 || kv->opt_force_narrow;
-      int S = narrow ? (kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::min(512 / (kv->cfg.n_kv_heads * tiles), ((ctx + 31) / 32) / 2))
-                     : (kv->opt_splits_wide > 0 ? kv->opt_splits_wide : std::min(256 / (kv->cfg.n_kv_heads * rb), ((ctx + 31) / 32) / (2 * rb)));
-      S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
-      AttnArgs A{kv->view(layer), q16 + (size_t)s0 * NH * 256, d_pos, depth, Ms, s0, NH, S, 0, kv->pm, kv->pl, kv->pacc16,
+    const int slice = slice256(kv, M);
+    for (int s0 = 0; s0 < M; s0 += slice) {
+      const Part256 P = part256(kv, M, s0, slice);
+      AttnArgs A{kv->view(layer), q16 + (size_t)s0 * NH * 256, d_pos, depth, P.Ms, s0, NH, P.S, P.rows_per_block, kv->pm, kv->pl, kv->pacc16,
                  fuse256 ? k16 : nullptr, fuse256 ? v16 : nullptr};
       A.in_bf16 = bf16;
-      if (narrow) launch_attend256(A, st); else launch_attend256_wide(A, st);
-      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
+      if (P.narrow) launch_attend256(A, st); else launch_attend256_wide(A, st);
+      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
     }
     return;
   }

@@ -152,7 +152,8 @@ __device__ __forceinline__ void quant_store_word256(const KvView& kv, int kvh, i
 
 }  // namespace
 
-// grid (S, n_kv, ceil(6M / 128)), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 rows come in
+// grid (S, n_kv, row blocks), block 512; wave w owns rows [16 w, 16 (w+1)) of the block, waves beyond the block's rows only
+// help with the dequantization; BF: bf16 rows come in
 template <bool BF>
 __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   __shared__ __align__(16) uint8_t lds[2][kLdsBuf];
@@ -160,12 +161,13 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int pos = *A.d_pos;
   const int nrows = kG * A.M;
-  constexpr int RPB = 128;
+  const int RPB = A.rows_per_block;
 
-  // row of this lane column: R = rb*128 + wave*16 + i  ->  token R/6 of the slice, head kvh*6 + R%6
+  // row of this lane column: R = rb*RPB + wave*16 + i  ->  token R/6 of the slice, head kvh*6 + R%6
   const int row0 = rb * RPB + wave * 16;
   const int R = row0 + i;
-  const bool vrow = R < nrows;
+  const int row_end = min(nrows, (rb + 1) * RPB);           // one past the block's last row
+  const bool vrow = R < row_end;
   const int tl = R / kG, head = kvh * kG + R % kG;
   int len = 0;
   if (vrow) { const int tg = A.tok0 + tl; len = min(pos + (A.depth ? (int)A.depth[tg] : tg) + 1, A.kv.max_ctx); }
@@ -186,7 +188,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
     }
   };
   if constexpr (!BF) q_ready();
-  const bool has_rows = row0 < nrows;                       // wave uniform
+  const bool has_rows = row0 < row_end;                     // wave uniform
 
   // key range of the workgroup: its splits cut [0, maxlen) of the block's longest row into 32-key tiles
   const int tok_lo = (rb * RPB) / kG, tok_hi = min(A.M, (rb * RPB + RPB + kG - 1) / kG);
@@ -355,7 +357,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   for (int k = 0; k < 8; ++k) {
     const int jr = 2 * k + (lane >> 5);
     const int Rr = row0 + jr;
-    if (Rr < nrows) {
+    if (Rr < row_end) {
       const size_t p = ((size_t)(Rr / kG) * A.S + split) * A.n_heads + kvh * kG + Rr % kG;
       const uint4 v = *reinterpret_cast<const uint4*>(stage + jr * kOPitch + chunk * 16);
       *reinterpret_cast<uint4*>(A.pacc16 + p * kD2 + chunk * 8) = v;
@@ -364,7 +366,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
 }
 
 void launch_attend256_wide(const AttnArgs& A, hipStream_t st) {
-  const int rows = kG * A.M, rb = (rows + 127) / 128;
+  const int rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block;
   const dim3 grid(A.S, A.kv.n_kv, rb);
   if (A.in_bf16) hipLaunchKernelGGL(attend256_wide_kernel<true>, grid, dim3(NT), 0, st, A);
   else hipLaunchKernelGGL(attend256_wide_kernel<false>, grid, dim3(NT), 0, st, A);

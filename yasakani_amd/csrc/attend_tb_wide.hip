@@ -135,7 +135,7 @@ __device__ __forceinline__ void decode_to_lds(uint8_t* buf, int tid, const Raw& 
   reinterpret_cast<uint32_t*>(buf + kLdsS)[tid & 63] = R.sc;      // waves repeat each other (no divergent branch)
 }
 
-// grid (S, n_kv, ceil(6M / 128)), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 queries
+// grid (S, n_kv, row blocks), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 queries
 template <int KB, bool BF>
 __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   constexpr int kTabBytes = 4 << (8 + KB);
@@ -155,12 +155,13 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   }
   const int pos = *A.d_pos;
   const int nrows = kG * A.M;
-  constexpr int RPB = 128;
+  const int RPB = A.rows_per_block;
 
-  // row of this lane column: R = rb*128 + wave*16 + i  ->  token R/6 of the slice, head kvh*6 + R%6
+  // row of this lane column: R = rb*RPB + wave*16 + i  ->  token R/6 of the slice, head kvh*6 + R%6
   const int row0 = rb * RPB + wave * 16;
   const int R = row0 + i;
-  const bool vrow = R < nrows;
+  const int row_end = min(nrows, (rb + 1) * RPB);           // one past the block's last row
+  const bool vrow = R < row_end;
   const int tl = R / kG, head = kvh * kG + R % kG;
   int len = 0;
   if (vrow) { const int tg = A.tok0 + tl; len = min(pos + (A.depth ? (int)A.depth[tg] : tg) + 1, A.max_ctx); }
@@ -178,7 +179,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
     for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, qraw[t]);
   };
   if constexpr (!BF) q_ready();
-  const bool has_rows = row0 < nrows;                       // wave uniform
+  const bool has_rows = row0 < row_end;                     // wave uniform
 
   // key range of the workgroup: its splits cut [0, maxlen) of the block's longest row into 32-key tiles
   const int tok_lo = (rb * RPB) / kG, tok_hi = min(A.M, (rb * RPB + RPB + kG - 1) / kG);
@@ -316,7 +317,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   for (int k = 0; k < 8; ++k) {
     const int jr = 2 * k + (lane >> 5);
     const int Rr = row0 + jr;
-    if (Rr < nrows) {
+    if (Rr < row_end) {
       const size_t p = ((size_t)(Rr / kG) * A.S + split) * A.n_heads + kvh * kG + Rr % kG;
       const uint4 v = *reinterpret_cast<const uint4*>(stage + jr * kOPitch + chunk * 16);
       *reinterpret_cast<uint4*>(A.pacc16 + p * kD2 + chunk * 8) = v;
@@ -327,7 +328,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
 }  // namespace
 
 void launch_attend_tb_wide(const TbAttnArgs& A, int kb, hipStream_t st) {
-  const int rows = kG * A.M, rb = (rows + 127) / 128;
+  const int rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block;
   const dim3 grid(A.S, A.n_kv, rb);
   if (kb == 4 && A.in_bf16) hipLaunchKernelGGL((attend_tb_wide_kernel<4, true>), grid, dim3(NT), 0, st, A);
   else if (kb == 4) hipLaunchKernelGGL((attend_tb_wide_kernel<4, false>), grid, dim3(NT), 0, st, A);

@@ -60,7 +60,7 @@ struct AttnArgs {
   int tok0;     // index of the slice's first row inside the pass (row t sees keys [0, *d_pos + depth(tok0+t) + 1))
   int n_heads;
   int S;        // splits
-  int rows_per_block;  // wide kernel: query rows one workgroup owns (multiple of 32)
+  int rows_per_block;  // wide kernels: query rows one workgroup owns (a multiple of 32, 256-channel rows of 16; at most 128)
   float* pm; float* pl; uint16_t* pacc16;
   // k16/v16 != nullptr: fused quantize-on-append - the workgroups whose tiles hold the new rows quantize and store them
   // before reading them.  Narrow kernel (M <= 2): rows [0, M) of the pass; wide kernel: k16/v16 point at row 0 of the
@@ -132,6 +132,7 @@ struct TbAttnArgs {
   RowMap rows;  // narrow kernel only: multi-stream pass (one token per workgroup column; kpay .. vscl = container 0, `layer` = the profile's layer)
   int in_bf16 = 0;   // q16 is bf16 rows
   int adapt = 0;     // multi-stream pass: workgroups shared out by ms_share
+  int rows_per_block = 128;   // wide kernel only
 };
 void launch_attend_tb(const TbAttnArgs&, int kb, hipStream_t);        // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend_tb_wide(const TbAttnArgs&, int kb, hipStream_t);   // 3..64 rows: 128 query rows per workgroup, tiles decoded once into LDS
