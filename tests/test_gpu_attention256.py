@@ -303,3 +303,32 @@ def test_full_length_32768(native, oracle, M):
     expect = ref.attend_f32(q, ctx, threads=16, want_f32=True)[1]
     assert_attn_close(out, expect, f"32k M={M}")
     assert np.abs(out.astype(np.float64) - expect).max() <= 2e-3
+
+
+# The decode kernel's wave merge and its request pipeline: waves without a tile, with one, with several, a last split that is
+# nearly empty; one and two tokens (6 and 12 rows of the 16); both trellis widths beside the int4 rows.  Against the wide kernel
+# (a window of 3 rows, of which the first ones are compared), which shares neither.
+@pytest.mark.parametrize("kk", [0, 4, 5])
+@pytest.mark.parametrize("M,ctx,splits", [(1, 0, 0), (1, 31, 2), (2, 32, 0), (1, 127, 2), (2, 160, 2), (1, 290, 3), (2, 2047, 1), (1, 2047, 0), (2, 1000, 200)])
+def test_decode_merge_against_the_wide_kernel(native, kk, M, ctx, splits):
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(M + ctx + kk)
+
+    def rows(n, heads):
+        return rng.standard_normal((n, heads, 256)).astype(np.float16)
+
+    with native.KvCache(max_ctx=2304, head_dim=256, max_rows=2048) as kv:
+        if kk:
+            kv.set_profile(kvqp.synthetic(layers=1, kk=kk, seed=9))
+        if ctx:
+            kv.append_host(0, rows(ctx, 4), rows(ctx, 4), 0)
+        q, k, v = rows(3, 24), rows(3, 4), rows(3, 4)
+        kv.poison_workspace()
+        wide = kv.layer_call(0, q, k, v, ctx)[:M].astype(np.float32)
+        if splits:
+            kv.set_opt(1, splits)
+        kv.poison_workspace()
+        out = kv.layer_call(0, q[:M], k[:M], v[:M], ctx).astype(np.float32)
+    # the same codes; P (times the V scale) and the outputs are fp16 on both sides, 2^-11 each
+    assert np.isfinite(out).all()
+    assert np.linalg.norm(out - wide) <= 1e-3 * np.linalg.norm(wide)

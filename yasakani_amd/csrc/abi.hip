@@ -172,7 +172,9 @@ int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
 // Row blocks of one slice get the same number of rows, in whole waves: the fragment reads of the waves that have rows set
 // the pace of a tile, so 144 rows are 80 + 64 and not 128 + 16 (24 rows at 9,001 tokens: 25.0 us per
 // layer call against 26.1).
-// Splits: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
+// Splits of the decode kernels: one workgroup per CU (the waves keep the next tile in flight and the combiner has half the
+// rows to read: 205 against 225 us for 16 layers at 20,011 tokens, 167 / 204 at 3,000, 97 / 101 for 2 layers at 200,000).
+// Of the wide ones: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
 // rounds of 256 workgroups best.
 struct Part256 { int Ms, S, rows_per_block; bool narrow; };
 int slice256(const yka_kv* kv, int M) { return M > kMaxSlice && !kv->opt_force_narrow ? 1024 : kMaxSlice; }
@@ -181,7 +183,7 @@ Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
   const int Ms = std::min(slice, M - s0), rows = kG * Ms, rb = (rows + 127) / 128, base = kv->cfg.n_kv_heads * rb;
   const bool narrow = Ms <= 2 || kv->opt_force_narrow;
   int S;
-  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min(512 / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
+  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min(256 / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
   else if (kv->opt_splits_wide > 0) S = kv->opt_splits_wide;
   else if (Ms <= kMaxSlice) S = std::min(256 / base, ctx_tiles / (2 * rb));
   else {
@@ -281,7 +283,7 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     return;
   }
   if (kv->r256()) {
-    // 256-channel rows: rows of at most 2 tokens (or option key 3) run on row tiles of 2 tokens x 6 heads, two workgroups
+    // 256-channel rows: rows of at most 2 tokens (or option key 3) run on row tiles of 2 tokens x 6 heads, one workgroup
     // per CU; wider slices on workgroups of 8 waves and up to 128 rows, one per CU.  Both kernels store the rows of a pass of
     // one slice themselves; a wide pass forced through the decode kernel and a pass of several slices launch the append first.
     const bool fuse256 = k16 && (M <= 2 || (M <= kMaxSlice && !kv->opt_force_narrow));

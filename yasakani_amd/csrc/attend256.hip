@@ -15,6 +15,7 @@
 // [7,3,6,2,5,1,4,0]; the query fragments are loaded in the same order.
 #include "yka_internal.h"
 #include "rot256_device.h"
+#include "merge256_device.h"
 #include <hip/hip_fp16.h>
 
 namespace yka {
@@ -184,7 +185,8 @@ struct Raw256 {        // what one lane holds of a 32-key tile
 };
 struct Offs256 { uint32_t kw, sc, vw; };
 
-__device__ __forceinline__ void load_tile256(const uint8_t* pg, int tp, const Offs256& L, Raw256& R) {
+// The two halves of a tile are requested apart: each one tile ahead, as soon as the registers it lands in are free.
+__device__ __forceinline__ void load_k256(const uint8_t* pg, int tp, const Offs256& L, Raw256& R) {
   const uint8_t* rows = pg + (uint32_t)tp * 128u;          // code rows of the tile (K and V planes)
   const uint8_t* sc = pg + (uint32_t)tp * 4u;              // scale entries of the tile
 #pragma unroll
@@ -192,8 +194,13 @@ __device__ __forceinline__ void load_tile256(const uint8_t* pg, int tp, const Of
     R.kw[kt][0] = *reinterpret_cast<const uint4*>(rows + kP2Kw + L.kw + 2048 * kt);
     R.kw[kt][1] = *reinterpret_cast<const uint4*>(rows + kP2Kw + L.kw + 2048 * kt + 16);
     R.ksc[kt] = *reinterpret_cast<const f4*>(sc + kP2Ks + L.sc + 64 * kt);
-    R.vsc[kt] = *reinterpret_cast<const f4*>(sc + kP2Vs + L.sc + 64 * kt);
   }
+}
+__device__ __forceinline__ void load_v256(const uint8_t* pg, int tp, const Offs256& L, Raw256& R) {
+  const uint8_t* rows = pg + (uint32_t)tp * 128u;
+  const uint8_t* sc = pg + (uint32_t)tp * 4u;
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) R.vsc[kt] = *reinterpret_cast<const f4*>(sc + kP2Vs + L.sc + 64 * kt);
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
@@ -211,7 +218,7 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   constexpr int TPT = MS ? 1 : 2;
   __shared__ float s_m[4][16], s_l[4][16];
   __shared__ __align__(16) float s_wn[16][4];
-  __shared__ float s_acc[4][16][kD2 + 4];
+  __shared__ __align__(16) float s_acc[4 * m256_wave<TPT * kG>()];
   int split = blockIdx.x, rt = blockIdx.z;
   const int kvh = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -328,9 +335,17 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
 #pragma unroll
   for (int b = 0; b < 16; ++b) o[b] = f4{0.f, 0.f, 0.f, 0.f};
 
+  // K words of the wave's next tile are requested behind the scores of this one, V words behind its PV product: no second
+  // register set, and every request has half a tile of work to hide under.  Past the end K is the last tile once more (an
+  // unconditional request: the compiler then knows how many loads are in flight at each wait).
   Raw256 cur;
+  if (tile0 + wave < tile1) {
+    const int t0 = (tile0 + wave) << 5;
+    const uint8_t* pg = page256(A.kv, kvh, t0);
+    load_k256(pg, t0 % kPageTok, offs, cur);
+    load_v256(pg, t0 % kPageTok, offs, cur);
+  }
   for (int T = tile0 + wave; T < tile1; T += 4) {
-    load_tile256(page256(A.kv, kvh, T << 5), (T << 5) % kPageTok, offs, cur);
     const int t0 = T << 5;
     const bool need_mask = t0 + 32 > minlen;
     // ---- scores: per 16-key tile 8 chained MFMAs (one per word of the lane), then one multiply by the key's scale ----
@@ -350,6 +365,9 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[4 * kt + r] = part[r] * cur.ksc[kt][r];      // key t0 + 16kt + 4g + r against row i
     }
+    const int tn = min(T + 4, tile1 - 1) << 5;
+    const uint8_t* const pgn = page256(A.kv, kvh, tn);
+    load_k256(pgn, tn % kPageTok, offs, cur);
     if (need_mask) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) { const int key = t0 + 16 * (e >> 2) + 4 * g + (e & 3); s[e] = key < len ? s[e] : -INFINITY; }
@@ -394,60 +412,25 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
         o[hh * 8 + 7 - 2 * bb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vlo, pf, o[hh * 8 + 7 - 2 * bb], 0, 0, 0);
         o[hh * 8 + 6 - 2 * bb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vhi, pf, o[hh * 8 + 6 - 2 * bb], 0, 0, 0);
       }
+    load_v256(pgn, tn % kPageTok, offs, cur);
   }
-  // ---- merge the 4 waves, write one partial per (row, split): o[hh*8 + el][r] = channel 8 (4g + r + 16 hh) + el of row i ----
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
-  if (g == 0) { s_m[wave][i] = m_run; s_l[wave][i] = l_run; }
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-    for (int el = 0; el < 8; ++el)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s_acc[wave][i][8 * (4 * g + r + 16 * hh) + el] = o[hh * 8 + el][r];
-  __syncthreads();
-  // per row: the weight of each wave's accumulator, already divided by the row's sum - computed once per row by 4 lanes,
-  // not once per output element
-  if (threadIdx.x < 64) {
-    const int j = threadIdx.x >> 2, w = threadIdx.x & 3;
-    const float mw = s_m[w][j];
-    float M2 = fmaxf(mw, __shfl_xor(mw, 1, 64));
-    M2 = fmaxf(M2, __shfl_xor(M2, 2, 64));
-    const float ww = exp2f(mw - M2);
-    float L = ww * s_l[w][j];
-    L += __shfl_xor(L, 1, 64);
-    L += __shfl_xor(L, 2, 64);
-    s_wn[j][w] = L > 0.f ? ww / L : 0.f;
-    const int tj = TPT * rt + j / kG;
-    if (w == 0 && j < TPT * kG && tj < A.M) {
-      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
-      A.pm[p] = M2; A.pl[p] = L;
-    }
-  }
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < TPT * kG * kD2; idx += 256) {
-    const int j = idx >> 8, d = idx & (kD2 - 1);
-    const int tj = TPT * rt + j / kG;
-    if (tj >= A.M) continue;
-    const f4 w4 = *reinterpret_cast<const f4*>(s_wn[j]);
-    const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
-    const float y = w4[0] * s_acc[0][j][d] + w4[1] * s_acc[1][j][d] + w4[2] * s_acc[2][j][d] + w4[3] * s_acc[3][j][d];
-    A.pacc16[p * kD2 + d] = __half_as_ushort(__float2half_rn(y));
-  }
+  merge_waves256<TPT * kG>(o, m_run, l_run, wave, min(TPT, A.M - TPT * rt) * kG, kvh, A.n_heads, 1.f, nullptr, s_m, s_l, s_wn, s_acc, A.pm, A.pl, A.pacc16,
+                           [&](int j) __attribute__((always_inline)) { return pair_of(TPT * rt + j / kG); });
 }
 
 // combiner (src/attention_kv4q.cu:325-332) for 256-channel rows: grid (n_heads, M), block 256 = 8 split lanes x 32 channel
 // lanes of 8 channels; the split lanes run in parallel and are summed through LDS.  S <= 256.  kInFlight = partial rows a
-// split lane requests before it uses any: 16 covers 128 splits (decode: few, long workgroups; 32 for up to 256 splits), 4 covers
+// split lane requests before it uses any: 8 covers the 64 splits of decode (16 for 128, 32 for 256), 4 covers
 // 32 and keeps the register count low where thousands of workgroups run (wide windows).
-template <int kInFlight>
+// MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
+template <int kInFlight, bool MS>
 __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
   __shared__ float s_w[256];
   __shared__ float s_o[8][kD2 + 4];
   __shared__ float s_wsum[8];
   const int head = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x;
   size_t pair0 = (size_t)tok * A.S;
-  if (A.rows.pos) {
+  if constexpr (MS) {
     const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
     A.S = __builtin_amdgcn_readlane(P.mine, tok);
     pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
@@ -493,7 +476,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
       wsum += w;
     }
     s0 += 8 * kInFlight;
-    if (s0 >= A.S) break;
+    if (!MS || s0 >= A.S) break;
     request(s0);
   }
 #pragma unroll
@@ -523,14 +506,15 @@ void launch_attend256(const AttnArgs& A, hipStream_t st) {
 }
 void launch_combine256(const CombineArgs& A, hipStream_t st) {
   if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most): half of them with 2 streams
-    if (A.M < 8) hipLaunchKernelGGL(combine256_kernel<16>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-    else hipLaunchKernelGGL(combine256_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    if (A.M < 8) hipLaunchKernelGGL((combine256_kernel<16, true>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    else hipLaunchKernelGGL((combine256_kernel<4, true>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
     return;
   }
   // 8 split lanes x kInFlight rows each must cover the S <= 256 splits
-  if (A.S > 128) hipLaunchKernelGGL(combine256_kernel<32>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else if (A.S > 32) hipLaunchKernelGGL(combine256_kernel<16>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else hipLaunchKernelGGL(combine256_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  if (A.S > 128) hipLaunchKernelGGL((combine256_kernel<32, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  else if (A.S > 64) hipLaunchKernelGGL((combine256_kernel<16, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  else if (A.S > 32) hipLaunchKernelGGL((combine256_kernel<8, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  else hipLaunchKernelGGL((combine256_kernel<4, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
 }
 void launch_export_rows256(const KvView& kv, int pos0, int n, uint32_t* kw, float* ks, uint32_t* vw, float* vs, hipStream_t st) {
   hipLaunchKernelGGL(xfer256_kernel<false>, dim3(n, kv.n_kv), dim3(64), 0, st, kv, pos0, n, kw, ks, vw, vs);

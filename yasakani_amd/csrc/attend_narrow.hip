@@ -512,7 +512,8 @@ void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
 // kInFlight = partial rows a split lane requests before it uses any: 16 covers 256 splits in one memory round trip, 8
 // covers the 128 splits of decode over long contexts (few, long workgroups); 4 keeps the register count low where
 // thousands of workgroups run (wide windows).
-template <int kInFlight>
+// MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
+template <int kInFlight, bool MS>
 __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   __shared__ float s_w[256];
   __shared__ float s_o[16][kD + 4];
@@ -523,7 +524,7 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
     if (A.S == 1 && A.direct) return;
   }
   size_t pair0 = (size_t)tok * A.S;
-  if (A.rows.pos) {
+  if constexpr (MS) {
     const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
     A.S = __builtin_amdgcn_readlane(P.mine, tok);
     pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
@@ -570,7 +571,7 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
       wsum += w;
     }
     s0 += 16 * kInFlight;
-    if (s0 >= A.S) break;
+    if (!MS || s0 >= A.S) break;
     request(s0);
   }
 #pragma unroll
@@ -656,7 +657,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
   if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most)
-    hipLaunchKernelGGL(combine_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    hipLaunchKernelGGL((combine_kernel<4, true>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
     return;
   }
   if (A.S <= 32 && !A.unrot && A.M >= 8) {
@@ -665,9 +666,9 @@ void launch_combine(const CombineArgs& A, hipStream_t st) {
     else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, A);
     return;
   }
-  if (A.S > 128) hipLaunchKernelGGL(combine_kernel<16>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);   // S <= 256
-  else if (A.S > 64) hipLaunchKernelGGL(combine_kernel<8>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else hipLaunchKernelGGL(combine_kernel<4>, dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);   // S <= 256
+  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  else hipLaunchKernelGGL((combine_kernel<4, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
 }
 
 }  // namespace yka

@@ -18,6 +18,7 @@
 //   * a mean row of K shifts every score of a query row by the same q.mu and cancels in the softmax: it is not added.
 //     A mean row of V is added to the normalised partial (the probabilities of a split sum to one).
 #include "yka_internal.h"
+#include "merge256_device.h"
 #include <hip/hip_fp16.h>
 
 namespace yka {
@@ -57,11 +58,10 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
   constexpr int TPT = MS ? 1 : 2;                    // tokens per row tile
   constexpr int NW = 2 * KB;                         // words per chunk
   constexpr int kTabBytes = 4 << (8 + KB);           // one pair table
-  constexpr int kAccBytes = 4 * 16 * (kD2 + 4) * 4;
+  constexpr int kAccBytes = 16 * m256_wave<TPT * kG>();
   __shared__ float s_m[4][16], s_l[4][16];
   __shared__ __align__(16) float s_wn[16][4];
   __shared__ __align__(16) uint8_t s_buf[kAccBytes > 2 * kTabBytes ? kAccBytes : 2 * kTabBytes];   // pair tables, then the wave merge
-  float (*s_acc)[16][kD2 + 4] = reinterpret_cast<float (*)[16][kD2 + 4]>(s_buf);
   const uint8_t* const s_tabK = s_buf;
   const uint8_t* const s_tabV = s_buf + kTabBytes;
   int split = blockIdx.x, rt = blockIdx.z;
@@ -293,46 +293,9 @@ __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
     }
   }
   __syncthreads();                                   // every wave is done with the tables: their space now holds the merge
-  // ---- merge the 4 waves, write one partial per (row, split): o[hh*8 + el][r] = channel 8 (4g + r + 16 hh) + el of row i ----
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
-  if (g == 0) { s_m[wave][i] = m_run; s_l[wave][i] = l_run; }
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-    for (int el = 0; el < 8; ++el)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s_acc[wave][i][8 * (4 * g + r + 16 * hh) + el] = o[hh * 8 + el][r];
-  __syncthreads();
-  // per row: the weight of each wave's accumulator, already divided by the row's sum and multiplied by gain / 256 of the
-  // V table - computed once per row by 4 lanes, not once per output element
-  if (threadIdx.x < 64) {
-    const int j = threadIdx.x >> 2, w = threadIdx.x & 3;
-    const float mw = s_m[w][j];
-    float M2 = fmaxf(mw, __shfl_xor(mw, 1, 64));
-    M2 = fmaxf(M2, __shfl_xor(M2, 2, 64));
-    const float ww = exp2f(mw - M2);
-    float L = ww * s_l[w][j];
-    L += __shfl_xor(L, 1, 64);
-    L += __shfl_xor(L, 2, 64);
-    s_wn[j][w] = L > 0.f ? ww * A.gfac[gV] / L : 0.f;
-    const int tj = TPT * rt + j / kG;
-    if (w == 0 && j < TPT * kG && tj < A.M) {
-      const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
-      A.pm[p] = M2; A.pl[p] = L;
-    }
-  }
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < TPT * kG * kD2; idx += 256) {
-    const int j = idx >> 8, d = idx & (kD2 - 1);
-    const int tj = TPT * rt + j / kG;
-    if (tj >= A.M) continue;
-    const f4 w4 = *reinterpret_cast<const f4*>(s_wn[j]);
-    const size_t p = pair_of(tj) * A.n_heads + kvh * kG + j % kG;
-    float y = w4[0] * s_acc[0][j][d] + w4[1] * s_acc[1][j][d] + w4[2] * s_acc[2][j][d] + w4[3] * s_acc[3][j][d];
-    if (A.mu && w4[0] + w4[1] + w4[2] + w4[3] > 0.f) y += A.mu[(size_t)gV * 256 + d];
-    A.pacc16[p * kD2 + d] = __half_as_ushort(__float2half_rn(y));
-  }
+  merge_waves256<TPT * kG>(o, m_run, l_run, wave, min(TPT, A.M - TPT * rt) * kG, kvh, A.n_heads, A.gfac[gV], A.mu ? A.mu + (size_t)gV * 256 : nullptr,
+                           s_m, s_l, s_wn, reinterpret_cast<float*>(s_buf), A.pm, A.pl, A.pacc16,
+                           [&](int j) __attribute__((always_inline)) { return pair_of(TPT * rt + j / kG); });
 }
 
 }  // namespace
