@@ -1,0 +1,39 @@
+"""Decode over trellis-coded rows: the encoder's search rides in the attention launch, which attends to the rows in front of the
+position; the combiner adds the new rows.  Against the general path (option 3: encoder launches first, every key in the
+attention launch), from the empty cache to the last row of the container."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kk", [4, 5])
+@pytest.mark.parametrize("M,ctx,opts", [(1, 0, []), (2, 0, []), (1, 1, []), (2, 31, []), (2, 32, []), (1, 500, [(4, 1)]), (2, 1023, [(1, 200)]),
+                                        (2, 2046, []), (1, 2047, []), (1, 700, [(11, 1)]), (2, 65, [(11, 1)])])
+def test_against_the_general_path(native, kk, M, ctx, opts):
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(100 * M + ctx + kk)
+    bf16 = (11, 1) in opts
+
+    def rows(n, heads):
+        x = rng.standard_normal((n, heads, 256)).astype(np.float32)
+        return native.bf16_bits(x) if bf16 else x.astype(np.float16)
+
+    with native.KvCache(n_layers=2, max_ctx=2048, head_dim=256, max_rows=2048) as kv:
+        kv.set_profile(kvqp.synthetic(layers=2, kk=kk, seed=11))
+        for key, val in opts:
+            kv.set_opt(key, val)
+        if ctx:
+            kv.append_host(1, rows(ctx, 4), rows(ctx, 4), 0)
+        q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
+        kv.poison_workspace()
+        out = kv.layer_call(1, q, k, v, ctx)
+        kv.set_opt(3, 1)
+        kv.poison_workspace()
+        ref = kv.layer_call(1, q, k, v, ctx)
+    if bf16:
+        out, ref = native.bf16_to_f32(out), native.bf16_to_f32(ref)
+    out, ref = out.astype(np.float32), ref.astype(np.float32)
+    assert np.isfinite(out).all()
+    # the same codes; the general path rounds P (times the V scale) and its partials to fp16, both round the output (bf16: 2^-8 each)
+    assert np.linalg.norm(out - ref) <= (1e-3 + (2 * 2.0 ** -8 if bf16 else 0)) * np.linalg.norm(ref)

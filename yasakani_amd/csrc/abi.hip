@@ -210,20 +210,25 @@ void check_tb_layer(const yka_kv* kv, int layer) {
   if (kv->tb && layer >= kv->tb->layers) throw std::runtime_error("the profile has no groups for this layer");
 }
 constexpr int kTbTileTok = 128;     // tokens per launch of the trellis encoder (its scratch holds that many)
+TbEncArgs tb_encoder_args(const yka_kv* kv, int layer, int container, const uint16_t* k16, const uint16_t* v16, int t0, int M, const int* d_pos) {
+  const yka_kv::Tb& T = *kv->tb;
+  TbEncArgs A{};
+  A.blob = T.blob; A.nm = T.nm; A.has_trellis = 1; A.desc = T.desc; A.ngrp = T.ngrp; A.mult_off = T.mult_off;
+  A.k16 = k16; A.v16 = v16; A.in_bf16 = kv->opt_io_bf16; A.d_pos = d_pos; A.layer = layer; A.tok0 = t0; A.n_kv = kv->cfg.n_kv_heads;
+  A.max_ctx = kv->cfg.max_ctx;
+  A.nrow = std::min(kTbTileTok, M - t0) * 2 * kv->cfg.n_kv_heads;
+  A.scr = T.scr; A.scr_w_ofs = T.scr_w_ofs;
+  A.pay0 = T.kpay(container); A.pay1 = T.vpay(container); A.scl0 = T.kscl(container); A.scl1 = T.vscl(container); A.stride = T.stride;
+  return A;
+}
 // trellis encoder over the rows of a pass: fp32 rows, or fp16 rows if k32 == nullptr
 void tb_append(yka_kv* kv, int layer, const float* k32, const float* v32, const uint16_t* k16, const uint16_t* v16, int M, const int* d_pos,
                int rot, hipStream_t st, int pos_limit = 0, const RowMap* rows = nullptr) {
-  const yka_kv::Tb& T = *kv->tb;
   const int container = rows ? 0 : layer;            // multi-stream pass: containers are streams, `layer` only names the groups
   check_tb_layer(kv, layer);
   for (int t0 = 0; t0 < M; t0 += kTbTileTok) {
-    TbEncArgs A{};
-    A.blob = T.blob; A.nm = T.nm; A.has_trellis = 1; A.desc = T.desc; A.ngrp = T.ngrp; A.mult_off = T.mult_off;
-    A.k32 = k32; A.v32 = v32; A.k16 = k16; A.v16 = v16; A.in_bf16 = kv->opt_io_bf16; A.d_pos = d_pos; A.layer = layer; A.tok0 = t0; A.n_kv = kv->cfg.n_kv_heads;
-    A.max_ctx = kv->cfg.max_ctx; A.rot = rot; A.pos_limit = pos_limit;
-    A.nrow = std::min(kTbTileTok, M - t0) * 2 * kv->cfg.n_kv_heads;
-    A.scr = T.scr; A.scr_w_ofs = T.scr_w_ofs;
-    A.pay0 = T.kpay(container); A.pay1 = T.vpay(container); A.scl0 = T.kscl(container); A.scl1 = T.vscl(container); A.stride = T.stride;
+    TbEncArgs A = tb_encoder_args(kv, layer, container, k16, v16, t0, M, d_pos);
+    A.k32 = k32; A.v32 = v32; A.rot = rot; A.pos_limit = pos_limit;
     if (rows) A.rows = *rows;
     launch_tb_encode(A, st);
   }
@@ -269,7 +274,9 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     // tiles of 2 tokens x 6 heads, wider slices on 128-row workgroups that decode every tile once into LDS
     const yka_kv::Tb& T = *kv->tb;
     check_tb_layer(kv, layer);
-    if (k16) do_append(kv, layer, k16, v16, M, d_pos, st);
+    // decode without a depth table: the encoder's search rides in the attention launch, which leaves the new rows to the combiner
+    const bool fuse = k16 && M <= 2 && !depth && mode == 0 && !kv->opt_force_narrow;
+    if (k16 && !fuse) do_append(kv, layer, k16, v16, M, d_pos, st);
     const int slice = slice256(kv, M);
     for (int s0 = 0; s0 < M; s0 += slice) {
       const Part256 P = part256(kv, M, s0, slice);
@@ -277,8 +284,14 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
                    T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, layer, q16 + (size_t)s0 * NH * 256, d_pos, depth, P.Ms, s0, NH, P.S,
                    kv->pm, kv->pl, kv->pacc16, RowMap{}, bf16};
       A.rows_per_block = P.rows_per_block;
+      const CombineArgs C{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
+      if (fuse) {
+        launch_tb_encode_attend(tb_encoder_args(kv, layer, layer, k16, v16, 0, M, d_pos), A, T.kb, st);
+        launch_combine256_new(C, A, T.kb, st);
+        return;
+      }
       if (P.narrow) launch_attend_tb(A, T.kb, st); else launch_attend_tb_wide(A, T.kb, st);
-      if (mode != 2) launch_combine256(CombineArgs{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16}, st);
+      if (mode != 2) launch_combine256(C, st);
     }
     return;
   }

@@ -423,8 +423,22 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
 // split lane requests before it uses any: 8 covers the 64 splits of decode (16 for 128, 32 for 256), 4 covers
 // 32 and keeps the register count low where thousands of workgroups run (wide windows).
 // MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
-template <int kInFlight, bool MS>
-__global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
+// KB != 0: partials of launch_tb_encode_attend, which leave out the rows of the pass; token t also sees the keys *d_pos + u, u <=
+// t, which are decoded here from the rows the encoder has stored (thread = channel; N names them) and join the sum as
+// splits of one key each, in fp32.
+template <int KB> struct NewKeyArgs { TbAttnArgs N; };
+template <> struct NewKeyArgs<0> {};
+// table integer of element d of a trellis-coded row: the last 8 stream bits up to the end of its field name the state
+template <int KB>
+__device__ __forceinline__ float tb_element(const uint8_t* row, int d, const uint32_t* pairs) {
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(row) + (d >> 6) * (2 * KB);
+  const int last = KB * ((d & 63) + 1) - 1, j = last >> 5;
+  const uint32_t lo = w[j], hi = j > 0 ? w[j - 1] : 0u;
+  const uint32_t state = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)(31 - (last & 31))) & 255u;
+  return __half2float(__ushort_as_half((uint16_t)(pairs[state] >> 16)));     // entry i: the values of states (i >> KB) & 255 and i & 255
+}
+template <int kInFlight, bool MS, int KB>
+__global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyArgs<KB> X) {
   __shared__ float s_w[256];
   __shared__ float s_o[8][kD2 + 4];
   __shared__ float s_wsum[8];
@@ -451,6 +465,36 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
     }
   };
   request(0);
+  float new_s[2] = {-1e30f, -1e30f}, new_v[2] = {0.f, 0.f};       // score in log2 units and V value (channel tid) of the new keys
+  if constexpr (KB != 0) {
+    __shared__ float s_dot[2][4];
+    const TbAttnArgs& N = X.N;
+    const int kvh = head / kG, gK = (N.layer * N.n_kv + kvh) * 2, gV = gK + 1, pos = *N.d_pos;
+    const uint32_t *pk = N.pairs + ((size_t)gK << (8 + KB)), *pv = N.pairs + ((size_t)gV << (8 + KB));
+    const float q = row16_value(N.q16[((size_t)tok * A.n_heads + head) * kD2 + tid], N.in_bf16);
+    float ksc[2] = {0.f, 0.f}, dot[2] = {0.f, 0.f};
+    bool seen[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int r = pos + u;
+      seen[u] = u <= tok && r >= 0 && r < N.max_ctx;               // uniform over the workgroup
+      if (!seen[u]) continue;
+      const size_t row = (size_t)kvh * N.max_ctx + r;
+      ksc[u] = N.kscl[row];
+      dot[u] = q * tb_element<KB>(N.kpay + row * N.stride, tid, pk);
+      new_v[u] = tb_element<KB>(N.vpay + row * N.stride, tid, pv) * N.vscl[row] * N.gfac[gV] + (N.mu ? N.mu[(size_t)gV * 256 + tid] : 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int o = 32; o; o >>= 1) dot[u] += __shfl_xor(dot[u], o, 64);
+      if ((tid & 63) == 0) s_dot[u][tid >> 6] = dot[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (seen[u]) new_s[u] = (s_dot[u][0] + s_dot[u][1] + s_dot[u][2] + s_dot[u][3]) * ksc[u] * (kLog2e * 0.0625f * N.gfac[gK]);
+  }
   float pmv = -1e30f, plv = 0.f;
   if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
   float M2 = pmv;
@@ -459,6 +503,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
   if ((tid & 63) == 0) s_wsum[tid >> 6] = M2;
   __syncthreads();
   M2 = fmaxf(fmaxf(s_wsum[0], s_wsum[1]), fmaxf(s_wsum[2], s_wsum[3]));
+  if constexpr (KB != 0) M2 = fmaxf(M2, fmaxf(new_s[0], new_s[1]));
   __syncthreads();
   s_w[tid] = (tid < A.S && pmv > -1e29f) ? exp2f(pmv - M2) * plv : 0.f;
   __syncthreads();
@@ -486,6 +531,13 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A) {
   float o = 0.f, L = 0.f;
 #pragma unroll
   for (int k = 0; k < 8; ++k) { o += s_o[k][tid]; L += s_wsum[k]; }
+  if constexpr (KB != 0) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float w = new_s[u] > -1e29f ? exp2f(new_s[u] - M2) : 0.f;
+      o += w * new_v[u]; L += w;
+    }
+  }
   float y = L > 0.f ? __fdiv_rn(o, L) : 0.f;
   if (A.unrot) y = rotate256(y, s_w, true);        // inverse of the rotation of the V rows (src/q35_kernels.cu:1421); s_w is free again
   A.out16[((size_t)tok * A.n_heads + head) * kD2 + tid] = A.out_bf16 ? f2bf_bits(y) : __half_as_ushort(__float2half_rn(y));
@@ -506,15 +558,26 @@ void launch_attend256(const AttnArgs& A, hipStream_t st) {
 }
 void launch_combine256(const CombineArgs& A, hipStream_t st) {
   if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most): half of them with 2 streams
-    if (A.M < 8) hipLaunchKernelGGL((combine256_kernel<16, true>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-    else hipLaunchKernelGGL((combine256_kernel<4, true>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    if (A.M < 8) hipLaunchKernelGGL((combine256_kernel<16, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
+    else hipLaunchKernelGGL((combine256_kernel<4, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
     return;
   }
   // 8 split lanes x kInFlight rows each must cover the S <= 256 splits
-  if (A.S > 128) hipLaunchKernelGGL((combine256_kernel<32, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else if (A.S > 64) hipLaunchKernelGGL((combine256_kernel<16, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else if (A.S > 32) hipLaunchKernelGGL((combine256_kernel<8, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else hipLaunchKernelGGL((combine256_kernel<4, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  if (A.S > 128) hipLaunchKernelGGL((combine256_kernel<32, false, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
+  else if (A.S > 64) hipLaunchKernelGGL((combine256_kernel<16, false, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
+  else if (A.S > 32) hipLaunchKernelGGL((combine256_kernel<8, false, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
+  else hipLaunchKernelGGL((combine256_kernel<4, false, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
+}
+template <int KB>
+static void launch_combine_new(const CombineArgs& A, const TbAttnArgs& N, hipStream_t st) {
+  const dim3 grid(A.n_heads, A.M);
+  const NewKeyArgs<KB> X{N};
+  if (A.S > 128) hipLaunchKernelGGL((combine256_kernel<32, false, KB>), grid, dim3(256), 0, st, A, X);
+  else if (A.S > 64) hipLaunchKernelGGL((combine256_kernel<16, false, KB>), grid, dim3(256), 0, st, A, X);
+  else hipLaunchKernelGGL((combine256_kernel<8, false, KB>), grid, dim3(256), 0, st, A, X);
+}
+void launch_combine256_new(const CombineArgs& A, const TbAttnArgs& N, int kb, hipStream_t st) {
+  if (kb == 4) launch_combine_new<4>(A, N, st); else launch_combine_new<5>(A, N, st);
 }
 void launch_export_rows256(const KvView& kv, int pos0, int n, uint32_t* kw, float* ks, uint32_t* vw, float* vs, hipStream_t st) {
   hipLaunchKernelGGL(xfer256_kernel<false>, dim3(n, kv.n_kv), dim3(64), 0, st, kv, pos0, n, kw, ks, vw, vs);

@@ -17,6 +17,7 @@
 // blocks.  3-bit fields keep a plainer form (group minima gathered through LDS, one lane walks back).
 #include "yka_internal.h"
 #include "rot256_device.h"
+#include "attend_tb_device.h"
 #include <hip/hip_fp16.h>
 
 namespace yka {
@@ -420,10 +421,10 @@ __device__ __forceinline__ void wave_chunk3(const int* xi, const int (&ci4)[4], 
   walk_back<KK, false>(best_final(cost, sid), bp, st_out);
 }
 
-// grid rows * nm, block 256: block = (row, multiplier); wave c = chunk c.  Writes the 256 states of the row under this
+// grid rows * nm, block 256: block `job` = (row, multiplier); wave c = chunk c.  Writes the 256 states of the row under this
 // multiplier and the 8 partial error sums to scratch.
 template <bool BF>
-__global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) {
+__device__ __forceinline__ void search_body(const TbEncArgs& A, const int block) {
   __shared__ float part8[8];
   __shared__ float rot_buf[256];
   __shared__ int target[256];
@@ -431,7 +432,7 @@ __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) {
   __shared__ uint8_t chosen[256];
   __shared__ int16_t table[256];
   const int d = threadIdx.x, wave = d >> 6, lane = d & 63;
-  const int row = blockIdx.x / A.nm, mult = blockIdx.x % A.nm;
+  const int row = block / A.nm, mult = block % A.nm;
   const Profile P{A.blob, A.desc, A.ngrp, A.mult_off};
   const RowRef R = locate_row<BF>(A, row, rot_buf);
   const GroupRec G = read_group(P, R.group);
@@ -466,6 +467,21 @@ __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) {
   const size_t job = (size_t)row * A.nm + mult;
   if ((d & 31) == 0) reinterpret_cast<float*>(A.scr + A.scr_w_ofs)[job * 8 + (d >> 5)] = sq;
   A.scr[job * 256 + d] = (uint8_t)state;
+}
+template <bool BF>
+__global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) { search_body<BF>(A, blockIdx.x); }
+
+// Decode (one or two tokens, no depth table): the search for the new rows' codes and the attention over the rows already in
+// the cache need nothing from each other, and neither fills the chip - 72 or 144 workgroups, each a serial chain of 64
+// steps, beside one attention workgroup per CU.  One launch runs both: the first `n_search` workgroups search, the others
+// attend to the keys in front of *d_pos.  The select launch stores the coded rows, the combiner adds them as keys of its own
+// (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 in four launches (search 9.3, select 4.7,
+// attention 12.5, combiner 4.5), 22.4 in three (13.7, 4.8, 5.3).
+template <int KB, bool BF>
+__global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(TbEncArgs E, TbAttnArgs A, int n_search) {
+  if ((int)blockIdx.x < n_search) { search_body<BF>(E, blockIdx.x); return; }
+  const int b = blockIdx.x - n_search, kvh = b / A.S;
+  tbd::attend_tb_body<KB, false>(A, b % A.S, kvh, 0, true);
 }
 
 // word d of a row's MSB-first stream of KB-bit fields: the fields that overlap bits [32 d, 32 d + 32)
@@ -624,6 +640,16 @@ void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
   }
   if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<false>, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
   hipLaunchKernelGGL(tb_select_kernel<false>, dim3(A.nrow), dim3(256), 0, st, A);
+}
+void launch_tb_encode_attend(const TbEncArgs& E, const TbAttnArgs& A, int kb, hipStream_t st) {
+  const int n_search = E.nrow * E.nm;
+  const dim3 grid(n_search + A.S * A.n_kv);
+  if (kb == 4 && E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<4, true>), grid, dim3(256), 0, st, E, A, n_search);
+  else if (kb == 4) hipLaunchKernelGGL((tb_search_attend_kernel<4, false>), grid, dim3(256), 0, st, E, A, n_search);
+  else if (E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<5, true>), grid, dim3(256), 0, st, E, A, n_search);
+  else hipLaunchKernelGGL((tb_search_attend_kernel<5, false>), grid, dim3(256), 0, st, E, A, n_search);
+  if (E.in_bf16) hipLaunchKernelGGL(tb_select_kernel<true>, dim3(E.nrow), dim3(256), 0, st, E);
+  else hipLaunchKernelGGL(tb_select_kernel<false>, dim3(E.nrow), dim3(256), 0, st, E);
 }
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t st) {

@@ -137,6 +137,8 @@ struct TbAttnArgs {
 void launch_attend_tb(const TbAttnArgs&, int kb, hipStream_t);        // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend_tb_wide(const TbAttnArgs&, int kb, hipStream_t);   // 3..64 rows: 128 query rows per workgroup, tiles decoded once into LDS
 void launch_tb_encode(const TbEncArgs&, hipStream_t);
+// one or two tokens: encoder and attention over the keys in front of *d_pos; the combiner has to add the new rows
+void launch_tb_encode_attend(const TbEncArgs&, const TbAttnArgs&, int kb, hipStream_t);
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t);
 
@@ -155,6 +157,7 @@ void launch_rotate_q256(const float* x32, int rows, uint16_t* q16, hipStream_t);
 void launch_attend256(const AttnArgs&, hipStream_t);       // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend256_wide(const AttnArgs&, hipStream_t);  // 3..64 rows: 128 query rows per workgroup, tiles dequantized once into LDS
 void launch_combine256(const CombineArgs&, hipStream_t);
+void launch_combine256_new(const CombineArgs&, const TbAttnArgs&, int kb, hipStream_t);   // the partials of launch_tb_encode_attend and the new rows
 void launch_export_rows256(const KvView&, int pos0, int n, uint32_t* kw, float* ks, uint32_t* vw, float* vs, hipStream_t);
 void launch_import_rows256(const KvView&, int pos0, int n, const uint32_t* kw, const float* ks, const uint32_t* vw, const float* vs, hipStream_t);
 // canonical <-> physical
