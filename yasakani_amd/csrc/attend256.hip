@@ -223,6 +223,12 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   const int kvh = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  uint16_t fresh_k[2] = {0, 0}, fresh_v[2] = {0, 0};       // single-stream pass: channel threadIdx.x of the rows it may have to store
+  if (!MS && A.k16) {
+    const size_t e = ((size_t)A.tok0 * A.kv.n_kv + kvh) * kD2 + threadIdx.x;
+    fresh_k[0] = request16(A.k16 + e); fresh_v[0] = request16(A.v16 + e);
+    if (A.M > 1) { const size_t e1 = e + (size_t)A.kv.n_kv * kD2; fresh_k[1] = request16(A.k16 + e1); fresh_v[1] = request16(A.v16 + e1); }
+  }
   int pos, slot = 0; bool row_ok = true;
   MsShare share{};
   if (MS) {
@@ -292,16 +298,17 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
     __shared__ float a_red[4];
     __shared__ uint8_t a_fld[256];
     bool mine = false;
-    for (int t = 0; t < A.M; ++t) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {              // a fused pass has at most two rows
+      if (t >= A.M) break;
       const int r = pos + A.tok0 + t;
       // A row no query row of this launch can see (a depth table may say so) lies past the last tile when it opens a new
       // one: nobody reads it now, the last workgroup in use stores it.  All conditions are uniform over the workgroup.
       const bool held = (r >> 5) >= tile0 && (r >> 5) < tile1, unseen = (r >> 5) >= ntiles && split == s_used - 1;
       if (r < 0 || r >= A.kv.max_ctx || !(held || unseen)) continue;
       mine = true;
-      const size_t e = ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD2 + threadIdx.x;
-      quant_store_row256(A.kv, kvh, r, false, row16_value(A.k16[e], A.in_bf16), threadIdx.x, a_red, a_fld);
-      quant_store_row256(A.kv, kvh, r, true, row16_value(A.v16[e], A.in_bf16), threadIdx.x, a_red, a_fld);
+      quant_store_row256(A.kv, kvh, r, false, row16_value(fresh_k[t], A.in_bf16), threadIdx.x, a_red, a_fld);
+      quant_store_row256(A.kv, kvh, r, true, row16_value(fresh_v[t], A.in_bf16), threadIdx.x, a_red, a_fld);
     }
     if (mine) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

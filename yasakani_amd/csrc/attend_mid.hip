@@ -127,6 +127,19 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
     const int tg = A.tok0 + tl;
     dep[rt] = v ? (A.depth ? (int)A.depth[tg] : tg) : -1;
   }
+  // the pass's first 16 K and 16 V rows, requested by every workgroup: the one that has to store them finds them here instead
+  // of asking for them once the position has told it so (8 rows at 32,037 tokens, 16 layers: 280 us against 289)
+  uint2 fresh[2][2] = {};
+  const int nst_max = rb == (int)gridDim.z - 1 ? A.M : min(A.M, tokb + ntok);
+  if (A.k16) {
+    const int c = tid & 15, slot = tid >> 4;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int hh = it * 16 + slot, t = hh >> 1;
+      const uint64_t* src = reinterpret_cast<const uint64_t*>(((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD + 8 * c);
+      if (t < nst_max) { fresh[it][0] = request64(src); fresh[it][1] = request64(src + 1); }
+    }
+  }
   const int pos = *A.d_pos;
   rows16_to_f16(qraw, A.in_bf16);
 #pragma unroll
@@ -168,7 +181,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
   bool stale = false;                                          // this wave's first tile holds rows this workgroup stores below
   if (A.k16) {
     const int nvis = min(A.M, tokb + ntok);                    // rows of the slice this block may read
-    const int nst = rb == (int)gridDim.z - 1 ? A.M : nvis;     // rows it stores if they are its own
+    const int nst = nst_max;                                   // rows it stores if they are its own
     const int r_lo = pos + A.tok0, r_hi = r_lo + nst - 1;
     const bool lastb = rb == (int)gridDim.z - 1;
     bool any_mine = false;                                     // uniform over the workgroup; a slice spans at most 3 tiles
@@ -182,7 +195,8 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
         for (int it = 0; it < 2; ++it) {
           const int hh = h0 + it * 16 + slot, t = hh >> 1;
           const uint16_t* src = ((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD + 8 * c;
-          rawv[it] = t < nst ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
+          if (h0 == 0) rawv[it] = make_uint4(fresh[it][0].x, fresh[it][0].y, fresh[it][1].x, fresh[it][1].y);
+          else rawv[it] = t < nst ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
         }
         rows16_to_f16(rawv, A.in_bf16);
 #pragma unroll

@@ -300,6 +300,15 @@ __device__ __forceinline__ uint64_t ms_new_rows(const RowMap& R, int M, int slot
   return __ballot(mine);
 }
 
+// A 16-bit value of a new row, requested before the position is known: whether the workgroup has to store the row is decided by
+// the position, and a load that waited for that decision would be a trip to memory of its own.  Atomic (relaxed, workgroup
+// scope: a plain load instruction) so that the compiler leaves the request where it stands instead of moving it to its use.
+__device__ __forceinline__ uint2 request64(const uint64_t* p) {
+  const uint64_t v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+}
+__device__ __forceinline__ uint16_t request16(const uint16_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+
 // start of the (page, kv head) block that holds token t
 __device__ __forceinline__ uint8_t* kv_page(const KvView& kv, int kvh, int t) {
   const int lp = t / kPageTok;
