@@ -235,10 +235,8 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
     if (A.adapt) {
       share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, split + A.S * rt);
       if (share.row < 0) return;
-      split = share.split; rt = share.row;
-    }
-    pos = A.rows.pos[rt];
-    slot = A.rows.slot[rt];
+      split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
+    } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }
     row_ok = pos >= 0 && pos < A.kv.max_ctx && slot >= 0 && slot < A.rows.n_slots;   // a bad row reads nothing and yields zeros
     A.kv = slot_view(A.kv, A.rows, row_ok ? slot : 0);
   } else {
@@ -564,8 +562,10 @@ void launch_attend256(const AttnArgs& A, hipStream_t st) {
   else hipLaunchKernelGGL(attend256_kernel<false>, dim3(A.S, A.kv.n_kv, (A.M + 1) / 2), dim3(256), 0, st, A);
 }
 void launch_combine256(const CombineArgs& A, hipStream_t st) {
-  if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most): half of them with 2 streams
-    if (A.M < 8) hipLaunchKernelGGL((combine256_kernel<16, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
+  // a stream may hold any share of the splits (256 at most, in batches of 8 * kInFlight).  5 streams of up to 3,000 tokens, us a
+  // pass: 15.2 with 16 in flight (and 198 registers), 12.4 with 4 and splits of 4 tiles.
+  if (A.rows.pos) {
+    if (A.M < 4) hipLaunchKernelGGL((combine256_kernel<8, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
     else hipLaunchKernelGGL((combine256_kernel<4, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
     return;
   }

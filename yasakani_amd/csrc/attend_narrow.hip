@@ -199,10 +199,8 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
     if (A.adapt) {
       share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, split + A.S * rt);
       if (share.row < 0) return;
-      split = share.split; rt = share.row;
-    }
-    pos = A.rows.pos[rt];
-    slot = A.rows.slot[rt];
+      split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
+    } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }
     row_ok = pos >= 0 && pos < A.kv.max_ctx && slot >= 0 && slot < A.rows.n_slots;   // a bad row reads nothing and yields zeros
     A.kv = slot_view(A.kv, A.rows, row_ok ? slot : 0);
   } else {

@@ -75,13 +75,12 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
   int pos; bool row_ok = true;
   MsShare share{};
   if (MS) {
+    int slot;
     if (A.adapt) {
       share = ms_share(A.rows, A.M, A.max_ctx, A.S * A.M, split + A.S * rt);
       if (share.row < 0) return;
-      split = share.split; rt = share.row;
-    }
-    pos = A.rows.pos[rt];
-    const int slot = A.rows.slot[rt];
+      split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
+    } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }
     row_ok = pos >= 0 && pos < A.max_ctx && slot >= 0 && slot < A.rows.n_slots;   // a bad row reads nothing and yields zeros
     const size_t off = row_ok ? (size_t)slot * A.rows.slot_bytes : 0;
     A.kpay += off; A.vpay += off;

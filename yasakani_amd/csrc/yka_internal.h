@@ -249,44 +249,48 @@ __device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n
 
 // Multi-stream pass: how the W workgroups of one kv head are shared out over the pass's M <= 64 rows.  Streams differ in
 // length, and with the same number of splits for each the workgroups of the longest set the pace: every split is given
-// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 2 and no row more than 256.  c =
+// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 4 (one per wave) and no row more than 256.  c =
 // (tiles of all rows) / (W - M) always fits, since every row may round up by one; four halvings look for a smaller one.
 // 16 streams of 2,000 to 32,000 tokens: 36.7 us a pass with 16 splits each (the longest stream's workgroups walk 62 tiles,
 // the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.  Row t's splits are
 // workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by every wave from the
 // row map (lane t looks at row t), again by the combiner: whole numbers, so that both agree.
-struct MsShare { int row, split, n; size_t base; };
-__device__ __forceinline__ int ms_row_tiles(const RowMap& R, int t, int max_ctx) {      // 0: a row that names no container or position
-  const int pos = R.pos[t], slot = R.slot[t];
-  return pos >= 0 && pos < max_ctx && slot >= 0 && slot < R.n_slots ? (pos + 32) >> 5 : 0;
+// The sums run through lane-crossing moves (a shift inside rows of 16 lanes, then two row broadcasts), not through LDS: this
+// stands in front of everything else a workgroup does (5 trellis streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128
+// channels 14.9 and 13.9).
+template <class Op>
+__device__ __forceinline__ int wave_scan(int v, Op op) {            // inclusive over the lanes; 0 is the neutral value
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));        // row_shr:1, 2, 4, 8
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));        // row_bcast:15 into rows 1 and 3
+  return op(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));     // row_bcast:31 into rows 2 and 3
 }
-struct MsPlan { int mine, incl; };                 // of row `lane`: its splits, and the splits up to and including it
+__device__ __forceinline__ int wave_scan_add(int v) { return wave_scan(v, [](int a, int b) { return a + b; }); }
+struct MsShare { int row, split, n, pos, slot; size_t base; };
+struct MsPlan { int mine, incl, pos, slot; };      // of row `lane`: its splits, the splits up to and including it, its place
 __device__ __forceinline__ MsPlan ms_plan(const RowMap& R, int M, int max_ctx, int W) {
-  const int lane = threadIdx.x & 63, tiles = lane < M ? ms_row_tiles(R, lane, max_ctx) : 0;
-  int total = tiles, most = tiles;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) { total += __shfl_xor(total, o, 64); most = max(most, __shfl_xor(most, o, 64)); }
-  int lo = max(2, max((most + 255) >> 8, (total + W - 1) / W)), c = max(lo, (total + W - M - 1) / (W - M));
-  int mine = (tiles + c - 1) / c;
+  const int lane = threadIdx.x & 63, pos = lane < M ? R.pos[lane] : -1, slot = lane < M ? R.slot[lane] : -1;
+  // 0 tiles: a row that names no container or position
+  const int tiles = pos >= 0 && pos < max_ctx && slot >= 0 && slot < R.n_slots ? (pos + 32) >> 5 : 0;
+  const int total = __builtin_amdgcn_readlane(wave_scan_add(tiles), 63);
+  const int most = __builtin_amdgcn_readlane(wave_scan(tiles, [](int a, int b) { return max(a, b); }), 63);
+  int lo = max(4, max((most + 255) >> 8, (total + W - 1) / W)), c = max(lo, (total + W - M - 1) / (W - M));
+  int mine = (tiles + c - 1) / c, incl = wave_scan_add(mine);
   for (int it = 0; it < 4 && lo < c; ++it) {       // c always fits; a smaller one may
-    const int mid = (lo + c) >> 1, want = (tiles + mid - 1) / mid;
-    int sum = want;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
-    if (__builtin_amdgcn_readfirstlane(sum) <= W) { c = mid; mine = want; } else lo = mid + 1;
+    const int mid = (lo + c) >> 1, want = (tiles + mid - 1) / mid, sum = wave_scan_add(want);
+    if (__builtin_amdgcn_readlane(sum, 63) <= W) { c = mid; mine = want; incl = sum; } else lo = mid + 1;
   }
-  int incl = mine;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) { const int up = __shfl_up(incl, o, 64); incl += lane >= o ? up : 0; }
-  return {mine, incl};
+  return {mine, incl, pos, slot};
 }
 // workgroup b of the kv head; row = -1: nothing left for it
 __device__ __forceinline__ MsShare ms_share(const RowMap& R, int M, int max_ctx, int W, int b) {
   const MsPlan P = ms_plan(R, M, max_ctx, W);
   const int row = __popcll(__ballot(P.incl <= b));
-  if (row >= M) return {-1, 0, 0, 0};
+  if (row >= M) return {-1, 0, 0, 0, 0, 0};
   const int n = __builtin_amdgcn_readlane(P.mine, row), base = __builtin_amdgcn_readlane(P.incl, row) - n;
-  return {row, b - base, n, (size_t)base};
+  return {row, b - base, n, __builtin_amdgcn_readlane(P.pos, row), __builtin_amdgcn_readlane(P.slot, row), (size_t)base};
 }
 
 // Multi-stream pass of at most 64 rows whose attention launch stores the new rows itself: the rows of the pass (bit t = row
