@@ -221,42 +221,8 @@ __device__ __forceinline__ uint4 pack_out8(const float* y, int bf16) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Splits a slice of a prefill chunk uses, of the `S` its launch provides for.  The host sizes the grid without knowing the
-// position, so the choice is made on the device, by every wave of the attention launch and again by the combiner: lane s - 1
-// prices s splits, the cheapest wins (ties: the fewest).  Whole numbers only, so that two compilations cannot disagree.
-// Times are in sixteenths of the time a workgroup takes for one 32-key tile (0.56 us): a workgroup costs kChunkOverhead
-// tiles before and after its loop (about 10 us: launch, query, first tile, merge, stores), one workgroup runs per CU, the
-// longest start first, and more than one split costs a combiner pass over M * s partial rows.
-// 1,500 rows on an empty cache in containers of 8,192 tokens, us per layer call: 105 with slices of 1,024 tokens in 4 and 8
-// splits (39 + 39 in the attention, 23 in the combiners), 48 with one split (44 in the attention, which then waits for its
-// longest workgroup: 47 tiles).  2,048 rows behind 131,072: the same with 2 splits of one slice as with 4 of two.
-constexpr int kChunkOverhead = 18, kChunkMaxSplits = 64;
-__device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n_kv, int max_ctx, int S) {
-  const int base = n_kv * ((kG * M + 127) / 128), s = (int)(threadIdx.x & 63) + 1;
-  const int first = max(0, min(pos + tok0 + min(M, 128 / kG + 1), max_ctx)), last = max(0, min(pos + tok0 + M, max_ctx));
-  const int lo = ((first + 31) >> 5) * 16 / s + 16 * kChunkOverhead, hi = ((last + 31) >> 5) * 16 / s + 16 * kChunkOverhead;
-  const int n = base * s, idle = (256 - (n & 255)) & 255;            // workgroups, and CUs without one in the last round
-  int t = max(hi, (n >> 1) * (lo + hi) / 256 + lo * idle / 256);
-  if (s > 1) t += 96 + M * s / 13;
-  int best = s <= S ? t : 0x7fffffff, at = s;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int bt = __shfl_xor(best, o, 64), ba = __shfl_xor(at, o, 64);
-    if (bt < best || (bt == best && ba < at)) { best = bt; at = ba; }
-  }
-  return __builtin_amdgcn_readfirstlane(at);
-}
-
-// Multi-stream pass: how the W workgroups of one kv head are shared out over the pass's M <= 64 rows.  Streams differ in
-// length, and with the same number of splits for each the workgroups of the longest set the pace: every split is given
-// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 4 (one per wave) and no row more than 256.  c =
-// (tiles of all rows) / (W - M) always fits, since every row may round up by one; four halvings look for a smaller one.
-// 16 streams of 2,000 to 32,000 tokens: 36.7 us a pass with 16 splits each (the longest stream's workgroups walk 62 tiles,
-// the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.  Row t's splits are
-// workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by every wave from the
-// row map (lane t looks at row t), again by the combiner: whole numbers, so that both agree.
-// The sums run through lane-crossing moves (a shift inside rows of 16 lanes, then two row broadcasts), not through LDS: this
-// stands in front of everything else a workgroup does (5 trellis streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128
+// Sums and maxima of the plans below run through lane-crossing moves (a shift inside rows of 16 lanes, then two row broadcasts),
+// not through LDS: a plan stands in front of everything else a workgroup does (multi-stream passes, 5 trellis streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128
 // channels 14.9 and 13.9).
 template <class Op>
 __device__ __forceinline__ int wave_scan(int v, Op op) {            // inclusive over the lanes; 0 is the neutral value
@@ -268,6 +234,38 @@ __device__ __forceinline__ int wave_scan(int v, Op op) {            // inclusive
   return op(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));     // row_bcast:31 into rows 2 and 3
 }
 __device__ __forceinline__ int wave_scan_add(int v) { return wave_scan(v, [](int a, int b) { return a + b; }); }
+
+// Splits a slice of a prefill chunk uses, of the `S` its launch provides for.  The host sizes the grid without knowing the
+// position, so the choice is made on the device, by every wave of the attention launch and again by the combiner: lane s - 1
+// prices s splits, the cheapest wins (ties: the fewest).  Whole numbers only, so that two compilations cannot disagree.
+// Times are in sixteenths of the time a workgroup takes for one 32-key tile (0.56 us): a workgroup costs kChunkOverhead
+// tiles before and after its loop (about 10 us: launch, query, first tile, merge, stores), one workgroup runs per CU, the
+// longest start first, and more than one split costs a combiner pass over M * s partial rows.
+// 1,500 rows on an empty cache in containers of 8,192 tokens, us per layer call: 105 with slices of 1,024 tokens in 4 and 8
+// splits (39 + 39 in the attention, 23 in the combiners), 46 with one split (42 in the attention, which then waits for its
+// longest workgroup: 47 tiles; 48 and 44 while the choice went through LDS).  2,048 rows behind 131,072: the same with 2 splits of one slice as with 4 of two.
+constexpr int kChunkOverhead = 18, kChunkMaxSplits = 64;
+__device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n_kv, int max_ctx, int S) {
+  const int base = n_kv * ((kG * M + 127) / 128), s = (int)(threadIdx.x & 63) + 1;
+  const int first = max(0, min(pos + tok0 + min(M, 128 / kG + 1), max_ctx)), last = max(0, min(pos + tok0 + M, max_ctx));
+  const int lo = ((first + 31) >> 5) * 16 / s + 16 * kChunkOverhead, hi = ((last + 31) >> 5) * 16 / s + 16 * kChunkOverhead;
+  const int n = base * s, idle = (256 - (n & 255)) & 255;            // workgroups, and CUs without one in the last round
+  int t = max(hi, (n >> 1) * (lo + hi) / 256 + lo * idle / 256);
+  if (s > 1) t += 96 + M * s / 13;
+  // lowest price, then fewest splits: the largest key (lane 0 always has one)
+  const int key = s <= S ? 0x7fffffff - ((max(0, min(t, 0x1fffffe)) << 6) | (s - 1)) : 0;
+  const int top = __builtin_amdgcn_readlane(wave_scan(key, [](int a, int b) { return max(a, b); }), 63);
+  return ((0x7fffffff - top) & 63) + 1;
+}
+
+// Multi-stream pass: how the W workgroups of one kv head are shared out over the pass's M <= 64 rows.  Streams differ in
+// length, and with the same number of splits for each the workgroups of the longest set the pace: every split is given
+// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 4 (one per wave) and no row more than 256.  c =
+// (tiles of all rows) / (W - M) always fits, since every row may round up by one; four halvings look for a smaller one.
+// 16 streams of 2,000 to 32,000 tokens: 36.7 us a pass with 16 splits each (the longest stream's workgroups walk 62 tiles,
+// the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.  Row t's splits are
+// workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by every wave from the
+// row map (lane t looks at row t), again by the combiner: whole numbers, so that both agree.
 struct MsShare { int row, split, n, pos, slot; size_t base; };
 struct MsPlan { int mine, incl, pos, slot; };      // of row `lane`: its splits, the splits up to and including it, its place
 __device__ __forceinline__ MsPlan ms_plan(const RowMap& R, int M, int max_ctx, int W) {
