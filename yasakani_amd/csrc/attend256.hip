@@ -45,8 +45,7 @@ __device__ __forceinline__ uint8_t* page256(const KvView& kv, int kvh, int t) {
 // all 256 threads of a workgroup (three barriers inside); red[4] and fld[256] are its LDS scratch.
 __device__ __forceinline__ void quant_store_row256(const KvView& kv, int kvh, int pos, bool isv, float x, int d, float* red, uint8_t* fld) {
   float am = fabsf(x);
-#pragma unroll
-  for (int o = 32; o; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
+  am = lane_rows(lane_row16(am, LaneMax{}), LaneMax{});
   __syncthreads();                               // the scratch of a previous row is no longer read
   if ((d & 63) == 0) red[d >> 6] = am;
   __syncthreads();
@@ -252,8 +251,7 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
     len = min(len, A.kv.max_ctx);
   }
   int maxlen = len, minlen = vrow ? len : 0x7fffffff;
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) { maxlen = max(maxlen, __shfl_xor(maxlen, o, 64)); minlen = min(minlen, __shfl_xor(minlen, o, 64)); }
+  maxlen = lane_row16(maxlen, LaneMax{}); minlen = lane_row16(minlen, LaneMin{});
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
   // as many of the launched splits as the length found on the device justifies (two 32-key tiles per workgroup at
   // least); the others leave the "no keys" marker, whose rows the combiner does not read
@@ -381,8 +379,7 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
     float tmax = s[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, s[e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    tmax = lane_rows(tmax, LaneMax{});
     const float m_new = fmaxf(m_run, tmax * sc_log2);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     const bool first = m_run < -1e29f;
@@ -503,8 +500,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   float pmv = -1e30f, plv = 0.f;
   if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
   float M2 = pmv;
-#pragma unroll
-  for (int o = 32; o; o >>= 1) M2 = fmaxf(M2, __shfl_xor(M2, o, 64));
+  M2 = lane_rows(lane_row16(M2, LaneMax{}), LaneMax{});
   if ((tid & 63) == 0) s_wsum[tid >> 6] = M2;
   __syncthreads();
   M2 = fmaxf(fmaxf(s_wsum[0], s_wsum[1]), fmaxf(s_wsum[2], s_wsum[3]));

@@ -130,8 +130,7 @@ __device__ __forceinline__ void quant_store_word256(const KvView& kv, int kvh, i
   float am = fabsf(x[0]);
 #pragma unroll
   for (int e = 1; e < 8; ++e) am = fmaxf(am, fabsf(x[e]));
-#pragma unroll
-  for (int o = 1; o < 32; o <<= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
+  am = lane_op16(lane_row16(am, LaneMax{}), LaneMax{});
   float s7 = __fdiv_rn(am, 7.f);
   if (s7 == 0.f) s7 = 1.f;
   uint32_t word = 0u;                          // channel 8c + e in bits [28 - 4e, 32 - 4e): the first field on top
@@ -302,8 +301,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
       for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, s[e]);
       tmax *= sc_log2;
       if (__any(tmax > m_run + kRaise)) {
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        tmax = lane_rows(tmax, LaneMax{});
         const float m_new = fmaxf(m_run, tmax);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new; l_run *= alpha;
@@ -342,8 +340,7 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   constexpr int kOPitch = 2 * kD2 + 16;                      // bytes per staged row
   uint8_t* stage = &lds[0][0] + wave * 16 * kOPitch;         // 8 waves x 8448 bytes of the 84480
   float l = l_run;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = lane_rows(l, LaneAdd{});
   const size_t pidx = ((size_t)tl * A.S + split) * A.n_heads + head;
   if (vrow && g == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
   const float inv = l > 0.f ? 1.f / l : 0.f;

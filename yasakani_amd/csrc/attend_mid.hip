@@ -156,8 +156,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
     maxlen = max(maxlen, lenr[rt]);
     if (dep[rt] >= 0) minlen = min(minlen, lenr[rt]);
   }
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) { maxlen = max(maxlen, __shfl_xor(maxlen, o, 64)); minlen = min(minlen, __shfl_xor(minlen, o, 64)); }
+  maxlen = lane_row16(maxlen, LaneMax{}); minlen = lane_row16(minlen, LaneMin{});
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
 
   // The grid is sized for the context the caller expects.  A workgroup none of whose waves has a tile (short contexts)
@@ -343,8 +342,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
       // 2^kRaiseMid (or on the row's first keys), so the accumulators are rescaled on almost no tile
       float tmax = fmaxf(fmaxf(fmaxf(e[0], e[1]), fmaxf(e[2], e[3])), fmaxf(fmaxf(e[4], e[5]), fmaxf(e[6], e[7])));
       if (__any(tmax > (first ? -INFINITY : kRaiseMid))) {
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        tmax = lane_rows(tmax, LaneMax{});
         const bool seen = tmax > -INFINITY;      // false: every key of the tile lies past the row's length
         const float d = first ? (seen ? tmax : 0.f) : fmaxf(tmax, 0.f);
         const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-d);
@@ -415,8 +413,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
   //      one normalised fp16 partial row piece.  o[rt][b][r] of lane (row i, group g) is channel 8 (4g + r) + b. ----
   auto stage = [&](int rt) __attribute__((always_inline)) {
     float l = l_run[rt];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = lane_rows(l, LaneAdd{});
     if (g == 0) { s_m[rt][wave][i] = m_run[rt]; s_l[rt][wave][i] = l; }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {

@@ -155,7 +155,7 @@ __device__ __forceinline__ void combine_column(const AttnArgs& A, int kvh, int r
         }
         // the wave's 4 split lanes (lane bits 4 and 5), then the 4 waves through LDS
 #pragma unroll
-        for (int c = 0; c < 8; ++c) { acc[c] += __shfl_xor(acc[c], 16, 64); acc[c] += __shfl_xor(acc[c], 32, 64); }
+        for (int c = 0; c < 8; ++c) acc[c] = lane_rows(acc[c], LaneAdd{});
         if ((tid & 48) == 0) {
           float* d = s_o + (wave * kG + h0 + hh) * kD + c8;
           *reinterpret_cast<float4*>(d) = make_float4(acc[0], acc[1], acc[2], acc[3]);
@@ -218,8 +218,7 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
     len = min(len, A.kv.max_ctx);
   }
   int maxlen = len, minlen = vrow ? len : 0x7fffffff;
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) { maxlen = max(maxlen, __shfl_xor(maxlen, o, 64)); minlen = min(minlen, __shfl_xor(minlen, o, 64)); }
+  maxlen = lane_row16(maxlen, LaneMax{}); minlen = lane_row16(minlen, LaneMin{});
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
   // The grid is sized for long contexts; how many of its splits a row tile uses follows from the length it finds on the
   // device: at least two 32-key tiles per workgroup.  The other workgroups leave the "no keys" marker and exit, and
@@ -317,8 +316,7 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
       float qs = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) qs += (float)c[e];
-      qs += __shfl_xor(qs, 16, 64);
-      qs += __shfl_xor(qs, 32, 64);
+      qs = lane_rows(qs, LaneAdd{});
       const float c0 = -32.f * kTwoM24 * qs;       // -8 per code, in the units of the products: 4 q n 2^-24
       kinit[m] = f4{c0, c0, c0, c0};
     }
@@ -371,8 +369,7 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
     float tmax = s[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, s[e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    tmax = lane_rows(tmax, LaneMax{});
     const float m_new = fmaxf(m_run, tmax * sc_log2);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);    // 0 on the first tile (m_run = -1e30): nothing to rescale yet
     const bool first = m_run < -1e29f;
@@ -450,8 +447,7 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
     }
   }
   // ---- merge the 4 waves of the workgroup, write one partial per (row, split) ----
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = lane_rows(l_run, LaneAdd{});
   if (g == 0) { s_m[wave][i] = m_run; s_l[wave][i] = l_run; }
   // o[b][r] of lane (row i, group g) is channel 8 (4g + r) + b: eight consecutive channels per r, two 16-byte writes
 #pragma unroll
@@ -548,8 +544,7 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   float pmv = -1e30f, plv = 0.f;
   if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
   float M2 = pmv;
-#pragma unroll
-  for (int o = 32; o; o >>= 1) M2 = fmaxf(M2, __shfl_xor(M2, o, 64));
+  M2 = lane_rows(lane_row16(M2, LaneMax{}), LaneMax{});
   if ((tid & 63) == 0) s_wsum[tid >> 6] = M2;
   __syncthreads();
   M2 = fmaxf(fmaxf(s_wsum[0], s_wsum[1]), fmaxf(s_wsum[2], s_wsum[3]));
@@ -627,8 +622,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
   float pmv = -1e30f, plv = 0.f;
   if (lane < A.S) { pmv = A.pm[p0 + (size_t)lane * A.n_heads]; plv = A.pl[p0 + (size_t)lane * A.n_heads]; }
   float M2 = pmv;
-#pragma unroll
-  for (int o = 32; o; o >>= 1) M2 = fmaxf(M2, __shfl_xor(M2, o, 64));
+  M2 = lane_rows(lane_row16(M2, LaneMax{}), LaneMax{});
   const float wl = (lane < A.S && pmv > -1e29f) ? exp2f(pmv - M2) * plv : 0.f;     // weight of split `lane`
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float wsum = 0.f;
@@ -643,8 +637,8 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
     wsum += w;
   }
 #pragma unroll
-  for (int c = 0; c < 8; ++c) { acc[c] += __shfl_xor(acc[c], 16, 64); acc[c] += __shfl_xor(acc[c], 32, 64); }
-  wsum += __shfl_xor(wsum, 16, 64); wsum += __shfl_xor(wsum, 32, 64);
+  for (int c = 0; c < 8; ++c) acc[c] = lane_rows(acc[c], LaneAdd{});
+  wsum = lane_rows(wsum, LaneAdd{});
   if (sl == 0) {
     const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
     float yv[8];

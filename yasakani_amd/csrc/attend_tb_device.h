@@ -100,8 +100,7 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
     len = min(len, A.max_ctx);
   }
   int maxlen = len, minlen = vrow ? len : 0x7fffffff;
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) { maxlen = max(maxlen, __shfl_xor(maxlen, o, 64)); minlen = min(minlen, __shfl_xor(minlen, o, 64)); }
+  maxlen = lane_row16(maxlen, LaneMax{}); minlen = lane_row16(minlen, LaneMin{});
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
   const int ntiles = (maxlen + 31) >> 5;
   const int s_used = MS && A.adapt ? share.n : min(A.S, max(1, ntiles >> 1));
@@ -244,8 +243,7 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
     float tmax = s[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, s[e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    tmax = lane_rows(tmax, LaneMax{});
     const float m_new = fmaxf(m_run, tmax * sc_log2);          // the table's gain is positive (checked when the profile is set)
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     const bool first_tile = m_run < -1e29f;

@@ -269,8 +269,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
       for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, s[e]);
       tmax *= sc_log2;
       if (__any(tmax > m_run + kRaise)) {
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        tmax = lane_rows(tmax, LaneMax{});
         const float m_new = fmaxf(m_run, tmax);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new; l_run *= alpha;
@@ -309,8 +308,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   constexpr int kOPitch = 2 * kD2 + 16;                      // bytes per staged row
   uint8_t* stage = &lds[0][0] + wave * 16 * kOPitch;         // 8 waves x 8448 bytes of the 84480
   float l = l_run;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = lane_rows(l, LaneAdd{});
   const size_t pidx = ((size_t)tl * A.S + split) * A.n_heads + head;
   if (vrow && g == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
   const float inv = l > 0.f ? A.gfac[gV] / l : 0.f;          // gain / 256 of the V table joins the normalisation

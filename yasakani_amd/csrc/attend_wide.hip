@@ -395,7 +395,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
       if (__any(tmax > (first ? -INFINITY : kRaise))) {
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        tmax = lane_op32(tmax, LaneMax{});
         const bool seen = tmax > -INFINITY;                       // false: every key of the tile lies past the row's length
         const float d = first ? (seen ? tmax : 0.f) : fmaxf(tmax, 0.f);
         const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-d);   // a first tile finds zeros in l and o
@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");     // the image has been read before the wave overwrites it
   uint8_t* stage = &lds[0][0][0] + wave * (64 * 64 * 4);     // 4 waves x 8704 bytes, 16384 bytes apart
   float l = l_run;
-  l += __shfl_xor(l, 32, 64);
+  l = lane_op32(l, LaneAdd{});
   const bool direct = CHUNK && A.S == 1 && A.out16;          // uniform over the grid
   if (!direct && vrow && h == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
   const float inv = l > 0.f ? 1.f / l : 0.f;

@@ -17,8 +17,7 @@ __device__ __forceinline__ int k_code_byte(int j) { return 4 * k_phys_dword(j >>
 // one lane = one channel; lanes of a 32-lane half-wave form one scale group
 __device__ __forceinline__ void quant_lane(float x, int& code, uint16_t& s16) {
   float am = fabsf(x);
-#pragma unroll
-  for (int o = 16; o; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 32));
+  am = lane_op16(lane_row16(am, LaneMax{}), LaneMax{});
   const float s32 = __fdiv_rn(am, 7.0f);
   s16 = __half_as_ushort(__float2half_rn(s32));
   if ((s16 & 0x7fffu) == 0) s16 = 0x3c00u;
@@ -38,7 +37,7 @@ __device__ __forceinline__ void quant_store_row(const KvView& kv, int kvh, int p
 __device__ __forceinline__ void quant_store_value(const KvView& kv, int kvh, int pos, bool isv, float x, int d) {
   int code; uint16_t s16;
   quant_lane(x, code, s16);
-  const int nb = __shfl_xor(code, 1, 64);
+  const int nb = lane_xor1(code);
   uint8_t* pg = kv_page(kv, kvh, pos);
   const int tp = pos % kPageTok;
   if ((d & 1) == 0) {
@@ -63,8 +62,8 @@ __device__ __forceinline__ void quant_store_chunk8(const KvView& kv, int kvh, in
   float am = fabsf(x[0]);
 #pragma unroll
   for (int e = 1; e < 8; ++e) am = fmaxf(am, fabsf(x[e]));
-  am = fmaxf(am, __shfl_xor(am, 1, 64));
-  am = fmaxf(am, __shfl_xor(am, 2, 64));
+  am = fmaxf(am, lane_xor1(am));
+  am = fmaxf(am, lane_xor2(am));
   const float s32 = __fdiv_rn(am, 7.0f);
   uint16_t s16 = __half_as_ushort(__float2half_rn(s32));
   if ((s16 & 0x7fffu) == 0) s16 = 0x3c00u;

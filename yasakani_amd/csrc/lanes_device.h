@@ -1,0 +1,53 @@
+// Exchanges between lanes without LDS (gfx950): a __shfl is an LDS instruction with its round trip, on the critical path of a wave
+// that has its SIMD to itself (the decode kernels); a DPP move or a row / half swap is one or two vector instructions.
+// 16 layers of one token, 128 channels: 1,003 tokens 121 -> 113 us, 8,003 127 -> 122, 32,741 178 -> 171; 256 channels at 9,000
+// 177 -> 169; 4 rows at 2,003 tokens 170 -> 162, 64 rows 345 -> 335.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace yka {
+
+typedef unsigned lanes_u32x2 __attribute__((ext_vector_type(2)));
+
+// the value a DPP control names, every lane valid
+template <int CTRL, class T>
+__device__ __forceinline__ T lane_dpp(T v) {
+  static_assert(sizeof(T) == 4, "one register");
+  const int b = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(b, b, CTRL, 0xf, 0xf, false));
+}
+template <class T> __device__ __forceinline__ T lane_xor1(T v) { return lane_dpp<0xB1>(v); }     // quad_perm [1,0,3,2]
+template <class T> __device__ __forceinline__ T lane_xor2(T v) { return lane_dpp<0x4E>(v); }     // quad_perm [2,3,0,1]
+template <class T> __device__ __forceinline__ T lane_xor8(T v) { return lane_dpp<0x128>(v); }    // row_ror:8
+// op(v, v of lane ^ 16) and op(v, v of lane ^ 32): after swapping a register with a copy of itself the two results hold, in
+// every lane, the values of the lane and of its partner (op commutes)
+template <class T, class Op>
+__device__ __forceinline__ T lane_op16(T v, Op op) {
+  const unsigned b = __builtin_bit_cast(unsigned, v);
+  const lanes_u32x2 r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const unsigned r0 = r[0], r1 = r[1];
+  return op(__builtin_bit_cast(T, r0), __builtin_bit_cast(T, r1));
+}
+template <class T, class Op>
+__device__ __forceinline__ T lane_op32(T v, Op op) {
+  const unsigned b = __builtin_bit_cast(unsigned, v);
+  const lanes_u32x2 r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  const unsigned r0 = r[0], r1 = r[1];
+  return op(__builtin_bit_cast(T, r0), __builtin_bit_cast(T, r1));
+}
+struct LaneMax { template <class T> __device__ __forceinline__ T operator()(T a, T b) const { if constexpr (__is_same(T, float)) return fmaxf(a, b); else return a > b ? a : b; } };
+struct LaneMin { __device__ __forceinline__ int operator()(int a, int b) const { return a < b ? a : b; } };
+struct LaneAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
+// over the four lanes l, l ^ 16, l ^ 32, l ^ 48
+template <class T, class Op> __device__ __forceinline__ T lane_rows(T v, Op op) { return lane_op32(lane_op16(v, op), op); }
+// over a row of 16 lanes; op is a maximum or minimum (after two steps a quad holds one value, so the mirrored octet is lane ^ 4)
+template <class T, class Op>
+__device__ __forceinline__ T lane_row16(T v, Op op) {
+  v = op(v, lane_xor1(v));
+  v = op(v, lane_xor2(v));
+  v = op(v, lane_dpp<0x141>(v));                   // row_half_mirror
+  return op(v, lane_xor8(v));
+}
+
+}  // namespace yka

@@ -24,8 +24,7 @@ __device__ __forceinline__ void merge_waves256(const V4 (&o)[16], float m_run, f
                                                const float* mu, float (*s_m)[16], float (*s_l)[16], float (*s_wn)[4], float* s_acc,
                                                float* pm, float* pl, uint16_t* pacc16, PairOf pair_of) {
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = lane_rows(l_run, LaneAdd{});
   if (g == 0) { s_m[wave][i] = m_run; s_l[wave][i] = l_run; }
   if (i < rows) {
     float* const d = s_acc + wave * m256_wave<ROWS>() + m256_row(i);
@@ -44,12 +43,12 @@ __device__ __forceinline__ void merge_waves256(const V4 (&o)[16], float m_run, f
   if (threadIdx.x < 64) {
     const int j = threadIdx.x >> 2, w = threadIdx.x & 3;
     const float mw = s_m[w][j];
-    float M2 = fmaxf(mw, __shfl_xor(mw, 1, 64));
-    M2 = fmaxf(M2, __shfl_xor(M2, 2, 64));
+    float M2 = fmaxf(mw, lane_xor1(mw));
+    M2 = fmaxf(M2, lane_xor2(M2));
     const float ww = exp2f(mw - M2);
     float L = ww * s_l[w][j];
-    L += __shfl_xor(L, 1, 64);
-    L += __shfl_xor(L, 2, 64);
+    L += lane_xor1(L);
+    L += lane_xor2(L);
     s_wn[j][w] = L > 0.f ? ww * factor / L : 0.f;
     if (w == 0 && j < rows) {
       const size_t p = pair_of(j) * n_heads + kvh * kG + j % kG;
