@@ -81,7 +81,7 @@ YKA_API const char* yka_build_info(void);
  *        tiles; 128-channel rows only).  0 = never, at most 64 (wider windows than 16 rows then run as blocks of 16
  *        tokens).  Default 10: measured faster than the 128-row workgroups of the wide kernel up to there;
  * key 9: split count of that kernel (0 = automatic);
- * key 10: tokens per prefill slice (passes wider than 64 rows), 0 = 1024; 128 .. 4096;
+ * key 10: tokens per prefill slice (passes wider than 64 rows), 0 = 2048; 128 .. 4096;
  * key 11: 16-bit row type at the boundary: 0 = fp16 (default), 1 = bf16, the type of the reference's activations
  *        (q35_kernels.cu:1048,1062: Q, gate and attention outputs are bf16 there).  With 1, d_q16 / d_k16 / d_v16 of every
  *        entry point are bf16 and are converted to fp16 by the kernels that read them (round to nearest; exact for
@@ -114,8 +114,8 @@ YKA_API int yka_attend(yka_kv* kv, int layer, const uint16_t* d_q16, int M, cons
  * Engine35::attn_block (engine35.cpp:911-934).  The rows are quantized inside the attention launches (each 64-row
  * slice stores its own rows before it reads them; bit-identical to yka_append), so a layer call is two launches:
  * attention and the split combiner.  M may be as large as max_rows; a pass wider than 64 rows is a prefill chunk: its rows
- * are appended by one launch, then slices of up to 1024 tokens (option key 10) run through the wide kernel, one attention
- * and one combiner launch per slice (attn_block cuts such passes into 64-row slices, engine35.cpp:935-947). */
+ * are appended by one launch, then slices of up to 2048 tokens (option key 10; 256-channel rows: 1024) run through the wide kernel, one
+ * attention and one combiner launch per slice (attn_block cuts such passes into 64-row slices, engine35.cpp:935-947). */
 YKA_API int yka_append_attend(yka_kv* kv, int layer, const uint16_t* d_q16, const uint16_t* d_k16,
                               const uint16_t* d_v16, int M, const int* d_pos, const uint8_t* d_depth,
                               uint16_t* d_out16, void* hip_stream);
