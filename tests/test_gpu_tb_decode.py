@@ -37,3 +37,27 @@ def test_against_the_general_path(native, kk, M, ctx, opts):
     assert np.isfinite(out).all()
     # the same codes; the general path rounds P (times the V scale) and its partials to fp16, both round the output (bf16: 2^-8 each)
     assert np.linalg.norm(out - ref) <= (1e-3 + (2 * 2.0 ** -8 if bf16 else 0)) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("kk", [4, 5])
+def test_splits_change_with_the_position(native, kk):
+    """A container of more than 98,304 tokens: half of the launched splits are in use up to that position, all beyond it."""
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(kk)
+    half = lambda n, heads: rng.standard_normal((n, heads, 256)).astype(np.float16)    # noqa: E731
+    with native.KvCache(n_layers=1, max_ctx=98304 + 512, head_dim=256, max_rows=2048) as kv:
+        kv.set_profile(kvqp.synthetic(layers=1, kk=kk, seed=11))
+        k, v = half(2048, 4), half(2048, 4)
+        for at in range(0, 98304 + 2048, 2048):
+            n = min(2048, 98304 + 300 - at)
+            kv.append_host(0, np.roll(k, at // 2048, axis=2)[:n], np.roll(v, at // 2048 + 1, axis=0)[:n], at)
+        for ctx, M in ((0, 2), (1, 1), (300, 1), (4095, 2), (98302, 2), (98303, 2), (98304, 1), (98305, 2), (98304 + 511, 1), (98304 + 510, 2)):
+            q, kn, vn = half(M, 24), half(M, 4), half(M, 4)
+            got = []
+            for splits in (0, 48):
+                kv.set_opt(1, splits)
+                kv.poison_workspace()
+                got.append(kv.layer_call(0, q, kn, vn, ctx).astype(np.float32))
+            assert np.isfinite(got[0]).all(), ctx
+            # other splits: partials and outputs rounded to fp16 once each (2^-11), sums in fp32
+            assert np.linalg.norm(got[0] - got[1]) <= 1e-3 * np.linalg.norm(got[1]), ctx

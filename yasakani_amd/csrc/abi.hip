@@ -176,14 +176,16 @@ int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
 // rows to read: 205 against 225 us for 16 layers at 20,011 tokens, 167 / 204 at 3,000, 97 / 101 for 2 layers at 200,000).
 // Of the wide ones: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
 // rounds of 256 workgroups best.
-struct Part256 { int Ms, S, rows_per_block; bool narrow; };
+struct Part256 { int Ms, S, rows_per_block; bool narrow; int s_short; };
 int slice256(const yka_kv* kv, int M) { return M > kMaxSlice && !kv->opt_force_narrow ? 1024 : kMaxSlice; }
 Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
   const int ctx = kv->opt_ctx_hint > 0 ? std::min(kv->opt_ctx_hint, kv->cfg.max_ctx) : kv->cfg.max_ctx, ctx_tiles = (ctx + 31) / 32;
   const int Ms = std::min(slice, M - s0), rows = kG * Ms, rb = (rows + 127) / 128, base = kv->cfg.n_kv_heads * rb;
   const bool narrow = Ms <= 2 || kv->opt_force_narrow;
+  // trellis decode in containers longer than kShortPos: a second workgroup per CU, used from there on (splits_at)
+  const bool two = kv->tb && Ms <= 2 && !kv->opt_splits_narrow && ctx_tiles > kShortPos / 32;
   int S;
-  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min(256 / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
+  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min((two ? 512 : 256) / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
   else if (kv->opt_splits_wide > 0) S = kv->opt_splits_wide;
   else if (Ms <= kMaxSlice) S = std::min(256 / base, ctx_tiles / (2 * rb));
   else {
@@ -196,7 +198,7 @@ Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
   }
   const size_t pairs = Ms > kMaxSlice ? kv->ws_rows : kWsPairs;
   S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(pairs / (size_t)Ms));
-  return {Ms, S, ((rows + rb - 1) / rb + 15) / 16 * 16, narrow};
+  return {Ms, S, ((rows + rb - 1) / rb + 15) / 16 * 16, narrow, two ? std::min(S, std::max(2, 256 / kv->cfg.n_kv_heads)) : 0};
 }
 
 void check_layer(const yka_kv* kv, int layer) {
@@ -284,7 +286,8 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
                    T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, layer, q16 + (size_t)s0 * NH * 256, d_pos, depth, P.Ms, s0, NH, P.S,
                    kv->pm, kv->pl, kv->pacc16, RowMap{}, bf16};
       A.rows_per_block = P.rows_per_block;
-      const CombineArgs C{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
+      CombineArgs C{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
+      A.s_short = C.s_short = P.s_short; C.d_pos = d_pos;
       if (fuse) {
         launch_tb_encode_attend(tb_encoder_args(kv, layer, layer, k16, v16, 0, M, d_pos), A, T.kb, st);
         launch_combine256_new(C, A, T.kb, st);

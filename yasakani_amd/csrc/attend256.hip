@@ -451,6 +451,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
     A.S = __builtin_amdgcn_readlane(P.mine, tok);
     pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
   }
+  else if (A.s_short) A.S = splits_at(A.S, A.s_short, *A.d_pos);        // the partials keep the distance of the launched splits
   const size_t p0 = pair0 * A.n_heads + head;
   // 8 split lanes; each takes splits sl, sl + 8, ... (at most kInFlight of them: the launcher picks kInFlight so that
   // 8 * kInFlight >= S).  Their partial rows are requested first, together with the (m, l) pairs the weights come from:

@@ -6,7 +6,9 @@ namespace {
 
 template <int KB, bool MS>
 __global__ void __launch_bounds__(256, 2) attend_tb_kernel(TbAttnArgs A) {
-  tbd::attend_tb_body<KB, MS>(A, blockIdx.x, blockIdx.y, blockIdx.z, false);
+  int split = blockIdx.x, kvh = blockIdx.y;
+  if (!MS && A.s_short) tb_split_of(A, split + A.S * kvh, split, kvh);
+  tbd::attend_tb_body<KB, MS>(A, split, kvh, blockIdx.z, false);
 }
 
 }  // namespace

@@ -103,7 +103,7 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
   maxlen = lane_row16(maxlen, LaneMax{}); minlen = lane_row16(minlen, LaneMin{});
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
   const int ntiles = (maxlen + 31) >> 5;
-  const int s_used = MS && A.adapt ? share.n : min(A.S, max(1, ntiles >> 1));
+  const int s_used = MS && A.adapt ? share.n : min(MS ? A.S : splits_at(A.S, A.s_short, pos), max(1, ntiles >> 1));
   // partials of (token tj, split) start at pair * n_heads
   auto pair_of = [&](int tj) __attribute__((always_inline)) { return MS && A.adapt ? share.base + split : (size_t)tj * A.S + split; };
   if (split >= s_used) {                             // the "no keys" marker; the combiner does not read such rows

@@ -480,8 +480,9 @@ __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) { search_bo
 template <int KB, bool BF>
 __global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(TbEncArgs E, TbAttnArgs A, int n_search) {
   if ((int)blockIdx.x < n_search) { search_body<BF>(E, blockIdx.x); return; }
-  const int b = blockIdx.x - n_search, kvh = b / A.S;
-  tbd::attend_tb_body<KB, false>(A, b % A.S, kvh, 0, true);
+  int split, kvh;
+  tb_split_of(A, blockIdx.x - n_search, split, kvh);
+  tbd::attend_tb_body<KB, false>(A, split, kvh, 0, true);
 }
 
 // word d of a row's MSB-first stream of KB-bit fields: the fields that overlap bits [32 d, 32 d + 32)

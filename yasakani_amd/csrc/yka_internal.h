@@ -85,7 +85,8 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
   // adapt != 0: partials of launch_attend_chunk - the splits in use follow from *d_pos as they did there, and with direct != 0 a
   // slice that used one split has written its output already
   int adapt = 0; int direct = 0; const int* d_pos = nullptr; int tok0 = 0; int n_kv = 0; int max_ctx = 0;
-  RowMap rows; };        // rows.pos != nullptr: partials of a multi-stream pass shared out by ms_share
+  RowMap rows;           // rows.pos != nullptr: partials of a multi-stream pass shared out by ms_share
+  int s_short = 0; };    // trellis decode: as in TbAttnArgs (d_pos is set then)
 // projection outputs xq [M][n_heads][128], xk / xv [M][n_kv][128] fp32 -> q16 and the cache rows at *d_pos + t
 struct PostArgs {
   KvView kv; const float* xq; const float* xk; const float* xv; int M; int n_heads; const int* d_pos;
@@ -134,9 +135,15 @@ struct TbAttnArgs {
   int in_bf16 = 0;   // q16 is bf16 rows
   int adapt = 0;     // multi-stream pass: workgroups shared out by ms_share
   int rows_per_block = 128;   // wide kernel only
+  int s_short = 0;   // decode: splits in use at a position up to kShortPos, S beyond; 0: always S (splits_at)
 };
 void launch_attend_tb(const TbAttnArgs&, int kb, hipStream_t);        // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend_tb_wide(const TbAttnArgs&, int kb, hipStream_t);   // 3..64 rows: 128 query rows per workgroup, tiles decoded once into LDS
+// decode workgroup b -> split and kv head.  With s_short the splits that are always in use come first: the workgroups that
+// may exit then do not take the CUs the others would have had to themselves
+__device__ __forceinline__ void tb_split_of(const TbAttnArgs& A, int b, int& split, int& kvh) {
+  if (A.s_short) { split = b / A.n_kv; kvh = b % A.n_kv; } else { split = b % A.S; kvh = b / A.S; }
+}
 void launch_tb_encode(const TbEncArgs&, hipStream_t);
 // one or two tokens: encoder and attention over the keys in front of *d_pos; the combiner has to add the new rows
 void launch_tb_encode_attend(const TbEncArgs&, const TbAttnArgs&, int kb, hipStream_t);
@@ -258,6 +265,15 @@ __device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n
   const int top = __builtin_amdgcn_readlane(wave_scan(key, [](int a, int b) { return max(a, b); }), 63);
   return ((0x7fffffff - top) & 63) + 1;
 }
+
+// Trellis decode in containers that may hold more than kShortPos tokens: the grid provides two workgroups per CU and the
+// position, found on the device, says whether both are used.  A workgroup alone on its CU makes the combiner cheaper; on a long
+// context its waves wait for memory and LDS gathers that a second one fills.  us per layer call, one row of 5 bits, 64 / 128
+// splits: 23.8 / 27.8 at 16,000 tokens, 41.3 / 42.7 at 70,000, 58.7 / 56.5 at 130,000, 81.7 / 74.1 at 200,000; 4 bits 39.5 /
+// 41.6 at 70,000, 57.1 / 55.6 at 130,000.  (int4 rows of 256 channels gain nothing: 42.7 / 43.9 at 200,000.)
+// The workgroups that exit cost 1 us below kShortPos (23.4 -> 24.5 us at 16,000 tokens in a container of 262,144).
+constexpr int kShortPos = 98304;
+__device__ __forceinline__ int splits_at(int S, int s_short, int pos) { return s_short && pos <= kShortPos ? s_short : S; }
 
 // Multi-stream pass: how the W workgroups of one kv head are shared out over the pass's M <= 64 rows.  Streams differ in
 // length, and with the same number of splits for each the workgroups of the longest set the pace: every split is given
