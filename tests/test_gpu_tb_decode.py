@@ -61,3 +61,28 @@ def test_splits_change_with_the_position(native, kk):
             assert np.isfinite(got[0]).all(), ctx
             # other splits: partials and outputs rounded to fp16 once each (2^-11), sums in fp32
             assert np.linalg.norm(got[0] - got[1]) <= 1e-3 * np.linalg.norm(got[1]), ctx
+
+
+@pytest.mark.parametrize("kk", [4, 5])
+@pytest.mark.parametrize("M,bad,which", [(1, 0, "k"), (2, 0, "k"), (2, 1, "k"), (1, 0, "v"), (1, 0, "q"), (2, 1, "q")])
+def test_rows_that_are_not_numbers(native, kk, M, bad, which):
+    """A new K row with a NaN has a NaN scale: a query that sees its key has no softmax, whichever launch attends to the key.
+    500 tokens: the new keys share a workgroup's tiles with cached ones in the general path, too."""
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(kk + M)
+    half = lambda n, heads: rng.standard_normal((n, heads, 256)).astype(np.float16)    # noqa: E731
+    with native.KvCache(n_layers=1, max_ctx=1024, head_dim=256, max_rows=512) as kv:
+        kv.set_profile(kvqp.synthetic(layers=1, kk=kk, seed=11))
+        kv.append_host(0, half(500, 4), half(500, 4), 0)
+        new = dict(q=half(M, 24), k=half(M, 4), v=half(M, 4))
+        new[which][bad, 2, 17] = np.nan
+        out = kv.layer_call(0, new["q"], new["k"], new["v"], 500).astype(np.float32)
+        kv.set_opt(3, 1)
+        ref = kv.layer_call(0, new["q"], new["k"], new["v"], 500).astype(np.float32)
+    heads = slice(2, 3) if which == "q" else slice(12, 18)         # query head 2, or the query heads of KV head 2
+    touched = np.zeros(out.shape[:2], bool)
+    touched[bad if which == "q" else slice(bad, None), heads] = True
+    assert np.isnan(out[touched]).all() if which == "v" else not out[touched].any()
+    assert np.array_equal(np.isnan(out), np.isnan(ref)) and np.array_equal(out[touched] == 0, ref[touched] == 0)
+    # as in test_against_the_general_path
+    assert np.linalg.norm(out[~touched] - ref[~touched]) <= 1e-3 * np.linalg.norm(ref[~touched])

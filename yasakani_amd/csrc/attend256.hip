@@ -469,6 +469,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   };
   request(0);
   float new_s[2] = {-1e30f, -1e30f}, new_v[2] = {0.f, 0.f};       // score in log2 units and V value (channel tid) of the new keys
+  bool seen[2] = {false, false};               // uniform over the workgroup
   if constexpr (KB != 0) {
     __shared__ float s_dot[2][4];
     const TbAttnArgs& N = X.N;
@@ -476,11 +477,10 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
     const uint32_t *pk = N.pairs + ((size_t)gK << (8 + KB)), *pv = N.pairs + ((size_t)gV << (8 + KB));
     const float q = row16_value(N.q16[((size_t)tok * A.n_heads + head) * kD2 + tid], N.in_bf16);
     float ksc[2] = {0.f, 0.f}, dot[2] = {0.f, 0.f};
-    bool seen[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int r = pos + u;
-      seen[u] = u <= tok && r >= 0 && r < N.max_ctx;               // uniform over the workgroup
+      seen[u] = u <= tok && r >= 0 && r < N.max_ctx;
       if (!seen[u]) continue;
       const size_t row = (size_t)kvh * N.max_ctx + r;
       ksc[u] = N.kscl[row];
@@ -536,7 +536,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   if constexpr (KB != 0) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const float w = new_s[u] > -1e29f ? exp2f(new_s[u] - M2) : 0.f;
+      const float w = seen[u] ? exp2f(new_s[u] - M2) : 0.f;        // a score that is NaN ends in L: no softmax, zeros below
       o += w * new_v[u]; L += w;
     }
   }
