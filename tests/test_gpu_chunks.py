@@ -89,3 +89,34 @@ def test_256_channel_rows(native, kk, M, ctx, opts):
     assert np.isfinite(out).all()
     assert np.linalg.norm(out - ref) <= 1e-3 * np.linalg.norm(ref)
     assert (np.linalg.norm(out - ref, axis=2) / np.linalg.norm(ref, axis=2)).max() <= 4e-3
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("ctx", [0, 400])
+def test_query_rows_that_are_not_numbers(native, ctx, bf16):
+    """A query row with a NaN has no softmax: zeros, from a slice that writes its own output rows (one split) as from one whose
+    partials a combiner merges (a split count set by the caller)."""
+    rng = np.random.default_rng(ctx)
+
+    def rows(n, heads):
+        x = rng.standard_normal((n, heads, 128)).astype(np.float32)
+        return native.bf16_bits(x) if bf16 else x.astype(np.float16)
+
+    M, bad = 150, [(0, 0), (77, 5), (78, 23), (149, 11)]
+    with native.KvCache(max_ctx=1024, max_rows=512) as kv:
+        kv.set_opt(11, bf16)
+        if ctx:
+            kv.append_host(0, rows(ctx, 4), rows(ctx, 4), 0)
+        q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
+        clean = kv.layer_call(0, q, k, v, ctx)
+        for t, h in bad:
+            q.view(np.uint16)[t, h, 40] = 0x7fc0 if bf16 else 0x7e00
+        touched = np.zeros((M, 24), bool)
+        touched[tuple(np.array(bad).T)] = True
+        for splits in (0, 3):
+            kv.set_opt(2, splits)
+            kv.poison_workspace()
+            out = kv.layer_call(0, q, k, v, ctx)
+            assert not (out[touched].view(np.uint16) & 0x7fff).any(), splits
+            if splits == 0:                                        # the other rows do not notice
+                assert np.array_equal(out[~touched].view(np.uint16), clean[~touched].view(np.uint16))

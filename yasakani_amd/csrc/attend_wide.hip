@@ -486,6 +486,8 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   l = lane_op32(l, LaneAdd{});
   const bool direct = CHUNK && A.S == 1 && A.out16;          // uniform over the grid
   if (!direct && vrow && h == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
+  // a row none of whose scores is a number keeps the marker: the combiner drops its partial and writes zeros, and so does this
+  const bool none = direct && m_run < -1e29f;
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int a0 = 0; a0 < 2; ++a0)
@@ -501,6 +503,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
         for (int c = 0; c < 8; ++c) y[c] = o[c & 3][4 * (2 * (c >> 2) + a0) + b] * inv;
         packed = pack_out8(y, 1);
       }
+      if (CHUNK && none) packed = make_uint4(0, 0, 0, 0);
       *reinterpret_cast<uint4*>(stage + j * kOPitch + (64 * a0 + 32 * h + 8 * b) * 2) = packed;
     }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");     // the wave reads back what its own lanes wrote
