@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   const int total = CHUNK ? A.S * A.kv.n_kv * n_rb : (int)gridDim.x;
   if (CHUNK && (int)blockIdx.x >= total) return;
   int pair, rb;
-  if (CHUNK && A.adapt && (min(pos + A.tok0 + A.M, A.kv.max_ctx) + 31) / 32 * 4608 * A.kv.n_kv <= (4 << 20)) {
+  if (CHUNK && A.adapt && (long long)((min(pos + A.tok0 + A.M, A.kv.max_ctx) + 31) / 32) * 4608 * A.kv.n_kv <= (4 << 20)) {
     const int pairs = A.S * A.kv.n_kv;
     rb = n_rb - 1 - (int)blockIdx.x / pairs; pair = (int)blockIdx.x % pairs;
   } else {

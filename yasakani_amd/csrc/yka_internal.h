@@ -253,15 +253,26 @@ __device__ __forceinline__ int wave_scan_add(int v) { return wave_scan(v, [](int
 // splits (39 + 39 in the attention, 23 in the combiners), 46 with one split (42 in the attention, which then waits for its
 // longest workgroup: 47 tiles; 48 and 44 while the choice went through LDS).  2,048 rows behind 131,072: the same with 2 splits of one slice as with 4 of two.
 constexpr int kChunkOverhead = 18, kChunkMaxSplits = 64;
+// price of s splits in those units.  The sums of workgroups times tiles are taken in 64 bits: with 2,048 rows on 4 KV heads they pass 2^31
+// at 11 M tokens, and the two readers of a choice have to agree on it
+__host__ __device__ constexpr long long chunk_price(int pos, int tok0, int M, int n_kv, int max_ctx, int s) {
+  auto tiles16 = [&](int rows) {                                     // of the row block that ends `rows` rows into the slice
+    const long long len = (long long)pos + tok0 + rows;
+    return (int)(((len < 0 ? 0 : len < max_ctx ? len : max_ctx) + 31) >> 5) * 16;
+  };
+  const int base = n_kv * ((kG * M + 127) / 128), n = base * s, idle = (256 - (n & 255)) & 255;   // workgroups, and CUs without one in the last round
+  const int lo = tiles16(M < 128 / kG + 1 ? M : 128 / kG + 1) / s + 16 * kChunkOverhead, hi = tiles16(M) / s + 16 * kChunkOverhead;
+  const long long rounds = ((long long)(n >> 1) * ((long long)lo + hi) >> 8) + ((long long)lo * idle >> 8), t = hi > rounds ? hi : rounds;
+  return s > 1 ? t + 96 + M * s / 13 : t;
+}
+// (a constant expression cannot wrap: these would not compile in 32 bits)
+static_assert(chunk_price(1 << 24, 0, 2048, 4, 1 << 25, 2) > chunk_price(1 << 23, 0, 2048, 4, 1 << 25, 2), "longer contexts cost more");
+static_assert(chunk_price(0x7fffff00, 4096, 4096, 1024, 0x7fffff00, kChunkMaxSplits) > 0, "the largest container the library opens");
 __device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n_kv, int max_ctx, int S) {
-  const int base = n_kv * ((kG * M + 127) / 128), s = (int)(threadIdx.x & 63) + 1;
-  const int first = max(0, min(pos + tok0 + min(M, 128 / kG + 1), max_ctx)), last = max(0, min(pos + tok0 + M, max_ctx));
-  const int lo = ((first + 31) >> 5) * 16 / s + 16 * kChunkOverhead, hi = ((last + 31) >> 5) * 16 / s + 16 * kChunkOverhead;
-  const int n = base * s, idle = (256 - (n & 255)) & 255;            // workgroups, and CUs without one in the last round
-  int t = max(hi, (n >> 1) * (lo + hi) / 256 + lo * idle / 256);
-  if (s > 1) t += 96 + M * s / 13;
+  const int s = (int)(threadIdx.x & 63) + 1;
   // lowest price, then fewest splits: the largest key (lane 0 always has one)
-  const int key = s <= S ? 0x7fffffff - ((max(0, min(t, 0x1fffffe)) << 6) | (s - 1)) : 0;
+  const long long t = chunk_price(pos, tok0, M, n_kv, max_ctx, s);
+  const int key = s <= S ? 0x7fffffff - (((int)(t < 0x1fffffe ? t : 0x1fffffe) << 6) | (s - 1)) : 0;
   const int top = __builtin_amdgcn_readlane(wave_scan(key, [](int a, int b) { return max(a, b); }), 63);
   return ((0x7fffffff - top) & 63) + 1;
 }
@@ -289,9 +300,10 @@ __device__ __forceinline__ MsPlan ms_plan(const RowMap& R, int M, int max_ctx, i
   const int lane = threadIdx.x & 63, pos = lane < M ? R.pos[lane] : -1, slot = lane < M ? R.slot[lane] : -1;
   // 0 tiles: a row that names no container or position
   const int tiles = pos >= 0 && pos < max_ctx && slot >= 0 && slot < R.n_slots ? (pos + 32) >> 5 : 0;
-  const int total = __builtin_amdgcn_readlane(wave_scan_add(tiles), 63);
+  // unsigned: 64 rows of the longest container are just under 2^32 tiles
+  const unsigned total = max(1u, (unsigned)__builtin_amdgcn_readlane(wave_scan_add(tiles), 63));
   const int most = __builtin_amdgcn_readlane(wave_scan(tiles, [](int a, int b) { return max(a, b); }), 63);
-  int lo = max(4, max((most + 255) >> 8, (total + W - 1) / W)), c = max(lo, (total + W - M - 1) / (W - M));
+  int lo = max(4, max((most + 255) >> 8, (int)((total - 1) / (unsigned)W + 1))), c = max(lo, (int)((total - 1) / (unsigned)(W - M) + 1));
   int mine = (tiles + c - 1) / c, incl = wave_scan_add(mine);
   for (int it = 0; it < 4 && lo < c; ++it) {       // c always fits; a smaller one may
     const int mid = (lo + c) >> 1, want = (tiles + mid - 1) / mid, sum = wave_scan_add(want);
