@@ -507,16 +507,21 @@ void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
 // covers the 128 splits of decode over long contexts (few, long workgroups); 4 keeps the register count low where
 // thousands of workgroups run (wide windows).
 // MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
-template <int kInFlight, bool MS>
+// ADAPT: rows of a prefill slice that the rows form below does not take (inverse rotation, or more than 32 splits); as many
+// workgroups as the chip holds at once, each walks its share of the tokens, so that the choice of the splits is made 8 times per CU and
+// not once per row (1,024 rows at 9,000 tokens with the inverse rotation: 42.4 us with a workgroup per row, 37.9 so).
+template <int kInFlight, bool MS, bool ADAPT>
 __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   __shared__ float s_w[256];
   __shared__ float s_o[16][kD + 4];
   __shared__ float s_wsum[16];
-  const int head = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x;
-  if (A.adapt) {
+  const int head = blockIdx.x, tid = threadIdx.x;
+  int tok = blockIdx.y;
+  if constexpr (ADAPT) {
     A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S);
     if (A.S == 1 && A.direct) return;
   }
+  do {
   size_t pair0 = (size_t)tok * A.S;
   if constexpr (MS) {
     const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
@@ -595,6 +600,8 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
     }
   }
   if (tid < kD) A.out16[((size_t)tok * A.n_heads + head) * kD + tid] = A.out_bf16 ? f2bf_bits(y) : __half_as_ushort(__float2half_rn(y));
+  if constexpr (ADAPT) __syncthreads();            // the next token reuses the LDS arrays
+  } while (ADAPT && (tok += gridDim.y) < A.M);
 }
 // The combiner for wide passes (many rows, at most 32 splits, no un-rotation): one wave per (token, head) row, four
 // waves per workgroup, no LDS and no barrier.  Lane = (split lane 0..3, 8 channels); a split lane takes splits sl, sl + 4,
@@ -649,7 +656,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
   if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most)
-    hipLaunchKernelGGL((combine_kernel<4, true>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+    hipLaunchKernelGGL((combine_kernel<4, true, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
     return;
   }
   if (A.S <= 32 && !A.unrot && A.M >= 8) {
@@ -658,9 +665,14 @@ void launch_combine(const CombineArgs& A, hipStream_t st) {
     else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, A);
     return;
   }
-  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);   // S <= 256
-  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
-  else hipLaunchKernelGGL((combine_kernel<4, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  if (A.adapt) {                                   // S <= kChunkMaxSplits
+    static_assert(kChunkMaxSplits <= 64, "16 split lanes x 4 rows in flight");
+    hipLaunchKernelGGL((combine_kernel<4, false, true>), dim3(A.n_heads, min(A.M, max(1, 2048 / A.n_heads))), dim3(256), 0, st, A);
+    return;
+  }
+  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);   // S <= 256
+  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
+  else hipLaunchKernelGGL((combine_kernel<4, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
 }
 
 }  // namespace yka
