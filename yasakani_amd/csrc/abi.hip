@@ -32,6 +32,7 @@ struct yka_kv {
   float *pm = nullptr, *pl = nullptr; uint16_t* pacc16 = nullptr;
   int* tickets = nullptr;     // [n_kv_heads][64] split tickets of the decode kernel, all zero between launches
   size_t ws_rows = 0;              // capacity of the partial workspace in (token, split) pairs
+  int2* ms_plan = nullptr;         // [64] shares of a multi-stream pass, attention launch -> combiner
   int* d_pos = nullptr;            // position used by the host-pointer hooks
   hipStream_t stream = nullptr;    // stream of the host-pointer hooks
   int opt_splits_narrow = 0, opt_splits_wide = 0, opt_force_narrow = 0, opt_unrot = 0, opt_ctx_hint = 0, opt_profile_layer = 0, opt_merge_in_launch = 0;
@@ -374,11 +375,10 @@ void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const ui
       RowMap Rs = R; Rs.pos += s0; Rs.slot += s0;
       const TbAttnArgs A{T.kpay(0), T.vpay(0), T.kscl(0), T.vscl(0), kv->cfg.max_ctx, kv->cfg.n_kv_heads, T.stride,
                          T.pairs, T.gfac, T.has_mu ? T.mu : nullptr, pl, q16 + (size_t)s0 * NH * 256, nullptr, nullptr, Ms, s0, NH, S,
-                         kv->pm, kv->pl, kv->pacc16, Rs, bf16, share};
+                         kv->pm, kv->pl, kv->pacc16, Rs, bf16, share, kv->ms_plan};
       launch_attend_tb(A, T.kb, st);
       CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
-      C.max_ctx = kv->cfg.max_ctx;
-      if (share) C.rows = Rs;
+      if (share) C.plan = kv->ms_plan;
       launch_combine256(C, st);
     }
     return;
@@ -396,8 +396,7 @@ void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const ui
     AttnArgs A{kv->view(0), q16 + (size_t)s0 * NH * D, nullptr, nullptr, Ms, s0, NH, S, 128, kv->pm, kv->pl, kv->pacc16, nullptr, nullptr, Rs};
     A.in_bf16 = bf16;
     CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * D, kv->opt_unrot, bf16};
-    C.max_ctx = kv->cfg.max_ctx;
-    if (share && !one_launch) { A.adapt = 1; C.rows = Rs; }
+    if (share && !one_launch) { A.adapt = 1; A.plan = kv->ms_plan; C.plan = kv->ms_plan; }
     if (fuse) { A.k16 = k16; A.v16 = v16; }
     if (r256) { launch_attend256(A, st); launch_combine256(C, st); }
     else if (one_launch) {
@@ -470,6 +469,7 @@ yka_kv* yka_kv_open(const yka_kv_config* cfg) {
     HIPCHK(hipMalloc((void**)&kv->pacc16, np * cfg->head_dim * 2));
     HIPCHK(hipMalloc((void**)&kv->tickets, (size_t)cfg->n_kv_heads * kMaxSlice * 4));   // one counter per (kv head, row tile); zero between launches
     HIPCHK(hipMemset(kv->tickets, 0, (size_t)cfg->n_kv_heads * kMaxSlice * 4));
+    HIPCHK(hipMalloc((void**)&kv->ms_plan, kMaxSlice * sizeof(int2)));
     HIPCHK(hipMalloc((void**)&kv->d_pos, 4));
     HIPCHK(hipMemset(kv->d_pos, 0, 4));
     HIPCHK(hipStreamCreateWithFlags(&kv->stream, hipStreamNonBlocking));
@@ -492,7 +492,7 @@ void yka_kv_close(yka_kv* kv) {
     (void)hipFree(kv->tb->scr); (void)hipFree(kv->tb->stage);
     delete kv->tb;
   }
-  (void)hipFree(kv->pool); (void)hipFree(kv->tables); (void)hipFree(kv->pm); (void)hipFree(kv->pl); (void)hipFree(kv->pacc16); (void)hipFree(kv->d_pos); (void)hipFree(kv->tickets);
+  (void)hipFree(kv->pool); (void)hipFree(kv->tables); (void)hipFree(kv->pm); (void)hipFree(kv->pl); (void)hipFree(kv->pacc16); (void)hipFree(kv->d_pos); (void)hipFree(kv->tickets); (void)hipFree(kv->ms_plan);
   delete kv;
 }
 
@@ -587,6 +587,7 @@ int yka_kv_poison_workspace(yka_kv* kv) {
   HIPCHK(hipMemset(kv->pm, 0xff, rows * 4));
   HIPCHK(hipMemset(kv->pl, 0xff, rows * 4));
   HIPCHK(hipMemset(kv->pacc16, 0xff, rows * (size_t)kv->D() * 2));
+  HIPCHK(hipMemset(kv->ms_plan, 0xff, kMaxSlice * sizeof(int2)));
   HIPCHK(hipDeviceSynchronize());
   YKA_CATCH_INT
 }

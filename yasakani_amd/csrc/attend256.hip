@@ -232,7 +232,8 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   MsShare share{};
   if (MS) {
     if (A.adapt) {
-      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, split + A.S * rt);
+      const int b = split + A.S * rt;
+      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, b, A.plan, b == 0 && kvh == 0 && wave == 0);
       if (share.row < 0) return;
       split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
     } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }
@@ -447,9 +448,8 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   const int head = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x;
   size_t pair0 = (size_t)tok * A.S;
   if constexpr (MS) {
-    const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
-    A.S = __builtin_amdgcn_readlane(P.mine, tok);
-    pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
+    const int2 P = A.plan[tok];
+    pair0 = (size_t)P.x; A.S = P.y;
   }
   else if (A.s_short) A.S = splits_at(A.S, A.s_short, *A.d_pos);        // the partials keep the distance of the launched splits
   const size_t p0 = pair0 * A.n_heads + head;
@@ -561,7 +561,7 @@ void launch_attend256(const AttnArgs& A, hipStream_t st) {
 void launch_combine256(const CombineArgs& A, hipStream_t st) {
   // a stream may hold any share of the splits (256 at most, in batches of 8 * kInFlight).  5 streams of up to 3,000 tokens, us a
   // pass: 15.2 with 16 in flight (and 198 registers), 12.4 with 4 and splits of 4 tiles.
-  if (A.rows.pos) {
+  if (A.plan) {
     if (A.M < 4) hipLaunchKernelGGL((combine256_kernel<8, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
     else hipLaunchKernelGGL((combine256_kernel<4, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
     return;

@@ -197,7 +197,8 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(AttnArgs A) {
   MsShare share{};
   if (MS) {
     if (A.adapt) {
-      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, split + A.S * rt);
+      const int b = split + A.S * rt;
+      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, b, A.plan, b == 0 && kvh == 0 && wave == 0);
       if (share.row < 0) return;
       split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
     } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }
@@ -524,9 +525,8 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   do {
   size_t pair0 = (size_t)tok * A.S;
   if constexpr (MS) {
-    const MsPlan P = ms_plan(A.rows, A.M, A.max_ctx, A.S * A.M);
-    A.S = __builtin_amdgcn_readlane(P.mine, tok);
-    pair0 = (size_t)(__builtin_amdgcn_readlane(P.incl, tok) - A.S);
+    const int2 P = A.plan[tok];
+    pair0 = (size_t)P.x; A.S = P.y;
   }
   const size_t p0 = pair0 * A.n_heads + head;                  // split s lives at p0 + s * n_heads
   // 16 split lanes; each takes splits sl, sl+16, ... (at most kInFlight of them: the launcher picks kInFlight so that
@@ -655,7 +655,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
   }  }
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
-  if (A.rows.pos) {                                // a stream may hold any share of the splits (256 at most)
+  if (A.plan) {                                    // a stream may hold any share of the splits (256 at most)
     hipLaunchKernelGGL((combine_kernel<4, true, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, A);
     return;
   }

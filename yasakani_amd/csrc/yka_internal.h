@@ -75,8 +75,10 @@ struct AttnArgs {
   int in_bf16 = 0;   // q16 / k16 / v16 are bf16 rows (rows16_to_f16)
   // wide kernel, slice of a prefill chunk (launch_attend_chunk): adapt != 0 lets the device choose how many of the S launched
   // splits the slice uses (chunk_splits_used); out16 != nullptr: a slice that uses one writes its output rows itself
-  // multi-stream pass: adapt != 0 shares the S * M workgroups of a kv head out by the streams' lengths (ms_share)
+  // multi-stream pass: adapt != 0 shares the S * M workgroups of a kv head out by the streams' lengths (ms_share) and leaves the
+  // shares in plan[M] for the combiner
   int adapt = 0;
+  int2* plan = nullptr;
 };
 // unrot != 0: the output row gets the inverse signed Hadamard rotation (7 butterfly stages, x 1/16, signs) before it is
 // rounded to fp16 - the counterpart of rotating V rows on their way into the cache (src/q35_kernels.cu:1421)
@@ -85,7 +87,7 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
   // adapt != 0: partials of launch_attend_chunk - the splits in use follow from *d_pos as they did there, and with direct != 0 a
   // slice that used one split has written its output already
   int adapt = 0; int direct = 0; const int* d_pos = nullptr; int tok0 = 0; int n_kv = 0; int max_ctx = 0;
-  RowMap rows;           // rows.pos != nullptr: partials of a multi-stream pass shared out by ms_share
+  const int2* plan = nullptr;   // partials of a multi-stream pass shared out by ms_share: first split and splits of every row
   int s_short = 0; };    // trellis decode: as in TbAttnArgs (d_pos is set then)
 // projection outputs xq [M][n_heads][128], xk / xv [M][n_kv][128] fp32 -> q16 and the cache rows at *d_pos + t
 struct PostArgs {
@@ -133,7 +135,8 @@ struct TbAttnArgs {
   float* pm; float* pl; uint16_t* pacc16;
   RowMap rows;  // narrow kernel only: multi-stream pass (one token per workgroup column; kpay .. vscl = container 0, `layer` = the profile's layer)
   int in_bf16 = 0;   // q16 is bf16 rows
-  int adapt = 0;     // multi-stream pass: workgroups shared out by ms_share
+  int adapt = 0;     // multi-stream pass: workgroups shared out by ms_share, the shares left in plan
+  int2* plan = nullptr;
   int rows_per_block = 128;   // wide kernel only
   int s_short = 0;   // decode: splits in use at a position up to kShortPos, S beyond; 0: always S (splits_at)
 };
@@ -293,10 +296,18 @@ __device__ __forceinline__ int splits_at(int S, int s_short, int pos) { return s
 // 16 streams of 2,000 to 32,000 tokens: 36.7 us a pass with 16 splits each (the longest stream's workgroups walk 62 tiles,
 // the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.  Row t's splits are
 // workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by every wave from the
-// row map (lane t looks at row t), again by the combiner: whole numbers, so that both agree.
+// row map (lane t looks at row t); the first wave of the launch leaves the shares in memory for the combiner, whose
+// workgroups have nothing to hide the computation under (48 streams of 300 tokens, 5 bits: its launch 6.0 us when it computed the shares, 4.6 since).
 struct MsShare { int row, split, n, pos, slot; size_t base; };
-struct MsPlan { int mine, incl, pos, slot; };      // of row `lane`: its splits, the splits up to and including it, its place
-__device__ __forceinline__ MsPlan ms_plan(const RowMap& R, int M, int max_ctx, int W) {
+// ceil(a / b) for quotients up to 2^16 and a below 2^27: the float quotient is off by one at most
+__device__ __forceinline__ int ms_tiles_per(int a, int b) {
+  const int n = a + b - 1;
+  int q = (int)((float)n * __builtin_amdgcn_rcpf((float)b));
+  const int r = n - q * b;
+  return q + (r >= b) - (r < 0);
+}
+// workgroup b of the kv head; row = -1: nothing left for it.  leave: this wave stores the plan
+__device__ __forceinline__ MsShare ms_share(const RowMap& R, int M, int max_ctx, int W, int b, int2* plan, bool leave) {
   const int lane = threadIdx.x & 63, pos = lane < M ? R.pos[lane] : -1, slot = lane < M ? R.slot[lane] : -1;
   // 0 tiles: a row that names no container or position
   const int tiles = pos >= 0 && pos < max_ctx && slot >= 0 && slot < R.n_slots ? (pos + 32) >> 5 : 0;
@@ -304,20 +315,16 @@ __device__ __forceinline__ MsPlan ms_plan(const RowMap& R, int M, int max_ctx, i
   const unsigned total = max(1u, (unsigned)__builtin_amdgcn_readlane(wave_scan_add(tiles), 63));
   const int most = __builtin_amdgcn_readlane(wave_scan(tiles, [](int a, int b) { return max(a, b); }), 63);
   int lo = max(4, max((most + 255) >> 8, (int)((total - 1) / (unsigned)W + 1))), c = max(lo, (int)((total - 1) / (unsigned)(W - M) + 1));
-  int mine = (tiles + c - 1) / c, incl = wave_scan_add(mine);
+  int mine = ms_tiles_per(tiles, c), incl = wave_scan_add(mine);
   for (int it = 0; it < 4 && lo < c; ++it) {       // c always fits; a smaller one may
-    const int mid = (lo + c) >> 1, want = (tiles + mid - 1) / mid, sum = wave_scan_add(want);
+    const int mid = (lo + c) >> 1, want = ms_tiles_per(tiles, mid), sum = wave_scan_add(want);
     if (__builtin_amdgcn_readlane(sum, 63) <= W) { c = mid; mine = want; incl = sum; } else lo = mid + 1;
   }
-  return {mine, incl, pos, slot};
-}
-// workgroup b of the kv head; row = -1: nothing left for it
-__device__ __forceinline__ MsShare ms_share(const RowMap& R, int M, int max_ctx, int W, int b) {
-  const MsPlan P = ms_plan(R, M, max_ctx, W);
-  const int row = __popcll(__ballot(P.incl <= b));
+  if (leave && lane < M) plan[lane] = make_int2(incl - mine, mine);
+  const int row = __popcll(__ballot(incl <= b));
   if (row >= M) return {-1, 0, 0, 0, 0, 0};
-  const int n = __builtin_amdgcn_readlane(P.mine, row), base = __builtin_amdgcn_readlane(P.incl, row) - n;
-  return {row, b - base, n, __builtin_amdgcn_readlane(P.pos, row), __builtin_amdgcn_readlane(P.slot, row), (size_t)base};
+  const int n = __builtin_amdgcn_readlane(mine, row), base = __builtin_amdgcn_readlane(incl, row) - n;
+  return {row, b - base, n, __builtin_amdgcn_readlane(pos, row), __builtin_amdgcn_readlane(slot, row), (size_t)base};
 }
 
 // Multi-stream pass of at most 64 rows whose attention launch stores the new rows itself: the rows of the pass (bit t = row
