@@ -200,3 +200,29 @@ def test_streams_of_very_different_lengths(native, dim, M):
             # the same kernel arithmetic with another split count: fp16 partials and outputs, 2^-11 each, summed in fp32
             assert np.linalg.norm(out[t].astype(np.float32) - ref) <= 1e-3 * np.linalg.norm(ref), f"row {t}: stream of {pos[t]} tokens"
         assert [kv.export_rows(int(slots[t]), int(pos[t]), 1)[0].any() for t in range(M) if t not in bad].count(False) == 0
+
+
+# 128-channel rows, numbers of streams whose whole splits leave a round of workgroups unfilled: long streams (48 tiles for each
+# workgroup of one round) use the second number of workgroups, short ones the first; both sides of that line, for 26 rows
+# (104 and 182 workgroups a kv head), 33 (99, 231), 48 (96, 192) and 51 (102, 255)
+@pytest.mark.parametrize("M,per_round", [(26, 104), (33, 99), (48, 96), (51, 102)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_the_line_between_short_and_long_streams(native, M, per_round, more):
+    rng = np.random.default_rng(M)
+    total = 48 * per_round - 1 + more                     # together 48 tiles a workgroup, or one tile less
+    tiles = np.full(M, total // M) + (np.arange(M) < total % M)
+    lens = tiles * 32 - rng.integers(1, 33, M)            # a row at position p has (p + 32) / 32 tiles
+    half = lambda n, heads: rng.standard_normal((n, heads, 128)).astype(np.float16)    # noqa: E731
+    pool_k, pool_v = half(6400, 4), half(6400, 4)
+    with native.KvCache(n_layers=M, max_ctx=8192, max_rows=6400) as kv:
+        for s in range(M):
+            n = int(lens[s])
+            kv.append_host(s, np.roll(pool_k, s, axis=0)[:n], np.roll(pool_v, 7 * s, axis=0)[:n], 0)
+        slots = rng.permutation(M).astype(np.int32)
+        pos = lens[slots].astype(np.int32)
+        q, k, v = half(M, 24), half(M, 4), half(M, 4)
+        kv.poison_workspace()
+        out = kv.ms_call(q, k, v, pos, slots).astype(np.float32)
+        for t in range(M):
+            ref = kv.layer_call(int(slots[t]), q[t:t + 1], k[t:t + 1], v[t:t + 1], int(pos[t])).astype(np.float32)[0]
+            assert np.linalg.norm(out[t] - ref) <= 1e-3 * np.linalg.norm(ref), f"row {t}: stream of {pos[t]} tokens"    # as above

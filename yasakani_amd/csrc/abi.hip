@@ -353,6 +353,27 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
   }
 }
 
+// Multi-stream pass, 128-channel rows: splits per row the launch provides for.  Two workgroups per CU, one round, as long as
+// whole splits of M rows fill it: streams of equal length get M times a whole number of workgroups, whatever the sharing-out.
+// Where one and a half or two rounds are filled a seventh better the grid is launched for those, and the device decides by
+// the streams' lengths which of the two it uses (ms_share; kMsLong).  us a pass, 512 / 768 / 1,024 workgroups provided:
+//   48 streams of equal length  8,000 tokens 56.9 / 50.7 / 52.7   16,000 102 / 89.4 / 91.8   2,000 24.6 / 24.8 / 26.1
+//   48 streams, a sixteenth up to 16,000 tokens 50.8 / 40.8 / 42.4   8,000 32.9 / 29.2 / 29.8   4,000 21.5 / 21.5 / 22.8
+//   33 streams of equal length 16,000 tokens 71.5 / 70.5 / 66.9   4,000 27.4 / 27.7 / 28.8
+// (before the sharing-out, 1,024 workgroups: 90.8 us for the 48 of 16,000, 65.7 for the 33)
+struct MsGrid { int S, in_short; };
+MsGrid ms_grid(const yka_kv* kv, int M) {
+  const int per = kv->cfg.n_kv_heads * M, S = std::max(2, std::min(kMaxSplits, 512 / per));
+  int best = S;
+  double fill = 1.15 * std::min(1.0, S * per / 512.0);
+  for (const int wgs : {768, 1024}) {
+    const int s = wgs / per;
+    if (s > S && s * per / (double)wgs >= fill) { fill = s * per / (double)wgs; best = s; }
+  }
+  const int fits = (int)(kWsPairs / (size_t)M);
+  return {std::min({best, kMaxSplits, fits}), best > S ? std::min(S, fits) * M : 0};
+}
+
 // Multi-stream pass: rows are appended (several rows of one stream may follow each other and read each other's keys) by the
 // attention launch or, beyond 64 rows and with a split count set by the caller, by a launch in front of it; every row attends to keys [0, pos[t]] of its own container.  One token per workgroup column.
 void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const uint16_t* v16, int M, const int* row_pos,
@@ -392,11 +413,13 @@ void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const ui
     const int Ms = std::min(kMaxSlice, M - s0);
     int S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : 512 / (kv->cfg.n_kv_heads * Ms);   // two workgroups per CU: one round
     S = std::min(std::max(2, std::min(kMaxSplits, S)), (int)(kWsPairs / (size_t)Ms));
+    const MsGrid G = share && !one_launch && !r256 ? ms_grid(kv, Ms) : MsGrid{S, 0};
+    S = G.S;
     RowMap Rs = R; Rs.pos += s0; Rs.slot += s0;
     AttnArgs A{kv->view(0), q16 + (size_t)s0 * NH * D, nullptr, nullptr, Ms, s0, NH, S, 128, kv->pm, kv->pl, kv->pacc16, nullptr, nullptr, Rs};
     A.in_bf16 = bf16;
     CombineArgs C{kv->pm, kv->pl, kv->pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * D, kv->opt_unrot, bf16};
-    if (share && !one_launch) { A.adapt = 1; A.plan = kv->ms_plan; C.plan = kv->ms_plan; }
+    if (share && !one_launch) { A.adapt = 1; A.ms_short = G.in_short; A.plan = kv->ms_plan; C.plan = kv->ms_plan; }
     if (fuse) { A.k16 = k16; A.v16 = v16; }
     if (r256) { launch_attend256(A, st); launch_combine256(C, st); }
     else if (one_launch) {

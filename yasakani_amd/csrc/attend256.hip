@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   if (MS) {
     if (A.adapt) {
       const int b = split + A.S * rt;
-      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, b, A.plan, b == 0 && kvh == 0 && wave == 0);
+      share = ms_share(A.rows, A.M, A.kv.max_ctx, A.S * A.M, 0, b, A.plan, b == 0 && kvh == 0 && wave == 0);
       if (share.row < 0) return;
       split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
     } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }

@@ -78,7 +78,7 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
     int slot;
     if (A.adapt) {
       const int b = split + A.S * rt;
-      share = ms_share(A.rows, A.M, A.max_ctx, A.S * A.M, b, A.plan, b == 0 && kvh == 0 && wave == 0);
+      share = ms_share(A.rows, A.M, A.max_ctx, A.S * A.M, 0, b, A.plan, b == 0 && kvh == 0 && wave == 0);
       if (share.row < 0) return;
       split = share.split; rt = share.row; pos = share.pos; slot = share.slot;
     } else { pos = A.rows.pos[rt]; slot = A.rows.slot[rt]; }

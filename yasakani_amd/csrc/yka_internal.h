@@ -79,6 +79,7 @@ struct AttnArgs {
   // shares in plan[M] for the combiner
   int adapt = 0;
   int2* plan = nullptr;
+  int ms_short = 0;  // workgroups of a kv head a pass over short streams uses (0: all S * M)
 };
 // unrot != 0: the output row gets the inverse signed Hadamard rotation (7 butterfly stages, x 1/16, signs) before it is
 // rounded to fp16 - the counterpart of rotating V rows on their way into the cache (src/q35_kernels.cu:1421)
@@ -306,14 +307,17 @@ __device__ __forceinline__ int ms_tiles_per(int a, int b) {
   const int r = n - q * b;
   return q + (r >= b) - (r < 0);
 }
-// workgroup b of the kv head; row = -1: nothing left for it.  leave: this wave stores the plan
-__device__ __forceinline__ MsShare ms_share(const RowMap& R, int M, int max_ctx, int W, int b, int2* plan, bool leave) {
+// workgroup b of the kv head; row = -1: nothing left for it.  leave: this wave stores the plan.  W_short: of the W launched
+// workgroups only so many are used while each of them would get fewer than kMsLong tiles (0: always all)
+constexpr unsigned kMsLong = 48;
+__device__ __forceinline__ MsShare ms_share(const RowMap& R, int M, int max_ctx, int W, int W_short, int b, int2* plan, bool leave) {
   const int lane = threadIdx.x & 63, pos = lane < M ? R.pos[lane] : -1, slot = lane < M ? R.slot[lane] : -1;
   // 0 tiles: a row that names no container or position
   const int tiles = pos >= 0 && pos < max_ctx && slot >= 0 && slot < R.n_slots ? (pos + 32) >> 5 : 0;
   // unsigned: 64 rows of the longest container are just under 2^32 tiles
   const unsigned total = max(1u, (unsigned)__builtin_amdgcn_readlane(wave_scan_add(tiles), 63));
   const int most = __builtin_amdgcn_readlane(wave_scan(tiles, [](int a, int b) { return max(a, b); }), 63);
+  if (W_short && total < kMsLong * (unsigned)W_short) W = W_short;
   int lo = max(4, max((most + 255) >> 8, (int)((total - 1) / (unsigned)W + 1))), c = max(lo, (int)((total - 1) / (unsigned)(W - M) + 1));
   int mine = ms_tiles_per(tiles, c), incl = wave_scan_add(mine);
   for (int it = 0; it < 4 && lo < c; ++it) {       // c always fits; a smaller one may
