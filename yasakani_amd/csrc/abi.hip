@@ -175,6 +175,9 @@ int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
 // layer call against 26.1).
 // Splits of the decode kernels: one workgroup per CU (the waves keep the next tile in flight and the combiner has half the
 // rows to read: 205 against 225 us for 16 layers at 20,011 tokens, 167 / 204 at 3,000, 97 / 101 for 2 layers at 200,000).
+// Windows forced through them (option key 3): two, where one would leave whole splits of the row tiles too long.  us per
+// layer call with 256 / 512 workgroups, 5 bits: 4 rows 26.3 / 28.6 at 1,000 tokens, 36.7 / 36.1 at 16,000, 8 rows 28.8 / 30.7 and
+// 47.9 / 45.4, 48 rows 64.2 / 62.3 and 187 / 145; int4: 16 rows 14.6 / 17.1 and 32.8 / 33.1, 48 rows 19.8 / 20.3 and 86.3 / 69.1.
 // Of the wide ones: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
 // rounds of 256 workgroups best.
 struct Part256 { int Ms, S, rows_per_block; bool narrow; int s_short; };
@@ -185,8 +188,9 @@ Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
   const bool narrow = Ms <= 2 || kv->opt_force_narrow;
   // trellis decode in containers longer than kShortPos: a second workgroup per CU, used from there on (splits_at)
   const bool two = kv->tb && Ms <= 2 && !kv->opt_splits_narrow && ctx_tiles > kShortPos / 32;
+  const int wgs = two || Ms > (kv->tb ? 4 : 16) ? 512 : 256;
   int S;
-  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min((two ? 512 : 256) / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
+  if (narrow) S = kv->opt_splits_narrow > 0 ? kv->opt_splits_narrow : std::max(2, std::min(wgs / (kv->cfg.n_kv_heads * ((Ms + 1) / 2)), ctx_tiles / 2));
   else if (kv->opt_splits_wide > 0) S = kv->opt_splits_wide;
   else if (Ms <= kMaxSlice) S = std::min(256 / base, ctx_tiles / (2 * rb));
   else {
