@@ -51,7 +51,10 @@ typedef struct yka_kv_config {
 
 /* replaces the KV reservation of yskn_open (yskn_abi.h:22; engine35.cpp:303-329). NULL on error.  Refused before any
  * device call: a configuration outside the ranges above, more than 1024 KV heads, or n_layers x max_ctx x n_kv_heads that
- * describes more than 1 TiB of cache. */
+ * describes more than 1 TiB of cache.
+ * Beside the containers a handle reserves the partial results of its split attention, n_heads * (2 * head_dim + 8) bytes
+ * for each of 4096 (token, split) pairs: 26 MB with 24 heads of 128 channels, 51 MB with 256.  With max_rows > 64 (prefill chunks)
+ * the largest demand of any slice decides: with 4 KV heads up to 10,899 pairs (69 MB) at 128 channels, 5,376 (67 MB) at 256. */
 YKA_API yka_kv* yka_kv_open(const yka_kv_config* cfg);
 /* replaces yskn_close (yskn_abi.h:23) for the KV containers */
 YKA_API void yka_kv_close(yka_kv* kv);

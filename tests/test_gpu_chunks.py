@@ -120,3 +120,23 @@ def test_query_rows_that_are_not_numbers(native, ctx, bf16):
             assert not (out[touched].view(np.uint16) & 0x7fff).any(), splits
             if splits == 0:                                        # the other rows do not notice
                 assert np.array_equal(out[~touched].view(np.uint16), clean[~touched].view(np.uint16))
+
+
+@pytest.mark.parametrize("dim,max_rows,pairs", [(128, 64, 4096), (128, 128, 4096), (128, 2048, 10899), (256, 341, 4096), (256, 2048, 5376)])
+def test_a_handle_reserves_what_its_slices_can_use(native, dim, max_rows, pairs):
+    """24 * (2 dim + 8) bytes for each (token, split) pair; everything else this handle holds is below 2 MB."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_bytes():
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    with native.KvCache(max_ctx=256, max_rows=max_rows, head_dim=dim):
+        pass                                                       # whatever the runtime itself keeps is there from now on
+    before = free_bytes()
+    with native.KvCache(max_ctx=32768 if max_rows > 64 else 256, max_rows=max_rows, head_dim=dim) as kv:
+        used = before - free_bytes()
+        cache = kv.max_ctx * 4 * (2 * (dim // 2) + (16 if dim == 128 else 8))
+    assert used - cache <= pairs * 24 * (2 * dim + 8) + (10 << 20), used       # each of six allocations rounds up to 2 MB at most

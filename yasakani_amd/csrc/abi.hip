@@ -105,9 +105,9 @@ void on_device(const yka_kv* kv) {
 }
 
 constexpr int kMaxSplits = 256;
-constexpr size_t kWsPairs = 4096;  // (token, split) pairs the partial workspace holds: 4096 * 24 * (256 + 8) bytes = 26 MB
-constexpr size_t kChunkPairs = 12288;   // where a handle takes prefill chunks (max_rows > 64): 2,048 rows x 6 splits, 78 MB
-size_t ws_pairs_of(const yka_kv* kv) { return kv->cfg.max_rows > kMaxSlice ? kChunkPairs : kWsPairs; }
+// (token, split) pairs of the partial workspace, n_heads * (2 * head_dim + 8) bytes each.  Windows and streams stay below kWsPairs (24
+// heads: 26 MB with 128 channels, 51 with 256); a slice of a prefill chunk may ask for more, kChunkPairs at most (ws_pairs_of)
+constexpr size_t kWsPairs = 4096, kChunkPairs = 12288;
 
 // splits for the narrow kernel: one workgroup per CU (256 of them) while a workgroup then walks at most 48 tiles - its
 // waves keep the next tile in flight, and half as many partial rows make the combiner cheaper (measured: 12.2 against
@@ -152,7 +152,7 @@ int mid_splits(const yka_kv* kv, int M, size_t ws_pairs = kWsPairs) {
 // device (chunk_splits_used: a chunk early in its context needs none); the grid provides the number between 1 and
 // kChunkMaxSplits that fills the rounds of 256 workgroups best on a long context - each split at least eight tiles of the
 // expected context, at most 2,048 workgroups and the partial workspace.
-constexpr int kChunkSlice = 2048;
+constexpr int kChunkSlice = 2048, kMaxChunkSlice = 4096, kChunkSlice256 = 1024;
 int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
   if (kv->opt_splits_wide > 0) return std::max(1, std::min(kv->opt_splits_wide, (int)(ws_pairs / (size_t)Ms)));
   const int rb = (kG * Ms + 127) / 128, base = kv->cfg.n_kv_heads * rb;
@@ -181,7 +181,7 @@ int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
 // Of the wide ones: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
 // rounds of 256 workgroups best.
 struct Part256 { int Ms, S, rows_per_block; bool narrow; int s_short; };
-int slice256(const yka_kv* kv, int M) { return M > kMaxSlice && !kv->opt_force_narrow ? 1024 : kMaxSlice; }
+int slice256(const yka_kv* kv, int M) { return M > kMaxSlice && !kv->opt_force_narrow ? kChunkSlice256 : kMaxSlice; }
 Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
   const int ctx = kv->opt_ctx_hint > 0 ? std::min(kv->opt_ctx_hint, kv->cfg.max_ctx) : kv->cfg.max_ctx, ctx_tiles = (ctx + 31) / 32;
   const int Ms = std::min(slice, M - s0), rows = kG * Ms, rb = (rows + 127) / 128, base = kv->cfg.n_kv_heads * rb;
@@ -204,6 +204,18 @@ Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
   const size_t pairs = Ms > kMaxSlice ? kv->ws_rows : kWsPairs;
   S = std::min(std::max(narrow ? 2 : 1, std::min(kMaxSplits, S)), (int)(pairs / (size_t)Ms));
   return {Ms, S, ((rows + rb - 1) / rb + 15) / 16 * 16, narrow, two ? std::min(S, std::max(2, 256 / kv->cfg.n_kv_heads)) : 0};
+}
+
+// Pairs a handle reserves: what the longest demand among the slices its max_rows allows comes to (a context hint only lowers it, a
+// split count set by the caller is cut to what is there).  4 KV heads: 4,096 up to 341 rows, then up to 10,899 (1,557 rows x 7
+// splits, 69 MB at 128 channels), with 256 channels 5,376 (67 MB).  1,500 rows behind 131,072 tokens take 3.26 ms with the 7 splits
+// that fill their rounds and 4.33 with the 2 that 4,096 pairs hold.
+size_t ws_pairs_of(const yka_kv* kv) {
+  size_t need = kWsPairs;
+  const int longest = std::min(kv->cfg.max_rows, kv->r256() ? kChunkSlice256 : kMaxChunkSlice);
+  for (int Ms = kMaxSlice + 1; Ms <= longest; ++Ms)
+    need = std::max(need, (size_t)Ms * (kv->r256() ? part256(kv, Ms, 0, kChunkSlice256).S : chunk_splits(kv, Ms, kChunkPairs)));
+  return need;
 }
 
 void check_layer(const yka_kv* kv, int layer) {
@@ -489,6 +501,7 @@ yka_kv* yka_kv_open(const yka_kv_config* cfg) {
       HIPCHK(hipMalloc((void**)&kv->tables, ident.size() * 4));
       HIPCHK(hipMemcpy(kv->tables, ident.data(), ident.size() * 4, hipMemcpyHostToDevice));
     }
+    kv->ws_rows = kChunkPairs;                     // the bound the demand is taken under
     kv->ws_rows = ws_pairs_of(kv);
     const size_t np = kv->ws_rows * cfg->n_heads;
     HIPCHK(hipMalloc((void**)&kv->pm, np * 4));
@@ -537,7 +550,7 @@ int yka_set_opt(yka_kv* kv, int key, int value) {
     case 8: if (value < 0 || value > kMaxSlice) throw std::runtime_error("widest window of the mid kernel must be in [0, 64]"); kv->opt_mid_rows = value; break;
     case 9: if (value < 0 || value > kMaxSplits) throw std::runtime_error("splits must be in [0, 256]"); kv->opt_splits_mid = value; break;
     case 11: if (value != 0 && value != 1) throw std::runtime_error("row type must be 0 (fp16) or 1 (bf16)"); kv->opt_io_bf16 = value; break;
-    case 10: if (value != 0 && (value < 128 || value > 4096)) throw std::runtime_error("prefill slice must be 0 or in [128, 4096] tokens"); kv->opt_chunk_slice = value; break;
+    case 10: if (value != 0 && (value < 128 || value > kMaxChunkSlice)) throw std::runtime_error("prefill slice must be 0 or in [128, 4096] tokens"); kv->opt_chunk_slice = value; break;
     default: throw std::runtime_error("unknown option key");
   }
   YKA_CATCH_INT
