@@ -120,3 +120,34 @@ def test_row256_probe_rejects_bad_arguments(native):
     x = np.zeros((2, 256), np.float32)
     with pytest.raises(native.YkaError):
         native.kvx256_probe(x, 2, 0)
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("M,offset", [(1, 1), (17, 1), (40, 3), (33, 7)])
+def test_append_of_rows_that_start_anywhere(native, bf16, M, offset):
+    """yka_append reads 16 bytes a lane where both row tensors start on a 16-byte boundary and values one by one elsewhere: K, V or
+    both `offset` values behind a boundary give the bytes of the aligned call."""
+    from tests.test_zz_no_alloc import _Hip
+    rng = np.random.default_rng(M + offset)
+    rows = [_edge_rows(rng)[:4 * M].reshape(M, 4, 128).astype(np.float32) for _ in range(2)]
+    k, v = (native.bf16_bits(x) if bf16 else x.astype(np.float16).view(np.uint16) for x in rows)
+    hip = _Hip()
+    try:
+        with native.KvCache(n_layers=4, max_ctx=256, max_rows=64) as kv:
+            kv.set_opt(11, bf16)
+            d_pos = hip.alloc(4)
+            hip.upload(d_pos, np.array([250 - M], np.int32))
+            base = [hip.alloc(2 * k.size + 64) for _ in range(2)]
+            for layer, shift in enumerate([(0, 0), (offset, 0), (0, offset), (offset, offset)]):
+                at = [b + 2 * n for b, n in zip(base, shift)]
+                for p, x in zip(at, (k, v)):
+                    hip.upload(p, x)
+                kv.append(layer, at[0], at[1], M, d_pos)
+                hip.sync()
+            want = kv.export_rows(0, 0, 256)
+            assert want[0][:, 250 - M:250].any()
+            for layer in (1, 2, 3):
+                for a, b in zip(kv.export_rows(layer, 0, 256), want):
+                    assert np.array_equal(a, b), layer
+    finally:
+        hip.free_all()

@@ -192,6 +192,8 @@ def test_streams_of_very_different_lengths(native, dim, M):
         q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
         kv.poison_workspace()
         out = kv.ms_call(q, k, v, pos, slots)
+        good = [t for t in range(M) if t not in bad]
+        stored = {t: kv.export_rows(int(slots[t]), int(pos[t]), 1) for t in good}
         for t in range(M):
             if t in bad:
                 assert not (out[t].view(np.uint16) & 0x7fff).any()
@@ -199,7 +201,10 @@ def test_streams_of_very_different_lengths(native, dim, M):
             ref = kv.layer_call(int(slots[t]), q[t:t + 1], k[t:t + 1], v[t:t + 1], int(pos[t])).astype(np.float32)[0]
             # the same kernel arithmetic with another split count: fp16 partials and outputs, 2^-11 each, summed in fp32
             assert np.linalg.norm(out[t].astype(np.float32) - ref) <= 1e-3 * np.linalg.norm(ref), f"row {t}: stream of {pos[t]} tokens"
-        assert [kv.export_rows(int(slots[t]), int(pos[t]), 1)[0].any() for t in range(M) if t not in bad].count(False) == 0
+        for t in good:                                    # the rows the pass stored are the rows one-row calls have stored since
+            assert stored[t][0].any()
+            for a, b in zip(stored[t], kv.export_rows(int(slots[t]), int(pos[t]), 1)):
+                assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), f"row {t}"
 
 
 # 128-channel rows, numbers of streams whose whole splits leave a round of workgroups unfilled: long streams (48 tiles for each
@@ -226,3 +231,46 @@ def test_the_line_between_short_and_long_streams(native, M, per_round, more):
         for t in range(M):
             ref = kv.layer_call(int(slots[t]), q[t:t + 1], k[t:t + 1], v[t:t + 1], int(pos[t])).astype(np.float32)[0]
             assert np.linalg.norm(out[t] - ref) <= 1e-3 * np.linalg.norm(ref), f"row {t}: stream of {pos[t]} tokens"    # as above
+
+
+# A pass that stores its rows inside the attention launch, with many consecutive rows of one stream: they lie in several tiles, on
+# both sides of a split boundary and of a 256-token page, and every workgroup stores those it reads.  Short streams and rows
+# that name nothing between them, the rows in any order.  Stored bytes and outputs against the oracle.
+@pytest.mark.parametrize("dim", [128, 256])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("first,n", [(236, 58), (200, 40), (505, 56), (0, 60)])
+def test_many_rows_of_one_stream_in_one_pass(native, oracle, dim, paged, first, n):
+    rng = np.random.default_rng(first + n + dim)
+    half = lambda m, heads: rng.standard_normal((m, heads, dim)).astype(np.float16)    # noqa: E731
+    lens = [first, 3, 0, 65]
+    with native.KvCache(n_layers=4, head_dim=dim, max_ctx=CTX, max_rows=512, paged=paged) as kv:
+        refs = []
+        for s, m in enumerate(lens):
+            if paged:
+                kv.set_page_table(rng.permutation(CTX // 256).astype(np.int32), layer=s)
+            refs.append(oracle.Cache(CTX, 24, 4, dim))
+            if m:
+                k, v = half(m, 4), half(m, 4)
+                for p in range(0, m, 512):
+                    kv.append_host(s, k[p:p + 512], v[p:p + 512], p)
+                refs[s].append(k, v, 0)
+        slots = np.array([0] * n + [1, 2, 3, 7], np.int32)
+        pos = np.array(list(range(first, first + n)) + [3, 0, 65, 9], np.int32)
+        order = rng.permutation(n + 4)
+        slots, pos = slots[order], pos[order]
+        q, k, v = half(n + 4, 24), half(n + 4, 4), half(n + 4, 4)
+        kv.poison_workspace()
+        out = kv.ms_call(q, k, v, pos, slots)
+        for t in np.argsort(pos, kind="stable"):
+            if slots[t] < 4:
+                refs[slots[t]].append(k[t:t + 1], v[t:t + 1], int(pos[t]))
+        for t, s in enumerate(slots):
+            if s == 7:
+                assert not (out[t].view(np.uint16) & 0x7fff).any()
+            else:                                         # first keys of a stream: two fp16 spacings on values in [2, 4] (tolerances.py)
+                assert_attn_close(out[t:t + 1], refs[s].attend_f32(q[t:t + 1], int(pos[t]), want_f32=True)[1], f"row {t} stream {s}", two_spacings=pos[t] < 64)
+        for s in range(4):
+            held = lens[s] + (n if s == 0 else 1)
+            for a, b in zip(kv.export_rows(s, 0, CTX), (refs[s].kc, refs[s].ks, refs[s].vc, refs[s].vs)):
+                a, b = a[:, :held].copy().view(np.uint8), b[:, :held].copy().view(np.uint8)
+                assert np.array_equal(a, b), f"rows of stream {s}"

@@ -13,8 +13,9 @@ up to half a spacing OF THE VALUE'S OWN BINADE off the exact product; a row made
 [4, 8) but whose output lies in [2, 4) carries up to one output spacing of such error before the output itself is
 rounded, and lands two spacings (3.9e-3) from the oracle's rounded value when the oracle's fp32 result sits next to a
 rounding boundary.  This EXCEEDS the plain 2e-3 bar.  It needs very short contexts (a row of a handful of keys); two
-shapes of a randomized sweep hit it (tests/test_gpu_sweep.py keeps both), each in one output value.  Those tests, and only
-those, use `two_spacings=True`: values with |ref| in [2, 4] may be two fp16 spacings off, everything else as above.
+shapes of a randomized sweep hit it (tests/test_gpu_sweep.py keeps both), each in one output value.  Those tests, and the
+ones whose rows see fewer than 64 keys (chunks and streams on a nearly empty cache), use `two_spacings=True`: values with
+|ref| in [2, 4] may be two fp16 spacings off, everything else as above.
 """
 import numpy as np
 
