@@ -208,8 +208,8 @@ def trellis_figures(native, ctx=32768, L=16, bits=5, torch=None):
 
 
 def prefill_chunk(native, reps=5, opts=()):
-    """A 2048-row prefill chunk on 131072 cached tokens: one append launch, then two 1024-token slices through the wide
-    kernel (128 rows per workgroup) and their combiner launches.  4 containers x 76.7 MB."""
+    """A 2048-row prefill chunk on 131072 cached tokens: one append launch, then one slice through the wide kernel
+    (128 rows per workgroup) and its combiner launch.  4 containers x 76.7 MB."""
     ctx, M, L = 131072, 2048, 4
     q, k, v = synth(31, ctx, M)
     kv = native.KvCache(n_layers=L, max_ctx=ctx + M, max_rows=M)
@@ -295,7 +295,7 @@ def sweep(native, which=("verify", "decode", "paged", "prefill"), reps=8, out=sy
         fill_cache(kv, k, v, ctx, chunk=16384)
         for slice_len in (0, 512, 683, 1024, 1366, 2048):
             for S in (0, 1, 2, 3, 4, 6, 8):
-                if slice_len * S > 4096 or (slice_len == 0 and 1024 * S > 4096):
+                if (slice_len or M) * S > 10899:
                     continue                                  # more (token, split) pairs than the partial workspace holds
                 opts = ((10, slice_len), (2, S))
                 emit("prefill chunk 2048 rows at 131072", opts, timed(kv, L, q, k[ctx:], v[ctx:], ctx, opts))

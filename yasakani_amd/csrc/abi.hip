@@ -289,7 +289,7 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
   const Workspace W = ws ? *ws : Workspace{kv->pm, kv->pl, kv->pacc16, kWsPairs, kv->tickets};
   const int bf16 = kv->opt_io_bf16;                // type of the 16-bit rows that come in and of the outputs
   if (kv->tb) {
-    // trellis-coded rows: the encoder runs first (two launches); rows of at most 2 tokens (or option key 3) run on row
+    // trellis-coded rows: the encoder runs first (two launches; not in decode, see below); rows of at most 2 tokens (or option key 3) run on row
     // tiles of 2 tokens x 6 heads, wider slices on 128-row workgroups that decode every tile once into LDS
     const yka_kv::Tb& T = *kv->tb;
     check_tb_layer(kv, layer);
@@ -1229,13 +1229,8 @@ int yka_append_host(yka_kv* kv, int layer, const uint16_t* k16, const uint16_t* 
   HIPCHK(hipMemcpy(dk.p, k16, nk * 2, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(dv.p, v16, nk * 2, hipMemcpyHostToDevice));
   HIPCHK(hipDeviceSynchronize());
-  // bf16 rows pass through staging rows that hold max_rows rows: such a handle takes the rows in pieces of that many
-  const int piece = kv->opt_io_bf16 ? kv->cfg.max_rows : M;
-  const size_t per_row = (size_t)kv->cfg.n_kv_heads * kv->D();
-  for (int r0 = 0; r0 < M; r0 += piece) {
-    launch_set_int(kv->d_pos, pos + r0, kv->stream);
-    do_append(kv, layer, dk.as<uint16_t>() + r0 * per_row, dv.as<uint16_t>() + r0 * per_row, std::min(piece, M - r0), kv->d_pos, kv->stream);
-  }
+  launch_set_int(kv->d_pos, pos, kv->stream);
+  do_append(kv, layer, dk.as<uint16_t>(), dv.as<uint16_t>(), M, kv->d_pos, kv->stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(kv->stream));
   YKA_CATCH_INT

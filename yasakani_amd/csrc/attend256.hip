@@ -209,7 +209,7 @@ __device__ __forceinline__ void load_v256(const uint8_t* pg, int tp, const Offs2
 
 }  // namespace
 
-// grid (S, n_kv, ceil(M/TPT)), block 256 (4 waves, 2 waves per SIMD).  Workgroup = (split, kv head, TPT tokens x 6 heads):
+// grid (S, n_kv, ceil(M/TPT)), block 256 (4 waves; decode launches one workgroup per CU, streams and forced windows two).  Workgroup = (split, kv head, TPT tokens x 6 heads):
 // TPT = 2 for a single-stream pass; MS (multi-stream pass, reference: src/q35_atxpk_ms.cu:13-33): one token per row
 // tile, which reads the container and the position its row map names.
 template <bool MS>
