@@ -353,7 +353,7 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     A.in_bf16 = bf16;
     CombineArgs C{W.pm, W.pl, W.pacc16, S, Ms, NH, out16 + (size_t)s0 * NH * kD, kv->opt_unrot, bf16};
     if (chunk && !kv->opt_splits_wide) {
-      A.adapt = C.adapt = 1; C.d_pos = d_pos; C.tok0 = s0; C.n_kv = kv->cfg.n_kv_heads; C.max_ctx = kv->cfg.max_ctx;
+      A.adapt = C.adapt = chunk_tile_cap(kv->cfg.n_kv_heads * ((kG * Ms + 127) / 128)); C.d_pos = d_pos; C.tok0 = s0; C.n_kv = kv->cfg.n_kv_heads; C.max_ctx = kv->cfg.max_ctx;
       if (!kv->opt_unrot && mode != 2) { A.out16 = C.out16; C.direct = 1; }
     }
     // option key 7, rows of at most 2 tokens: the last workgroup of each column merges the splits inside the attention launch

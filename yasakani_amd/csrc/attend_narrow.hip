@@ -519,7 +519,7 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
   const int head = blockIdx.x, tid = threadIdx.x;
   int tok = blockIdx.y;
   if constexpr (ADAPT) {
-    A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S);
+    A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S, A.adapt);
     if (A.S == 1 && A.direct) return;
   }
   do {
@@ -612,7 +612,7 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineArgs A) {
 template <bool ADAPT>
 __global__ void __launch_bounds__(256) combine_rows_kernel(CombineArgs A) {
   if constexpr (ADAPT) {
-    A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S);
+    A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S, A.adapt);
     if (A.S == 1 && A.direct) return;
   }
   for (int row = blockIdx.x * 4 + (threadIdx.x >> 6); row < A.M * A.n_heads; row += ADAPT ? 4 * (int)gridDim.x : A.M * A.n_heads) {   // row = tok * n_heads + head

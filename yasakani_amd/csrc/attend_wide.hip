@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   __shared__ __align__(16) uint8_t lds[2][2][kLdsBuf];               // [group][buffer]
   const int n_rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block;
   const int pos = *A.d_pos;
-  if constexpr (CHUNK) { if (A.adapt) A.S = chunk_splits_used(pos, A.tok0, A.M, A.kv.n_kv, A.kv.max_ctx, A.S); }
+  if constexpr (CHUNK) { if (A.adapt) A.S = chunk_splits_used(pos, A.tok0, A.M, A.kv.n_kv, A.kv.max_ctx, A.S, A.adapt); }
   const int total = CHUNK ? A.S * A.kv.n_kv * n_rb : (int)gridDim.x;
   if (CHUNK && (int)blockIdx.x >= total) return;
   int pair, rb;
@@ -487,7 +487,14 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   const bool direct = CHUNK && A.S == 1 && A.out16;          // uniform over the grid
   if (!direct && vrow && h == 0) { A.pm[pidx] = m_run; A.pl[pidx] = l; }
   // a row none of whose scores is a number keeps the marker: the combiner drops its partial and writes zeros, and so does this
-  const bool none = direct && m_run < -1e29f;
+  // (behind a branch: 64 selects here, or 32 on the packed rows, are 0.2 us of a slice, as instructions fetched for nothing)
+  if (CHUNK && direct && __any(m_run < -1e29f)) {
+    const bool none = m_run < -1e29f;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = none ? 0.f : o[dt][r];
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int a0 = 0; a0 < 2; ++a0)
@@ -503,7 +510,6 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
         for (int c = 0; c < 8; ++c) y[c] = o[c & 3][4 * (2 * (c >> 2) + a0) + b] * inv;
         packed = pack_out8(y, 1);
       }
-      if (CHUNK && none) packed = make_uint4(0, 0, 0, 0);
       *reinterpret_cast<uint4*>(stage + j * kOPitch + (64 * a0 + 32 * h + 8 * b) * 2) = packed;
     }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");     // the wave reads back what its own lanes wrote

@@ -73,8 +73,8 @@ struct AttnArgs {
   // draws the last ticket merges the column's partials into out16 and puts the counter back to zero
   int* tickets = nullptr; uint16_t* out16 = nullptr; int out_bf16 = 0;
   int in_bf16 = 0;   // q16 / k16 / v16 are bf16 rows (rows16_to_f16)
-  // wide kernel, slice of a prefill chunk (launch_attend_chunk): adapt != 0 lets the device choose how many of the S launched
-  // splits the slice uses (chunk_splits_used); out16 != nullptr: a slice that uses one writes its output rows itself
+  // wide kernel, slice of a prefill chunk (launch_attend_chunk): adapt != 0 (chunk_tile_cap) lets the device choose how many of the
+  // S launched splits the slice uses (chunk_splits_used); out16 != nullptr: a slice that uses one writes its output rows itself
   // multi-stream pass: adapt != 0 shares the S * M workgroups of a kv head out by the streams' lengths (ms_share) and leaves the
   // shares in plan[M] for the combiner
   int adapt = 0;
@@ -257,26 +257,26 @@ __device__ __forceinline__ int wave_scan_add(int v) { return wave_scan(v, [](int
 // splits (39 + 39 in the attention, 23 in the combiners), 46 with one split (42 in the attention, which then waits for its
 // longest workgroup: 47 tiles; 48 and 44 while the choice went through LDS).  2,048 rows behind 131,072: the same with 2 splits of one slice as with 4 of two.
 constexpr int kChunkOverhead = 18, kChunkMaxSplits = 64;
-// price of s splits in those units.  The sums of workgroups times tiles are taken in 64 bits: with 2,048 rows on 4 KV heads they pass 2^31
-// at 11 M tokens, and the two readers of a choice have to agree on it
-__host__ __device__ constexpr long long chunk_price(int pos, int tok0, int M, int n_kv, int max_ctx, int s) {
-  auto tiles16 = [&](int rows) {                                     // of the row block that ends `rows` rows into the slice
-    const long long len = (long long)pos + tok0 + rows;
-    return (int)(((len < 0 ? 0 : len < max_ctx ? len : max_ctx) + 31) >> 5) * 16;
-  };
-  const int base = n_kv * ((kG * M + 127) / 128), n = base * s, idle = (256 - (n & 255)) & 255;   // workgroups, and CUs without one in the last round
-  const int lo = tiles16(M < 128 / kG + 1 ? M : 128 / kG + 1) / s + 16 * kChunkOverhead, hi = tiles16(M) / s + 16 * kChunkOverhead;
-  const long long rounds = ((long long)(n >> 1) * ((long long)lo + hi) >> 8) + ((long long)lo * idle >> 8), t = hi > rounds ? hi : rounds;
-  return s > 1 ? t + 96 + M * s / 13 : t;
+// Price of s splits in those units, for a slice whose first and last row blocks walk so many tiles.  Workgroups times tiles would pass 2^31
+// with 2,048 rows on 4 KV heads at 11 M tokens, and the two readers of a choice have to agree on it: the caller cuts the tiles at
+// chunk_tile_cap (which changes no choice: beyond it the overhead is nothing).  That limit comes from the host, in `adapt`; 64-bit
+// products or a unit chosen here cost 1 % of a prompt's first slice, as instructions fetched cold in front of everything else.
+__host__ __device__ constexpr unsigned chunk_price(int first, int last, int base, int M, int s) {
+  const unsigned lo = first * 16 / s + 16 * kChunkOverhead, hi = last * 16 / s + 16 * kChunkOverhead;
+  const unsigned n = (unsigned)base * s, idle = (256 - (n & 255)) & 255;        // workgroups, and CUs without one in the last round
+  const unsigned rounds = (n >> 1) * (lo + hi) / 256 + lo * idle / 256, t = hi > rounds ? hi : rounds;
+  return s > 1 ? t + 96 + (unsigned)(M * s) / 13 : t;
 }
-// (a constant expression cannot wrap: these would not compile in 32 bits)
-static_assert(chunk_price(1 << 24, 0, 2048, 4, 1 << 25, 2) > chunk_price(1 << 23, 0, 2048, 4, 1 << 25, 2), "longer contexts cost more");
-static_assert(chunk_price(0x7fffff00, 4096, 4096, 1024, 0x7fffff00, kChunkMaxSplits) > 0, "the largest container the library opens");
-__device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n_kv, int max_ctx, int S) {
-  const int s = (int)(threadIdx.x & 63) + 1;
+constexpr int chunk_tile_cap(int base) { return base < 64 ? 1 << 20 : (1 << 26) / base; }
+static_assert(chunk_price(chunk_tile_cap(384), chunk_tile_cap(384), 384, 2048, 2) * 10u < chunk_price(chunk_tile_cap(384), chunk_tile_cap(384), 384, 2048, 1) * 9u,
+              "two splits fill 768 of 768 places, one 384 of 512, also on the longest contexts");
+static_assert(chunk_price(chunk_tile_cap(4), chunk_tile_cap(4), 4, 22, 1) < 0x1fffffeu, "a price and a split count share 31 bits");
+__device__ __forceinline__ int chunk_splits_used(int pos, int tok0, int M, int n_kv, int max_ctx, int S, int tile_cap) {
+  const int base = n_kv * ((kG * M + 127) / 128), s = (int)(threadIdx.x & 63) + 1;
+  const int first = max(0, min(pos + tok0 + min(M, 128 / kG + 1), max_ctx)), last = max(0, min(pos + tok0 + M, max_ctx));
+  const unsigned t = chunk_price(min((first + 31) >> 5, tile_cap), min((last + 31) >> 5, tile_cap), base, M, s);
   // lowest price, then fewest splits: the largest key (lane 0 always has one)
-  const long long t = chunk_price(pos, tok0, M, n_kv, max_ctx, s);
-  const int key = s <= S ? 0x7fffffff - (((int)(t < 0x1fffffe ? t : 0x1fffffe) << 6) | (s - 1)) : 0;
+  const int key = s <= S ? 0x7fffffff - (int)((min(t, 0x1fffffeu) << 6) | (unsigned)(s - 1)) : 0;
   const int top = __builtin_amdgcn_readlane(wave_scan(key, [](int a, int b) { return max(a, b); }), 63);
   return ((0x7fffffff - top) & 63) + 1;
 }
