@@ -78,7 +78,7 @@ YKA_API const char* yka_build_info(void);
  * key 7: 1 = the decode kernel (128-channel rows of at most 2 tokens, multi-stream passes, no option key 4) merges its
  *        splits inside the attention launch: the workgroup that finishes a column last combines it.  0 (default) = a
  *        second launch combines.  Same results to within the summation order.  On MI355X the second launch is the faster
- *        form (12.0 against 18.9 us per layer call at 32k tokens): the hand-over between XCDs costs three dependent
+ *        form (11.4 against 20.9 us per layer call at 32k tokens): the hand-over between XCDs costs three dependent
  *        trips to memory (store acknowledged, ticket, loads), more than the gap between two kernels;
  * key 8: widest window (rows) that runs on the kernel for small windows (a wave owns whole tiles and walks the window's row
  *        tiles; 128-channel rows only).  0 = never, at most 64 (wider windows than 16 rows then run as blocks of 16
