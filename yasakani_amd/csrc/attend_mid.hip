@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
 #pragma unroll
       for (int c = 0; c < 8; ++c) v[c] = (_Float16)(acc[c] * inv);
       const size_t p = ((size_t)(tokb + R / kG) * A.S + split) * A.n_heads + kvh * kG + R % kG;
-      *reinterpret_cast<uint4*>(A.pacc16 + p * kD + c8) = __builtin_bit_cast(uint4, v);
+      store_partial16(A.pacc16 + p * kD + c8, __builtin_bit_cast(uint4, v));
       if (c8 == 0) { A.pm[p] = M2; A.pl[p] = L; }
     }
   };

@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
     if (Rr < row_end) {
       const size_t p = ((size_t)(Rr / kG) * A.S + split) * A.n_heads + kvh * kG + Rr % kG;
       const uint4 v = *reinterpret_cast<const uint4*>(stage + jr * kOPitch + chunk * 16);
-      *reinterpret_cast<uint4*>(A.pacc16 + p * kD2 + chunk * 8) = v;
+      store_partial16(A.pacc16 + p * kD2 + chunk * 8, v);
     }
   }
 }

@@ -521,7 +521,8 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
     if (Rr < nrows && Rr < (rb + 1) * RPB) {
       const size_t p = ((size_t)(Rr / kG) * A.S + split) * A.n_heads + kvh * kG + Rr % kG;   // S == 1: also the output row
       const uint4 v = *reinterpret_cast<const uint4*>(stage + jr * kOPitch + chunk * 16);
-      *reinterpret_cast<uint4*>((direct ? A.out16 : A.pacc16) + p * kD + chunk * 8) = v;
+      if constexpr (CHUNK) *reinterpret_cast<uint4*>((direct ? A.out16 : A.pacc16) + p * kD + chunk * 8) = v;   // a slice in several splits gains nothing from writing through
+      else store_partial16(A.pacc16 + p * kD + chunk * 8, v);
     }
   }
 }

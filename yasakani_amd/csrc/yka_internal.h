@@ -233,6 +233,18 @@ __device__ __forceinline__ uint4 pack_out8(const float* y, int bf16) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// 16 bytes of a partial row, written through the XCD's L2 (agent scope) as it leaves the workgroup.  The combiner runs on other XCDs, so
+// what lies dirty in an L2 when the launch ends is written back then, with nothing else running: 9.6 MB of partials of 24
+// rows in 32 splits kept the combiner waiting 5 us behind the last workgroup, where 1.4 us are usual.  Written through, the
+// rows of the workgroups that end early are out before the last one ends.  us per 16 layers, ordinary / nontemporal / written through: 24
+// rows of 256 channels at 9,001 tokens 396 / 370 / 363, 64 rows of 128 at 32,768 741 / 733 / 730, 8 rows at 12,037 229 / 225 /
+// 225.  Decode leaves a few 100 KB, which nobody waits for, and its stores are in the way of its end: 173 / 173 / 176 and 16 streams
+// 27.2 / 27.8 / 28.0 a pass; it keeps ordinary stores.
+__device__ __forceinline__ void store_partial16(uint16_t* p, uint4 v) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)p, u32x4{v.x, v.y, v.z, v.w}, "agent");
+}
+
 // Sums and maxima of the plans below run through lane-crossing moves (a shift inside rows of 16 lanes, then two row broadcasts),
 // not through LDS: a plan stands in front of everything else a workgroup does (multi-stream passes, 5 trellis streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128
 // channels 14.9 and 13.9).
