@@ -88,7 +88,8 @@ __device__ __forceinline__ void pv_done(f4 (&o)[8]) {
 // The static check in tests/test_isa_inflight_loads.py reports exactly that; it has to pass before this file runs on
 // a GPU.)
 template <int NRT>
-__global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
+__global__ void __launch_bounds__(256, 1) attend_mid_kernel(const int* p_pos, uint8_t* p_base, const int32_t* p_table, int p_n_kv, int p_max_ctx, int p_s, AttnArgs A) {
+  A.d_pos = p_pos; A.kv = KvView{p_base, p_table, p_n_kv, p_max_ctx}; A.S = p_s;
   constexpr int TB = (16 * NRT) / kG;          // tokens per row block
   __shared__ __align__(16) uint4 s_q[NRT * 4 * 64];                 // [row tile][scale group][lane]: B operands of the score MFMAs
   // wave merge: up to four row tiles are staged at once (one barrier for the whole merge), more go through two buffers
@@ -474,11 +475,11 @@ void launch_attend_mid(const AttnArgs& A, hipStream_t st) {
   const int tb = (16 * nrt) / kG, nb = (A.M + tb - 1) / tb;
   const dim3 grid(A.S, A.kv.n_kv, nb), block(256);
   switch (nrt) {
-    case 2: hipLaunchKernelGGL(attend_mid_kernel<2>, grid, block, 0, st, A); break;
-    case 3: hipLaunchKernelGGL(attend_mid_kernel<3>, grid, block, 0, st, A); break;
-    case 4: hipLaunchKernelGGL(attend_mid_kernel<4>, grid, block, 0, st, A); break;
-    case 5: hipLaunchKernelGGL(attend_mid_kernel<5>, grid, block, 0, st, A); break;
-    default: hipLaunchKernelGGL(attend_mid_kernel<6>, grid, block, 0, st, A); break;
+    case 2: hipLaunchKernelGGL(attend_mid_kernel<2>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
+    case 3: hipLaunchKernelGGL(attend_mid_kernel<3>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
+    case 4: hipLaunchKernelGGL(attend_mid_kernel<4>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
+    case 5: hipLaunchKernelGGL(attend_mid_kernel<5>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
+    default: hipLaunchKernelGGL(attend_mid_kernel<6>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
   }
 }
 

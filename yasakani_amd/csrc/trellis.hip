@@ -469,7 +469,7 @@ __device__ __forceinline__ void search_body(const TbEncArgs& A, const int block)
   A.scr[job * 256 + d] = (uint8_t)state;
 }
 template <bool BF>
-__global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) { search_body<BF>(A, blockIdx.x); }
+__global__ void __launch_bounds__(256) tb_search_kernel(const int* p_pos, const uint32_t* p_desc, TbEncArgs A) { A.d_pos = p_pos; A.desc = p_desc; search_body<BF>(A, blockIdx.x); }
 
 // Decode (one or two tokens, no depth table): the search for the new rows' codes and the attention over the rows already in
 // the cache need nothing from each other, and neither fills the chip - 72 or 144 workgroups, each a serial chain of 64
@@ -478,7 +478,8 @@ __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) { search_bo
 // (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 in four launches (search 9.3, select 4.7,
 // attention 12.5, combiner 4.5), 22.4 in three (13.7, 4.8, 5.3).
 template <int KB, bool BF>
-__global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(TbEncArgs E, TbAttnArgs A, int n_search) {
+__global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_pos, const uint32_t* p_desc, int n_search, TbEncArgs E, TbAttnArgs A) {
+  E.d_pos = A.d_pos = p_pos; E.desc = p_desc;
   if ((int)blockIdx.x < n_search) { search_body<BF>(E, blockIdx.x); return; }
   int split, kvh;
   tb_split_of(A, blockIdx.x - n_search, split, kvh);
@@ -545,7 +546,8 @@ __device__ __forceinline__ Coded code_trellis(const TbEncArgs& A, const Profile&
 // grid rows, block 256: codes the row (best multiplier of the search, or the flat quantizer), rebuilds what it decodes to,
 // packs the fields, stores payload / scale / projection coefficients
 template <bool BF>
-__global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
+__global__ void __launch_bounds__(256) tb_select_kernel(const int* p_pos, const uint32_t* p_desc, TbEncArgs A) {
+  A.d_pos = p_pos; A.desc = p_desc;
   __shared__ float part8[8];
   __shared__ float rot_buf[256];
   __shared__ uint8_t fld[256];
@@ -635,22 +637,22 @@ __global__ void __launch_bounds__(256) tb_unpack_kernel(const uint8_t* blob, con
 void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
   if (A.nrow <= 0) return;
   if (A.in_bf16) {                       // BF: k16 / v16 are bf16 rows
-    if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<true>, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
-    hipLaunchKernelGGL(tb_select_kernel<true>, dim3(A.nrow), dim3(256), 0, st, A);
+    if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<true>, dim3(A.nrow * A.nm), dim3(256), 0, st, A.d_pos, A.desc, A);
+    hipLaunchKernelGGL(tb_select_kernel<true>, dim3(A.nrow), dim3(256), 0, st, A.d_pos, A.desc, A);
     return;
   }
-  if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<false>, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
-  hipLaunchKernelGGL(tb_select_kernel<false>, dim3(A.nrow), dim3(256), 0, st, A);
+  if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<false>, dim3(A.nrow * A.nm), dim3(256), 0, st, A.d_pos, A.desc, A);
+  hipLaunchKernelGGL(tb_select_kernel<false>, dim3(A.nrow), dim3(256), 0, st, A.d_pos, A.desc, A);
 }
 void launch_tb_encode_attend(const TbEncArgs& E, const TbAttnArgs& A, int kb, hipStream_t st) {
   const int n_search = E.nrow * E.nm;
   const dim3 grid(n_search + A.S * A.n_kv);
-  if (kb == 4 && E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<4, true>), grid, dim3(256), 0, st, E, A, n_search);
-  else if (kb == 4) hipLaunchKernelGGL((tb_search_attend_kernel<4, false>), grid, dim3(256), 0, st, E, A, n_search);
-  else if (E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<5, true>), grid, dim3(256), 0, st, E, A, n_search);
-  else hipLaunchKernelGGL((tb_search_attend_kernel<5, false>), grid, dim3(256), 0, st, E, A, n_search);
-  if (E.in_bf16) hipLaunchKernelGGL(tb_select_kernel<true>, dim3(E.nrow), dim3(256), 0, st, E);
-  else hipLaunchKernelGGL(tb_select_kernel<false>, dim3(E.nrow), dim3(256), 0, st, E);
+  if (kb == 4 && E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<4, true>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
+  else if (kb == 4) hipLaunchKernelGGL((tb_search_attend_kernel<4, false>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
+  else if (E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<5, true>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
+  else hipLaunchKernelGGL((tb_search_attend_kernel<5, false>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
+  if (E.in_bf16) hipLaunchKernelGGL(tb_select_kernel<true>, dim3(E.nrow), dim3(256), 0, st, E.d_pos, E.desc, E);
+  else hipLaunchKernelGGL(tb_select_kernel<false>, dim3(E.nrow), dim3(256), 0, st, E.d_pos, E.desc, E);
 }
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t st) {

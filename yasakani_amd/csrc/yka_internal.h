@@ -90,6 +90,15 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
   int adapt = 0; int direct = 0; const int* d_pos = nullptr; int tok0 = 0; int n_kv = 0; int max_ctx = 0;
   const int2* plan = nullptr;   // partials of a multi-stream pass shared out by ms_share: first split and splits of every row
   int s_short = 0; };    // trellis decode: as in TbAttnArgs (d_pos is set then)
+// Kernels of the decode and small-window chain name what their first loads need as leading arguments of their own and are compiled
+// with -amdgpu-kernarg-preload-count: those arrive in scalar registers with the wave, and the position (the combiner's partials)
+// is asked for at once instead of 0.3 us later, behind the load of the argument block.  us per 16 layers without / with: one token at 32,741 tokens
+// 172.5 / 166.5, 8 rows at 12,037 223 / 217, one 5-bit trellis row at 16,001 382 / 371, one token at 1,003 115.4 / 113.8, 16
+// streams 27.1 / 26.7 a pass.  Not where it measured slower: the 256-channel kernels (273 / 280), wide windows (737 / 743).
+#define YKA_COMBINE_PARAMS const float *p_pm, const float *p_pl, const uint16_t *p_acc, const void *p_where, int p_s, int p_heads
+#define YKA_COMBINE_GIVE(A) (A).pm, (A).pl, (A).pacc16, (A).plan ? (const void*)(A).plan : (const void*)(A).d_pos, (A).S, (A).n_heads
+#define YKA_COMBINE_TAKE(A) \
+  A.pm = p_pm; A.pl = p_pl; A.pacc16 = p_acc; A.S = p_s; A.n_heads = p_heads; A.d_pos = static_cast<const int*>(p_where); A.plan = static_cast<const int2*>(p_where);
 // projection outputs xq [M][n_heads][128], xk / xv [M][n_kv][128] fp32 -> q16 and the cache rows at *d_pos + t
 struct PostArgs {
   KvView kv; const float* xq; const float* xk; const float* xv; int M; int n_heads; const int* d_pos;
