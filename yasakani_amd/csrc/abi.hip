@@ -45,7 +45,8 @@ struct yka_kv {
     int kb = 0, stride = 0, nm = 0, layers = 0; bool has_mu = false;   // layers: layers the profile has groups for
     uint8_t* blob = nullptr; uint32_t* desc = nullptr; int ngrp = 0; unsigned mult_off = 0; uint32_t* pairs = nullptr; float* gfac = nullptr; float* mu = nullptr;
     uint8_t* pool = nullptr; size_t layer_bytes = 0, pay_bytes = 0, scl_bytes = 0;
-    uint8_t* scr = nullptr; size_t scr_w_ofs = 0;
+    uint8_t* scr = nullptr; size_t scr_w_ofs = 0, scr_s_ofs = 0;
+    const float* mults = nullptr;    // scale multipliers, behind gfac
     float* stage = nullptr;          // fp32 K rows then V rows of one pass ([max_rows][n_kv][256] each): yka_attn_post -> encoder
     // 256 bytes in front of the first row: windows of the attention kernels begin in the word before a chunk
     uint8_t* kpay(int layer) const { return pool + 256 + (size_t)layer * layer_bytes; }
@@ -236,7 +237,8 @@ TbEncArgs tb_encoder_args(const yka_kv* kv, int layer, int container, const uint
   A.k16 = k16; A.v16 = v16; A.in_bf16 = kv->opt_io_bf16; A.d_pos = d_pos; A.layer = layer; A.tok0 = t0; A.n_kv = kv->cfg.n_kv_heads;
   A.max_ctx = kv->cfg.max_ctx;
   A.nrow = std::min(kTbTileTok, M - t0) * 2 * kv->cfg.n_kv_heads;
-  A.scr = T.scr; A.scr_w_ofs = T.scr_w_ofs;
+  A.scr = T.scr; A.scr_w_ofs = T.scr_w_ofs; A.scr_s_ofs = T.scr_s_ofs;
+  A.kb = T.kb; A.pairs = T.pairs; A.mu = T.has_mu ? T.mu : nullptr; A.mults = T.mults;
   A.pay0 = T.kpay(container); A.pay1 = T.vpay(container); A.scl0 = T.kscl(container); A.scl1 = T.vscl(container); A.stride = T.stride;
   return A;
 }
@@ -948,17 +950,19 @@ int yka_kv_set_profile(yka_kv* kv, const uint8_t* blob, size_t blob_len) {
   const size_t rows = (size_t)n_kv * kv->cfg.max_ctx;
   T->pay_bytes = rows * T->stride; T->scl_bytes = rows * 4; T->layer_bytes = 2 * T->pay_bytes + 2 * T->scl_bytes;
   const size_t jobs = (size_t)kTbTileTok * 2 * n_kv * I.nm;
-  T->scr_w_ofs = jobs * 256;
+  T->scr_w_ofs = jobs * 256; T->scr_s_ofs = T->scr_w_ofs + jobs * 32;
   HIPCHK(hipMalloc((void**)&T->blob, blob_len)); HIPCHK(hipMemcpy(T->blob, blob, blob_len, hipMemcpyHostToDevice));
   const std::vector<uint32_t> desc = tb_descriptors(blob, blob_len, I);
   T->ngrp = I.ngrp; T->mult_off = V.word(32);
   HIPCHK(hipMalloc((void**)&T->desc, desc.size() * 4)); HIPCHK(hipMemcpy(T->desc, desc.data(), desc.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc((void**)&T->pairs, pairs.size() * 4)); HIPCHK(hipMemcpy(T->pairs, pairs.data(), pairs.size() * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMalloc((void**)&T->gfac, gfac.size() * 4)); HIPCHK(hipMemcpy(T->gfac, gfac.data(), gfac.size() * 4, hipMemcpyHostToDevice));
+  gfac.resize((size_t)need + I.nm);
+  std::memcpy(gfac.data() + need, blob + V.multipliers(), (size_t)I.nm * 4);
+  HIPCHK(hipMalloc((void**)&T->gfac, gfac.size() * 4)); T->mults = T->gfac + need; HIPCHK(hipMemcpy(T->gfac, gfac.data(), gfac.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc((void**)&T->mu, mu.size() * 4)); HIPCHK(hipMemcpy(T->mu, mu.data(), mu.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc((void**)&T->pool, 256 + T->layer_bytes * kv->cfg.n_layers + 256));
   HIPCHK(hipMemset(T->pool, 0, 256 + T->layer_bytes * kv->cfg.n_layers + 256));     // unwritten rows: state 0 everywhere, scale 0
-  HIPCHK(hipMalloc((void**)&T->scr, T->scr_w_ofs + jobs * 32));
+  HIPCHK(hipMalloc((void**)&T->scr, T->scr_s_ofs + jobs * 4));
   HIPCHK(hipMalloc((void**)&T->stage, (size_t)2 * kv->cfg.max_rows * n_kv * 256 * sizeof(float)));
   HIPCHK(hipDeviceSynchronize());
   guard.done = true;

@@ -110,46 +110,29 @@ __device__ __forceinline__ float block_fold(float* part8, float v, float start) 
 }
 
 // ---- which row a block works on ----
+// Probe form: row r of the launch with its own group and position
 struct RowRef {
-  float x;             // element threadIdx.x of the row (after the optional rotation)
+  float x;             // element threadIdx.x of the row
   int group, pos;      // profile group and position
-  size_t index;        // probe form: the row's index in the arrays; cache form: kv head * max_ctx + position
-  int is_v;            // cache form: 0 K row, 1 V row
-  size_t container;    // cache form, multi-stream pass: byte offset of the row's container
-  bool valid;          // multi-stream pass: false if the row names no container
+  size_t index;        // the row's index in the arrays
 };
-// Probe form: rows with their own group and position.  Cache form: row r of the launch = (token r / (2 n_kv), K | V, kv head)
-template <bool BF>
-__device__ __forceinline__ RowRef locate_row(const TbEncArgs& A, int r, float* rot_buf) {
-  const int d = threadIdx.x;
-  RowRef R{};
-  R.valid = true;
-  if (A.yin) {
-    R.index = (size_t)(A.row0 + r);
-    R.group = A.grp[R.index]; R.pos = A.pos[R.index]; R.x = A.yin[R.index * 256 + d];
-  } else {
-    const int per_tok = 2 * A.n_kv, tok = A.tok0 + r / per_tok, within = r % per_tok;
-    R.is_v = within / A.n_kv;
-    const int kvh = within % A.n_kv;
-    if (A.rows.pos) {                                  // multi-stream pass: the row's own container and position
-      const int slot = A.rows.slot[tok];
-      R.pos = A.rows.pos[tok];
-      R.valid = slot >= 0 && slot < A.rows.n_slots;
-      R.container = R.valid ? (size_t)slot * A.rows.slot_bytes : 0;
-    } else {
-      R.pos = *A.d_pos + tok;
-    }
-    R.group = (A.layer * A.n_kv + kvh) * 2 + R.is_v;
-    const size_t src = ((size_t)tok * A.n_kv + kvh) * 256 + d;
-    R.x = A.k32 ? (R.is_v ? A.v32 : A.k32)[src] : row16_value((R.is_v ? A.v16 : A.k16)[src], BF);
-    R.index = (size_t)kvh * A.max_ctx + (size_t)max(0, min(R.pos, A.max_ctx - 1));
-  }
-  if (A.rot) R.x = rotate256(R.x, rot_buf, false);
-  return R;
+__device__ __forceinline__ RowRef locate_row(const TbEncArgs& A, int r) {
+  const size_t index = (size_t)(A.row0 + r);
+  return RowRef{A.yin[index * 256 + threadIdx.x], A.grp[index], A.pos[index], index};
+}
+// Cache form: row r of the launch = (token r / (2 n_kv), K | V, kv head)
+struct CacheRow { int tok, is_v, kvh, group; };
+__device__ __forceinline__ CacheRow cache_row(const TbEncArgs& A, int r) {
+  const int per_tok = 2 * A.n_kv, within = r % per_tok, is_v = within / A.n_kv, kvh = within % A.n_kv;
+  return CacheRow{A.tok0 + r / per_tok, is_v, kvh, (A.layer * A.n_kv + kvh) * 2 + is_v};
 }
 
 // ---- the step before coding (src/kvq_fast.cuh:63-76): remove the mean row, project out up to two directions with
 //      coefficients rounded to fp16, measure the rms of what is left ----
+__device__ __forceinline__ float rms_of(float sum_sq) {
+  const float rms = sqrtf(__fdiv_rn(sum_sq, 256.f));     // sqrtf is correctly rounded on this target
+  return rms == 0.f ? 1.f : rms;
+}
 struct Residual { float r, mean, coef[2], dir[2], rms; };
 __device__ __forceinline__ Residual residual_of(float* part8, const Profile& P, const GroupRec& G, float x) {
   const unsigned d = threadIdx.x;
@@ -163,9 +146,7 @@ __device__ __forceinline__ Residual residual_of(float* part8, const Profile& P, 
     Q.coef[k] = round_f16(block_fold<AddRn>(part8, __fmul_rn(Q.r, Q.dir[k]), 0.f));
     Q.r = __fsub_rn(Q.r, __fmul_rn(Q.coef[k], Q.dir[k]));
   }
-  const float mean_sq = __fdiv_rn(block_fold<AddRn>(part8, __fmul_rn(Q.r, Q.r), 0.f), 256.f);
-  Q.rms = sqrtf(mean_sq);                              // sqrtf is correctly rounded on this target
-  if (Q.rms == 0.f) Q.rms = 1.f;
+  Q.rms = rms_of(block_fold<AddRn>(part8, __fmul_rn(Q.r, Q.r), 0.f));
   return Q;
 }
 // scale tried for a multiplier: rms * multiplier rounded to fp32, then to fp16; 0 -> 1
@@ -438,19 +419,65 @@ __device__ __forceinline__ void wave_chunk3(const int* xi, const int (&ci4)[4], 
 }
 
 // grid rows * nm, block 256: block `job` = (row, multiplier); wave c = chunk c.  Writes the 256 states of the row under this
-// multiplier and the 8 partial error sums to scratch.
-template <bool BF>
+// multiplier and the 8 partial error sums to scratch; cache form: the scale that was tried as well.
+struct SearchLds {
+  float part8[8];
+  int target[256];
+  uint8_t back[4][64 * 32];
+  uint8_t chosen[256];
+  int16_t table[256];
+};
+// the end of a job: squared error of this multiplier (element d of the row is lane d & 63 of wave d >> 6; summed per run of 32
+// elements) and the states
+__device__ __forceinline__ void leave_job(const TbEncArgs& A, SearchLds& L, size_t job, float r, float s, float gain) {
+  const int d = threadIdx.x, state = L.chosen[d];
+  const float miss = __fsub_rn(r, __fmul_rn(table_value((int)L.table[state], gain), s));
+  const float sq = run_fold<AddRn>(__fmul_rn(miss, miss));
+  if ((d & 31) == 0) reinterpret_cast<float*>(A.scr + A.scr_w_ofs)[job * 8 + (d >> 5)] = sq;
+  A.scr[job * 256 + d] = (uint8_t)state;
+}
+// integer target of an element: the residual in units of s / 256, clamped
+__device__ __forceinline__ int target_of(float r, float s) {
+  return (int)fminf(fmaxf(rintf(__fmul_rn(__fdiv_rn(r, s), 256.f)), -2048.f), 2048.f);
+}
+// Cache form.  The profile of a handle is trellis-coded throughout with KB bits, without guard positions and directions
+// (yka_kv_set_profile), and its tables and mean rows lie in arrays indexed by the group: the row, the table, the mean, the gain and
+// the multiplier are asked for together, in one trip to memory (through the group's record they were three: a block of a
+// 16-row window reached its first step after 3.8 us).  The position is not needed here.
+template <int KB, bool BF>
 __device__ __forceinline__ void search_body(const TbEncArgs& A, const int block) {
-  __shared__ float part8[8];
+  __shared__ __align__(16) SearchLds L;
   __shared__ float rot_buf[256];
-  __shared__ int target[256];
-  __shared__ __align__(16) uint8_t back[4][64 * 32];
-  __shared__ uint8_t chosen[256];
-  __shared__ int16_t table[256];
-  const int d = threadIdx.x, wave = d >> 6, lane = d & 63;
+  const int d = threadIdx.x, wave = d >> 6;
   const int row = block / A.nm, mult = block % A.nm;
+  const CacheRow R = cache_row(A, row);
+  const size_t src = ((size_t)R.tok * A.n_kv + R.kvh) * 256 + d;
+  float x = A.k32 ? (R.is_v ? A.v32 : A.k32)[src] : row16_value((R.is_v ? A.v16 : A.k16)[src], BF);
+  // the first 256 entries of the group's pair table hold the table: entry i ends with the value of state i, an exact integer
+  const uint32_t pair = A.pairs[((size_t)R.group << (8 + KB)) + d];
+  const float mean = A.mu ? A.mu[(size_t)R.group * 256 + d] : 0.f;
+  const float gain = __uint_as_float(A.desc[8 * (size_t)R.group + 5]), mult_value = A.mults[mult];
+  if (A.rot) x = rotate256(x, rot_buf, false);
+  L.table[d] = (int16_t)(int)__half2float(__ushort_as_half((uint16_t)(pair >> 16)));
+  const float r = A.mu ? __fsub_rn(x, mean) : x;
+  const float s = trial_scale(rms_of(block_fold<AddRn>(L.part8, __fmul_rn(r, r), 0.f)), mult_value);    // its barriers publish the table
+  const StepConsts C = step_consts<KB>([&](int state) { return (int)L.table[state]; });
+  L.target[d] = target_of(r, s);
+  __syncthreads();
+  wave_chunk<KB>(L.target + 64 * wave, C, L.back[wave], L.chosen + 64 * wave);
+  const size_t job = (size_t)row * A.nm + mult;
+  leave_job(A, L, job, r, s, gain);
+  if (d == 0) reinterpret_cast<float*>(A.scr + A.scr_s_ofs)[job] = s;
+}
+template <int KB, bool BF>
+__global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) { search_body<KB, BF>(A, blockIdx.x); }
+// Probe form: any profile, every row with its own group
+__global__ void __launch_bounds__(256) tb_search_probe_kernel(TbEncArgs A) {
+  __shared__ __align__(16) SearchLds L;
+  const int d = threadIdx.x, wave = d >> 6, lane = d & 63;
+  const int row = blockIdx.x / A.nm, mult = blockIdx.x % A.nm;
   const Profile P{A.blob, A.desc, A.ngrp, A.mult_off};
-  const RowRef R = locate_row<BF>(A, row, rot_buf);
+  const RowRef R = locate_row(A, row);
   const GroupRec G = read_group(P, R.group);
   if (!G.present || R.pos < G.guard || G.mode != 0) return;                // uniform over the block: nothing to search
   // everything the search needs from memory is requested before the residual's block reductions
@@ -465,25 +492,16 @@ __device__ __forceinline__ void search_body(const TbEncArgs& A, const int block)
     for (int k = 0; k < 4; ++k) ci4[k] = tab(lane + 64 * k);
   }
   const float mult_value = P.multiplier(mult);
-  table[d] = (int16_t)tab(d);                            // published by the barriers of the block reductions
-  const Residual Q = residual_of(part8, P, G, R.x);
+  L.table[d] = (int16_t)tab(d);                          // published by the barriers of the block reductions
+  const Residual Q = residual_of(L.part8, P, G, R.x);
   const float s = trial_scale(Q.rms, mult_value);
-  // integer target of element d: the residual in units of s / 256, clamped
-  target[d] = (int)fminf(fmaxf(rintf(__fmul_rn(__fdiv_rn(Q.r, s), 256.f)), -2048.f), 2048.f);
+  L.target[d] = target_of(Q.r, s);
   __syncthreads();
-  if (G.bits == 5) wave_chunk<5>(target + 64 * wave, C, back[wave], chosen + 64 * wave);
-  else if (G.bits == 4) wave_chunk<4>(target + 64 * wave, C, back[wave], chosen + 64 * wave);
-  else wave_chunk3(target + 64 * wave, ci4, back[wave], chosen + 64 * wave);
-  // squared error of this multiplier: element d of the row is lane `lane` of wave `wave`; summed per run of 32 elements
-  const int state = chosen[d];
-  const float miss = __fsub_rn(Q.r, __fmul_rn(table_value((int)table[state], T.gain), s));
-  const float sq = run_fold<AddRn>(__fmul_rn(miss, miss));
-  const size_t job = (size_t)row * A.nm + mult;
-  if ((d & 31) == 0) reinterpret_cast<float*>(A.scr + A.scr_w_ofs)[job * 8 + (d >> 5)] = sq;
-  A.scr[job * 256 + d] = (uint8_t)state;
+  if (G.bits == 5) wave_chunk<5>(L.target + 64 * wave, C, L.back[wave], L.chosen + 64 * wave);
+  else if (G.bits == 4) wave_chunk<4>(L.target + 64 * wave, C, L.back[wave], L.chosen + 64 * wave);
+  else wave_chunk3(L.target + 64 * wave, ci4, L.back[wave], L.chosen + 64 * wave);
+  leave_job(A, L, (size_t)row * A.nm + mult, Q.r, s, T.gain);
 }
-template <bool BF>
-__global__ void __launch_bounds__(256) tb_search_kernel(const int* p_pos, const uint32_t* p_desc, TbEncArgs A) { A.d_pos = p_pos; A.desc = p_desc; search_body<BF>(A, blockIdx.x); }
 
 // Decode (one or two tokens, no depth table): the search for the new rows' codes and the attention over the rows already in
 // the cache need nothing from each other, and neither fills the chip - 72 or 144 workgroups, each a serial chain of 64
@@ -492,9 +510,9 @@ __global__ void __launch_bounds__(256) tb_search_kernel(const int* p_pos, const 
 // (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 in four launches (search 9.3, select 4.7,
 // attention 12.5, combiner 4.5), 22.4 in three (13.7, 4.8, 5.3).
 template <int KB, bool BF>
-__global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_pos, const uint32_t* p_desc, int n_search, TbEncArgs E, TbAttnArgs A) {
-  E.d_pos = A.d_pos = p_pos; E.desc = p_desc;
-  if ((int)blockIdx.x < n_search) { search_body<BF>(E, blockIdx.x); return; }
+__global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_pos, int n_search, TbEncArgs E, TbAttnArgs A) {
+  A.d_pos = p_pos;
+  if ((int)blockIdx.x < n_search) { search_body<KB, BF>(E, blockIdx.x); return; }
   int split, kvh;
   tb_split_of(A, blockIdx.x - n_search, split, kvh);
   tbd::attend_tb_body<KB, false>(A, split, kvh, 0, true);
@@ -557,18 +575,54 @@ __device__ __forceinline__ Coded code_trellis(const TbEncArgs& A, const Profile&
   return Coded{state & ((1 << G.bits) - 1), G.bits, s, value, true};
 }
 
+// What a row is stored as after the search (cache form), by a wave: the multiplier whose search left the smallest squared error (its 8
+// partial sums added in order from 0; the first of equal errors), the four states of elements 4 lane .. 4 lane + 3 it chose, its scale.
+__device__ __forceinline__ void pick_job(const TbEncArgs& A, int row, int lane, uint32_t& states, float& scale) {
+  const size_t job0 = (size_t)row * A.nm;
+  uint32_t all[kMaxMult];
+#pragma unroll
+  for (int i = 0; i < kMaxMult; ++i) all[i] = i < A.nm ? reinterpret_cast<const uint32_t*>(A.scr + (job0 + i) * 256)[lane] : 0u;
+  float4 e0 = make_float4(0, 0, 0, 0), e1 = e0;
+  float s = 0.f;
+  if (lane < A.nm) {
+    const float4* err = reinterpret_cast<const float4*>(A.scr + A.scr_w_ofs) + (job0 + lane) * 2;
+    e0 = err[0]; e1 = err[1];
+    s = reinterpret_cast<const float*>(A.scr + A.scr_s_ofs)[job0 + lane];
+  }
+  float total = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) total = __fadd_rn(total, (&e0.x)[k]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) total = __fadd_rn(total, (&e1.x)[k]);
+  float least = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(total), 0));
+  int keep = 0;
+  states = all[0];
+#pragma unroll
+  for (int i = 1; i < kMaxMult; ++i) {
+    const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(total), i));
+    const bool better = i < A.nm && v < least;           // uniform over the wave
+    least = better ? v : least; keep = better ? i : keep; states = better ? all[i] : states;
+  }
+  scale = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s), __builtin_amdgcn_readfirstlane(keep)));
+}
+// packs and stores the fields of those states (fld: 256 bytes of LDS private to the wave)
+template <int KB>
+__device__ __forceinline__ void store_coded_row(uint8_t* dst, uint8_t* fld, int lane, uint32_t states) {
+  reinterpret_cast<uint32_t*>(fld)[lane] = states & (0x01010101u * ((1u << KB) - 1u));
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  if (lane < 8 * KB) reinterpret_cast<uint32_t*>(dst)[lane] = pack_word<KB>(fld, lane);
+}
+
 // grid rows, block 256: codes the row (best multiplier of the search, or the flat quantizer), rebuilds what it decodes to,
 // packs the fields, stores payload / scale / projection coefficients
-template <bool BF>
-__global__ void __launch_bounds__(256) tb_select_kernel(const int* p_pos, const uint32_t* p_desc, TbEncArgs A) {
-  A.d_pos = p_pos; A.desc = p_desc;
+// (probe form)
+__global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
   __shared__ float part8[8];
-  __shared__ float rot_buf[256];
   __shared__ uint8_t fld[256];
   __shared__ float totals[kMaxMult], mults[kMaxMult];
   const int d = threadIdx.x, row = blockIdx.x;
   const Profile P{A.blob, A.desc, A.ngrp, A.mult_off};
-  const RowRef R = locate_row<BF>(A, row, rot_buf);
+  const RowRef R = locate_row(A, row);
   const GroupRec G = read_group(P, R.group);
   Coded C{0, 4, 1.f, R.x, false};
   float rebuilt = R.x;                                   // rows that stay uncoded come back as they are
@@ -586,10 +640,8 @@ __global__ void __launch_bounds__(256) tb_select_kernel(const int* p_pos, const 
     if (G.has_mean) rebuilt = __fadd_rn(rebuilt, Q.mean);
     coef_bits = (unsigned)__half_as_ushort(__float2half_rn(Q.coef[0])) | ((unsigned)__half_as_ushort(__float2half_rn(Q.coef[1])) << 16);
   }
-  const bool storable = A.yin || (R.valid && R.pos >= 0 && R.pos < A.max_ctx && (A.pos_limit == 0 || R.pos < A.pos_limit));
-  uint8_t* const plane = R.is_v ? A.pay1 : A.pay0;
-  if (plane && storable) {
-    uint32_t* const words = reinterpret_cast<uint32_t*>(plane + R.container + R.index * (size_t)A.stride);
+  if (A.pay0) {
+    uint32_t* const words = reinterpret_cast<uint32_t*>(A.pay0 + R.index * (size_t)A.stride);
     fld[d] = (uint8_t)C.field;
     __syncthreads();
     if (d < (A.stride >> 2)) {
@@ -598,13 +650,36 @@ __global__ void __launch_bounds__(256) tb_select_kernel(const int* p_pos, const 
       words[d] = w;
     }
     if (d == 0) {
-      float* const scales = R.is_v ? A.scl1 : A.scl0;
-      if (scales) reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(scales) + R.container)[R.index] = C.scale;
       if (A.side) { A.side[2 * R.index] = __float_as_uint(C.scale); A.side[2 * R.index + 1] = coef_bits; }
       if (A.coded) A.coded[R.index] = C.any ? 1 : 0;
     }
   }
   if (A.yout) A.yout[R.index * 256 + d] = rebuilt;
+}
+
+// Cache form: a wave per row.  Every multiplier's states (a word of four per lane), error sums and scale are requested at once with the
+// position; what the row is coded with then costs no further trip: the search has left the scales, so neither the row nor its
+// mean is read again.
+template <int KB>
+__global__ void __launch_bounds__(256) tb_store_kernel(const int* p_pos, const uint8_t* p_scr, int p_nm, TbEncArgs A) {
+  A.d_pos = p_pos; A.scr = const_cast<uint8_t*>(p_scr); A.nm = p_nm;
+  __shared__ uint32_t fld[4][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = blockIdx.x * 4 + wave;
+  if (row >= A.nrow) return;                             // no barrier below
+  uint32_t states; float scale;
+  pick_job(A, row, lane, states, scale);
+  const CacheRow R = cache_row(A, row);
+  int pos; size_t container = 0; bool ok = true;
+  if (A.rows.pos) {                                      // multi-stream pass: the row's own container and position
+    const int slot = A.rows.slot[R.tok];
+    pos = A.rows.pos[R.tok];
+    ok = slot >= 0 && slot < A.rows.n_slots;
+    if (ok) container = (size_t)slot * A.rows.slot_bytes;
+  } else pos = *A.d_pos + R.tok;
+  if (!ok || pos < 0 || pos >= A.max_ctx || (A.pos_limit != 0 && pos >= A.pos_limit)) return;
+  const size_t index = (size_t)R.kvh * A.max_ctx + (size_t)pos;
+  store_coded_row<KB>((R.is_v ? A.pay1 : A.pay0) + container + index * (size_t)A.stride, reinterpret_cast<uint8_t*>(fld[wave]), lane, states);
+  if (lane == 0) reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(R.is_v ? A.scl1 : A.scl0) + container)[index] = scale;
 }
 
 // n <= 13 bits that start at bit `first` of an MSB-first stream of words (bits past the last word read as zero)
@@ -648,25 +723,33 @@ __global__ void __launch_bounds__(256) tb_unpack_kernel(const uint8_t* blob, con
 
 }  // namespace
 
+template <int KB>
+static void launch_store(const TbEncArgs& A, hipStream_t st) {
+  hipLaunchKernelGGL(tb_store_kernel<KB>, dim3((A.nrow + 3) / 4), dim3(256), 0, st, A.d_pos, A.scr, A.nm, A);
+}
+template <int KB>
+static void launch_encode(const TbEncArgs& A, hipStream_t st) {
+  if (A.in_bf16) hipLaunchKernelGGL((tb_search_kernel<KB, true>), dim3(A.nrow * A.nm), dim3(256), 0, st, A);   // k16 / v16 are bf16 rows
+  else hipLaunchKernelGGL((tb_search_kernel<KB, false>), dim3(A.nrow * A.nm), dim3(256), 0, st, A);
+  launch_store<KB>(A, st);
+}
 void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
   if (A.nrow <= 0) return;
-  if (A.in_bf16) {                       // BF: k16 / v16 are bf16 rows
-    if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<true>, dim3(A.nrow * A.nm), dim3(256), 0, st, A.d_pos, A.desc, A);
-    hipLaunchKernelGGL(tb_select_kernel<true>, dim3(A.nrow), dim3(256), 0, st, A.d_pos, A.desc, A);
+  if (A.yin) {
+    if (A.has_trellis) hipLaunchKernelGGL(tb_search_probe_kernel, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
+    hipLaunchKernelGGL(tb_select_kernel, dim3(A.nrow), dim3(256), 0, st, A);
     return;
   }
-  if (A.has_trellis) hipLaunchKernelGGL(tb_search_kernel<false>, dim3(A.nrow * A.nm), dim3(256), 0, st, A.d_pos, A.desc, A);
-  hipLaunchKernelGGL(tb_select_kernel<false>, dim3(A.nrow), dim3(256), 0, st, A.d_pos, A.desc, A);
+  if (A.kb == 4) launch_encode<4>(A, st); else launch_encode<5>(A, st);
 }
 void launch_tb_encode_attend(const TbEncArgs& E, const TbAttnArgs& A, int kb, hipStream_t st) {
   const int n_search = E.nrow * E.nm;
   const dim3 grid(n_search + A.S * A.n_kv);
-  if (kb == 4 && E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<4, true>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
-  else if (kb == 4) hipLaunchKernelGGL((tb_search_attend_kernel<4, false>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
-  else if (E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<5, true>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
-  else hipLaunchKernelGGL((tb_search_attend_kernel<5, false>), grid, dim3(256), 0, st, A.d_pos, E.desc, n_search, E, A);
-  if (E.in_bf16) hipLaunchKernelGGL(tb_select_kernel<true>, dim3(E.nrow), dim3(256), 0, st, E.d_pos, E.desc, E);
-  else hipLaunchKernelGGL(tb_select_kernel<false>, dim3(E.nrow), dim3(256), 0, st, E.d_pos, E.desc, E);
+  if (kb == 4 && E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<4, true>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
+  else if (kb == 4) hipLaunchKernelGGL((tb_search_attend_kernel<4, false>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
+  else if (E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<5, true>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
+  else hipLaunchKernelGGL((tb_search_attend_kernel<5, false>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
+  if (kb == 4) launch_store<4>(E, st); else launch_store<5>(E, st);
 }
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t st) {

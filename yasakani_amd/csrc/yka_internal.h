@@ -130,6 +130,9 @@ struct TbEncArgs {
   float* yout; uint32_t* side; int* coded;
   int nrow;
   uint8_t* scr; size_t scr_w_ofs;     // scratch: states [nrow * nm][256] bytes, then at scr_w_ofs error sums [nrow * nm][8] fp32
+  // cache form (every group trellis-coded with kb bits, no guard positions, no directions): pair tables and mean rows by group (TbAttnArgs),
+  // multipliers as aligned floats, and in the scratch at scr_s_ofs the scale every job tried [nrow * nm] fp32
+  int kb; const uint32_t* pairs; const float* mu; const float* mults; size_t scr_s_ofs;
   uint8_t* pay0; uint8_t* pay1; float* scl0; float* scl1; int stride;
   int pos_limit;                      // cache form: rows at positions >= pos_limit are not stored (0: no limit besides max_ctx)
   RowMap rows;                        // cache form, multi-stream pass: token t sits at rows.pos[t] of container rows.slot[t] (pay / scl = container 0)
