@@ -86,3 +86,30 @@ def test_rows_that_are_not_numbers(native, kk, M, bad, which):
     assert np.array_equal(np.isnan(out), np.isnan(ref)) and np.array_equal(out[touched] == 0, ref[touched] == 0)
     # as in test_against_the_general_path
     assert np.linalg.norm(out[~touched] - ref[~touched]) <= 1e-3 * np.linalg.norm(ref[~touched])
+
+
+@pytest.mark.parametrize("kk", [4, 5])
+@pytest.mark.parametrize("heads,n_mult", [(1, 1), (1, 16), (2, 9), (3, 2)])
+@pytest.mark.parametrize("M,post", [(1, False), (2, False), (3, False), (5, False), (1, True)])
+def test_rows_as_the_oracle_codes_them(native, oracle, kk, heads, n_mult, M, post):
+    """Rows coded by the combiner of a decode pass (M <= 2) and by a wave per row (wider; `post`: fp32 rows), in handles whose rows do not fill
+    the waves of a workgroup (2 to 30 rows, four to a workgroup), with one multiplier and with as many as a profile may have."""
+    from yasakani_amd import kvqp
+    blob = kvqp.synthetic(layers=1, kv_heads=heads, kk=kk, seed=kk, n_mult=n_mult, mu=M == 2)
+    rng = np.random.default_rng(10 * M + heads)
+    k, v = (rng.standard_normal((M, heads, 256)).astype(np.float16) for _ in range(2))
+    k[0, 0] = 0                                                    # a row of zeros: its residual has no length
+    q = rng.standard_normal((M, 6 * heads, 256)).astype(np.float16)
+    pos = 256 - M                                                  # up to the last row of the container
+    with native.KvCache(n_heads=6 * heads, n_kv_heads=heads, max_ctx=256, head_dim=256, max_rows=8) as kv:
+        kv.set_profile(blob)
+        if post:
+            kv.append256_f32_host(0, k.astype(np.float32), v.astype(np.float32), pos, rotate=False)
+        else:
+            kv.layer_call(0, q, k, v, pos)
+        kw, ks, vw, vs = kv.export_rows(0, pos, M)
+    for kind, x, words, scales in ((0, k, kw, ks), (1, v, vw, vs)):
+        for h in range(heads):
+            ref = oracle.tb_encode_rows(blob, np.full(M, 2 * h + kind, np.int32), np.arange(M, dtype=np.int32), x[:, h].astype(np.float32))
+            assert np.array_equal(words[h], ref["words"][:, :8 * kk]), (kind, h)
+            assert np.array_equal(np.asarray(scales[h]).view(np.uint32), np.asarray(ref["scale"]).view(np.uint32)), (kind, h)

@@ -308,8 +308,9 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
       CombineArgs C{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
       A.s_short = C.s_short = P.s_short; C.d_pos = d_pos;
       if (fuse) {
-        launch_tb_encode_attend(tb_encoder_args(kv, layer, layer, k16, v16, 0, M, d_pos), A, T.kb, st);
-        launch_combine256_new(C, A, T.kb, st);
+        const TbEncArgs E = tb_encoder_args(kv, layer, layer, k16, v16, 0, M, d_pos);
+        launch_tb_encode_attend(E, A, T.kb, st);
+        launch_combine256_new(C, A, tb_jobs(E), T.kb, st);
         return;
       }
       if (P.narrow) launch_attend_tb(A, T.kb, st); else launch_attend_tb_wide(A, T.kb, st);

@@ -16,6 +16,7 @@
 #include "yka_internal.h"
 #include "rot256_device.h"
 #include "merge256_device.h"
+#include "tb_store_device.h"
 #include <hip/hip_fp16.h>
 
 namespace yka {
@@ -427,19 +428,12 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
 // 32 and keeps the register count low where thousands of workgroups run (wide windows).
 // MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
 // KB != 0: partials of launch_tb_encode_attend, which leave out the rows of the pass; token t also sees the keys *d_pos + u, u <=
-// t, which are decoded here from the rows the encoder has stored (thread = channel; N names them) and join the sum as
-// splits of one key each, in fp32.
-template <int KB> struct NewKeyArgs { TbAttnArgs N; };
+// t, which join the sum as splits of one key each, in fp32 (thread = channel; N names the rows).  The searches have left what the
+// rows may be coded with: wave 2 u + v of a workgroup picks the code of the K (v = 0) or V row of token u, and the workgroups of a kv head's first
+// query head store them.  Everything that takes is requested with the partials.  5 bits at 16,001 tokens, 16 layers: 356 us with a
+// launch between that stored the rows and their values read back here, 312 us so.
+template <int KB> struct NewKeyArgs { TbAttnArgs N; TbJobs J; };
 template <> struct NewKeyArgs<0> {};
-// table integer of element d of a trellis-coded row: the last 8 stream bits up to the end of its field name the state
-template <int KB>
-__device__ __forceinline__ float tb_element(const uint8_t* row, int d, const uint32_t* pairs) {
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(row) + (d >> 6) * (2 * KB);
-  const int last = KB * ((d & 63) + 1) - 1, j = last >> 5;
-  const uint32_t lo = w[j], hi = j > 0 ? w[j - 1] : 0u;
-  const uint32_t state = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)(31 - (last & 31))) & 255u;
-  return __half2float(__ushort_as_half((uint16_t)(pairs[state] >> 16)));     // entry i: the values of states (i >> KB) & 255 and i & 255
-}
 template <int kInFlight, bool MS, int KB>
 __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyArgs<KB> X) {
   __shared__ float s_w[256];
@@ -472,20 +466,41 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   bool seen[2] = {false, false};               // uniform over the workgroup
   if constexpr (KB != 0) {
     __shared__ float s_dot[2][4];
+    __shared__ float s_tab[2][256];              // K and V table of the kv head
+    __shared__ uint32_t s_code[4][64], s_fld[4][64];
+    __shared__ float s_scale[4];
     const TbAttnArgs& N = X.N;
-    const int kvh = head / kG, gK = (N.layer * N.n_kv + kvh) * 2, gV = gK + 1, pos = *N.d_pos;
-    const uint32_t *pk = N.pairs + ((size_t)gK << (8 + KB)), *pv = N.pairs + ((size_t)gV << (8 + KB));
+    const int kvh = head / kG, gK = (N.layer * N.n_kv + kvh) * 2, gV = gK + 1;
+    const int wave = tid >> 6, lane = tid & 63, u_w = wave >> 1;
+    // entry i of a pair table ends with the value of state i & 255
+    const uint32_t tk = N.pairs[((size_t)gK << (8 + KB)) + tid], tv = N.pairs[((size_t)gV << (8 + KB)) + tid];
     const float q = row16_value(N.q16[((size_t)tok * A.n_heads + head) * kD2 + tid], N.in_bf16);
+    const float mu = N.mu ? N.mu[(size_t)gV * 256 + tid] : 0.f;
+    const int pos = *N.d_pos;
+    if (u_w <= tok) {                            // uniform over the wave
+      uint32_t states; float scale;
+      pick_job(X.J, (2 * u_w + (wave & 1)) * N.n_kv + kvh, lane, states, scale);
+      s_code[wave][lane] = states;
+      if (lane == 0) s_scale[wave] = scale;
+      const int r = pos + u_w;
+      if (tok == A.M - 1 && head % kG == 0 && r >= 0 && r < N.max_ctx) {
+        const size_t row = (size_t)kvh * N.max_ctx + r;
+        store_coded_row<KB>(const_cast<uint8_t*>((wave & 1) ? N.vpay : N.kpay) + row * N.stride, reinterpret_cast<uint8_t*>(s_fld[wave]), lane, states);
+        if (lane == 0) const_cast<float*>((wave & 1) ? N.vscl : N.kscl)[row] = scale;
+      }
+    }
+    s_tab[0][tid] = __half2float(__ushort_as_half((uint16_t)(tk >> 16)));
+    s_tab[1][tid] = __half2float(__ushort_as_half((uint16_t)(tv >> 16)));
+    __syncthreads();
     float ksc[2] = {0.f, 0.f}, dot[2] = {0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int r = pos + u;
       seen[u] = u <= tok && r >= 0 && r < N.max_ctx;
       if (!seen[u]) continue;
-      const size_t row = (size_t)kvh * N.max_ctx + r;
-      ksc[u] = N.kscl[row];
-      dot[u] = q * tb_element<KB>(N.kpay + row * N.stride, tid, pk);
-      new_v[u] = tb_element<KB>(N.vpay + row * N.stride, tid, pv) * N.vscl[row] * N.gfac[gV] + (N.mu ? N.mu[(size_t)gV * 256 + tid] : 0.f);
+      ksc[u] = s_scale[2 * u];
+      dot[u] = q * s_tab[0][reinterpret_cast<const uint8_t*>(s_code[2 * u])[tid]];
+      new_v[u] = s_tab[1][reinterpret_cast<const uint8_t*>(s_code[2 * u + 1])[tid]] * s_scale[2 * u + 1] * N.gfac[gV] + mu;
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -573,15 +588,15 @@ void launch_combine256(const CombineArgs& A, hipStream_t st) {
   else hipLaunchKernelGGL((combine256_kernel<4, false, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
 }
 template <int KB>
-static void launch_combine_new(const CombineArgs& A, const TbAttnArgs& N, hipStream_t st) {
+static void launch_combine_new(const CombineArgs& A, const TbAttnArgs& N, const TbJobs& J, hipStream_t st) {
   const dim3 grid(A.n_heads, A.M);
-  const NewKeyArgs<KB> X{N};
+  const NewKeyArgs<KB> X{N, J};
   if (A.S > 128) hipLaunchKernelGGL((combine256_kernel<32, false, KB>), grid, dim3(256), 0, st, A, X);
   else if (A.S > 64) hipLaunchKernelGGL((combine256_kernel<16, false, KB>), grid, dim3(256), 0, st, A, X);
   else hipLaunchKernelGGL((combine256_kernel<8, false, KB>), grid, dim3(256), 0, st, A, X);
 }
-void launch_combine256_new(const CombineArgs& A, const TbAttnArgs& N, int kb, hipStream_t st) {
-  if (kb == 4) launch_combine_new<4>(A, N, st); else launch_combine_new<5>(A, N, st);
+void launch_combine256_new(const CombineArgs& A, const TbAttnArgs& N, const TbJobs& J, int kb, hipStream_t st) {
+  if (kb == 4) launch_combine_new<4>(A, N, J, st); else launch_combine_new<5>(A, N, J, st);
 }
 void launch_export_rows256(const KvView& kv, int pos0, int n, uint32_t* kw, float* ks, uint32_t* vw, float* vs, hipStream_t st) {
   hipLaunchKernelGGL(xfer256_kernel<false>, dim3(n, kv.n_kv), dim3(64), 0, st, kv, pos0, n, kw, ks, vw, vs);

@@ -18,6 +18,7 @@
 #include "yka_internal.h"
 #include "rot256_device.h"
 #include "attend_tb_device.h"
+#include "tb_store_device.h"
 #include <hip/hip_fp16.h>
 
 namespace yka {
@@ -506,9 +507,9 @@ __global__ void __launch_bounds__(256) tb_search_probe_kernel(TbEncArgs A) {
 // Decode (one or two tokens, no depth table): the search for the new rows' codes and the attention over the rows already in
 // the cache need nothing from each other, and neither fills the chip - 72 or 144 workgroups, each a serial chain of 64
 // steps, beside one attention workgroup per CU.  One launch runs both: the first `n_search` workgroups search, the others
-// attend to the keys in front of *d_pos.  The select launch stores the coded rows, the combiner adds them as keys of its own
-// (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 in four launches (search 9.3, select 4.7,
-// attention 12.5, combiner 4.5), 22.4 in three (13.7, 4.8, 5.3).
+// attend to the keys in front of *d_pos.  The combiner picks the codes of the new rows, stores them and adds them as keys of its own
+// (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 with the encoder in launches of its own, 22.2
+// with the rows stored by a launch between these two, 19.5 so.
 template <int KB, bool BF>
 __global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_pos, int n_search, TbEncArgs E, TbAttnArgs A) {
   A.d_pos = p_pos;
@@ -516,19 +517,6 @@ __global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_p
   int split, kvh;
   tb_split_of(A, blockIdx.x - n_search, split, kvh);
   tbd::attend_tb_body<KB, false>(A, split, kvh, 0, true);
-}
-
-// word d of a row's MSB-first stream of KB-bit fields: the fields that overlap bits [32 d, 32 d + 32)
-template <int KB>
-__device__ __forceinline__ uint32_t pack_word(const uint8_t* fld, int d) {
-  const int e0 = (32 * d) / KB;                          // first field with bits in the word (division by a constant)
-  uint32_t w = 0u;
-#pragma unroll
-  for (int k = 0; k < 32 / KB + 2; ++k) {
-    const int e = e0 + k, sh = 32 * d + 32 - KB * (e + 1);   // distance of the field's last bit from the word's last bit
-    if (e < 256 && sh > -KB) w |= sh >= 0 ? (uint32_t)fld[e] << sh : (uint32_t)fld[e] >> -sh;
-  }
-  return w;
 }
 
 // what a row is stored as: one field per element, the field width, the row scale
@@ -545,7 +533,6 @@ __device__ __forceinline__ Coded code_flat(float* part8, float r) {
 // the first of equal errors), the state the search chose for this element under it.  What that needs from memory is
 // requested before the residual is computed, for all multipliers at once (the choice then costs no further round trip):
 // the states of this element, and - by thread i < multipliers - multiplier i and the error total of its search.
-constexpr int kMaxMult = 16;
 struct SearchResults { int state[kMaxMult]; };
 __device__ __forceinline__ SearchResults fetch_search_results(const TbEncArgs& A, const Profile& P, int row, float* totals, float* mults) {
   SearchResults S;
@@ -573,44 +560,6 @@ __device__ __forceinline__ Coded code_trellis(const TbEncArgs& A, const Profile&
   float value = 0.f;
   if (A.yout) { const TableRec T = read_table(P, G); value = __fmul_rn(table_value(table_int(P, T, state), T.gain), s); }
   return Coded{state & ((1 << G.bits) - 1), G.bits, s, value, true};
-}
-
-// What a row is stored as after the search (cache form), by a wave: the multiplier whose search left the smallest squared error (its 8
-// partial sums added in order from 0; the first of equal errors), the four states of elements 4 lane .. 4 lane + 3 it chose, its scale.
-__device__ __forceinline__ void pick_job(const TbEncArgs& A, int row, int lane, uint32_t& states, float& scale) {
-  const size_t job0 = (size_t)row * A.nm;
-  uint32_t all[kMaxMult];
-#pragma unroll
-  for (int i = 0; i < kMaxMult; ++i) all[i] = i < A.nm ? reinterpret_cast<const uint32_t*>(A.scr + (job0 + i) * 256)[lane] : 0u;
-  float4 e0 = make_float4(0, 0, 0, 0), e1 = e0;
-  float s = 0.f;
-  if (lane < A.nm) {
-    const float4* err = reinterpret_cast<const float4*>(A.scr + A.scr_w_ofs) + (job0 + lane) * 2;
-    e0 = err[0]; e1 = err[1];
-    s = reinterpret_cast<const float*>(A.scr + A.scr_s_ofs)[job0 + lane];
-  }
-  float total = 0.f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) total = __fadd_rn(total, (&e0.x)[k]);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) total = __fadd_rn(total, (&e1.x)[k]);
-  float least = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(total), 0));
-  int keep = 0;
-  states = all[0];
-#pragma unroll
-  for (int i = 1; i < kMaxMult; ++i) {
-    const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(total), i));
-    const bool better = i < A.nm && v < least;           // uniform over the wave
-    least = better ? v : least; keep = better ? i : keep; states = better ? all[i] : states;
-  }
-  scale = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s), __builtin_amdgcn_readfirstlane(keep)));
-}
-// packs and stores the fields of those states (fld: 256 bytes of LDS private to the wave)
-template <int KB>
-__device__ __forceinline__ void store_coded_row(uint8_t* dst, uint8_t* fld, int lane, uint32_t states) {
-  reinterpret_cast<uint32_t*>(fld)[lane] = states & (0x01010101u * ((1u << KB) - 1u));
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  if (lane < 8 * KB) reinterpret_cast<uint32_t*>(dst)[lane] = pack_word<KB>(fld, lane);
 }
 
 // grid rows, block 256: codes the row (best multiplier of the search, or the flat quantizer), rebuilds what it decodes to,
@@ -667,7 +616,7 @@ __global__ void __launch_bounds__(256) tb_store_kernel(const int* p_pos, const u
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = blockIdx.x * 4 + wave;
   if (row >= A.nrow) return;                             // no barrier below
   uint32_t states; float scale;
-  pick_job(A, row, lane, states, scale);
+  pick_job(tb_jobs(A), row, lane, states, scale);
   const CacheRow R = cache_row(A, row);
   int pos; size_t container = 0; bool ok = true;
   if (A.rows.pos) {                                      // multi-stream pass: the row's own container and position
@@ -749,7 +698,6 @@ void launch_tb_encode_attend(const TbEncArgs& E, const TbAttnArgs& A, int kb, hi
   else if (kb == 4) hipLaunchKernelGGL((tb_search_attend_kernel<4, false>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
   else if (E.in_bf16) hipLaunchKernelGGL((tb_search_attend_kernel<5, true>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
   else hipLaunchKernelGGL((tb_search_attend_kernel<5, false>), grid, dim3(256), 0, st, A.d_pos, n_search, E, A);
-  if (kb == 4) launch_store<4>(E, st); else launch_store<5>(E, st);
 }
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t st) {

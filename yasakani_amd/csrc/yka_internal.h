@@ -138,6 +138,9 @@ struct TbEncArgs {
   RowMap rows;                        // cache form, multi-stream pass: token t sits at rows.pos[t] of container rows.slot[t] (pay / scl = container 0)
   int in_bf16;                        // cache form: k16 / v16 are bf16 rows
 };
+// what the searches of a launch have left in the scratch (TbEncArgs): nm jobs per row
+struct TbJobs { const uint8_t* scr; size_t w_ofs, s_ofs; int nm; };
+__host__ __device__ inline TbJobs tb_jobs(const TbEncArgs& A) { return TbJobs{A.scr, A.scr_w_ofs, A.scr_s_ofs, A.nm}; }
 // attention over trellis-coded rows (attend_tb.hip).  pairs [groups][2^(8 + kb)]: entry i = the table's integers, as two
 // fp16 values, of the states (i >> kb) & 255 and i & 255 (two consecutive elements from 8 + kb stream bits); gfac [groups]:
 // gain / 256; mu [groups][256] fp32 mean rows (zero rows where a group has none) or nullptr if no group has one
@@ -161,7 +164,7 @@ __device__ __forceinline__ void tb_split_of(const TbAttnArgs& A, int b, int& spl
   if (A.s_short) { split = b / A.n_kv; kvh = b % A.n_kv; } else { split = b % A.S; kvh = b / A.S; }
 }
 void launch_tb_encode(const TbEncArgs&, hipStream_t);
-// one or two tokens: encoder and attention over the keys in front of *d_pos; the combiner has to add the new rows
+// one or two tokens: searches of the encoder and attention over the keys in front of *d_pos; the combiner has to store the new rows and add them
 void launch_tb_encode_attend(const TbEncArgs&, const TbAttnArgs&, int kb, hipStream_t);
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t);
@@ -181,7 +184,7 @@ void launch_rotate_q256(const float* x32, int rows, uint16_t* q16, hipStream_t);
 void launch_attend256(const AttnArgs&, hipStream_t);       // row tiles of 2 tokens x 6 heads (decode; any width)
 void launch_attend256_wide(const AttnArgs&, hipStream_t);  // 3..64 rows: 128 query rows per workgroup, tiles dequantized once into LDS
 void launch_combine256(const CombineArgs&, hipStream_t);
-void launch_combine256_new(const CombineArgs&, const TbAttnArgs&, int kb, hipStream_t);   // the partials of launch_tb_encode_attend and the new rows
+void launch_combine256_new(const CombineArgs&, const TbAttnArgs&, const TbJobs&, int kb, hipStream_t);   // the partials of launch_tb_encode_attend and the new rows
 void launch_export_rows256(const KvView&, int pos0, int n, uint32_t* kw, float* ks, uint32_t* vw, float* vs, hipStream_t);
 void launch_import_rows256(const KvView&, int pos0, int n, const uint32_t* kw, const float* ks, const uint32_t* vw, const float* vs, hipStream_t);
 // canonical <-> physical
