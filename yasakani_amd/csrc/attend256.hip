@@ -104,23 +104,26 @@ __global__ void __launch_bounds__(256) attn_post256_kernel(PostArgs A) {
   __shared__ uint8_t fld[256];
   const int blk = blockIdx.x, tok = blockIdx.y, d = threadIdx.x;
   const int NH = A.n_heads, KVH = A.kv.n_kv;
+  // as in attn_post_kernel: value and weight are requested with the position, the rotary factors as soon as it is known
+  const bool gate = blk >= NH + 2 * KVH, isq = blk < NH, isk = !isq && blk < NH + KVH;
+  const int head = gate ? blk - NH - 2 * KVH : isq ? blk : (isk ? blk - NH : blk - NH - KVH);
+  const float* src = (gate ? A.xgate : isq ? A.xq : isk ? A.xk : A.xv) + ((size_t)tok * (gate || isq ? NH : KVH) + head) * kD2;
+  const float raw = __hip_atomic_load(src + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  const uint16_t* weights = isq ? A.qn_w16 : A.kn_w16;
+  const uint16_t wraw = isq || isk ? request16(weights + d) : (uint16_t)0;
   const int pos = *A.d_pos + tok;
   if (pos < 0 || pos >= A.kv.max_ctx || (A.rd > 0 && pos >= A.rope_rows)) return;   // rows outside the container are dropped
-  if (blk >= NH + 2 * KVH) {                       // gate rows: the projection rounded to the 16-bit type
-    const size_t e = ((size_t)tok * NH + (blk - NH - 2 * KVH)) * kD2 + d;
-    A.gate16[e] = A.io_bf16 ? f2bf_bits(A.xgate[e]) : __half_as_ushort(__float2half_rn(A.xgate[e]));
+  if (gate) {                                      // gate rows: the projection rounded to the 16-bit type
+    A.gate16[((size_t)tok * NH + head) * kD2 + d] = A.io_bf16 ? f2bf_bits(raw) : __half_as_ushort(__float2half_rn(raw));
     return;
   }
-  const bool isq = blk < NH, isk = !isq && blk < NH + KVH;
-  const int head = isq ? blk : (isk ? blk - NH : blk - NH - KVH);
-  const float* src = isq ? A.xq + ((size_t)tok * NH + head) * kD2
-                         : (isk ? A.xk : A.xv) + ((size_t)tok * KVH + head) * kD2;
-  const float y = f16r256(src[d]);
+  const int hr = A.rd >> 1;
+  float2 cs = make_float2(0.f, 0.f);
+  if (d < A.rd && (isq || isk)) cs = reinterpret_cast<const float2*>(A.rope)[(size_t)pos * hr + (d < hr ? d : d - hr)];
+  const float y = f16r256(raw);
   float out;
   if (isq || isk) {
-    float ss = __fmul_rn(y, y);
-#pragma unroll
-    for (int o = 16; o; o >>= 1) ss = __fadd_rn(ss, __shfl_xor(ss, o, 64));
+    const float ss = lane_run32(__fmul_rn(y, y), [](float a, float b) { return __fadd_rn(a, b); });
     if ((d & 31) == 0) red[d >> 5] = ss;
     __syncthreads();
     float tot = 0.f;
@@ -128,16 +131,13 @@ __global__ void __launch_bounds__(256) attn_post256_kernel(PostArgs A) {
     for (int w = 0; w < 8; ++w) tot = __fadd_rn(tot, red[w]);
     // sqrtf, not __fsqrt_rn: only the former is correctly rounded on this target
     const float r = __fdiv_rn(1.f, sqrtf(__fadd_rn(__fdiv_rn(tot, 256.f), A.eps)));
-    const float w = __half2float(__ushort_as_half((isq ? A.qn_w16 : A.kn_w16)[d]));
+    const float w = __half2float(__ushort_as_half(wraw));
     const float xn = f16r256(__fmul_rn(__fmul_rn(y, r), __fadd_rn(1.f, w)));
     out = xn;
-    const int hr = A.rd >> 1;
     if (hr > 0) {
       buf[d] = xn;
       __syncthreads();
       if (d < A.rd) {
-        const int i = d < hr ? d : d - hr;
-        const float2 cs = reinterpret_cast<const float2*>(A.rope)[(size_t)pos * hr + i];
         const float partner = d < hr ? -buf[d + hr] : buf[d - hr];
         out = f16r256(__fadd_rn(f16r256(__fmul_rn(xn, cs.x)), f16r256(__fmul_rn(partner, cs.y))));
       }
@@ -504,8 +504,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-#pragma unroll
-      for (int o = 32; o; o >>= 1) dot[u] += __shfl_xor(dot[u], o, 64);
+      dot[u] = lane_run32(lane_op32(dot[u], LaneAdd{}), LaneAdd{});
       if ((tid & 63) == 0) s_dot[u][tid >> 6] = dot[u];
     }
     __syncthreads();

@@ -587,11 +587,7 @@ __global__ void __launch_bounds__(256) combine_kernel(YKA_COMBINE_PARAMS, Combin
   }
   if (A.unrot) {                                   // uniform over the grid
     // inverse signed Hadamard rotation over the row's 128 channels (threads 0..127 = two waves)
-#pragma unroll
-    for (int h = 1; h < 64; h *= 2) {
-      const float b = __shfl_xor(y, h, 64);
-      y = (tid & h) ? b - y : y + b;
-    }
+    y = wave_hadamard(y, tid);
     __syncthreads();
     if (tid < kD) s_w[tid] = y;
     __syncthreads();

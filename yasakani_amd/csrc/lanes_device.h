@@ -19,6 +19,13 @@ __device__ __forceinline__ T lane_dpp(T v) {
 }
 template <class T> __device__ __forceinline__ T lane_xor1(T v) { return lane_dpp<0xB1>(v); }     // quad_perm [1,0,3,2]
 template <class T> __device__ __forceinline__ T lane_xor2(T v) { return lane_dpp<0x4E>(v); }     // quad_perm [2,3,0,1]
+// two shifts inside rows of 16, each into the banks of 4 lanes whose partner lies that way
+template <class T> __device__ __forceinline__ T lane_xor4(T v) {
+  static_assert(sizeof(T) == 4, "one register");
+  const int b = __builtin_bit_cast(int, v);
+  const int up = __builtin_amdgcn_update_dpp(b, b, 0x104, 0xf, 0x5, false);                         // row_shl:4 into banks 0 and 2
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(up, b, 0x114, 0xf, 0xa, false));         // row_shr:4 into banks 1 and 3
+}
 template <class T> __device__ __forceinline__ T lane_xor8(T v) { return lane_dpp<0x128>(v); }    // row_ror:8
 // op(v, v of lane ^ 16) and op(v, v of lane ^ 32): after swapping a register with a copy of itself the two results hold, in
 // every lane, the values of the lane and of its partner (op commutes)
@@ -41,6 +48,34 @@ struct LaneMin { __device__ __forceinline__ int operator()(int a, int b) const {
 struct LaneAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
 // over the four lanes l, l ^ 16, l ^ 32, l ^ 48
 template <class T, class Op> __device__ __forceinline__ T lane_rows(T v, Op op) { return lane_op32(lane_op16(v, op), op); }
+// the butterfly v = op(v, v of lane ^ o), o = 16 .. 1, inside each half of the wave (the reference's reduction of a run of 32
+// elements); lane ^ 4 as a rotation by four, since lanes l and l ^ 8 hold one value by then
+template <class T, class Op>
+__device__ __forceinline__ T lane_run32(T v, Op op) {
+  v = lane_op16(v, op);
+  v = op(v, lane_xor8(v));
+  v = op(v, lane_dpp<0x124>(v));                   // row_ror:4
+  v = op(v, lane_xor2(v));
+  return op(v, lane_xor1(v));
+}
+// one stage of a Hadamard transform: a + b in the lane whose bit H is 0, b - a (b: the partner's value) in the other
+template <int H>
+__device__ __forceinline__ float lane_hadamard(float a, int lane) {
+  if constexpr (H >= 16) {
+    const unsigned u = __builtin_bit_cast(unsigned, a);
+    const lanes_u32x2 r = H == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const unsigned r0 = r[0], r1 = r[1];           // in both lanes of a pair: the value of the lower and of the upper one
+    const float lo = __builtin_bit_cast(float, r0), hi = __builtin_bit_cast(float, r1);
+    return (lane & H) ? __fsub_rn(lo, hi) : __fadd_rn(lo, hi);
+  } else {
+    const float b = H == 1 ? lane_xor1(a) : H == 2 ? lane_xor2(a) : H == 4 ? lane_xor4(a) : lane_xor8(a);
+    return (lane & H) ? __fsub_rn(b, a) : __fadd_rn(a, b);
+  }
+}
+__device__ __forceinline__ float wave_hadamard(float a, int lane) {
+  a = lane_hadamard<1>(a, lane); a = lane_hadamard<2>(a, lane); a = lane_hadamard<4>(a, lane);
+  a = lane_hadamard<8>(a, lane); a = lane_hadamard<16>(a, lane); return lane_hadamard<32>(a, lane);
+}
 // over a row of 16 lanes; op is a maximum or minimum (after two steps a quad holds one value, so the mirrored octet is lane ^ 4)
 template <class T, class Op>
 __device__ __forceinline__ T lane_row16(T v, Op op) {

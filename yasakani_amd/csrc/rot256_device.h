@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "lanes_device.h"
 #include "sign_device.h"
 
 namespace yka {
@@ -13,11 +14,7 @@ namespace yka {
 __device__ __forceinline__ float rotate256(float x, float* buf, bool inverse) {
   const int d = threadIdx.x;
   float a = inverse ? x : __fmul_rn(x, channel_sign(d));
-#pragma unroll
-  for (int h = 1; h < 64; h *= 2) {
-    const float b = __shfl_xor(a, h, 64);
-    a = (d & h) ? __fsub_rn(b, a) : __fadd_rn(a, b);
-  }
+  a = wave_hadamard(a, d);
 #pragma unroll
   for (int h = 64; h < 256; h *= 2) {
     __syncthreads();

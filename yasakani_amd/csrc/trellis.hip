@@ -86,17 +86,8 @@ __device__ __forceinline__ float round_f16(float v) { asm volatile("" : "+v"(v))
 // 32 elements the butterfly a[i] = op(a[i], a[i ^ o]), o = 16 .. 1, then the 8 run results folded in order from `start`.
 struct AddRn { __device__ static float op(float a, float b) { return __fadd_rn(a, b); } };
 struct MaxOp { __device__ static float op(float a, float b) { return fmaxf(a, b); } };
-// The butterfly inside a run goes through lane-crossing moves: lane ^ 16, lane ^ 8, then lane ^ 4 as a rotation by four in the row
-// of 16 (after the step before it lanes l and l ^ 8 hold one value), then inside the quad.
 template <class Op>
-__device__ __forceinline__ float run_fold(float v) {
-  const auto op = [](float a, float b) { return Op::op(a, b); };
-  v = lane_op16(v, op);
-  v = op(v, lane_xor8(v));
-  v = op(v, lane_dpp<0x124>(v));                         // row_ror:4
-  v = op(v, lane_xor2(v));
-  return op(v, lane_xor1(v));
-}
+__device__ __forceinline__ float run_fold(float v) { return lane_run32(v, [](float a, float b) { return Op::op(a, b); }); }
 template <class Op>
 __device__ __forceinline__ float block_fold(float* part8, float v, float start) {
   v = run_fold<Op>(v);
