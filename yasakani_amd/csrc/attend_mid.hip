@@ -88,8 +88,7 @@ __device__ __forceinline__ void pv_done(f4 (&o)[8]) {
 // The static check in tests/test_isa_inflight_loads.py reports exactly that; it has to pass before this file runs on
 // a GPU.)
 template <int NRT>
-__global__ void __launch_bounds__(256, 1) attend_mid_kernel(const int* p_pos, uint8_t* p_base, const int32_t* p_table, int p_n_kv, int p_max_ctx, int p_s, AttnArgs A) {
-  A.d_pos = p_pos; A.kv = KvView{p_base, p_table, p_n_kv, p_max_ctx}; A.S = p_s;
+__global__ void __launch_bounds__(256, 1) attend_mid_kernel(AttnArgs A) {
   constexpr int TB = (16 * NRT) / kG;          // tokens per row block
   __shared__ __align__(16) uint4 s_q[NRT * 4 * 64];                 // [row tile][scale group][lane]: B operands of the score MFMAs
   // wave merge: up to four row tiles are staged at once (one barrier for the whole merge), more go through two buffers
@@ -444,7 +443,9 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(const int* p_pos, ui
 #pragma unroll
       for (int c = 0; c < 8; ++c) v[c] = (_Float16)(acc[c] * inv);
       const size_t p = ((size_t)(tokb + R / kG) * A.S + split) * A.n_heads + kvh * kG + R % kG;
-      store_partial16(A.pacc16 + p * kD + c8, __builtin_bit_cast(uint4, v));
+      // megabytes of partials are written through (store_partial16): 6 rows or more, every split in use
+      if (NRT >= 3 && 4 * A.S <= ntiles) store_partial16(A.pacc16 + p * kD + c8, __builtin_bit_cast(uint4, v));
+      else *reinterpret_cast<uint4*>(A.pacc16 + p * kD + c8) = __builtin_bit_cast(uint4, v);
       if (c8 == 0) { A.pm[p] = M2; A.pl[p] = L; }
     }
   };
@@ -475,11 +476,11 @@ void launch_attend_mid(const AttnArgs& A, hipStream_t st) {
   const int tb = (16 * nrt) / kG, nb = (A.M + tb - 1) / tb;
   const dim3 grid(A.S, A.kv.n_kv, nb), block(256);
   switch (nrt) {
-    case 2: hipLaunchKernelGGL(attend_mid_kernel<2>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
-    case 3: hipLaunchKernelGGL(attend_mid_kernel<3>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
-    case 4: hipLaunchKernelGGL(attend_mid_kernel<4>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
-    case 5: hipLaunchKernelGGL(attend_mid_kernel<5>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
-    default: hipLaunchKernelGGL(attend_mid_kernel<6>, grid, block, 0, st, A.d_pos, A.kv.base, A.kv.table, A.kv.n_kv, A.kv.max_ctx, A.S, A); break;
+    case 2: hipLaunchKernelGGL(attend_mid_kernel<2>, grid, block, 0, st, A); break;
+    case 3: hipLaunchKernelGGL(attend_mid_kernel<3>, grid, block, 0, st, A); break;
+    case 4: hipLaunchKernelGGL(attend_mid_kernel<4>, grid, block, 0, st, A); break;
+    case 5: hipLaunchKernelGGL(attend_mid_kernel<5>, grid, block, 0, st, A); break;
+    default: hipLaunchKernelGGL(attend_mid_kernel<6>, grid, block, 0, st, A); break;
   }
 }
 

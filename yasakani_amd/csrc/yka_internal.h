@@ -90,11 +90,12 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
   int adapt = 0; int direct = 0; const int* d_pos = nullptr; int tok0 = 0; int n_kv = 0; int max_ctx = 0;
   const int2* plan = nullptr;   // partials of a multi-stream pass shared out by ms_share: first split and splits of every row
   int s_short = 0; };    // trellis decode: as in TbAttnArgs (d_pos is set then)
-// Kernels of the decode and small-window chain name what their first loads need as leading arguments of their own and are compiled
+// Decode, its combiner and the trellis kernels of decode name what their first loads need as leading arguments of their own and are compiled
 // with -amdgpu-kernarg-preload-count: those arrive in scalar registers with the wave, and the position (the combiner's partials)
-// is asked for at once instead of 0.3 us later, behind the load of the argument block.  us per 16 layers without / with: one token at 32,741 tokens
-// 172.5 / 166.5, 8 rows at 12,037 223 / 217, one 5-bit trellis row at 16,001 382 / 371, one token at 1,003 115.4 / 113.8, 16
-// streams 27.1 / 26.7 a pass.  Not where it measured slower: the 256-channel kernels (273 / 280), wide windows (737 / 743).
+// is asked for at once instead of 0.3 us later, behind the load of the argument block.  us per 16 layers without / with: one token at 32,741
+// tokens 172.5 / 166.5, one 5-bit trellis row at 16,001 382 / 371, 8 rows at 12,037 (the combiner alone) 226 / 220, one token at
+// 1,003 115.4 / 113.8, 16 streams 27.1 / 26.7 a pass.  Not where it measured slower: the 256-channel kernels (273 / 280), wide
+// windows (737 / 743), windows of 3 to 5 rows in the mid kernel (212 / 218; 8 rows 220 / 218).
 #define YKA_COMBINE_PARAMS const float *p_pm, const float *p_pl, const uint16_t *p_acc, const void *p_where, int p_s, int p_heads
 #define YKA_COMBINE_GIVE(A) (A).pm, (A).pl, (A).pacc16, (A).plan ? (const void*)(A).plan : (const void*)(A).d_pos, (A).S, (A).n_heads
 #define YKA_COMBINE_TAKE(A) \
@@ -253,8 +254,8 @@ __device__ __forceinline__ uint4 pack_out8(const float* y, int bf16) {
 // rows in 32 splits kept the combiner waiting 5 us behind the last workgroup, where 1.4 us are usual.  Written through, the
 // rows of the workgroups that end early are out before the last one ends.  us per 16 layers, ordinary / nontemporal / written through: 24
 // rows of 256 channels at 9,001 tokens 396 / 370 / 363, 64 rows of 128 at 32,768 741 / 733 / 730, 8 rows at 12,037 229 / 225 /
-// 225.  Decode leaves a few 100 KB, which nobody waits for, and its stores are in the way of its end: 173 / 173 / 176 and 16 streams
-// 27.2 / 27.8 / 28.0 a pass; it keeps ordinary stores.
+// 225.  Decode and the smallest windows leave little, which nobody waits for, and such stores are in the way of their end: one token at
+// 32,741 tokens 173 / 173 / 176, 16 streams 27.2 / 27.8 / 28.0 a pass, 4 rows at 32,768 259 ordinary and 263; they keep ordinary stores.
 __device__ __forceinline__ void store_partial16(uint16_t* p, uint4 v) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)p, u32x4{v.x, v.y, v.z, v.w}, "agent");
