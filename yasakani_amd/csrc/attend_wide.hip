@@ -15,11 +15,11 @@
 //   * a wave owns one tile of 32 rows (MFMA 32x32x16: one K or V fragment read from LDS serves 32 rows) and stays
 //     under 256 registers, so the two waves of a SIMD (one of each group) fit and all MFMA results live in ordinary
 //     VGPRs (no accumulator-file copies);
-//   * a step of a group has two phases with a workgroup barrier after each: a MATRIX phase (the PV product of the
-//     previous tile, the score MFMAs of this tile with the scale multiply-adds in their shadow, fragment reads) and a
-//     VECTOR phase (softmax, dequantization of the group's next tile, requests for the tile after that).  The groups run
-//     half a step apart: while one is in its matrix phase the other is in its vector phase, so the two waves of a SIMD
-//     never compete for the matrix pipe and vector work of one wave runs under the MFMAs of the other.  Two waves
+//   * a step of a group has two phases: a MATRIX phase (the PV product of the previous tile, the score MFMAs of this tile
+//     with the scale multiply-adds in their shadow, fragment reads) and a VECTOR phase (softmax, dequantization of the
+//     group's next tile, requests for the tile after that).  The groups run half a step apart - between two workgroup barriers
+//     one runs matrix, then vector phase, the other vector, then matrix phase - so the two waves of a SIMD
+//     do not compete for the matrix pipe and vector work of one wave runs under the MFMAs of the other.  Two waves
 //     left to themselves do not find this arrangement: measured, two independent 4-wave workgroups per compute unit
 //     take as long as the same two one after the other;
 //   * the group scales of K are applied to the fp32 partial sum of each 32-channel group (two chained MFMAs per
@@ -287,10 +287,10 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
     asm volatile("" ::: "memory");             // the tile loads below are instructions the compiler does not see as loads
   }
 
-  // tiles of this group: tile0 + grp + 2u, u = 0 .. nu-1; both groups walk nsteps steps (a group one tile short idles in
-  // its last step) so that every wave of the workgroup meets the same number of barriers
+  // tiles of this group: tile0 + grp + 2u, u = 0 .. nu-1; both groups walk nstep steps (idle where they have no tile left) so
+  // that every wave of the workgroup meets the same number of barriers
   const int ntl = max(0, tile1 - tile0);
-  const int nsteps = (ntl + 1) >> 1, nu = (ntl + 1 - grp) >> 1;
+  const int nu = (ntl + 1 - grp) >> 1;
   auto tile_of = [&](int u) __attribute__((always_inline)) { return tile0 + grp + 2 * min(u, nu - 1); };   // past the end: the last tile again
 
   float m_run = -1e30f, l_run = 0.f;           // m_run in log2 units, shared by the two lanes of a row
@@ -311,12 +311,9 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
     wait_raw<0>(raw0);
     if constexpr (BF) q_ready();               // every load has been answered: the query costs no trip to memory of its own
     dequant_to_lds(lds[grp][0], gt, raw0, magic, sc_log2);
-    load_tile_raw(tile_of(1), raw1);
-    load_tile_raw(tile_of(2), raw0);
   }
-  __syncthreads();
 
-  // The probabilities and the V fragments of a tile stay in registers across the two barriers of a step; their eight
+  // The probabilities and the V fragments of a tile stay in registers until the next matrix phase; their eight
   // MFMAs open the NEXT matrix phase.  The first one multiplies zeros; the product of the last tile follows the loop.
   h8 pf[2], vfr[8];
 #pragma unroll
@@ -370,15 +367,8 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
     for (int c = 0; c < 8; ++c)
       vfr[c] = __builtin_bit_cast(h8, *reinterpret_cast<const uint4*>(buf + kLdsV + (32 * (c >> 1) + j) * kVPitch + (16 * (c & 1) + 8 * h) * 2));
   };
-  // ---- vector phase of tile u: softmax of its scores; `rs` holds the raw codes of tile u+1, which are dequantized into
-  //      the group's other buffer (unconditionally: after the last tile that buffer is read by nobody) and replaced by
-  //      the request for tile u+3 ----
-  auto vector_phase = [&](const int u, const int cb, Raw& rs) __attribute__((always_inline)) {
-    // The wave in its vector phase goes first when both waves of a SIMD have an instruction to issue.  At equal priority
-    // the older wave (group 0) wins in both of its phases and the younger group sets the pace of every phase: its vector
-    // phase, the longer stream, measured 1,580 cycles against group 0's 1,190.  With this, both groups take about 1,200
-    // cycles in either phase.
-    __builtin_amdgcn_s_setprio(2);
+  // ---- vector phase of tile u: softmax of its scores ----
+  auto softmax = [&](const int u) __attribute__((always_inline)) {
     if (has_rows) {
       const int t0 = tile_of(u) << 5;
       // online softmax with a lazily raised maximum: a row's offset m_run only moves when a score exceeds it by more
@@ -420,32 +410,67 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
       }
       l_run += lsum0 + lsum1;
     }
+  };
+  // ---- the group's tile k + 1, whose raw codes `rs` holds, goes to the buffer that tile k does not occupy (after the last tile that
+  //      buffer is read by nobody); the request for tile k + 3 replaces them (past the end: the last tile again, so that the
+  //      count of loads in flight is static) ----
+  auto feed = [&](const int k, const int cb, Raw& rs) __attribute__((always_inline)) {
     wait_raw<6>(rs);                           // the six loads of the other register set stay in flight
     dequant_to_lds(lds[grp][cb ^ 1], gt, rs, magic, sc_log2);
-    load_tile_raw(tile_of(u + 3), rs);         // always issued (past the end: the last tile again), so that the count of loads in flight is static
-    __builtin_amdgcn_s_setprio(0);
+    load_tile_raw(tile_of(k + 3), rs);
   };
-  // Group 1 starts one barrier late and group 0 ends with one barrier more: the groups stay a phase apart, and every
-  // wave executes 2 * nsteps + 1 barriers whatever its group (a group one tile short only meets the barriers of its
-  // last step).  cb and the register set are literals at every call site.
-  if (grp == 1) __syncthreads();
-  for (int u = 0; u < nu; u += 2) {
-    matrix_phase(u, 0);
-    __syncthreads();
-    vector_phase(u, 0, raw1);
-    __syncthreads();
-    if (u + 1 < nu) {
-      matrix_phase(u + 1, 1);
+  // One workgroup barrier per step.  Between two barriers group 0 runs the matrix and then the vector phase of its tile k, group 1
+  // the vector phase of its tile k - 1 and then the matrix phase of its tile k: each time one group's MFMAs run under the other's
+  // vector work.  Both dequantize tile k + 1 in step k, into the buffer of tile k - 1, which nobody has read since the barrier
+  // before.  The wave in its vector phase goes first when both waves of a SIMD have an instruction to issue: at equal priority the
+  // older wave (group 0) wins in both of its phases and the younger group sets the pace.
+  // With a barrier behind either phase the waves waited 130 cycles behind the matrix phase and 250 behind the vector phase of a step
+  // of 2,780.  us, two barriers / one: 16 layers of 1,500 rows on an empty cache 742 / 704, of 64 rows at 32,768 tokens 731 / 716.
+  // 2,048 rows at 131,072 tokens, 2 layers 8,131 / 8,111: 1,420 / 1,332 cycles a tile, but the chip lowers its clock from 2.24 to 2.15
+  // GHz - a long slice is bound by power, and only work left out shortens it.
+  // The loads of a group live inside its own branch from the request to the last wait (a join would copy their registers).
+  const int nstep = max((ntl + 1) >> 1, (ntl >> 1) + 1);
+  auto requests = [&]() __attribute__((always_inline)) { if (nu > 0) { load_tile_raw(tile_of(1), raw1); load_tile_raw(tile_of(2), raw0); } };
+  if (grp == 0) {
+    auto step = [&](const int k, const int cb, Raw& rs) __attribute__((always_inline)) {
+      if (k < nu) {
+        matrix_phase(k, cb);
+        __builtin_amdgcn_s_setprio(2);
+        softmax(k);
+        feed(k, cb, rs);
+        __builtin_amdgcn_s_setprio(0);
+      }
       __syncthreads();
-      vector_phase(u + 1, 1, raw0);
-      __syncthreads();
+    };
+    requests();
+    __syncthreads();
+    for (int k = 0; k < nstep; k += 2) {
+      step(k, 0, raw1);
+      if (k + 1 < nstep) step(k + 1, 1, raw0);
     }
+    wait_raw<0>(raw0);                         // every request has been answered before the registers it names are given up
+    wait_raw<0>(raw1);
+  } else {
+    auto step = [&](const int k, const int cb, Raw& rs) __attribute__((always_inline)) {
+      __builtin_amdgcn_s_setprio(2);
+      if (k > 0 && k <= nu) softmax(k - 1);
+      if (k < nu) {
+        feed(k, cb, rs);
+        __builtin_amdgcn_s_setprio(0);
+        matrix_phase(k, cb);
+      }
+      __syncthreads();
+    };
+    requests();
+    __syncthreads();
+    for (int k = 0; k < nstep; k += 2) {
+      step(k, 0, raw1);
+      if (k + 1 < nstep) step(k + 1, 1, raw0);
+    }
+    wait_raw<0>(raw0);
+    wait_raw<0>(raw1);
   }
-  for (int u = nu; u < nsteps; ++u) { __syncthreads(); __syncthreads(); }
-  if (grp == 0) __syncthreads();
-  // every request has been answered before the registers it names are given up
-  wait_raw<0>(raw0);
-  wait_raw<0>(raw1);
+  __builtin_amdgcn_s_setprio(0);
   if (has_rows) pv();
 
   // ---- the two groups' states of a row are merged: group 1 leaves its registers in LDS (the tile buffers are free
