@@ -36,6 +36,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int NT = 512;                        // threads per workgroup (8 waves x 16 rows)
 constexpr int kKPitch = 544, kVPitch = 96;     // conflict-free for the fragment reads (see attend256_wide.hip)
 constexpr int kLdsK = 0, kLdsV = 32 * kKPitch, kLdsS = kLdsV + kD2 * kVPitch, kLdsBuf = kLdsS + 256;   // 42240
+enum { kFeedOnly, kFeedFirst, kComputeFirst };    // what a wave does in a tile step, and in which order
 constexpr float kRaise = 8.f;                  // log2 slack before a running maximum is raised
 
 // byte offset (entry index x 4) into a pair table for the KB + 8 bits that end at bit `endbit` (exclusive) of the bit
@@ -152,7 +153,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   const uint8_t* const tabK = tabs;
   const uint8_t* const tabV = tabs + kTabBytes;
   const int split = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int gK = (A.layer * A.n_kv + kvh) * 2, gV = gK + 1;
   const int pos = *A.d_pos;
   const int nrows = kG * A.M;
@@ -218,19 +219,21 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   __syncthreads();                             // pair tables
   if (tile0 < tile1) {
     decode_to_lds<KB>(lds[0], tid, raw, offs, tabK, tabV);
-    load_tile_raw(min(tile0 + 1, tile1 - 1), raw);
   }
-  __syncthreads();
 
   // One tile: `rs` holds the raw words of tile T+1, which are decoded into the other LDS buffer (unconditionally: after
   // the last tile that buffer is read by nobody) and replaced by the request for tile T+2 (past the end: the last tile
   // again); cb is a literal at both call sites.
-  auto tile_step = [&](auto compute_tag, const int T, const int cb, Raw& rs) __attribute__((always_inline)) {
-    constexpr bool kCompute = decltype(compute_tag)::value;
+  auto tile_step = [&](auto order_tag, const int T, const int cb, Raw& rs) __attribute__((always_inline)) {
+    constexpr int kOrder = decltype(order_tag)::value;
+    constexpr bool kCompute = kOrder != kFeedOnly;
     const uint8_t* buf = lds[cb];
-    wait_raw(rs);
-    decode_to_lds<KB>(lds[cb ^ 1], tid, rs, offs, tabK, tabV);
-    load_tile_raw(min(T + 2, tile1 - 1), rs);
+    auto feed = [&]() __attribute__((always_inline)) {
+      wait_raw(rs);
+      decode_to_lds<KB>(lds[cb ^ 1], tid, rs, offs, tabK, tabV);
+      load_tile_raw(min(T + 2, tile1 - 1), rs);
+    };
+    if constexpr (kOrder != kComputeFirst) feed();
     if constexpr (kCompute) {
       const int t0 = T << 5;
       // ---- scores: per 16-key block 8 chained MFMAs over the 256 channels, then one multiply by the key's scale ----
@@ -292,16 +295,23 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
 #pragma unroll
       for (int b = 0; b < 8; ++b) o[b + 8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[b], pf, o[b + 8], 0, 0, 0);
     }
+    if constexpr (kOrder == kComputeFirst) feed();
     __syncthreads();
   };
-  auto run = [&](auto compute_tag) __attribute__((always_inline)) {
+  auto run = [&](auto order_tag) __attribute__((always_inline)) {      // the requests of a branch live inside it (a join would copy their registers)
+    if (tile0 < tile1) load_tile_raw(min(tile0 + 1, tile1 - 1), raw);
+    __syncthreads();
     for (int T = tile0; T < tile1; T += 2) {
-      tile_step(compute_tag, T, 0, raw);
-      if (T + 1 < tile1) tile_step(compute_tag, T + 1, 1, raw);
+      tile_step(order_tag, T, 0, raw);
+      if (T + 1 < tile1) tile_step(order_tag, T + 1, 1, raw);
     }
+    wait_raw(raw);                             // the loads past the last tile
   };
-  if (has_rows) run(std::true_type{}); else run(std::false_type{});
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // the loads past the last tile
+  // the two waves of a SIMD take the halves of a step in opposite order: one's MFMAs run under the other's vector work and LDS writes
+  // (16 layers of 16 rows of 5 bits at 16,384 tokens: 764 us with the image first in every wave, 747 so)
+  if (!has_rows) run(std::integral_constant<int, kFeedOnly>{});
+  else if (wave < 4) run(std::integral_constant<int, kFeedFirst>{});
+  else run(std::integral_constant<int, kComputeFirst>{});
   if (!has_rows) return;                       // no barrier follows
   // ---- partials: normalised fp16.  o[b][r] of lane (row i, group g) is channel 16b + 4g + r.  Rows go through LDS (the
   //      tile buffers are free after the last barrier) so that every store instruction writes whole 512-byte rows ----
