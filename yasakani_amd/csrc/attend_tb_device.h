@@ -72,7 +72,21 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int gK = (A.layer * A.n_kv + kvh) * 2, gV = gK + 1;
-  int pos; bool row_ok = true;
+  // The K and V pair tables of this kv head (global, in L2 -> LDS) are requested before the position, the query and the first K tile
+  // behind it, and only then are the tables waited for: one trip to memory instead of four (one row of 5 bits at 16,001 tokens, 16 layers: 307 us before, 298 so; 30 streams of 4 bits 96.6 and 94.8).
+  int pos = 0;
+  if (!MS) pos = *A.d_pos;
+  constexpr int kTabLoads = kTabBytes / 16 / 256;    // per thread and table
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  u32x4 tk[kTabLoads], tv[kTabLoads];
+  {
+    const u32x4* srcK = reinterpret_cast<const u32x4*>(A.pairs + (size_t)gK * (kTabBytes / 4)) + threadIdx.x;
+    const u32x4* srcV = reinterpret_cast<const u32x4*>(A.pairs + (size_t)gV * (kTabBytes / 4)) + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kTabLoads; ++k) { tk[k] = srcK[256 * k]; tv[k] = srcV[256 * k]; }
+    asm volatile("" ::: "memory");                   // the requests stay in front of the branches below
+  }
+  bool row_ok = true;
   MsShare share{};
   if (MS) {
     int slot;
@@ -87,8 +101,6 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
     A.kpay += off; A.vpay += off;
     A.kscl = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(A.kscl) + off);
     A.vscl = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(A.vscl) + off);
-  } else {
-    pos = *A.d_pos;
   }
   const int tl = TPT * rt + i / kG;
   const bool vrow = i < TPT * kG && tl < A.M && row_ok;
@@ -115,23 +127,16 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
     }
     return;
   }
-  {                                                  // the K and V pair tables of this kv head: global (L2) -> LDS
-    const uint4* srcK = reinterpret_cast<const uint4*>(A.pairs + (size_t)gK * (kTabBytes / 4));
-    const uint4* srcV = reinterpret_cast<const uint4*>(A.pairs + (size_t)gV * (kTabBytes / 4));
-    uint4* dst = reinterpret_cast<uint4*>(s_buf);
-#pragma unroll 4
-    for (int x = threadIdx.x; x < kTabBytes / 16; x += 256) { dst[x] = srcK[x]; dst[kTabBytes / 16 + x] = srcV[x]; }
-  }
-  __syncthreads();
   const int tps = (ntiles + s_used - 1) / s_used;
   const int tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
 
   h8 qf[8];                                          // k-step t: channels 64 g + 8 t .. + 7 of row i
   uint4 qraw[8];
   {
-    const uint16_t* qrow = A.q16 + ((size_t)tl * A.n_heads + head) * kD2 + 64 * g;
+    // padding lanes read row 0 (memory that exists) and drop it below: no branch between the requests
+    const uint16_t* qrow = A.q16 + (vrow ? ((size_t)tl * A.n_heads + head) * kD2 : (size_t)0) + 64 * g;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) qraw[t] = vrow ? *reinterpret_cast<const uint4*>(qrow + 8 * t) : make_uint4(0, 0, 0, 0);
+    for (int t = 0; t < 8; ++t) qraw[t] = *reinterpret_cast<const uint4*>(qrow + 8 * t);
   }
   const float sc_log2 = kLog2e * 0.0625f * A.gfac[gK];      // log2(e) / sqrt(256) x gain / 256 of the K table
   const size_t row0 = (size_t)kvh * A.max_ctx;
@@ -180,9 +185,15 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
     }
   };
   if (tile0 + wave < tile1) load_k(tile0 + wave);
+  {
+    u32x4* dst = reinterpret_cast<u32x4*>(s_buf) + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kTabLoads; ++k) { dst[256 * k] = tk[k]; dst[kTabBytes / 16 + 256 * k] = tv[k]; }
+  }
+  __syncthreads();
   rows16_to_f16(qraw, A.in_bf16);                    // behind the first tile's requests: a bf16 query does not hold them up
 #pragma unroll
-  for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, qraw[t]);
+  for (int t = 0; t < 8; ++t) qf[t] = __builtin_bit_cast(h8, vrow ? qraw[t] : make_uint4(0, 0, 0, 0));
   for (int T = tile0 + wave; T < tile1; T += 4) {
     const int t0 = T << 5;
     f4 vsc[2];
