@@ -437,7 +437,7 @@ template <> struct NewKeyArgs<0> {};
 template <int kInFlight, bool MS, int KB>
 __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyArgs<KB> X) {
   __shared__ float s_w[256];
-  __shared__ float s_o[8][kD2 + 4];
+  __shared__ __align__(16) float s_o[8][kD2 + 4];
   __shared__ float s_wsum[8];
   const int head = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x;
   size_t pair0 = (size_t)tok * A.S;
@@ -464,8 +464,12 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   request(0);
   float new_s[2] = {-1e30f, -1e30f}, new_v[2] = {0.f, 0.f};       // score in log2 units and V value (channel tid) of the new keys
   bool seen[2] = {false, false};               // uniform over the workgroup
+  float ksc[2] = {0.f, 0.f};
+  float kfac = 0.f;
+  __shared__ float s_dot[2][4], s_max[4];
+  float pmv = -1e30f, plv = 0.f;               // the split this thread weighs
+  if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
   if constexpr (KB != 0) {
-    __shared__ float s_dot[2][4];
     __shared__ float s_tab[2][256];              // K and V table of the kv head
     __shared__ uint32_t s_code[4][64], s_fld[4][64];
     __shared__ float s_scale[4];
@@ -476,6 +480,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
     const uint32_t tk = N.pairs[((size_t)gK << (8 + KB)) + tid], tv = N.pairs[((size_t)gV << (8 + KB)) + tid];
     const float q = row16_value(N.q16[((size_t)tok * A.n_heads + head) * kD2 + tid], N.in_bf16);
     const float mu = N.mu ? N.mu[(size_t)gV * 256 + tid] : 0.f;
+    const float gk = N.gfac[gK], gv = N.gfac[gV];
     const int pos = *N.d_pos;
     if (u_w <= tok) {                            // uniform over the wave
       uint32_t states; float scale;
@@ -492,35 +497,35 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
     s_tab[0][tid] = __half2float(__ushort_as_half((uint16_t)(tk >> 16)));
     s_tab[1][tid] = __half2float(__ushort_as_half((uint16_t)(tv >> 16)));
     __syncthreads();
-    float ksc[2] = {0.f, 0.f}, dot[2] = {0.f, 0.f};
+    float dot[2] = {0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int r = pos + u;
       seen[u] = u <= tok && r >= 0 && r < N.max_ctx;
       if (!seen[u]) continue;
       ksc[u] = s_scale[2 * u];
+      kfac = kLog2e * 0.0625f * gk;
       dot[u] = q * s_tab[0][reinterpret_cast<const uint8_t*>(s_code[2 * u])[tid]];
-      new_v[u] = s_tab[1][reinterpret_cast<const uint8_t*>(s_code[2 * u + 1])[tid]] * s_scale[2 * u + 1] * N.gfac[gV] + mu;
+      new_v[u] = s_tab[1][reinterpret_cast<const uint8_t*>(s_code[2 * u + 1])[tid]] * s_scale[2 * u + 1] * gv + mu;
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       dot[u] = lane_run32(lane_op32(dot[u], LaneAdd{}), LaneAdd{});
       if ((tid & 63) == 0) s_dot[u][tid >> 6] = dot[u];
     }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-      if (seen[u]) new_s[u] = (s_dot[u][0] + s_dot[u][1] + s_dot[u][2] + s_dot[u][3]) * ksc[u] * (kLog2e * 0.0625f * N.gfac[gK]);
   }
-  float pmv = -1e30f, plv = 0.f;
-  if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
+  // the splits' maximum goes to LDS in front of the barrier the new keys' scores need anyway
   float M2 = pmv;
   M2 = lane_rows(lane_row16(M2, LaneMax{}), LaneMax{});
-  if ((tid & 63) == 0) s_wsum[tid >> 6] = M2;
+  if ((tid & 63) == 0) s_max[tid >> 6] = M2;
   __syncthreads();
-  M2 = fmaxf(fmaxf(s_wsum[0], s_wsum[1]), fmaxf(s_wsum[2], s_wsum[3]));
-  if constexpr (KB != 0) M2 = fmaxf(M2, fmaxf(new_s[0], new_s[1]));
-  __syncthreads();
+  M2 = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+  if constexpr (KB != 0) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (seen[u]) new_s[u] = (s_dot[u][0] + s_dot[u][1] + s_dot[u][2] + s_dot[u][3]) * ksc[u] * kfac;
+    M2 = fmaxf(M2, fmaxf(new_s[0], new_s[1]));
+  }
   s_w[tid] = (tid < A.S && pmv > -1e29f) ? exp2f(pmv - M2) * plv : 0.f;
   __syncthreads();
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -540,8 +545,8 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
     if (!MS || s0 >= A.S) break;
     request(s0);
   }
-#pragma unroll
-  for (int c = 0; c < 8; ++c) s_o[sl][c8 + c] = acc[c];
+  *reinterpret_cast<float4*>(&s_o[sl][c8]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  *reinterpret_cast<float4*>(&s_o[sl][c8 + 4]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
   if ((tid & 31) == 0) s_wsum[sl] = wsum;
   __syncthreads();
   float o = 0.f, L = 0.f;

@@ -516,7 +516,7 @@ template <int kInFlight, bool MS, bool ADAPT>
 __global__ void __launch_bounds__(256) combine_kernel(YKA_COMBINE_PARAMS, CombineArgs A) {
   YKA_COMBINE_TAKE(A)
   __shared__ float s_w[256];
-  __shared__ float s_o[16][kD + 4];
+  __shared__ __align__(16) float s_o[16][kD + 4];
   __shared__ float s_wsum[16];
   const int head = blockIdx.x, tid = threadIdx.x;
   int tok = blockIdx.y;
@@ -574,8 +574,8 @@ __global__ void __launch_bounds__(256) combine_kernel(YKA_COMBINE_PARAMS, Combin
     if (!MS || s0 >= A.S) break;
     request(s0);
   }
-#pragma unroll
-  for (int c = 0; c < 8; ++c) s_o[sl][c8 + c] = acc[c];
+  *reinterpret_cast<float4*>(&s_o[sl][c8]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  *reinterpret_cast<float4*>(&s_o[sl][c8 + 4]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
   if ((tid & 15) == 0) s_wsum[sl] = wsum;
   __syncthreads();
   float y = 0.f;

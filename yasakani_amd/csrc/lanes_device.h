@@ -44,6 +44,7 @@ __device__ __forceinline__ T lane_op32(T v, Op op) {
   return op(__builtin_bit_cast(T, r0), __builtin_bit_cast(T, r1));
 }
 struct LaneMax { template <class T> __device__ __forceinline__ T operator()(T a, T b) const { if constexpr (__is_same(T, float)) return fmaxf(a, b); else return a > b ? a : b; } };
+struct LaneMinF { __device__ __forceinline__ float operator()(float a, float b) const { return fminf(a, b); } };
 struct LaneMin { __device__ __forceinline__ int operator()(int a, int b) const { return a < b ? a : b; } };
 struct LaneAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
 // over the four lanes l, l ^ 16, l ^ 32, l ^ 48

@@ -38,16 +38,17 @@ __device__ __forceinline__ void pick_job(const TbJobs& A, int row, int lane, uin
   for (int k = 0; k < 4; ++k) total = __fadd_rn(total, (&e0.x)[k]);
 #pragma unroll
   for (int k = 0; k < 4; ++k) total = __fadd_rn(total, (&e1.x)[k]);
-  float least = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(total), 0));
-  int keep = 0;
-  states = all[0];
+  // the smallest total, the first of equal ones; one that is not a number never wins, except by being the first multiplier's
+  const float inf = __builtin_huge_valf(), mine = lane < A.nm && total == total ? total : inf;
+  const float least = lane_row16(mine, LaneMinF{});
+  const uint64_t at = __ballot(lane < A.nm && mine == least), first_bad = __ballot(lane == 0 && total != total);
+  const int keep = __builtin_amdgcn_readfirstlane(first_bad ? 0 : __builtin_ctzll(at));
 #pragma unroll
-  for (int i = 1; i < kMaxMult; ++i) {
-    const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(total), i));
-    const bool better = i < A.nm && v < least;           // uniform over the wave
-    least = better ? v : least; keep = better ? i : keep; states = better ? all[i] : states;
-  }
-  scale = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s), __builtin_amdgcn_readfirstlane(keep)));
+  for (int b = kMaxMult / 2; b; b >>= 1)
+#pragma unroll
+    for (int i = 0; i < b; ++i) all[i] = (keep & b) ? all[i + b] : all[i];       // uniform over the wave
+  states = all[0];
+  scale = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s), keep));
 }
 // packs and stores the fields of those states (fld: 256 bytes of LDS private to the wave)
 template <int KB>
