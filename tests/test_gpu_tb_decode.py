@@ -113,3 +113,39 @@ def test_rows_as_the_oracle_codes_them(native, oracle, kk, heads, n_mult, M, pos
             ref = oracle.tb_encode_rows(blob, np.full(M, 2 * h + kind, np.int32), np.arange(M, dtype=np.int32), x[:, h].astype(np.float32))
             assert np.array_equal(words[h], ref["words"][:, :8 * kk]), (kind, h)
             assert np.array_equal(np.asarray(scales[h]).view(np.uint32), np.asarray(ref["scale"]).view(np.uint32)), (kind, h)
+
+
+@pytest.mark.parametrize("kk", [4, 5])
+@pytest.mark.parametrize("M", [3, 16, 17])                    # 17: stored by a launch of their own
+@pytest.mark.parametrize("pos,splits", [(0, 0), (30, 0), (250, 0), (250, 1), (250, 97), (1008 - 3, 0)])
+@pytest.mark.parametrize("siblings", [False, True])
+def test_windows_store_every_row(native, kk, M, pos, splits, siblings):
+    """Rows stored by the attention launch of a window: over two tiles, in a share of one split and of many, in front of the end of the
+    container, and siblings (a depth table of zeros) that no query row's tiles reach.  Against the rows of an append."""
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(M + pos)
+    half = lambda n, heads: rng.standard_normal((n, heads, 256)).astype(np.float16)    # noqa: E731
+    blob = kvqp.synthetic(layers=1, kk=kk, seed=11, mu=True)
+    q, k, v = half(M, 24), half(M, 4), half(M, 4)
+    old_k, old_v = half(max(pos, 1), 4), half(max(pos, 1), 4)
+    n = min(M, 1024 - pos)
+    stored, outs = [], []
+    for fused in (True, False):
+        with native.KvCache(max_ctx=1024, head_dim=256, max_rows=1024) as kv:
+            kv.set_profile(blob)
+            kv.set_opt(2, splits)
+            if pos:
+                kv.append_host(0, old_k[:pos], old_v[:pos], 0)
+            depth = np.zeros(M, np.uint8) if siblings else None
+            if fused:
+                kv.poison_workspace()
+                outs.append(kv.layer_call(0, q, k, v, pos, depth))
+            else:
+                kv.append_host(0, k, v, pos)
+                outs.append(kv.layer_call(0, q, None, None, pos, depth))
+            stored.append([np.ascontiguousarray(x).view(np.uint8) for x in kv.export_rows(0, 0, pos + n)])
+    for a, b in zip(*stored):
+        assert np.array_equal(a, b)
+    a, b = (x.astype(np.float32) for x in outs)
+    # the same rows, other split bounds: partials and outputs rounded to fp16 once each (2^-11), sums in fp32
+    assert np.isfinite(a).all() and np.linalg.norm(a - b) <= 1e-3 * np.linalg.norm(b)

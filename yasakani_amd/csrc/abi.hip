@@ -297,7 +297,10 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
     check_tb_layer(kv, layer);
     // decode without a depth table: the encoder's search rides in the attention launch, which leaves the new rows to the combiner
     const bool fuse = k16 && M <= 2 && !depth && mode == 0 && !kv->opt_force_narrow;
-    if (k16 && !fuse) do_append(kv, layer, k16, v16, M, d_pos, st);
+    const bool stores = k16 && M > 2 && M <= kTbFuseRows && !kv->opt_force_narrow;    // the wide kernel codes and stores the rows
+    TbEncArgs E{};
+    if (stores) launch_tb_search(E = tb_encoder_args(kv, layer, layer, k16, v16, 0, M, d_pos), st);
+    else if (k16 && !fuse) do_append(kv, layer, k16, v16, M, d_pos, st);
     const int slice = slice256(kv, M);
     for (int s0 = 0; s0 < M; s0 += slice) {
       const Part256 P = part256(kv, M, s0, slice);
@@ -307,6 +310,7 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
       A.rows_per_block = P.rows_per_block;
       CombineArgs C{kv->pm, kv->pl, kv->pacc16, P.S, P.Ms, NH, out16 + (size_t)s0 * NH * 256, kv->opt_unrot, bf16};
       A.s_short = C.s_short = P.s_short; C.d_pos = d_pos;
+      if (stores) A.jobs = tb_jobs(E);
       if (fuse) {
         const TbEncArgs E = tb_encoder_args(kv, layer, layer, k16, v16, 0, M, d_pos);
         launch_tb_encode_attend(E, A, T.kb, st);

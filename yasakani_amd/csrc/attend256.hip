@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   if (tid < A.S) { pmv = A.pm[p0 + (size_t)tid * A.n_heads]; plv = A.pl[p0 + (size_t)tid * A.n_heads]; }
   if constexpr (KB != 0) {
     __shared__ float s_tab[2][256];              // K and V table of the kv head
-    __shared__ uint32_t s_code[4][64], s_fld[4][64];
+    __shared__ uint32_t s_code[4][64];
     __shared__ float s_scale[4];
     const TbAttnArgs& N = X.N;
     const int kvh = head / kG, gK = (N.layer * N.n_kv + kvh) * 2, gV = gK + 1;
@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
       const int r = pos + u_w;
       if (tok == A.M - 1 && head % kG == 0 && r >= 0 && r < N.max_ctx) {
         const size_t row = (size_t)kvh * N.max_ctx + r;
-        store_coded_row<KB>(const_cast<uint8_t*>((wave & 1) ? N.vpay : N.kpay) + row * N.stride, reinterpret_cast<uint8_t*>(s_fld[wave]), lane, states);
+        store_coded_row<KB>(const_cast<uint8_t*>((wave & 1) ? N.vpay : N.kpay) + row * N.stride, lane, states);
         if (lane == 0) const_cast<float*>((wave & 1) ? N.vscl : N.kscl)[row] = scale;
       }
     }

@@ -14,7 +14,7 @@
 //   V  [256 channels][96 B] key 16kb + 4g + r sits at slot 8g + 4kb + r: the 8 keys whose probabilities an MFMA lane of
 //                           group g holds are 16 contiguous bytes
 //   SC [2][32] fp32        K scales, V scales of the tile's keys
-#include "yka_internal.h"
+#include "tb_store_device.h"
 #include <hip/hip_fp16.h>
 #include <type_traits>
 
@@ -188,8 +188,49 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   if (A.depth) { for (int t = tok_lo; t < tok_hi; ++t) { const int dp = (int)A.depth[A.tok0 + t]; maxdep = max(maxdep, dp); mindep = min(mindep, dp); } }
   else { mindep = A.tok0 + tok_lo; maxdep = A.tok0 + tok_hi - 1; }
   const int maxlen = min(pos + maxdep + 1, A.max_ctx), minlen = min(pos + mindep + 1, A.max_ctx);
-  const int ntiles = (maxlen + 31) >> 5, tps = (ntiles + A.S - 1) / A.S;
-  const int tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
+  const int ntiles = (maxlen + 31) >> 5;
+  int tps = (ntiles + A.S - 1) / A.S, tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
+  // where the rows of the pass are stored here (below) the last split owns the tiles that hold them and as many in front of them as its share
+  // leaves once the coding is paid for, about two tiles; the others share the rest evenly
+  if (A.jobs.scr && A.S > 1) {
+    constexpr int kStoreCost = 2;
+    const int Tw = min(min(ntiles, max(0, pos + A.tok0) >> 5), (A.S - 1) * ((ntiles + kStoreCost + A.S - 1) / A.S));
+    tps = (Tw + A.S - 2) / (A.S - 1);
+    tile0 = split == A.S - 1 ? Tw : min(Tw, split * tps);
+    tile1 = split == A.S - 1 ? ntiles : min(Tw, tile0 + tps);
+  }
+
+  // ---- the rows of the pass: a workgroup codes and stores those that lie in the tiles of its own range before it reads them, from what
+  //      the searches have left, a wave per row.  Row blocks of one kv head write identical bytes; a row past the last tile of the last
+  //      row block (no query row of the pass sees it: a depth table may say so) is stored by that block's last split.  Writer and
+  //      readers are waves of one CU and one write-through L1.  Every condition that guards the barrier is uniform over the workgroup. ----
+  if (A.jobs.scr) {
+    const int r0 = pos + A.tok0, Tn0 = r0 >> 5, Tn1 = (r0 + A.M - 1) >> 5;
+    const bool last_wg = split == A.S - 1 && rb == (int)gridDim.z - 1;
+    if ((Tn0 < tile1 && Tn1 >= tile0) || (last_wg && Tn1 >= ntiles)) {
+      constexpr int kRows = 2 * kTbFuseRows / 8;             // rows of a wave at most
+      JobTotals errors[kRows];
+      uint32_t states[kRows];
+      float scale[kRows];
+      auto job_row = [&](int it) { return min(8 * it + wave, 2 * A.M - 1) * A.n_kv + kvh; };    // K (even) or V row of token (8 it + wave) / 2
+#pragma unroll
+      for (int it = 0; it < kRows; ++it) errors[it] = request_errors(A.jobs, job_row(it), lane);
+#pragma unroll
+      for (int it = 0; it < kRows; ++it) states[it] = job_states(A.jobs, job_row(it), choose_job(A.jobs, lane, errors[it], scale[it]), lane);
+#pragma unroll
+      for (int it = 0; it < kRows; ++it) {
+        const int h = 8 * it + wave, r = r0 + (h >> 1), T = r >> 5;
+        if (h < 2 * A.M && r >= 0 && r < A.max_ctx && ((T >= tile0 && T < tile1) || (last_wg && T >= ntiles))) {   // uniform over the wave
+          const size_t row = (size_t)kvh * A.max_ctx + r;
+          store_coded_row<KB>(const_cast<uint8_t*>((h & 1) ? A.vpay : A.kpay) + row * A.stride, lane, states[it]);
+          if (lane == 0) const_cast<float*>((h & 1) ? A.vscl : A.kscl)[row] = scale[it];
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __syncthreads();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+  }
 
   const float sc_log2 = kLog2e * 0.0625f * A.gfac[gK];      // log2(e) / sqrt(256) x gain / 256 of the K table (positive)
   float m_run = -1e30f, l_run = 0.f;           // m_run in log2 units, shared by the four lanes of a row

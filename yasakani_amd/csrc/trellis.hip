@@ -603,8 +603,7 @@ __global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
 template <int KB>
 __global__ void __launch_bounds__(256) tb_store_kernel(const int* p_pos, const uint8_t* p_scr, int p_nm, TbEncArgs A) {
   A.d_pos = p_pos; A.scr = const_cast<uint8_t*>(p_scr); A.nm = p_nm;
-  __shared__ uint32_t fld[4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = blockIdx.x * 4 + wave;
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= A.nrow) return;                             // no barrier below
   uint32_t states; float scale;
   pick_job(tb_jobs(A), row, lane, states, scale);
@@ -618,7 +617,7 @@ __global__ void __launch_bounds__(256) tb_store_kernel(const int* p_pos, const u
   } else pos = *A.d_pos + R.tok;
   if (!ok || pos < 0 || pos >= A.max_ctx || (A.pos_limit != 0 && pos >= A.pos_limit)) return;
   const size_t index = (size_t)R.kvh * A.max_ctx + (size_t)pos;
-  store_coded_row<KB>((R.is_v ? A.pay1 : A.pay0) + container + index * (size_t)A.stride, reinterpret_cast<uint8_t*>(fld[wave]), lane, states);
+  store_coded_row<KB>((R.is_v ? A.pay1 : A.pay0) + container + index * (size_t)A.stride, lane, states);
   if (lane == 0) reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(R.is_v ? A.scl1 : A.scl0) + container)[index] = scale;
 }
 
@@ -668,11 +667,11 @@ static void launch_store(const TbEncArgs& A, hipStream_t st) {
   hipLaunchKernelGGL(tb_store_kernel<KB>, dim3((A.nrow + 3) / 4), dim3(256), 0, st, A.d_pos, A.scr, A.nm, A);
 }
 template <int KB>
-static void launch_encode(const TbEncArgs& A, hipStream_t st) {
+static void launch_search(const TbEncArgs& A, hipStream_t st) {
   if (A.in_bf16) hipLaunchKernelGGL((tb_search_kernel<KB, true>), dim3(A.nrow * A.nm), dim3(256), 0, st, A);   // k16 / v16 are bf16 rows
   else hipLaunchKernelGGL((tb_search_kernel<KB, false>), dim3(A.nrow * A.nm), dim3(256), 0, st, A);
-  launch_store<KB>(A, st);
 }
+void launch_tb_search(const TbEncArgs& A, hipStream_t st) { if (A.kb == 4) launch_search<4>(A, st); else launch_search<5>(A, st); }
 void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
   if (A.nrow <= 0) return;
   if (A.yin) {
@@ -680,7 +679,8 @@ void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
     hipLaunchKernelGGL(tb_select_kernel, dim3(A.nrow), dim3(256), 0, st, A);
     return;
   }
-  if (A.kb == 4) launch_encode<4>(A, st); else launch_encode<5>(A, st);
+  launch_tb_search(A, st);
+  if (A.kb == 4) launch_store<4>(A, st); else launch_store<5>(A, st);
 }
 void launch_tb_encode_attend(const TbEncArgs& E, const TbAttnArgs& A, int kb, hipStream_t st) {
   const int n_search = E.nrow * E.nm;

@@ -155,6 +155,7 @@ struct TbAttnArgs {
   int adapt = 0;     // multi-stream pass: workgroups shared out by ms_share, the shares left in plan
   int2* plan = nullptr;
   int rows_per_block = 128;   // wide kernel only
+  TbJobs jobs{};     // wide kernel: searches of the rows of the pass (at most kTbFuseRows), which its workgroups then store; scr == nullptr: they are stored
   int s_short = 0;   // decode: splits in use at a position up to kShortPos, S beyond; 0: always S (splits_at)
 };
 void launch_attend_tb(const TbAttnArgs&, int kb, hipStream_t);        // row tiles of 2 tokens x 6 heads (decode; any width)
@@ -165,10 +166,17 @@ __device__ __forceinline__ void tb_split_of(const TbAttnArgs& A, int b, int& spl
   if (A.s_short) { split = b / A.n_kv; kvh = b % A.n_kv; } else { split = b % A.S; kvh = b / A.S; }
 }
 void launch_tb_encode(const TbEncArgs&, hipStream_t);
+void launch_tb_search(const TbEncArgs&, hipStream_t);     // the searches alone (cache form): TbAttnArgs::jobs has their results stored
 // one or two tokens: searches of the encoder and attention over the keys in front of *d_pos; the combiner has to store the new rows and add them
 void launch_tb_encode_attend(const TbEncArgs&, const TbAttnArgs&, int kb, hipStream_t);
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t);
+
+// Trellis windows of at most so many rows are coded and stored by the attention launch, the others by a launch of their own: the workgroup that
+// holds the window codes 2 rows per token, 8 at a time, which costs about two tiles of its share (its range is shorter by so much) and saves
+// the launch between.  us per 16 layers, launch / here: 16 rows of 5 bits at 16,384 tokens 743 / 687; per 4 layers at 500 tokens 3 rows 87.9 /
+// 81.8, 10 rows 107.9 / 103.8, 16 rows 138.2 / 138.9 (nothing hides the coding there), 16 rows of 4 bits at 3,000 156.2 / 145.3.
+constexpr int kTbFuseRows = 16;
 
 // launchers (each checks nothing: the C layer validates shapes first)
 void launch_append(const AppendArgs&, hipStream_t);
