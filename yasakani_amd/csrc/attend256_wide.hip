@@ -196,8 +196,19 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   if (A.depth) { for (int t = tok_lo; t < tok_hi; ++t) { const int dp = (int)A.depth[A.tok0 + t]; maxdep = max(maxdep, dp); mindep = min(mindep, dp); } }
   else { mindep = A.tok0 + tok_lo; maxdep = A.tok0 + tok_hi - 1; }
   const int maxlen = min(pos + maxdep + 1, A.kv.max_ctx), minlen = min(pos + mindep + 1, A.kv.max_ctx);
-  const int ntiles = (maxlen + 31) >> 5, tps = (ntiles + A.S - 1) / A.S;
-  const int tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
+  const int ntiles = (maxlen + 31) >> 5;
+  int tps = (ntiles + A.S - 1) / A.S, tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
+  // where the rows of the pass are stored here (below) the last split owns the tiles that hold them and as many in front of them as its share
+  // leaves once the quantization is paid for; the others share the rest evenly
+  // (in windows of more than 32 rows and on short contexts more workgroups than one should quantize: 64 rows at 1,600 tokens, 4 layers: 86 us a
+  // pass, 98 with all rows in the last split; 4 rows at 3,000 49.5 and 46.3, 16 at 4,090 73.3 and 68.9, 8 at 8,180 62.1 and 58.4)
+  if (A.k16 && A.M <= 32 && A.S > 1 && ntiles >= 2 * A.S) {
+    const int cost = 1 + A.M / 16;
+    const int Tw = min(min(ntiles, max(0, pos + A.tok0) >> 5), (A.S - 1) * ((ntiles + cost + A.S - 1) / A.S));
+    tps = (Tw + A.S - 2) / (A.S - 1);
+    tile0 = split == A.S - 1 ? Tw : min(Tw, split * tps);
+    tile1 = split == A.S - 1 ? ntiles : min(Tw, tile0 + tps);
+  }
 
   // ---- fused quantize-on-append (a slice of at most 64 tokens): a workgroup stores the rows of this pass that lie in
   //      the tiles of its own range before it reads them, so no workgroup reads a row another one has to store.  Row
@@ -212,21 +223,27 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
     const bool last_wg = split == A.S - 1 && rb == (int)gridDim.z - 1;
     if ((Tn0 < tile1 && Tn1 >= tile0) || (last_wg && Tn1 >= ntiles)) {
       const int slot = tid >> 5, c = tid & 31;
-      uint4 rawv[8];
-      bool mine[8];
+      auto store_rows = [&](auto steps) __attribute__((always_inline)) {           // 8 tokens a step
+        constexpr int kSteps = decltype(steps)::value;
+        uint4 rawv[kSteps];
+        bool mine[kSteps];
 #pragma unroll
-      for (int it = 0; it < 8; ++it) {
-        const int hh = it * 16 + slot, t = hh >> 1, r = r0 + t, T = r >> 5;
-        mine[it] = t < A.M && r >= 0 && r < A.kv.max_ctx && ((T >= tile0 && T < tile1) || (last_wg && T >= ntiles));
-        const uint16_t* src = ((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD2 + 8 * c;
-        rawv[it] = mine[it] ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
-      }
-      if constexpr (BF) rows16_to_f16(rawv);
+        for (int it = 0; it < kSteps; ++it) {
+          const int hh = it * 16 + slot, t = hh >> 1, r = r0 + t, T = r >> 5;
+          mine[it] = t < A.M && r >= 0 && r < A.kv.max_ctx && ((T >= tile0 && T < tile1) || (last_wg && T >= ntiles));
+          const uint16_t* src = ((hh & 1) ? A.v16 : A.k16) + ((size_t)(A.tok0 + t) * A.kv.n_kv + kvh) * kD2 + 8 * c;
+          rawv[it] = mine[it] ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
+        }
+        if constexpr (BF) rows16_to_f16(rawv);
 #pragma unroll
-      for (int it = 0; it < 8; ++it) {
-        const int hh = it * 16 + slot;
-        quant_store_word256(A.kv, kvh, r0 + (hh >> 1), hh & 1, rawv[it], c, mine[it]);
-      }
+        for (int it = 0; it < kSteps; ++it) {
+          const int hh = it * 16 + slot;
+          quant_store_word256(A.kv, kvh, r0 + (hh >> 1), hh & 1, rawv[it], c, mine[it]);
+        }
+      };
+      if (A.M <= 16) store_rows(std::integral_constant<int, 2>{});
+      else if (A.M <= 32) store_rows(std::integral_constant<int, 4>{});
+      else store_rows(std::integral_constant<int, 8>{});
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
       __syncthreads();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
