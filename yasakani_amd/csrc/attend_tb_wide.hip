@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   // key range of the workgroup: its splits cut [0, maxlen) of the block's longest row into 32-key tiles
   const int tok_lo = (rb * RPB) / kG, tok_hi = min(A.M, (rb * RPB + RPB + kG - 1) / kG);
   int maxdep = 0, mindep = 0x7fffffff;
-  if (A.depth) { for (int t = tok_lo; t < tok_hi; ++t) { const int dp = (int)A.depth[A.tok0 + t]; maxdep = max(maxdep, dp); mindep = min(mindep, dp); } }
+  if (A.depth) depth_range(A.depth + A.tok0, tok_lo, tok_hi, mindep, maxdep);
   else { mindep = A.tok0 + tok_lo; maxdep = A.tok0 + tok_hi - 1; }
   const int maxlen = min(pos + maxdep + 1, A.max_ctx), minlen = min(pos + mindep + 1, A.max_ctx);
   const int ntiles = (maxlen + 31) >> 5;

@@ -269,6 +269,15 @@ __device__ __forceinline__ void store_partial16(uint16_t* p, uint4 v) {
   __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)p, u32x4{v.x, v.y, v.z, v.w}, "agent");
 }
 
+// least and greatest depth of tokens tok_lo .. tok_hi - 1 (at most 64), a token per lane: one trip to memory (a loop over them was one each:
+// 4 layers of 16 rows with a depth table at 9,000 tokens 68.9 us, 63.7 so, of 24 rows of 256 channels 88.8 and 85.8, of 16 trellis rows 177 and 172)
+__device__ __forceinline__ void depth_range(const uint8_t* depth, int tok_lo, int tok_hi, int& least, int& most) {
+  const int t = tok_lo + (int)(threadIdx.x & 63), last = max(tok_lo, tok_hi - 1);
+  const int dp = depth[min(t, last)];
+  least = __builtin_amdgcn_readfirstlane(lane_rows(lane_row16(dp, LaneMin{}), LaneMin{}));
+  most = __builtin_amdgcn_readfirstlane(lane_rows(lane_row16(dp, LaneMax{}), LaneMax{}));
+}
+
 // Sums and maxima of the plans below run through lane-crossing moves (a shift inside rows of 16 lanes, then two row broadcasts),
 // not through LDS: a plan stands in front of everything else a workgroup does (multi-stream passes, 5 trellis streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128
 // channels 14.9 and 13.9).
