@@ -513,8 +513,8 @@ void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
 // workgroups as the chip holds at once, each walks its share of the tokens, so that the choice of the splits is made 8 times per CU and
 // not once per row (1,024 rows at 9,000 tokens with the inverse rotation: 42.4 us with a workgroup per row, 37.9 so).
 template <int kInFlight, bool MS, bool ADAPT>
-__global__ void __launch_bounds__(256) combine_kernel(YKA_COMBINE_PARAMS, CombineArgs A) {
-  YKA_COMBINE_TAKE(A)
+__global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, CombineArgs A) {
+  take_head(A, head_args);
   __shared__ float s_w[256];
   __shared__ __align__(16) float s_o[16][kD + 4];
   __shared__ float s_wsum[16];
@@ -608,8 +608,8 @@ __global__ void __launch_bounds__(256) combine_kernel(YKA_COMBINE_PARAMS, Combin
 // ADAPT: rows of a prefill slice; as many workgroups as the chip holds at once (8 per CU), each walks its share - most slices on
 // short contexts find nothing to do here and should not pay for dispatching thousands of workgroups to find out.
 template <bool ADAPT>
-__global__ void __launch_bounds__(256) combine_rows_kernel(YKA_COMBINE_PARAMS, CombineArgs A) {
-  YKA_COMBINE_TAKE(A)
+__global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args, CombineArgs A) {
+  take_head(A, head_args);
   if constexpr (ADAPT) {
     A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S, A.adapt);
     if (A.S == 1 && A.direct) return;
@@ -655,23 +655,23 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(YKA_COMBINE_PARAMS, C
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
   if (A.plan) {                                    // a stream may hold any share of the splits (256 at most)
-    hipLaunchKernelGGL((combine_kernel<4, true, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);
+    hipLaunchKernelGGL((combine_kernel<4, true, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);
     return;
   }
   if (A.S <= 32 && !A.unrot && A.M >= 8) {
     const int wgs = (A.M * A.n_heads + 3) / 4;
-    if (A.adapt) hipLaunchKernelGGL(combine_rows_kernel<true>, dim3(min(wgs, 2048)), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);
-    else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);
+    if (A.adapt) hipLaunchKernelGGL(combine_rows_kernel<true>, dim3(min(wgs, 2048)), dim3(256), 0, st, combine_head(A), A);
+    else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, combine_head(A), A);
     return;
   }
   if (A.adapt) {                                   // S <= kChunkMaxSplits
     static_assert(kChunkMaxSplits <= 64, "16 split lanes x 4 rows in flight");
-    hipLaunchKernelGGL((combine_kernel<4, false, true>), dim3(A.n_heads, min(A.M, max(1, 2048 / A.n_heads))), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);
+    hipLaunchKernelGGL((combine_kernel<4, false, true>), dim3(A.n_heads, min(A.M, max(1, 2048 / A.n_heads))), dim3(256), 0, st, combine_head(A), A);
     return;
   }
-  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);   // S <= 256
-  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);
-  else hipLaunchKernelGGL((combine_kernel<4, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, YKA_COMBINE_GIVE(A), A);
+  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);   // S <= 256
+  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);
+  else hipLaunchKernelGGL((combine_kernel<4, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);
 }
 
 }  // namespace yka

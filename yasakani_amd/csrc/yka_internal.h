@@ -96,10 +96,19 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
 // tokens 172.5 / 166.5, one 5-bit trellis row at 16,001 382 / 371, 8 rows at 12,037 (the combiner alone) 226 / 220, one token at
 // 1,003 115.4 / 113.8, 16 streams 27.1 / 26.7 a pass.  Not where it measured slower: the 256-channel kernels (273 / 280), wide
 // windows (737 / 743), windows of 3 to 5 rows in the mid kernel (212 / 218; 8 rows 220 / 218).
-#define YKA_COMBINE_PARAMS const float *p_pm, const float *p_pl, const uint16_t *p_acc, const void *p_where, int p_s, int p_heads
-#define YKA_COMBINE_GIVE(A) (A).pm, (A).pl, (A).pacc16, (A).plan ? (const void*)(A).plan : (const void*)(A).d_pos, (A).S, (A).n_heads
-#define YKA_COMBINE_TAKE(A) \
-  A.pm = p_pm; A.pl = p_pl; A.pacc16 = p_acc; A.S = p_s; A.n_heads = p_heads; A.d_pos = static_cast<const int*>(p_where); A.plan = static_cast<const int2*>(p_where);
+// One leading argument of eight words, not six: every argument of a launch costs the host, and a decode call issued outside a graph is as long as
+// the host takes (one token at 26,630 tokens, 2 layers: 25.7 us without, 28.1 with six, 26.1 so).
+typedef uint32_t CombineHead __attribute__((ext_vector_type(8)));     // pm, pl, pacc16 (two words each), S, n_heads
+inline CombineHead combine_head(const CombineArgs& A) {
+  const uint64_t pm = (uint64_t)(uintptr_t)A.pm, pl = (uint64_t)(uintptr_t)A.pl, acc = (uint64_t)(uintptr_t)A.pacc16;
+  return CombineHead{(uint32_t)pm, (uint32_t)(pm >> 32), (uint32_t)pl, (uint32_t)(pl >> 32), (uint32_t)acc, (uint32_t)(acc >> 32), (uint32_t)A.S, (uint32_t)A.n_heads};
+}
+__device__ __forceinline__ void take_head(CombineArgs& A, CombineHead H) {
+  A.pm = reinterpret_cast<const float*>((uintptr_t)H[0] | ((uintptr_t)H[1] << 32));
+  A.pl = reinterpret_cast<const float*>((uintptr_t)H[2] | ((uintptr_t)H[3] << 32));
+  A.pacc16 = reinterpret_cast<const uint16_t*>((uintptr_t)H[4] | ((uintptr_t)H[5] << 32));
+  A.S = (int)H[6]; A.n_heads = (int)H[7];
+}
 // projection outputs xq [M][n_heads][128], xk / xv [M][n_kv][128] fp32 -> q16 and the cache rows at *d_pos + t
 struct PostArgs {
   KvView kv; const float* xq; const float* xk; const float* xv; int M; int n_heads; const int* d_pos;
