@@ -332,3 +332,32 @@ def test_decode_merge_against_the_wide_kernel(native, kk, M, ctx, splits):
     # the same codes; P (times the V scale) and the outputs are fp16 on both sides, 2^-11 each
     assert np.isfinite(out).all()
     assert np.linalg.norm(out - wide) <= 1e-3 * np.linalg.norm(wide)
+
+
+@pytest.mark.parametrize("M", [3, 16, 17, 32, 33])            # steps of the quantizer, and the widest window whose rows one split owns
+@pytest.mark.parametrize("pos,splits", [(0, 2), (127, 2), (128, 2), (700, 3), (700, 11), (1024 - 33, 4), (250, 1), (505, 0)])
+@pytest.mark.parametrize("siblings", [False, True])
+def test_windows_store_every_row_whoever_owns_it(native, M, pos, splits, siblings):
+    """Rows stored by the window launch - in the last split's share where every split has two tiles or more (pos 127: exactly two, with 32
+    rows more than two), in the tiles' own splits otherwise; siblings (a depth table of zeros) beyond every query row's tiles; rows up to
+    the end of the container.  Against the rows of an append and attention over them."""
+    rng = np.random.default_rng(M + pos)
+    half = lambda n, heads: rng.standard_normal((n, heads, 256)).astype(np.float16)    # noqa: E731
+    q, k, v = half(M, 24), half(M, 4), half(M, 4)
+    old_k, old_v = half(max(pos, 1), 4), half(max(pos, 1), 4)
+    depth = np.zeros(M, np.uint8) if siblings else None
+    stored, outs = [], []
+    for fused in (True, False):
+        with native.KvCache(max_ctx=1024, head_dim=256, max_rows=1024) as kv:
+            kv.set_opt(2, splits)
+            if pos:
+                kv.append_host(0, old_k[:pos], old_v[:pos], 0)
+            kv.poison_workspace()
+            if not fused:
+                kv.append_host(0, k, v, pos)
+            outs.append(kv.layer_call(0, q, k if fused else None, v if fused else None, pos, depth).astype(np.float32))
+            stored.append([np.ascontiguousarray(x).view(np.uint8) for x in kv.export_rows(0, 0, pos + M)])
+    for a, b in zip(*stored):
+        assert np.array_equal(a, b)
+    # the same rows, other split bounds: partials and outputs rounded to fp16 once each (2^-11), sums in fp32
+    assert np.isfinite(outs[0]).all() and np.linalg.norm(outs[0] - outs[1]) <= 1e-3 * np.linalg.norm(outs[1])
