@@ -183,8 +183,8 @@ __device__ __forceinline__ void combine_column(const AttnArgs& A, int kvh, int r
 // TPT = 2 for a single-stream pass; MS (multi-stream pass, reference: src/q35_atxpk_ms.cu:13-33): one token per tile,
 // which reads the container and the position its row map names.
 template <bool MS>
-__global__ void __launch_bounds__(256, 2) attend_narrow_kernel(const int* p_pos, const int* p_slot, int p_m, AttnArgs A) {
-  if (MS) { A.rows.pos = p_pos; A.rows.slot = p_slot; A.M = p_m; } else A.d_pos = p_pos;
+__global__ void __launch_bounds__(256, 2) attend_narrow_kernel(std::conditional_t<MS, RowsHead, uint64_t> H, AttnArgs A) {
+  if constexpr (MS) take_head(A, H); else A.d_pos = head_ptr<const int>((uint32_t)H, (uint32_t)(H >> 32));
   __shared__ float s_m[4][16], s_l[4][16];
   __shared__ __align__(16) float s_acc[4][16][kD + 4];     // 8448 floats; the fused combiner needs 4672 of them
   __shared__ int s_ticket;
@@ -498,8 +498,8 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(const int* p_pos,
 }
 
 void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
-  if (A.rows.pos) hipLaunchKernelGGL(attend_narrow_kernel<true>, dim3(A.S, A.kv.n_kv, A.M), dim3(256), 0, st, A.rows.pos, A.rows.slot, A.M, A);
-  else hipLaunchKernelGGL(attend_narrow_kernel<false>, dim3(A.S, A.kv.n_kv, (A.M + 1) / 2), dim3(256), 0, st, A.d_pos, nullptr, A.M, A);
+  if (A.rows.pos) hipLaunchKernelGGL(attend_narrow_kernel<true>, dim3(A.S, A.kv.n_kv, A.M), dim3(256), 0, st, rows_head(A), A);
+  else hipLaunchKernelGGL(attend_narrow_kernel<false>, dim3(A.S, A.kv.n_kv, (A.M + 1) / 2), dim3(256), 0, st, (uint64_t)(uintptr_t)A.d_pos, A);
 }
 
 // combiner (reference: src/attention_kv4q.cu:325-332): M2 = max pm; w_s = pm_s > -1e29 ? 2^(pm_s - M2) * pl_s : 0;
@@ -513,8 +513,8 @@ void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
 // workgroups as the chip holds at once, each walks its share of the tokens, so that the choice of the splits is made 8 times per CU and
 // not once per row (1,024 rows at 9,000 tokens with the inverse rotation: 42.4 us with a workgroup per row, 37.9 so).
 template <int kInFlight, bool MS, bool ADAPT>
-__global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, CombineArgs A) {
-  take_head(A, head_args);
+__global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, CombineTail tail_args) {
+  CombineArgs A = combine_args(head_args, tail_args);
   __shared__ float s_w[256];
   __shared__ __align__(16) float s_o[16][kD + 4];
   __shared__ float s_wsum[16];
@@ -608,8 +608,8 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
 // ADAPT: rows of a prefill slice; as many workgroups as the chip holds at once (8 per CU), each walks its share - most slices on
 // short contexts find nothing to do here and should not pay for dispatching thousands of workgroups to find out.
 template <bool ADAPT>
-__global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args, CombineArgs A) {
-  take_head(A, head_args);
+__global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args, CombineTail tail_args) {
+  CombineArgs A = combine_args(head_args, tail_args);
   if constexpr (ADAPT) {
     A.S = chunk_splits_used(*A.d_pos, A.tok0, A.M, A.n_kv, A.max_ctx, A.S, A.adapt);
     if (A.S == 1 && A.direct) return;
@@ -655,23 +655,23 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
   if (A.plan) {                                    // a stream may hold any share of the splits (256 at most)
-    hipLaunchKernelGGL((combine_kernel<4, true, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);
+    hipLaunchKernelGGL((combine_kernel<4, true, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), combine_tail(A));
     return;
   }
   if (A.S <= 32 && !A.unrot && A.M >= 8) {
     const int wgs = (A.M * A.n_heads + 3) / 4;
-    if (A.adapt) hipLaunchKernelGGL(combine_rows_kernel<true>, dim3(min(wgs, 2048)), dim3(256), 0, st, combine_head(A), A);
-    else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, combine_head(A), A);
+    if (A.adapt) hipLaunchKernelGGL(combine_rows_kernel<true>, dim3(min(wgs, 2048)), dim3(256), 0, st, combine_head(A), combine_tail(A));
+    else hipLaunchKernelGGL(combine_rows_kernel<false>, dim3(wgs), dim3(256), 0, st, combine_head(A), combine_tail(A));
     return;
   }
   if (A.adapt) {                                   // S <= kChunkMaxSplits
     static_assert(kChunkMaxSplits <= 64, "16 split lanes x 4 rows in flight");
-    hipLaunchKernelGGL((combine_kernel<4, false, true>), dim3(A.n_heads, min(A.M, max(1, 2048 / A.n_heads))), dim3(256), 0, st, combine_head(A), A);
+    hipLaunchKernelGGL((combine_kernel<4, false, true>), dim3(A.n_heads, min(A.M, max(1, 2048 / A.n_heads))), dim3(256), 0, st, combine_head(A), combine_tail(A));
     return;
   }
-  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);   // S <= 256
-  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);
-  else hipLaunchKernelGGL((combine_kernel<4, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), A);
+  if (A.S > 128) hipLaunchKernelGGL((combine_kernel<16, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), combine_tail(A));   // S <= 256
+  else if (A.S > 64) hipLaunchKernelGGL((combine_kernel<8, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), combine_tail(A));
+  else hipLaunchKernelGGL((combine_kernel<4, false, false>), dim3(A.n_heads, A.M), dim3(256), 0, st, combine_head(A), combine_tail(A));
 }
 
 }  // namespace yka
