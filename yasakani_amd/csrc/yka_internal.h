@@ -98,8 +98,8 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
 // windows (737 / 743), windows of 3 to 5 rows in the mid kernel (212 / 218; 8 rows 220 / 218).
 // Such a pointer travels as an integer, and the combiners' arguments are split into head and tail, not repeated: a pointer among a
 // launch's arguments costs the host 0.2 us, and the 136 bytes of a repeated block 0.45 us more than these 96.  A call issued outside a graph
-// is as long as the host takes; 16 layers of one token at 1,622 tokens, us: 179 without preloaded arguments, 193 with three plain
-// arguments here and the block repeated, 185 with an integer here, 177 with the split.
+// is as long as the host takes; 16 layers of one token at 1,622 tokens, us: 177 without preloaded arguments, 192 with pointers
+// and the block repeated, 185 with integers, 178 with the split.
 typedef uint32_t CombineHead __attribute__((ext_vector_type(8)));     // pm, pl, pacc16 (two words each), S, n_heads
 struct CombineTail { uint16_t* out16; const int* d_pos; const int2* plan; int M, unrot, out_bf16, adapt, direct, tok0, n_kv, max_ctx, s_short; };
 inline CombineHead combine_head(const CombineArgs& A) {
@@ -109,24 +109,13 @@ inline CombineHead combine_head(const CombineArgs& A) {
 inline CombineTail combine_tail(const CombineArgs& A) {
   return CombineTail{A.out16, A.d_pos, A.plan, A.M, A.unrot, A.out_bf16, A.adapt, A.direct, A.tok0, A.n_kv, A.max_ctx, A.s_short};
 }
-// two words of such an argument as a pointer into global memory; without the address space the loads behind it are flat ones
-template <typename T> __device__ __forceinline__ T* head_ptr(uint32_t lo, uint32_t hi) {
-  return (T*)(__attribute__((address_space(1))) T*)((uintptr_t)lo | ((uintptr_t)hi << 32));
-}
+// such an integer, or two words of a head, as a pointer into global memory; without the address space the loads behind it are flat ones
+template <typename T> __device__ __forceinline__ T* head_ptr(uint64_t word) { return (T*)(__attribute__((address_space(1))) T*)word; }
+template <typename T> __device__ __forceinline__ T* head_ptr(uint32_t lo, uint32_t hi) { return head_ptr<T>((uint64_t)lo | ((uint64_t)hi << 32)); }
 __device__ __forceinline__ CombineArgs combine_args(CombineHead H, const CombineTail& T) {
   CombineArgs A{head_ptr<const float>(H[0], H[1]), head_ptr<const float>(H[2], H[3]), head_ptr<const uint16_t>(H[4], H[5]), (int)H[6], T.M, (int)H[7],
                 T.out16, T.unrot, T.out_bf16, T.adapt, T.direct, T.d_pos, T.tok0, T.n_kv, T.max_ctx, T.plan, T.s_short};
   return A;
-}
-typedef uint32_t RowsHead __attribute__((ext_vector_type(8)));        // of a multi-stream pass: positions, slots (two words each), M
-inline RowsHead rows_head(const AttnArgs& A) {
-  const uint64_t pos = (uint64_t)(uintptr_t)A.rows.pos, slot = (uint64_t)(uintptr_t)A.rows.slot;
-  return RowsHead{(uint32_t)pos, (uint32_t)(pos >> 32), (uint32_t)slot, (uint32_t)(slot >> 32), (uint32_t)A.M, 0, 0, 0};
-}
-__device__ __forceinline__ void take_head(AttnArgs& A, RowsHead H) {
-  A.rows.pos = head_ptr<const int>(H[0], H[1]);
-  A.rows.slot = head_ptr<const int>(H[2], H[3]);
-  A.M = (int)H[4];
 }
 // projection outputs xq [M][n_heads][128], xk / xv [M][n_kv][128] fp32 -> q16 and the cache rows at *d_pos + t
 struct PostArgs {
