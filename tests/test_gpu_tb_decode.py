@@ -90,10 +90,11 @@ def test_rows_that_are_not_numbers(native, kk, M, bad, which):
 
 @pytest.mark.parametrize("kk", [4, 5])
 @pytest.mark.parametrize("heads,n_mult", [(1, 1), (1, 16), (2, 9), (3, 2)])
-@pytest.mark.parametrize("M,post", [(1, False), (2, False), (3, False), (5, False), (1, True)])
+@pytest.mark.parametrize("M,post", [(1, False), (2, False), (3, False), (5, False), (16, False), (17, False), (1, True)])
 def test_rows_as_the_oracle_codes_them(native, oracle, kk, heads, n_mult, M, post):
-    """Rows coded by the combiner of a decode pass (M <= 2) and by a wave per row (wider; `post`: fp32 rows), in handles whose rows do not fill
-    the waves of a workgroup (2 to 30 rows, four to a workgroup), with one multiplier and with as many as a profile may have."""
+    """Rows coded by the combiner of a decode pass (M <= 2), by the attention launch of a window (up to 16 rows) and by a launch of their own
+    (wider; `post`: fp32 rows), in handles whose rows do not fill the waves of a workgroup (2 to 102 rows, four to a workgroup), with one
+    multiplier and with as many as a profile may have."""
     from yasakani_amd import kvqp
     blob = kvqp.synthetic(layers=1, kv_heads=heads, kk=kk, seed=kk, n_mult=n_mult, mu=M == 2)
     rng = np.random.default_rng(10 * M + heads)
@@ -101,7 +102,7 @@ def test_rows_as_the_oracle_codes_them(native, oracle, kk, heads, n_mult, M, pos
     k[0, 0] = 0                                                    # a row of zeros: its residual has no length
     q = rng.standard_normal((M, 6 * heads, 256)).astype(np.float16)
     pos = 256 - M                                                  # up to the last row of the container
-    with native.KvCache(n_heads=6 * heads, n_kv_heads=heads, max_ctx=256, head_dim=256, max_rows=8) as kv:
+    with native.KvCache(n_heads=6 * heads, n_kv_heads=heads, max_ctx=256, head_dim=256, max_rows=24) as kv:
         kv.set_profile(blob)
         if post:
             kv.append256_f32_host(0, k.astype(np.float32), v.astype(np.float32), pos, rotate=False)
@@ -116,7 +117,7 @@ def test_rows_as_the_oracle_codes_them(native, oracle, kk, heads, n_mult, M, pos
 
 
 @pytest.mark.parametrize("kk", [4, 5])
-@pytest.mark.parametrize("M", [3, 16, 17])                    # 17: stored by a launch of their own
+@pytest.mark.parametrize("M", [3, 16])                        # 17: both passes below would be the same launches; see the test above and the next
 @pytest.mark.parametrize("pos,splits", [(0, 0), (30, 0), (250, 0), (250, 1), (250, 97), (1008 - 3, 0)])
 @pytest.mark.parametrize("siblings", [False, True])
 def test_windows_store_every_row(native, kk, M, pos, splits, siblings):
@@ -149,3 +150,37 @@ def test_windows_store_every_row(native, kk, M, pos, splits, siblings):
     a, b = (x.astype(np.float32) for x in outs)
     # the same rows, other split bounds: partials and outputs rounded to fp16 once each (2^-11), sums in fp32
     assert np.isfinite(a).all() and np.linalg.norm(a - b) <= 1e-3 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("form", ["kv4", "kv5", "256"])
+@pytest.mark.parametrize("M", [1, 2, 3, 16, 17, 21, 22, 32, 33])    # edges of who stores the rows, and of a row block (21 rows are one, 22 are two)
+@pytest.mark.parametrize("bf16", [False, True])
+def test_passes_read_the_rows_they_store(native, form, M, bf16):
+    """A pass over rows that others occupied, then the same pass over its own: the same launches, so the same bits, unless the first one read
+    something it had yet to store.  One split and many, over two tiles, up to the end of the container; a depth table."""
+    from yasakani_amd import kvqp
+    rng = np.random.default_rng(M)
+
+    def rows(n, heads):
+        x = rng.standard_normal((n, heads, 256)).astype(np.float32)
+        return native.bf16_bits(x) if bf16 else x.astype(np.float16)
+
+    with native.KvCache(max_ctx=1024, head_dim=256, max_rows=1024) as kv:
+        if form != "256":
+            kv.set_profile(kvqp.synthetic(layers=1, kk=int(form[2]), seed=11, mu=True))
+        kv.set_opt(11, int(bf16))
+        kv.append_host(0, rows(1024, 4), rows(1024, 4), 0)
+        q, k, v = rows(M, 24), rows(M, 4), rows(M, 4)
+        for pos, splits, tree in ((0, 0, False), (30, 3, True), (250, 1, False), (250, 97, False), (700, 5, True), (700, 0, False), (1024 - M, 0, False)):
+            kv.set_opt(2, splits)
+            if M <= 2:
+                kv.set_opt(1, splits)
+            depth = (np.arange(M) // 2).astype(np.uint8) if tree else None
+            kv.append_host(0, rows(M, 4), rows(M, 4), pos)
+            outs = []
+            for _ in range(2):
+                kv.poison_workspace()
+                outs.append(kv.layer_call(0, q, k, v, pos, depth).view(np.uint16))
+            f = native.bf16_to_f32(outs[0]) if bf16 else outs[0].view(np.float16)
+            assert np.isfinite(f.astype(np.float32)).all(), (pos, splits)
+            assert np.array_equal(outs[0], outs[1]), (pos, splits)
