@@ -27,7 +27,8 @@ SOURCES = ("attend_mid.hip",)
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-S", "--cuda-device-only"]
-EXTRA = {"attend_mid.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}      # as in the library's Makefile
+# as in the library's Makefile
+EXTRA = {"attend_mid.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "attend_narrow.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
 
 VMEM = re.compile(r"^(global|buffer|scratch|flat)_(load|store|atomic)")
 REG = re.compile(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b")
