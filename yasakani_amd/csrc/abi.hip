@@ -43,10 +43,10 @@ struct yka_kv {
   // [K payload n_kv * max_ctx * stride][V payload][K scales n_kv * max_ctx fp32][V scales]
   struct Tb {
     int kb = 0, stride = 0, nm = 0, layers = 0; bool has_mu = false;   // layers: layers the profile has groups for
-    uint8_t* blob = nullptr; uint32_t* desc = nullptr; int ngrp = 0; unsigned mult_off = 0; uint32_t* pairs = nullptr; float* gfac = nullptr; float* mu = nullptr;
+    uint32_t* pairs = nullptr; float* gfac = nullptr; float* mu = nullptr;
     uint8_t* pool = nullptr; size_t layer_bytes = 0, pay_bytes = 0, scl_bytes = 0;
     uint8_t* scr = nullptr; size_t scr_w_ofs = 0, scr_s_ofs = 0;
-    const float* mults = nullptr;    // scale multipliers, behind gfac
+    const float* mults = nullptr; const float* gains = nullptr;    // scale multipliers and the groups' table gains, behind gfac
     float* stage = nullptr;          // fp32 K rows then V rows of one pass ([max_rows][n_kv][256] each): yka_attn_post -> encoder
     // 256 bytes in front of the first row: windows of the attention kernels begin in the word before a chunk
     uint8_t* kpay(int layer) const { return pool + 256 + (size_t)layer * layer_bytes; }
@@ -233,12 +233,12 @@ constexpr int kTbTileTok = 128;     // tokens per launch of the trellis encoder 
 TbEncArgs tb_encoder_args(const yka_kv* kv, int layer, int container, const uint16_t* k16, const uint16_t* v16, int t0, int M, const int* d_pos) {
   const yka_kv::Tb& T = *kv->tb;
   TbEncArgs A{};
-  A.blob = T.blob; A.nm = T.nm; A.has_trellis = 1; A.desc = T.desc; A.ngrp = T.ngrp; A.mult_off = T.mult_off;
+  A.nm = T.nm;
   A.k16 = k16; A.v16 = v16; A.in_bf16 = kv->opt_io_bf16; A.d_pos = d_pos; A.layer = layer; A.tok0 = t0; A.n_kv = kv->cfg.n_kv_heads;
   A.max_ctx = kv->cfg.max_ctx;
   A.nrow = std::min(kTbTileTok, M - t0) * 2 * kv->cfg.n_kv_heads;
   A.scr = T.scr; A.scr_w_ofs = T.scr_w_ofs; A.scr_s_ofs = T.scr_s_ofs;
-  A.kb = T.kb; A.pairs = T.pairs; A.mu = T.has_mu ? T.mu : nullptr; A.mults = T.mults;
+  A.kb = T.kb; A.pairs = T.pairs; A.mu = T.has_mu ? T.mu : nullptr; A.gains = T.gains; A.mults = T.mults;
   A.pay0 = T.kpay(container); A.pay1 = T.vpay(container); A.scl0 = T.kscl(container); A.scl1 = T.vscl(container); A.stride = T.stride;
   return A;
 }
@@ -535,7 +535,7 @@ void yka_kv_close(yka_kv* kv) {
   (void)hipDeviceSynchronize();
   if (kv->stream) (void)hipStreamDestroy(kv->stream);
   if (kv->tb) {
-    (void)hipFree(kv->tb->blob); (void)hipFree(kv->tb->desc); (void)hipFree(kv->tb->pairs); (void)hipFree(kv->tb->gfac); (void)hipFree(kv->tb->mu); (void)hipFree(kv->tb->pool);
+    (void)hipFree(kv->tb->pairs); (void)hipFree(kv->tb->gfac); (void)hipFree(kv->tb->mu); (void)hipFree(kv->tb->pool);
     (void)hipFree(kv->tb->scr); (void)hipFree(kv->tb->stage);
     delete kv->tb;
   }
@@ -809,7 +809,7 @@ TbInfo tb_check_blob(const uint8_t* b, size_t n) {
   }
   return I;
 }
-// What the encoder kernels would otherwise look up in the blob by four dependent loads (layout: TbEncArgs::desc): a
+// What the encoder kernels would otherwise look up in the blob by four dependent loads (layout: TbProbeArgs::desc): a
 // record per group, then every table as aligned int16.  The blob has passed tb_check_blob.
 std::vector<uint32_t> tb_descriptors(const uint8_t* b, size_t n, const TbInfo& I) {
   const BlobView V{b, n};
@@ -860,13 +860,13 @@ int yka_tb_pack_unpack(const uint8_t* blob, size_t blob_len, const float* x, con
   for (int i = 0; i < 3; ++i) HIPCHK(hipEventCreate(&ev[i]));
   HIPCHK(hipEventRecord(ev[0], nullptr));
   for (int r0 = 0; r0 < rows; r0 += kTile) {
-    TbEncArgs A{};
+    TbProbeArgs A{};
     A.blob = db.as<uint8_t>(); A.nm = I.nm; A.has_trellis = I.has_trellis;
     A.desc = dd_desc.as<uint32_t>(); A.ngrp = I.ngrp; A.mult_off = BlobView{blob, blob_len}.word(32);
     A.yin = dx.as<float>(); A.grp = dg.as<int>(); A.pos = dp.as<int>(); A.row0 = r0; A.nrow = std::min(kTile, rows - r0);
     A.yout = dy.as<float>(); A.side = dside.as<uint32_t>(); A.scr = scr.as<uint8_t>(); A.scr_w_ofs = w_ofs;
-    A.pay0 = dpay.as<uint8_t>(); A.stride = stride;
-    launch_tb_encode(A, nullptr);
+    A.pay = dpay.as<uint8_t>(); A.stride = stride;
+    launch_tb_probe(A, nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipDeviceSynchronize());                  // the scratch block is reused by the next tile
   }
@@ -909,7 +909,7 @@ int yka_kv_set_profile(yka_kv* kv, const uint8_t* blob, size_t blob_len) {
   const BlobView V{blob, blob_len};
   // what the reference asks of a layer before it keeps packed rows for it (kvqaxpk_packable, src/kvq_atxpk.hpp:61-72)
   int kb = 0; bool has_mu = false;
-  std::vector<uint16_t> tabs((size_t)need * 256); std::vector<float> gfac(need), mu((size_t)need * 256, 0.f);
+  std::vector<uint16_t> tabs((size_t)need * 256); std::vector<float> gfac(need), gains(need), mu((size_t)need * 256, 0.f);
   std::vector<uint32_t> pairs;
   for (int g = 0; g < need; ++g) {
     const size_t rec = V.group_record(g);
@@ -922,7 +922,7 @@ int yka_kv_set_profile(yka_kv* kv, const uint8_t* blob, size_t blob_len) {
     const size_t trec = V.table_record(blob[rec + 2]);
     float gain; std::memcpy(&gain, blob + trec + 4, 4);
     if (!(gain > 0.f) || gain > 1e6f) throw std::runtime_error("profile blob: table gain must be positive and finite");
-    gfac[g] = 0.00390625f * gain;
+    gfac[g] = 0.00390625f * gain; gains[g] = gain;
     uint16_t* row = &tabs[(size_t)g * 256];
     for (int st = 0; st < 256; ++st) row[st] = int_to_f16_bits(V.table_int(trec, st));
     if (blob[rec + 5] == 0) continue;
@@ -945,7 +945,7 @@ int yka_kv_set_profile(yka_kv* kv, const uint8_t* blob, size_t blob_len) {
     ~TbGuard() {
       if (done || !kv->tb) return;
       yka_kv::Tb* t = kv->tb;
-      (void)hipFree(t->blob); (void)hipFree(t->desc); (void)hipFree(t->pairs); (void)hipFree(t->gfac); (void)hipFree(t->mu); (void)hipFree(t->pool); (void)hipFree(t->scr); (void)hipFree(t->stage);
+      (void)hipFree(t->pairs); (void)hipFree(t->gfac); (void)hipFree(t->mu); (void)hipFree(t->pool); (void)hipFree(t->scr); (void)hipFree(t->stage);
       delete t; kv->tb = nullptr;
     }
   } guard{kv};
@@ -956,14 +956,11 @@ int yka_kv_set_profile(yka_kv* kv, const uint8_t* blob, size_t blob_len) {
   T->pay_bytes = rows * T->stride; T->scl_bytes = rows * 4; T->layer_bytes = 2 * T->pay_bytes + 2 * T->scl_bytes;
   const size_t jobs = (size_t)kTbTileTok * 2 * n_kv * I.nm;
   T->scr_w_ofs = jobs * 256; T->scr_s_ofs = T->scr_w_ofs + jobs * 32;
-  HIPCHK(hipMalloc((void**)&T->blob, blob_len)); HIPCHK(hipMemcpy(T->blob, blob, blob_len, hipMemcpyHostToDevice));
-  const std::vector<uint32_t> desc = tb_descriptors(blob, blob_len, I);
-  T->ngrp = I.ngrp; T->mult_off = V.word(32);
-  HIPCHK(hipMalloc((void**)&T->desc, desc.size() * 4)); HIPCHK(hipMemcpy(T->desc, desc.data(), desc.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc((void**)&T->pairs, pairs.size() * 4)); HIPCHK(hipMemcpy(T->pairs, pairs.data(), pairs.size() * 4, hipMemcpyHostToDevice));
   gfac.resize((size_t)need + I.nm);
   std::memcpy(gfac.data() + need, blob + V.multipliers(), (size_t)I.nm * 4);
-  HIPCHK(hipMalloc((void**)&T->gfac, gfac.size() * 4)); T->mults = T->gfac + need; HIPCHK(hipMemcpy(T->gfac, gfac.data(), gfac.size() * 4, hipMemcpyHostToDevice));
+  gfac.insert(gfac.end(), gains.begin(), gains.end());
+  HIPCHK(hipMalloc((void**)&T->gfac, gfac.size() * 4)); T->mults = T->gfac + need; T->gains = T->mults + I.nm; HIPCHK(hipMemcpy(T->gfac, gfac.data(), gfac.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc((void**)&T->mu, mu.size() * 4)); HIPCHK(hipMemcpy(T->mu, mu.data(), mu.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc((void**)&T->pool, 256 + T->layer_bytes * kv->cfg.n_layers + 256));
   HIPCHK(hipMemset(T->pool, 0, 256 + T->layer_bytes * kv->cfg.n_layers + 256));     // unwritten rows: state 0 everywhere, scale 0

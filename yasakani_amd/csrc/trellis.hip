@@ -25,7 +25,7 @@ namespace yka {
 namespace {
 
 // ---- the profile blob, read where it lies (little-endian, no alignment assumed) ----
-// The encoder kernels also get what the host has already looked up in the blob (`desc`, see TbEncArgs): one aligned
+// The encoder of the probe form also gets what the host has already looked up in the blob (`desc`, see TbProbeArgs): one aligned
 // 32-byte record per group and the tables as aligned int16, so that a block reaches its table after ONE dependent load
 // instead of four (header -> offset of the group record -> record -> offset of the table record -> table).
 struct Profile {
@@ -108,7 +108,7 @@ struct RowRef {
   int group, pos;      // profile group and position
   size_t index;        // the row's index in the arrays
 };
-__device__ __forceinline__ RowRef locate_row(const TbEncArgs& A, int r) {
+__device__ __forceinline__ RowRef locate_row(const TbProbeArgs& A, int r) {
   const size_t index = (size_t)(A.row0 + r);
   return RowRef{A.yin[index * 256 + threadIdx.x], A.grp[index], A.pos[index], index};
 }
@@ -333,6 +333,9 @@ __device__ __forceinline__ void wave_chunk(const int* xi, const StepConsts& C, u
 #pragma unroll
   for (int g = 0; g < U; ++g) kept = lane == keeper_lane<KK>(g) ? g : kept;
   uint32_t* const rec = reinterpret_cast<uint32_t*>(bp) + (kept < 0 ? 0 : kept);
+  // A lone wave's steps slow down where 8-byte instructions straddle multiples of 8 bytes: 28 of the 44 of these four steps do not with 4 bits if
+  // the loop begins at such a multiple (16 if it begins 4 bytes on), 25 of 43 with 5 bits if the middle of the first two steps
+  // lies at one (18).  One token of 4 bits at 1,600 tokens, 4 layers: 59.5 us the other way, 58.7 so; of 5 bits at 600 55.9 and 55.4.
 #pragma unroll 1
   for (int t = 0; t < 64; t += 4) {
     uint32_t chosen4 = 0u;
@@ -355,6 +358,7 @@ __device__ __forceinline__ void wave_chunk(const int* xi, const StepConsts& C, u
           key[3] = add_rot3(m, mad24(nx, b1[3], a1[3]));
         }
       }
+      if (KK == 5 && h == 0) asm volatile(".p2align 3");
       {                                                // arrangement 1 -> 0
         int km = KK == 5 ? least : min(min(key[0], key[1]), min(key[2], key[3]));
         if constexpr (KK == 5) km = min_oct(min_xor2(min_xor1(km)));
@@ -421,12 +425,12 @@ struct SearchLds {
 };
 // the end of a job: squared error of this multiplier (element d of the row is lane d & 63 of wave d >> 6; summed per run of 32
 // elements) and the states
-__device__ __forceinline__ void leave_job(const TbEncArgs& A, SearchLds& L, size_t job, float r, float s, float gain) {
+__device__ __forceinline__ void leave_job(uint8_t* scr, size_t w_ofs, SearchLds& L, size_t job, float r, float s, float gain) {
   const int d = threadIdx.x, state = L.chosen[d];
   const float miss = __fsub_rn(r, __fmul_rn(table_value((int)L.table[state], gain), s));
   const float sq = run_fold<AddRn>(__fmul_rn(miss, miss));
-  if ((d & 31) == 0) reinterpret_cast<float*>(A.scr + A.scr_w_ofs)[job * 8 + (d >> 5)] = sq;
-  A.scr[job * 256 + d] = (uint8_t)state;
+  if ((d & 31) == 0) reinterpret_cast<float*>(scr + w_ofs)[job * 8 + (d >> 5)] = sq;
+  scr[job * 256 + d] = (uint8_t)state;
 }
 // integer target of an element: the residual in units of s / 256, clamped
 __device__ __forceinline__ int target_of(float r, float s) {
@@ -448,7 +452,7 @@ __device__ __forceinline__ void search_body(const TbEncArgs& A, const int block)
   // the first 256 entries of the group's pair table hold the table: entry i ends with the value of state i, an exact integer
   const uint32_t pair = A.pairs[((size_t)R.group << (8 + KB)) + d];
   const float mean = A.mu ? A.mu[(size_t)R.group * 256 + d] : 0.f;
-  const float gain = __uint_as_float(A.desc[8 * (size_t)R.group + 5]), mult_value = A.mults[mult];
+  const float gain = A.gains[R.group], mult_value = A.mults[mult];
   if (A.rot) x = rotate256(x, rot_buf, false);
   L.table[d] = (int16_t)(int)__half2float(__ushort_as_half((uint16_t)(pair >> 16)));
   const float r = A.mu ? __fsub_rn(x, mean) : x;
@@ -458,13 +462,13 @@ __device__ __forceinline__ void search_body(const TbEncArgs& A, const int block)
   __syncthreads();
   wave_chunk<KB>(L.target + 64 * wave, C, L.back[wave], L.chosen + 64 * wave);
   const size_t job = (size_t)row * A.nm + mult;
-  leave_job(A, L, job, r, s, gain);
+  leave_job(A.scr, A.scr_w_ofs, L, job, r, s, gain);
   if (d == 0) reinterpret_cast<float*>(A.scr + A.scr_s_ofs)[job] = s;
 }
 template <int KB, bool BF>
 __global__ void __launch_bounds__(256) tb_search_kernel(TbEncArgs A) { search_body<KB, BF>(A, blockIdx.x); }
 // Probe form: any profile, every row with its own group
-__global__ void __launch_bounds__(256) tb_search_probe_kernel(TbEncArgs A) {
+__global__ void __launch_bounds__(256) tb_search_probe_kernel(TbProbeArgs A) {
   __shared__ __align__(16) SearchLds L;
   const int d = threadIdx.x, wave = d >> 6, lane = d & 63;
   const int row = blockIdx.x / A.nm, mult = blockIdx.x % A.nm;
@@ -492,7 +496,7 @@ __global__ void __launch_bounds__(256) tb_search_probe_kernel(TbEncArgs A) {
   if (G.bits == 5) wave_chunk<5>(L.target + 64 * wave, C, L.back[wave], L.chosen + 64 * wave);
   else if (G.bits == 4) wave_chunk<4>(L.target + 64 * wave, C, L.back[wave], L.chosen + 64 * wave);
   else wave_chunk3(L.target + 64 * wave, ci4, L.back[wave], L.chosen + 64 * wave);
-  leave_job(A, L, (size_t)row * A.nm + mult, Q.r, s, T.gain);
+  leave_job(A.scr, A.scr_w_ofs, L, (size_t)row * A.nm + mult, Q.r, s, T.gain);
 }
 
 // Decode (one or two tokens, no depth table): the search for the new rows' codes and the attention over the rows already in
@@ -525,7 +529,7 @@ __device__ __forceinline__ Coded code_flat(float* part8, float r) {
 // requested before the residual is computed, for all multipliers at once (the choice then costs no further round trip):
 // the states of this element, and - by thread i < multipliers - multiplier i and the error total of its search.
 struct SearchResults { int state[kMaxMult]; };
-__device__ __forceinline__ SearchResults fetch_search_results(const TbEncArgs& A, const Profile& P, int row, float* totals, float* mults) {
+__device__ __forceinline__ SearchResults fetch_search_results(const TbProbeArgs& A, const Profile& P, int row, float* totals, float* mults) {
   SearchResults S;
   const int d = threadIdx.x;
 #pragma unroll
@@ -540,7 +544,7 @@ __device__ __forceinline__ SearchResults fetch_search_results(const TbEncArgs& A
   }
   return S;                                              // totals / mults: visible after the next barrier
 }
-__device__ __forceinline__ Coded code_trellis(const TbEncArgs& A, const Profile& P, const GroupRec& G, const Residual& Q, const SearchResults& S,
+__device__ __forceinline__ Coded code_trellis(const TbProbeArgs& A, const Profile& P, const GroupRec& G, const Residual& Q, const SearchResults& S,
                                               const float* totals, const float* mults) {
   int keep = 0; float least = totals[0];
   for (int i = 1; i < A.nm; ++i) { const float total = totals[i]; if (total < least) { least = total; keep = i; } }
@@ -548,15 +552,13 @@ __device__ __forceinline__ Coded code_trellis(const TbEncArgs& A, const Profile&
   int state = 0;
 #pragma unroll
   for (int i = 0; i < kMaxMult; ++i) state = i == keep ? S.state[i] : state;
-  float value = 0.f;
-  if (A.yout) { const TableRec T = read_table(P, G); value = __fmul_rn(table_value(table_int(P, T, state), T.gain), s); }
-  return Coded{state & ((1 << G.bits) - 1), G.bits, s, value, true};
+  const TableRec T = read_table(P, G);
+  return Coded{state & ((1 << G.bits) - 1), G.bits, s, __fmul_rn(table_value(table_int(P, T, state), T.gain), s), true};
 }
 
 // grid rows, block 256: codes the row (best multiplier of the search, or the flat quantizer), rebuilds what it decodes to,
-// packs the fields, stores payload / scale / projection coefficients
-// (probe form)
-__global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
+// packs the fields, stores payload / scale / projection coefficients (probe form)
+__global__ void __launch_bounds__(256) tb_select_kernel(TbProbeArgs A) {
   __shared__ float part8[8];
   __shared__ uint8_t fld[256];
   __shared__ float totals[kMaxMult], mults[kMaxMult];
@@ -580,21 +582,16 @@ __global__ void __launch_bounds__(256) tb_select_kernel(TbEncArgs A) {
     if (G.has_mean) rebuilt = __fadd_rn(rebuilt, Q.mean);
     coef_bits = (unsigned)__half_as_ushort(__float2half_rn(Q.coef[0])) | ((unsigned)__half_as_ushort(__float2half_rn(Q.coef[1])) << 16);
   }
-  if (A.pay0) {
-    uint32_t* const words = reinterpret_cast<uint32_t*>(A.pay0 + R.index * (size_t)A.stride);
-    fld[d] = (uint8_t)C.field;
-    __syncthreads();
-    if (d < (A.stride >> 2)) {
-      uint32_t w = 0u;
-      if (C.any && d < 8 * C.bits) w = C.bits == 5 ? pack_word<5>(fld, d) : C.bits == 4 ? pack_word<4>(fld, d) : pack_word<3>(fld, d);
-      words[d] = w;
-    }
-    if (d == 0) {
-      if (A.side) { A.side[2 * R.index] = __float_as_uint(C.scale); A.side[2 * R.index + 1] = coef_bits; }
-      if (A.coded) A.coded[R.index] = C.any ? 1 : 0;
-    }
+  uint32_t* const words = reinterpret_cast<uint32_t*>(A.pay + R.index * (size_t)A.stride);
+  fld[d] = (uint8_t)C.field;
+  __syncthreads();
+  if (d < (A.stride >> 2)) {
+    uint32_t w = 0u;
+    if (C.any && d < 8 * C.bits) w = C.bits == 5 ? pack_word<5>(fld, d) : C.bits == 4 ? pack_word<4>(fld, d) : pack_word<3>(fld, d);
+    words[d] = w;
   }
-  if (A.yout) A.yout[R.index * 256 + d] = rebuilt;
+  if (d == 0) { A.side[2 * R.index] = __float_as_uint(C.scale); A.side[2 * R.index + 1] = coef_bits; }
+  A.yout[R.index * 256 + d] = rebuilt;
 }
 
 // Cache form: a wave per row.  Every multiplier's states (a word of four per lane), error sums and scale are requested at once with the
@@ -674,13 +671,12 @@ static void launch_search(const TbEncArgs& A, hipStream_t st) {
 void launch_tb_search(const TbEncArgs& A, hipStream_t st) { if (A.kb == 4) launch_search<4>(A, st); else launch_search<5>(A, st); }
 void launch_tb_encode(const TbEncArgs& A, hipStream_t st) {
   if (A.nrow <= 0) return;
-  if (A.yin) {
-    if (A.has_trellis) hipLaunchKernelGGL(tb_search_probe_kernel, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
-    hipLaunchKernelGGL(tb_select_kernel, dim3(A.nrow), dim3(256), 0, st, A);
-    return;
-  }
   launch_tb_search(A, st);
   if (A.kb == 4) launch_store<4>(A, st); else launch_store<5>(A, st);
+}
+void launch_tb_probe(const TbProbeArgs& A, hipStream_t st) {
+  if (A.has_trellis) hipLaunchKernelGGL(tb_search_probe_kernel, dim3(A.nrow * A.nm), dim3(256), 0, st, A);
+  hipLaunchKernelGGL(tb_select_kernel, dim3(A.nrow), dim3(256), 0, st, A);
 }
 void launch_tb_encode_attend(const TbEncArgs& E, const TbAttnArgs& A, int kb, hipStream_t st) {
   const int n_search = E.nrow * E.nm;

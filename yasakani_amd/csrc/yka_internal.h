@@ -131,30 +131,33 @@ struct PostArgs {
   int io_bf16 = 0;   // 16-bit rows that leave (q16, gate16) are bf16 instead of fp16
 };
 
-// Trellis-coded rows (trellis.hip; reference TbFastArgs, src/kvq_fast.hpp:16-37).  Probe form (yin != nullptr): rows
-// row0 .. row0 + nrow - 1 of yin with their own group and position; results indexed by row.  Cache form: row rj of the
-// launch is (token rj / (2 n_kv), K | V, kv head) of the pass, read from k32 / v32 [M][n_kv][256]; its payload goes to
-// pay0 (K) / pay1 (V) + (kvh * max_ctx + pos) * stride and its scale to scl0 / scl1 [kvh * max_ctx + pos].
+// Trellis-coded rows on their way into the cache (trellis.hip).  Row rj of the launch is (token rj / (2 n_kv), K | V, kv head) of the
+// pass, read from k32 / v32 [M][n_kv][256]; its payload goes to pay0 (K) / pay1 (V) + (kvh * max_ctx + pos) * stride and its
+// scale to scl0 / scl1 [kvh * max_ctx + pos].  Every group is trellis-coded with kb bits, without guard positions and directions.
 struct TbEncArgs {
+  const float* k32; const float* v32; const uint16_t* k16; const uint16_t* v16;   // fp32 rows, or 16-bit rows if k32 == nullptr
+  const int* d_pos; int layer, tok0, n_kv, max_ctx, rot;
+  int nrow, nm;                       // rows of the launch, scale multipliers of the profile: nrow * nm searches
+  uint8_t* scr; size_t scr_w_ofs, scr_s_ofs;   // scratch: states [nrow * nm][256] bytes, at scr_w_ofs error sums [nrow * nm][8] fp32, at scr_s_ofs the scales tried [nrow * nm] fp32
+  // pair tables and mean rows by group (TbAttnArgs), table gains by group, multipliers
+  int kb; const uint32_t* pairs; const float* mu; const float* gains; const float* mults;
+  uint8_t* pay0; uint8_t* pay1; float* scl0; float* scl1; int stride;
+  int pos_limit;                      // rows at positions >= pos_limit are not stored (0: no limit besides max_ctx)
+  RowMap rows;                        // multi-stream pass: token t sits at rows.pos[t] of container rows.slot[t] (pay / scl = container 0)
+  int in_bf16;                        // k16 / v16 are bf16 rows
+};
+// The codec alone (reference TbFastArgs, src/kvq_fast.hpp:16-37): rows row0 .. row0 + nrow - 1 of yin with their own group and position,
+// any profile; results indexed by row.
+struct TbProbeArgs {
   const uint8_t* blob; int nm; int has_trellis;
   // what the host looked up in the blob (see tb_descriptors in abi.hip): [ngrp][8] words
   //   { mode | bits << 8 | table << 16 | guard << 24, directions | has_mean << 8, byte offset of the mean row, of the
   //     first direction, index (in int16 units, from desc) of the group's table as aligned int16, gain bits, 0, 0 }
   // followed by the tables; mult_off: byte offset of the scale multipliers in the blob
   const uint32_t* desc; int ngrp; unsigned mult_off;
-  const float* k32; const float* v32; const uint16_t* k16; const uint16_t* v16;   // cache form: fp32 rows, or fp16 rows if k32 == nullptr
-  const int* d_pos; int layer, tok0, n_kv, max_ctx, rot;
-  const float* yin; const int* grp; const int* pos; int row0;
-  float* yout; uint32_t* side; int* coded;
-  int nrow;
-  uint8_t* scr; size_t scr_w_ofs;     // scratch: states [nrow * nm][256] bytes, then at scr_w_ofs error sums [nrow * nm][8] fp32
-  // cache form (every group trellis-coded with kb bits, no guard positions, no directions): pair tables and mean rows by group (TbAttnArgs),
-  // multipliers as aligned floats, and in the scratch at scr_s_ofs the scale every job tried [nrow * nm] fp32
-  int kb; const uint32_t* pairs; const float* mu; const float* mults; size_t scr_s_ofs;
-  uint8_t* pay0; uint8_t* pay1; float* scl0; float* scl1; int stride;
-  int pos_limit;                      // cache form: rows at positions >= pos_limit are not stored (0: no limit besides max_ctx)
-  RowMap rows;                        // cache form, multi-stream pass: token t sits at rows.pos[t] of container rows.slot[t] (pay / scl = container 0)
-  int in_bf16;                        // cache form: k16 / v16 are bf16 rows
+  const float* yin; const int* grp; const int* pos; int row0, nrow;
+  float* yout; uint32_t* side; uint8_t* pay; int stride;
+  uint8_t* scr; size_t scr_w_ofs;     // states and error sums, as above
 };
 // what the searches of a launch have left in the scratch (TbEncArgs): nm jobs per row
 struct TbJobs { const uint8_t* scr; size_t w_ofs, s_ofs; int nm; };
@@ -162,7 +165,9 @@ __host__ __device__ inline TbJobs tb_jobs(const TbEncArgs& A) { return TbJobs{A.
 // attention over trellis-coded rows (attend_tb.hip).  pairs [groups][2^(8 + kb)]: entry i = the table's integers, as two
 // fp16 values, of the states (i >> kb) & 255 and i & 255 (two consecutive elements from 8 + kb stream bits); gfac [groups]:
 // gain / 256; mu [groups][256] fp32 mean rows (zero rows where a group has none) or nullptr if no group has one
-struct TbAttnArgs {
+// At a multiple of 64 bytes among a kernel's arguments: what a decode workgroup asks of it first does not straddle two cache lines, whatever stands in
+// front (4 layers of one token of 4 bits at 16,000 tokens 65.2 us with the rows' pointers across two lines, 64.3 so).
+struct alignas(64) TbAttnArgs {
   const uint8_t* kpay; const uint8_t* vpay; const float* kscl; const float* vscl; int max_ctx, n_kv, stride;
   const uint32_t* pairs; const float* gfac; const float* mu; int layer;
   const uint16_t* q16; const int* d_pos; const uint8_t* depth; int M, tok0, n_heads, S;
@@ -183,7 +188,8 @@ __device__ __forceinline__ void tb_split_of(const TbAttnArgs& A, int b, int& spl
   if (A.s_short) { split = b / A.n_kv; kvh = b % A.n_kv; } else { split = b % A.S; kvh = b / A.S; }
 }
 void launch_tb_encode(const TbEncArgs&, hipStream_t);
-void launch_tb_search(const TbEncArgs&, hipStream_t);     // the searches alone (cache form): TbAttnArgs::jobs has their results stored
+void launch_tb_search(const TbEncArgs&, hipStream_t);     // the searches alone: TbAttnArgs::jobs has their results stored
+void launch_tb_probe(const TbProbeArgs&, hipStream_t);
 // one or two tokens: searches of the encoder and attention over the keys in front of *d_pos; the combiner has to store the new rows and add them
 void launch_tb_encode_attend(const TbEncArgs&, const TbAttnArgs&, int kb, hipStream_t);
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
