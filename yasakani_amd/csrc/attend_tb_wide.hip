@@ -145,6 +145,8 @@ __device__ __forceinline__ void decode_to_lds(uint8_t* buf, int tid, const Raw& 
 }
 
 // grid (S, n_kv, row blocks), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 queries
+// No register is left: 256 with 4 bits; with 5 bits a pair that is live across the tile loop is stored to scratch in front of it and read again
+// behind it.  The build walks the generated code (isa_check.py), since a load in flight must not be what is spilled.
 template <int KB, bool BF>
 __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   constexpr int kTabBytes = 4 << (8 + KB);

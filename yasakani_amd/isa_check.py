@@ -19,11 +19,11 @@ import subprocess
 from concurrent.futures import ThreadPoolExecutor
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
-# Walked: the kernel whose waits are unconditional (one register set, `s_waitcnt vmcnt(0)` at one site).  The other
-# attention kernels leave a number of loads in flight that depends on wave-uniform conditions correlated across branches
-# (a younger tile was requested or not; a wave group has tiles or not), which a walk over all branch outcomes cannot
-# follow: it reports paths that no wave takes.
-SOURCES = ("attend_mid.hip",)
+# Walked: the kernels whose waits are unconditional (one register set, `s_waitcnt vmcnt(0)`), among them the one that has no register
+# left and spills (attend_tb_wide.hip, 5 bits).  The other attention kernels leave a number of loads in flight that depends on
+# wave-uniform conditions correlated across branches (a younger tile was requested or not; a wave group has tiles or not),
+# which a walk over all branch outcomes cannot follow: it reports paths that no wave takes.
+SOURCES = ("attend_mid.hip", "attend_tb_wide.hip")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-S", "--cuda-device-only"]
