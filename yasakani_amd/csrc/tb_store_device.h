@@ -6,19 +6,6 @@
 namespace yka {
 
 constexpr int kMaxMult = 16;
-// word d of a row's MSB-first stream of KB-bit fields: the fields that overlap bits [32 d, 32 d + 32)
-template <int KB>
-__device__ __forceinline__ uint32_t pack_word(const uint8_t* fld, int d) {
-  const int e0 = (32 * d) / KB;                          // first field with bits in the word (division by a constant)
-  uint32_t w = 0u;
-#pragma unroll
-  for (int k = 0; k < 32 / KB + 2; ++k) {
-    const int e = e0 + k, sh = 32 * d + 32 - KB * (e + 1);   // distance of the field's last bit from the word's last bit
-    if (e < 256 && sh > -KB) w |= sh >= 0 ? (uint32_t)fld[e] << sh : (uint32_t)fld[e] >> -sh;
-  }
-  return w;
-}
-
 // What a row is stored as after the search (cache form), by a wave: the multiplier whose search left the smallest squared error (its 8
 // partial sums added in order from 0; the first of equal errors), the four states of elements 4 lane .. 4 lane + 3 it chose, its scale.
 // choose_job: which job, from what request_errors has asked for.  A wave with one row asks for the states of all jobs beside that

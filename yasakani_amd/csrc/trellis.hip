@@ -514,6 +514,19 @@ __global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_p
   tbd::attend_tb_body<KB, false>(A, split, kvh, 0, true);
 }
 
+// word d of a row's MSB-first stream of KB-bit fields: the fields that overlap bits [32 d, 32 d + 32)
+template <int KB>
+__device__ __forceinline__ uint32_t pack_word(const uint8_t* fld, int d) {
+  const int e0 = (32 * d) / KB;                          // first field with bits in the word (division by a constant)
+  uint32_t w = 0u;
+#pragma unroll
+  for (int k = 0; k < 32 / KB + 2; ++k) {
+    const int e = e0 + k, sh = 32 * d + 32 - KB * (e + 1);   // distance of the field's last bit from the word's last bit
+    if (e < 256 && sh > -KB) w |= sh >= 0 ? (uint32_t)fld[e] << sh : (uint32_t)fld[e] >> -sh;
+  }
+  return w;
+}
+
 // what a row is stored as: one field per element, the field width, the row scale
 struct Coded { int field, bits; float scale, value; bool any; };
 // flat groups: symmetric int4 with scale max|r| / 7 (src/kvq_fast.cuh:194-198)
