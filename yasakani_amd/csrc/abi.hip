@@ -106,8 +106,9 @@ void on_device(const yka_kv* kv) {
 }
 
 constexpr int kMaxSplits = 256;
-// (token, split) pairs of the partial workspace, n_heads * (2 * head_dim + 8) bytes each.  Windows and streams stay below kWsPairs (24
-// heads: 26 MB with 128 channels, 51 with 256); a slice of a prefill chunk may ask for more, kChunkPairs at most (ws_pairs_of)
+// (token, split) pairs of the partial workspace, n_heads * (2 * head_dim + 8) bytes each.  Windows and streams stay below
+// kWsPairs (24 heads: 26 MB with 128 channels, 51 with 256); a slice of a prefill chunk may ask for more, kChunkPairs at
+// most (ws_pairs_of)
 constexpr size_t kWsPairs = 4096, kChunkPairs = 12288;
 
 // splits for the narrow kernel: one workgroup per CU (256 of them) while a workgroup then walks at most 48 tiles - its
@@ -169,18 +170,20 @@ int chunk_splits(const yka_kv* kv, int Ms, size_t ws_pairs) {
   return best;
 }
 
-// 256-channel rows, both formats: how a pass is cut.  Passes of more than 64 rows (prompt chunks) go through the wide kernels
-// in slices of up to 1,024 tokens: in slices of 64 a chunk on a short context is mostly launches (1,500 first rows, int4: 533 us per layer call in 24 slices, 146 in two).
+// 256-channel rows, both formats: how a pass is cut.  Passes of more than 64 rows (prompt chunks) go through the wide
+// kernels in slices of up to 1,024 tokens: in slices of 64 a chunk on a short context is mostly launches (1,500 first rows,
+// int4: 533 us per layer call in 24 slices, 146 in two).
 // Row blocks of one slice get the same number of rows, in whole waves: the fragment reads of the waves that have rows set
-// the pace of a tile, so 144 rows are 80 + 64 and not 128 + 16 (24 rows at 9,001 tokens: 25.0 us per
-// layer call against 26.1).
+// the pace of a tile, so 144 rows are 80 + 64 and not 128 + 16 (24 rows at 9,001 tokens: 25.0 us per layer call against
+// 26.1).
 // Splits of the decode kernels: one workgroup per CU (the waves keep the next tile in flight and the combiner has half the
 // rows to read: 205 against 225 us for 16 layers at 20,011 tokens, 167 / 204 at 3,000, 97 / 101 for 2 layers at 200,000).
 // Windows forced through them (option key 3): two, where one would leave whole splits of the row tiles too long.  us per
-// layer call with 256 / 512 workgroups, 5 bits: 4 rows 26.3 / 28.6 at 1,000 tokens, 36.7 / 36.1 at 16,000, 8 rows 28.8 / 30.7 and
-// 47.9 / 45.4, 48 rows 64.2 / 62.3 and 187 / 145; int4: 16 rows 14.6 / 17.1 and 32.8 / 33.1, 48 rows 19.8 / 20.3 and 86.3 / 69.1.
-// Of the wide ones: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of at most four
-// rounds of 256 workgroups best.
+// layer call with 256 / 512 workgroups, 5 bits: 4 rows 26.3 / 28.6 at 1,000 tokens, 36.7 / 36.1 at 16,000, 8 rows 28.8 /
+// 30.7 and 47.9 / 45.4, 48 rows 64.2 / 62.3 and 187 / 145; int4: 16 rows 14.6 / 17.1 and 32.8 / 33.1, 48 rows 19.8 / 20.3
+// and 86.3 / 69.1.
+// Of the wide ones: one workgroup per CU, at least 2 * row blocks tiles each; of a chunk the fewest that fill the last of
+// at most four rounds of 256 workgroups best.
 struct Part256 { int Ms, S, rows_per_block; bool narrow; int s_short; };
 int slice256(const yka_kv* kv, int M) { return M > kMaxSlice && !kv->opt_force_narrow ? kChunkSlice256 : kMaxSlice; }
 Part256 part256(const yka_kv* kv, int M, int s0, int slice) {
@@ -291,8 +294,10 @@ void do_attend(yka_kv* kv, int layer, const uint16_t* q16, int M, const int* d_p
   const Workspace W = ws ? *ws : Workspace{kv->pm, kv->pl, kv->pacc16, kWsPairs, kv->tickets};
   const int bf16 = kv->opt_io_bf16;                // type of the 16-bit rows that come in and of the outputs
   if (kv->tb) {
-    // trellis-coded rows: the encoder runs first (two launches; not in decode, see below); rows of at most 2 tokens (or option key 3) run on row
-    // tiles of 2 tokens x 6 heads, wider slices on 128-row workgroups that decode every tile once into LDS
+    // trellis-coded rows: the encoder runs first, in two launches (search, store); windows of up to kTbFuseRows rows launch
+    // the search alone and the attention stores, decode launches nothing in front (see below).  Rows of at most 2 tokens
+    // (or option key 3) run on row tiles of 2 tokens x 6 heads, wider slices on 128-row workgroups that decode every tile
+    // once into LDS
     const yka_kv::Tb& T = *kv->tb;
     check_tb_layer(kv, layer);
     // decode without a depth table: the encoder's search rides in the attention launch, which leaves the new rows to the combiner
@@ -398,7 +403,8 @@ MsGrid ms_grid(const yka_kv* kv, int M) {
 }
 
 // Multi-stream pass: rows are appended (several rows of one stream may follow each other and read each other's keys) by the
-// attention launch or, beyond 64 rows and with a split count set by the caller, by a launch in front of it; every row attends to keys [0, pos[t]] of its own container.  One token per workgroup column.
+// attention launch or, beyond 64 rows and with a split count set by the caller, by a launch in front of it; every row
+// attends to keys [0, pos[t]] of its own container.  One token per workgroup column.
 void do_attend_ms(yka_kv* kv, const uint16_t* q16, const uint16_t* k16, const uint16_t* v16, int M, const int* row_pos,
                   const int* row_slot, uint16_t* out16, hipStream_t st) {
   const int NH = kv->cfg.n_heads, D = kv->D();

@@ -210,9 +210,10 @@ __device__ __forceinline__ void load_v256(const uint8_t* pg, int tp, const Offs2
 
 }  // namespace
 
-// grid (S, n_kv, ceil(M/TPT)), block 256 (4 waves; decode launches one workgroup per CU, streams and forced windows two).  Workgroup = (split, kv head, TPT tokens x 6 heads):
-// TPT = 2 for a single-stream pass; MS (multi-stream pass, reference: src/q35_atxpk_ms.cu:13-33): one token per row
-// tile, which reads the container and the position its row map names.
+// grid (S, n_kv, ceil(M/TPT)), block 256 (4 waves; decode launches one workgroup per CU, streams and forced windows two).
+// Workgroup = (split, kv head, TPT tokens x 6 heads):
+// TPT = 2 for a single-stream pass; MS (multi-stream pass, reference: src/q35_atxpk_ms.cu:13-33): one token per row tile,
+// which reads the container and the position its row map names.
 template <bool MS>
 __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
   constexpr int TPT = MS ? 1 : 2;
@@ -424,14 +425,15 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(AttnArgs A) {
 
 // combiner (src/attention_kv4q.cu:325-332) for 256-channel rows: grid (n_heads, M), block 256 = 8 split lanes x 32 channel
 // lanes of 8 channels; the split lanes run in parallel and are summed through LDS.  S <= 256.  kInFlight = partial rows a
-// split lane requests before it uses any: 8 covers the 64 splits of decode (16 for 128, 32 for 256), 4 covers
-// 32 and keeps the register count low where thousands of workgroups run (wide windows).
+// split lane requests before it uses any: 8 covers the 64 splits of decode (16 for 128, 32 for 256), 4 covers 32 and keeps
+// the register count low where thousands of workgroups run (wide windows).
 // MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
-// KB != 0: partials of launch_tb_encode_attend, which leave out the rows of the pass; token t also sees the keys *d_pos + u, u <=
-// t, which join the sum as splits of one key each, in fp32 (thread = channel; N names the rows).  The searches have left what the
-// rows may be coded with: wave 2 u + v of a workgroup picks the code of the K (v = 0) or V row of token u, and the workgroups of a kv head's first
-// query head store them.  Everything that takes is requested with the partials.  5 bits at 16,001 tokens, 16 layers: 356 us with a
-// launch between that stored the rows and their values read back here, 312 us so.
+// KB != 0: partials of launch_tb_encode_attend, which leave out the rows of the pass; token t also sees the keys *d_pos +
+// u, u <= t, which join the sum as splits of one key each, in fp32 (thread = channel; N names the rows).  The searches have
+// left what the rows may be coded with: wave 2 u + v of a workgroup picks the code of the K (v = 0) or V row of token u,
+// and the workgroups of a kv head's first query head store them.  Everything that takes is requested with the partials.  5
+// bits at 16,001 tokens, 16 layers: 356 us with a launch between that stored the rows and their values read back here, 312
+// us so.
 template <int KB> struct NewKeyArgs { TbAttnArgs N; TbJobs J; };
 template <> struct NewKeyArgs<0> {};
 template <int kInFlight, bool MS, int KB>

@@ -8,8 +8,8 @@
 //     codes transposed (channel-major, the operand shape of the token-contracting MFMA), both scale vectors as they are;
 //   * a wave owns 16 rows (MFMA 16x16x32: 16 accumulator tiles of 4 registers cover the 256 output channels, the query
 //     fragments take 32 registers), so that two waves fit a SIMD;
-//   * LDS is double buffered: tile n+1 is dequantized before or behind the consumption of tile n; one barrier per tile; the tile loads are
-//     explicit instructions two tiles ahead with their own waits;
+//   * LDS is double buffered: tile n+1 is dequantized before or behind the consumption of tile n; one barrier per tile; the
+//     tile loads are explicit instructions two tiles ahead with their own waits;
 //   * quantize-on-append rides in the launch: a workgroup stores the rows of the pass that fall into the tiles of its own
 //     split before it reads them (32 lanes per row, a word of 8 channels each).
 // LDS image of one tile (42240 bytes):
@@ -198,10 +198,11 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
   const int maxlen = min(pos + maxdep + 1, A.kv.max_ctx), minlen = min(pos + mindep + 1, A.kv.max_ctx);
   const int ntiles = (maxlen + 31) >> 5;
   int tps = (ntiles + A.S - 1) / A.S, tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
-  // where the rows of the pass are stored here (below) the last split owns the tiles that hold them and as many in front of them as its share
-  // leaves once the quantization is paid for; the others share the rest evenly
-  // (in windows of more than 32 rows and on short contexts more workgroups than one should quantize: 64 rows at 1,600 tokens, 4 layers: 86 us a
-  // pass, 98 with all rows in the last split; 4 rows at 3,000 49.5 and 46.3, 16 at 4,090 73.3 and 68.9, 8 at 8,180 62.1 and 58.4)
+  // where the rows of the pass are stored here (below) the last split owns the tiles that hold them and as many in front of
+  // them as its share leaves once the quantization is paid for; the others share the rest evenly (in windows of more than
+  // 32 rows and on short contexts more workgroups than one should quantize: 64 rows at 1,600 tokens, 4 layers: 86 us a
+  // pass, 98 with all rows in the last split; 4 rows at 3,000 49.5 and 46.3, 16 at 4,090 73.3 and 68.9, 8 at 8,180 62.1 and
+  // 58.4)
   if (A.k16 && A.M <= 32 && A.S > 1 && ntiles >= 2 * A.S) {
     const int cost = 1 + A.M / 16;
     const int Tw = min(min(ntiles, max(0, pos + A.tok0) >> 5), (A.S - 1) * ((ntiles + cost + A.S - 1) / A.S));
@@ -359,8 +360,9 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(AttnArgs A) {
     wait_raw<0>(raw0);                         // the loads past the last tile
     wait_raw<0>(raw1);
   };
-  // the two waves of a SIMD take the halves of a step in opposite order: one's MFMAs run under the other's vector work and LDS writes
-  // (16 layers of 24 rows at 9,001 tokens: 363 us with the image first in every wave, 353 so; 8 rows and 1,024-row slices 2 to 5 %)
+  // the two waves of a SIMD take the halves of a step in opposite order: one's MFMAs run under the other's vector work and
+  // LDS writes (16 layers of 24 rows at 9,001 tokens: 363 us with the image first in every wave, 353 so; 8 rows and
+  // 1,024-row slices 2 to 5 %)
   if (!has_rows) run(std::integral_constant<int, kFeedOnly>{});
   else if (wave < 4) run(std::integral_constant<int, kFeedFirst>{});
   else run(std::integral_constant<int, kComputeFirst>{});

@@ -421,9 +421,10 @@ __global__ void __launch_bounds__(256, 2) attend_narrow_kernel(uint64_t p_pos, u
       request(T0 + 4, tb);
       q_ready(std::integral_constant<int, 2 * kTileLoads>{});
       for (int T = T0; T < tile1; T += 8) {
-        // The loop begins at a multiple of 8 bytes, where seven in ten of its 8-byte instructions begin at one too; 4 bytes on they straddle two:
-        // 16 layers of one token at 32,741 tokens 169.9 us instead of 166.6, of two 181.4 and 178.3, whatever moved the code (an
-        // instruction or an argument more in front of it).
+        // The loop begins at a multiple of 8 bytes, where seven in ten of its 8-byte instructions begin at one too; 4 bytes
+        // on they straddle two:
+        // 16 layers of one token at 32,741 tokens 169.9 us instead of 166.6, of two 181.4 and 178.3, whatever moved the
+        // code (an instruction or an argument more in front of it).
         asm volatile(".p2align 3");
         if (T + 4 >= tile1) asm volatile("s_waitcnt vmcnt(0)");
         wait_tile<kTileLoads>(ta);
@@ -508,15 +509,15 @@ void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
 }
 
 // combiner (reference: src/attention_kv4q.cu:325-332): M2 = max pm; w_s = pm_s > -1e29 ? 2^(pm_s - M2) * pl_s : 0;
-// y = sum w_s * (acc_s / l_s) / sum w_s.  grid (n_heads, M), block 256: 16 lanes x 8 channels cover a row, 16 split
-// lanes run in parallel and are summed through LDS.  S <= 256.
-// kInFlight = partial rows a split lane requests before it uses any: 16 covers 256 splits in one memory round trip, 8
-// covers the 128 splits of decode over long contexts (few, long workgroups); 4 keeps the register count low where
-// thousands of workgroups run (wide windows).
+// y = sum w_s * (acc_s / l_s) / sum w_s.  grid (n_heads, M), block 256: 16 lanes x 8 channels cover a row, 16 split lanes
+// run in parallel and are summed through LDS.  S <= 256. kInFlight = partial rows a split lane requests before it uses any:
+// 16 covers 256 splits in one memory round trip, 8 covers the 128 splits of decode over long contexts (few, long
+// workgroups); 4 keeps the register count low where thousands of workgroups run (wide windows).
 // MS: a stream's share of the splits may exceed what is in flight at once (a loop over batches; 256 at most).
 // ADAPT: rows of a prefill slice that the rows form below does not take (inverse rotation, or more than 32 splits); as many
-// workgroups as the chip holds at once, each walks its share of the tokens, so that the choice of the splits is made 8 times per CU and
-// not once per row (1,024 rows at 9,000 tokens with the inverse rotation: 42.4 us with a workgroup per row, 37.9 so).
+// workgroups as the chip holds at once, each walks its share of the tokens, so that the choice of the splits is made 8
+// times per CU and not once per row (1,024 rows at 9,000 tokens with the inverse rotation: 42.4 us with a workgroup per
+// row, 37.9 so).
 template <int kInFlight, bool MS, bool ADAPT>
 __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, CombineTail tail_args) {
   CombineArgs A = combine_args(head_args, tail_args);

@@ -72,8 +72,9 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int gK = (A.layer * A.n_kv + kvh) * 2, gV = gK + 1;
-  // The K and V pair tables of this kv head (global, in L2 -> LDS) are requested before the position, the query and the first K tile
-  // behind it, and only then are the tables waited for: one trip to memory instead of four (one row of 5 bits at 16,001 tokens, 16 layers: 307 us before, 298 so; 30 streams of 4 bits 96.6 and 94.8).
+  // The K and V pair tables of this kv head (global, in L2 -> LDS) are requested before the position, the query and the
+  // first K tile behind it, and only then are the tables waited for: one trip to memory instead of four (one row of 5 bits
+  // at 16,001 tokens, 16 layers: 307 us before, 298 so; 30 streams of 4 bits 96.6 and 94.8).
   int pos = 0;
   if (!MS) pos = *A.d_pos;
   constexpr int kTabLoads = kTabBytes / 16 / 256;    // per thread and table

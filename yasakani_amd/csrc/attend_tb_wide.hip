@@ -1,5 +1,6 @@
 // Split-KV attention over trellis-coded rows (the reference's KV4 / KV5 packed streams) for windows of 3..64 query tokens.
-// gfx950.  reference: launch_q35_prefill_atx_pk / q35_atxpk4_kernel on packed rows (src/q35_atxpk.hpp:21, src/q35_atxpk4.cuh:71-499).
+// gfx950.  reference: launch_q35_prefill_atx_pk / q35_atxpk4_kernel on packed rows (src/q35_atxpk.hpp:21,
+// src/q35_atxpk4.cuh:71-499).
 //
 // The compute side is the wide kernel of the flat 256-channel rows (attend256_wide.hip): a workgroup of 8 waves owns 128
 // query rows and one split of the keys, every 32-key tile is decoded ONCE per workgroup into a double-buffered LDS image
@@ -145,8 +146,9 @@ __device__ __forceinline__ void decode_to_lds(uint8_t* buf, int tid, const Raw& 
 }
 
 // grid (S, n_kv, row blocks), block 512; wave w owns rows [16 w, 16 (w+1)) of the block; BF: bf16 queries
-// No register is left: 256 with 4 bits; with 5 bits a pair that is live across the tile loop is stored to scratch in front of it and read again
-// behind it.  The build walks the generated code (isa_check.py), since a load in flight must not be what is spilled.
+// No register is left: 256 with 4 bits; with 5 bits a pair that is live across the tile loop is stored to scratch in front
+// of it and read again behind it.  The build walks the generated code (isa_check.py), since a load in flight must not be
+// what is spilled.
 template <int KB, bool BF>
 __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   constexpr int kTabBytes = 4 << (8 + KB);
@@ -195,8 +197,8 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
   const int maxlen = min(pos + maxdep + 1, A.max_ctx), minlen = min(pos + mindep + 1, A.max_ctx);
   const int ntiles = (maxlen + 31) >> 5;
   int tps = (ntiles + A.S - 1) / A.S, tile0 = split * tps, tile1 = min(ntiles, tile0 + tps);
-  // where the rows of the pass are stored here (below) the last split owns the tiles that hold them and as many in front of them as its share
-  // leaves once the coding is paid for, about two tiles; the others share the rest evenly
+  // where the rows of the pass are stored here (below) the last split owns the tiles that hold them and as many in front of
+  // them as its share leaves once the coding is paid for, about two tiles; the others share the rest evenly
   if (A.jobs.scr && A.S > 1) {
     constexpr int kStoreCost = 2;
     const int Tw = min(min(ntiles, max(0, pos + A.tok0) >> 5), (A.S - 1) * ((ntiles + kStoreCost + A.S - 1) / A.S));
@@ -205,10 +207,11 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
     tile1 = split == A.S - 1 ? ntiles : min(Tw, tile0 + tps);
   }
 
-  // ---- the rows of the pass: a workgroup codes and stores those that lie in the tiles of its own range before it reads them, from what
-  //      the searches have left, a wave per row.  Row blocks of one kv head write identical bytes; a row past the last tile of the last
-  //      row block (no query row of the pass sees it: a depth table may say so) is stored by that block's last split.  Writer and
-  //      readers are waves of one CU and one write-through L1.  Every condition that guards the barrier is uniform over the workgroup. ----
+  // ---- the rows of the pass: a workgroup codes and stores those that lie in the tiles of its own range before it reads
+  //      them, from what the searches have left, a wave per row.  Row blocks of one kv head write identical bytes; a row past
+  //      the last tile of the last row block (no query row of the pass sees it: a depth table may say so) is stored by that
+  //      block's last split.  Writer and readers are waves of one CU and one write-through L1.  Every condition that guards
+  //      the barrier is uniform over the workgroup. ----
   if (A.jobs.scr) {
     const int r0 = pos + A.tok0, Tn0 = r0 >> 5, Tn1 = (r0 + A.M - 1) >> 5;
     const bool last_wg = split == A.S - 1 && rb == (int)gridDim.z - 1;
@@ -353,8 +356,8 @@ __global__ void __launch_bounds__(NT, 1) attend_tb_wide_kernel(TbAttnArgs A) {
     }
     wait_raw(raw);                             // the loads past the last tile
   };
-  // the two waves of a SIMD take the halves of a step in opposite order: one's MFMAs run under the other's vector work and LDS writes
-  // (16 layers of 16 rows of 5 bits at 16,384 tokens: 764 us with the image first in every wave, 747 so)
+  // the two waves of a SIMD take the halves of a step in opposite order: one's MFMAs run under the other's vector work and
+  // LDS writes (16 layers of 16 rows of 5 bits at 16,384 tokens: 764 us with the image first in every wave, 747 so)
   if (!has_rows) run(std::integral_constant<int, kFeedOnly>{});
   else if (wave < 4) run(std::integral_constant<int, kFeedFirst>{});
   else run(std::integral_constant<int, kComputeFirst>{});

@@ -411,23 +411,24 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
       l_run += lsum0 + lsum1;
     }
   };
-  // ---- the group's tile k + 1, whose raw codes `rs` holds, goes to the buffer that tile k does not occupy (after the last tile that
-  //      buffer is read by nobody); the request for tile k + 3 replaces them (past the end: the last tile again, so that the
-  //      count of loads in flight is static) ----
+  // ---- the group's tile k + 1, whose raw codes `rs` holds, goes to the buffer that tile k does not occupy (after the last
+  //      tile that buffer is read by nobody); the request for tile k + 3 replaces them (past the end: the last tile again, so
+  //      that the count of loads in flight is static) ----
   auto feed = [&](const int k, const int cb, Raw& rs) __attribute__((always_inline)) {
     wait_raw<6>(rs);                           // the six loads of the other register set stay in flight
     dequant_to_lds(lds[grp][cb ^ 1], gt, rs, magic, sc_log2);
     load_tile_raw(tile_of(k + 3), rs);
   };
-  // One workgroup barrier per step.  Between two barriers group 0 runs the matrix and then the vector phase of its tile k, group 1
-  // the vector phase of its tile k - 1 and then the matrix phase of its tile k: each time one group's MFMAs run under the other's
-  // vector work.  Both dequantize tile k + 1 in step k, into the buffer of tile k - 1, which nobody has read since the barrier
-  // before.  The wave in its vector phase goes first when both waves of a SIMD have an instruction to issue: at equal priority the
-  // older wave (group 0) wins in both of its phases and the younger group sets the pace.
-  // With a barrier behind either phase the waves waited 130 cycles behind the matrix phase and 250 behind the vector phase of a step
-  // of 2,780.  us, two barriers / one: 16 layers of 1,500 rows on an empty cache 742 / 704, of 64 rows at 32,768 tokens 731 / 716.
-  // 2,048 rows at 131,072 tokens, 2 layers 8,131 / 8,111: 1,420 / 1,332 cycles a tile, but the chip lowers its clock from 2.24 to 2.15
-  // GHz - a long slice is bound by power, and only work left out shortens it.
+  // One workgroup barrier per step.  Between two barriers group 0 runs the matrix and then the vector phase of its tile k,
+  // group 1 the vector phase of its tile k - 1 and then the matrix phase of its tile k: each time one group's MFMAs run
+  // under the other's vector work.  Both dequantize tile k + 1 in step k, into the buffer of tile k - 1, which nobody has
+  // read since the barrier before.  The wave in its vector phase goes first when both waves of a SIMD have an instruction
+  // to issue: at equal priority the older wave (group 0) wins in both of its phases and the younger group sets the pace.
+  // With a barrier behind either phase the waves waited 130 cycles behind the matrix phase and 250 behind the vector phase
+  // of a step of 2,780.  us, two barriers / one: 16 layers of 1,500 rows on an empty cache 742 / 704, of 64 rows at 32,768
+  // tokens 731 / 716.
+  // 2,048 rows at 131,072 tokens, 2 layers 8,131 / 8,111: 1,420 / 1,332 cycles a tile, but the chip lowers its clock from
+  // 2.24 to 2.15 GHz - a long slice is bound by power, and only work left out shortens it.
   // The loads of a group live inside its own branch from the request to the last wait (a join would copy their registers).
   const int nstep = max((ntl + 1) >> 1, (ntl >> 1) + 1);
   auto requests = [&]() __attribute__((always_inline)) { if (nu > 0) { load_tile_raw(tile_of(1), raw1); load_tile_raw(tile_of(2), raw0); } };

@@ -6,11 +6,12 @@
 namespace yka {
 
 constexpr int kMaxMult = 16;
-// What a row is stored as after the search (cache form), by a wave: the multiplier whose search left the smallest squared error (its 8
-// partial sums added in order from 0; the first of equal errors), the four states of elements 4 lane .. 4 lane + 3 it chose, its scale.
-// choose_job: which job, from what request_errors has asked for.  A wave with one row asks for the states of all jobs beside that
-// (pick_job, one trip to memory; no branch stands between the requests, past the last multiplier it is asked for again); one with several rows
-// asks for the chosen states only, which are a ninth of the bytes.
+// What a row is stored as after the search (cache form), by a wave: the multiplier whose search left the smallest squared
+// error (its 8 partial sums added in order from 0; the first of equal errors), the four states of elements 4 lane .. 4 lane
+// + 3 it chose, its scale.
+// choose_job: which job, from what request_errors has asked for.  A wave with one row asks for the states of all jobs
+// beside that (pick_job, one trip to memory; no branch stands between the requests, past the last multiplier it is asked
+// for again); one with several rows asks for the chosen states only, which are a ninth of the bytes.
 typedef uint32_t JobStates __attribute__((ext_vector_type(kMaxMult)));
 typedef float JobErrors __attribute__((ext_vector_type(4)));
 struct JobTotals { JobErrors e0, e1; float s; };
@@ -44,8 +45,9 @@ __device__ __forceinline__ void pick_job(const TbJobs& A, int row, int lane, uin
   const auto a2 = (keep & 2) ? a4.hi : a4.lo;
   states = (keep & 1) ? a2.y : a2.x;
 }
-// packs the fields of those states and stores the row: 4 fields of a lane are 4 KB bits of the MSB-first stream; a word is made of the
-// bits of two lanes (4 bits: lane 2 w and the next) or of up to three (5 bits: 8 lanes are 5 words, word j starts in lane 8 j / 5)
+// packs the fields of those states and stores the row: 4 fields of a lane are 4 KB bits of the MSB-first stream; a word is
+// made of the bits of two lanes (4 bits: lane 2 w and the next) or of up to three (5 bits: 8 lanes are 5 words, word j
+// starts in lane 8 j / 5)
 template <int KB>
 __device__ __forceinline__ void store_coded_row(uint8_t* dst, int lane, uint32_t states) {
   constexpr uint32_t mask = (1u << KB) - 1u;

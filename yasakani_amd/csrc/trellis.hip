@@ -333,9 +333,10 @@ __device__ __forceinline__ void wave_chunk(const int* xi, const StepConsts& C, u
 #pragma unroll
   for (int g = 0; g < U; ++g) kept = lane == keeper_lane<KK>(g) ? g : kept;
   uint32_t* const rec = reinterpret_cast<uint32_t*>(bp) + (kept < 0 ? 0 : kept);
-  // A lone wave's steps slow down where 8-byte instructions straddle multiples of 8 bytes: 28 of the 44 of these four steps do not with 4 bits if
-  // the loop begins at such a multiple (16 if it begins 4 bytes on), 25 of 43 with 5 bits if the middle of the first two steps
-  // lies at one (18).  One token of 4 bits at 1,600 tokens, 4 layers: 59.5 us the other way, 58.7 so; of 5 bits at 600 55.9 and 55.4.
+  // A lone wave's steps slow down where 8-byte instructions straddle multiples of 8 bytes: 28 of the 44 of these four steps
+  // do not with 4 bits if the loop begins at such a multiple (16 if it begins 4 bytes on), 25 of 43 with 5 bits if the
+  // middle of the first two steps lies at one (18).  One token of 4 bits at 1,600 tokens, 4 layers: 59.5 us the other way,
+  // 58.7 so; of 5 bits at 600 55.9 and 55.4.
 #pragma unroll 1
   for (int t = 0; t < 64; t += 4) {
     uint32_t chosen4 = 0u;
@@ -502,9 +503,9 @@ __global__ void __launch_bounds__(256) tb_search_probe_kernel(TbProbeArgs A) {
 // Decode (one or two tokens, no depth table): the search for the new rows' codes and the attention over the rows already in
 // the cache need nothing from each other, and neither fills the chip - 72 or 144 workgroups, each a serial chain of 64
 // steps, beside one attention workgroup per CU.  One launch runs both: the first `n_search` workgroups search, the others
-// attend to the keys in front of *d_pos.  The combiner picks the codes of the new rows, stores them and adds them as keys of its own
-// (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 with the encoder in launches of its own, 22.2
-// with the rows stored by a launch between these two, 19.5 so.
+// attend to the keys in front of *d_pos.  The combiner picks the codes of the new rows, stores them and adds them as keys
+// of its own (combine256_kernel with new keys).  5 bits, 16,001 tokens, us per layer call: 29.0 with the encoder in
+// launches of its own, 22.2 with the rows stored by a launch between these two, 17.8 so.
 template <int KB, bool BF>
 __global__ void __launch_bounds__(256, 2) tb_search_attend_kernel(const int* p_pos, int n_search, TbEncArgs E, TbAttnArgs A) {
   A.d_pos = p_pos;
@@ -607,9 +608,9 @@ __global__ void __launch_bounds__(256) tb_select_kernel(TbProbeArgs A) {
   A.yout[R.index * 256 + d] = rebuilt;
 }
 
-// Cache form: a wave per row.  Every multiplier's states (a word of four per lane), error sums and scale are requested at once with the
-// position; what the row is coded with then costs no further trip: the search has left the scales, so neither the row nor its
-// mean is read again.
+// Cache form: a wave per row.  Every multiplier's states (a word of four per lane), error sums and scale are requested at
+// once with the position; what the row is coded with then costs no further trip: the search has left the scales, so neither
+// the row nor its mean is read again.
 template <int KB>
 __global__ void __launch_bounds__(256) tb_store_kernel(const int* p_pos, const uint8_t* p_scr, int p_nm, TbEncArgs A) {
   A.d_pos = p_pos; A.scr = const_cast<uint8_t*>(p_scr); A.nm = p_nm;

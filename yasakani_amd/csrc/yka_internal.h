@@ -90,16 +90,19 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
   int adapt = 0; int direct = 0; const int* d_pos = nullptr; int tok0 = 0; int n_kv = 0; int max_ctx = 0;
   const int2* plan = nullptr;   // partials of a multi-stream pass shared out by ms_share: first split and splits of every row
   int s_short = 0; };    // trellis decode: as in TbAttnArgs (d_pos is set then)
-// Decode, its combiner and the trellis kernels of decode name what their first loads need as leading arguments of their own and are compiled
-// with -amdgpu-kernarg-preload-count: those arrive in scalar registers with the wave, and the position (the combiner's partials)
-// is asked for at once instead of 0.3 us later, behind the load of the argument block.  us per 16 layers without / with: one token at 32,741
-// tokens 172.5 / 166.5, one 5-bit trellis row at 16,001 382 / 371, 8 rows at 12,037 (the combiner alone) 226 / 220, one token at
-// 1,003 115.4 / 113.8, 16 streams 27.1 / 26.7 a pass.  Not where it measured slower: the 256-channel kernels (273 / 280), wide
-// windows (737 / 743), windows of 3 to 5 rows in the mid kernel (212 / 218; 8 rows 220 / 218).
-// Such a pointer travels as an integer, and the combiners' arguments are split into head and tail, not repeated: a pointer among a
-// launch's arguments costs the host 0.2 us, and the 136 bytes of a repeated block 0.45 us more than these 96.  A call issued outside a graph
-// is as long as the host takes; 16 layers of one token at 1,622 tokens, us: 177 without preloaded arguments, 192 with pointers
-// and the block repeated, 185 with integers, 178 with the split.
+// Decode, its combiner and the trellis kernels of decode name what their first loads need as leading arguments of their own
+// and are compiled with -amdgpu-kernarg-preload-count: those arrive in scalar registers with the wave, and the position
+// (the combiner's partials) is asked for at once instead of 0.3 us later, behind the load of the argument block.  us per 16
+// layers without / with: one token at 32,741 tokens 172.5 / 166.5, one 5-bit trellis row at 16,001 382 / 371, 8 rows at
+// 12,037 (the combiner alone) 226 / 220, one token at 1,003 115.4 / 113.8, 16 streams 27.1 / 26.7 a pass.  Not where it
+// measured slower: the 256-channel kernels (273 / 280), wide windows (737 / 743), windows of 3 to 5 rows in the mid kernel
+// (212 / 218; 8 rows 220 / 218).
+// In the int4 decode kernel and the combiners such a pointer travels as an integer, and the combiners' arguments are split
+// into head and tail, not repeated: a pointer among a launch's arguments costs the host 0.2 us, and the 136 bytes of a
+// repeated block 0.45 us more than these 96.  A call issued outside a graph is as long as the host takes; 16 layers of one
+// token at 1,622 tokens, us: 177 without preloaded arguments, 192 with pointers and the block repeated, 185 with integers,
+// 178 with the split.  The trellis kernels keep pointers and repeat what they preload: over such rows the device takes
+// longer than the host on any context (one token at 600 tokens 13.8 us a layer against 11.8).
 typedef uint32_t CombineHead __attribute__((ext_vector_type(8)));     // pm, pl, pacc16 (two words each), S, n_heads
 struct CombineTail { uint16_t* out16; const int* d_pos; const int2* plan; int M, unrot, out_bf16, adapt, direct, tok0, n_kv, max_ctx, s_short; };
 inline CombineHead combine_head(const CombineArgs& A) {
@@ -109,7 +112,8 @@ inline CombineHead combine_head(const CombineArgs& A) {
 inline CombineTail combine_tail(const CombineArgs& A) {
   return CombineTail{A.out16, A.d_pos, A.plan, A.M, A.unrot, A.out_bf16, A.adapt, A.direct, A.tok0, A.n_kv, A.max_ctx, A.s_short};
 }
-// such an integer, or two words of a head, as a pointer into global memory; without the address space the loads behind it are flat ones
+// such an integer, or two words of a head, as a pointer into global memory; without the address space the loads behind it
+// are flat ones
 template <typename T> __device__ __forceinline__ T* head_ptr(uint64_t word) { return (T*)(__attribute__((address_space(1))) T*)word; }
 template <typename T> __device__ __forceinline__ T* head_ptr(uint32_t lo, uint32_t hi) { return head_ptr<T>((uint64_t)lo | ((uint64_t)hi << 32)); }
 __device__ __forceinline__ CombineArgs combine_args(CombineHead H, const CombineTail& T) {
@@ -131,9 +135,10 @@ struct PostArgs {
   int io_bf16 = 0;   // 16-bit rows that leave (q16, gate16) are bf16 instead of fp16
 };
 
-// Trellis-coded rows on their way into the cache (trellis.hip).  Row rj of the launch is (token rj / (2 n_kv), K | V, kv head) of the
-// pass, read from k32 / v32 [M][n_kv][256]; its payload goes to pay0 (K) / pay1 (V) + (kvh * max_ctx + pos) * stride and its
-// scale to scl0 / scl1 [kvh * max_ctx + pos].  Every group is trellis-coded with kb bits, without guard positions and directions.
+// Trellis-coded rows on their way into the cache (trellis.hip).  Row rj of the launch is (token rj / (2 n_kv), K | V, kv
+// head) of the pass, read from k32 / v32 [M][n_kv][256]; its payload goes to pay0 (K) / pay1 (V) + (kvh * max_ctx + pos) *
+// stride and its scale to scl0 / scl1 [kvh * max_ctx + pos].  Every group is trellis-coded with kb bits, without guard
+// positions and directions.
 struct TbEncArgs {
   const float* k32; const float* v32; const uint16_t* k16; const uint16_t* v16;   // fp32 rows, or 16-bit rows if k32 == nullptr
   const int* d_pos; int layer, tok0, n_kv, max_ctx, rot;
@@ -146,8 +151,8 @@ struct TbEncArgs {
   RowMap rows;                        // multi-stream pass: token t sits at rows.pos[t] of container rows.slot[t] (pay / scl = container 0)
   int in_bf16;                        // k16 / v16 are bf16 rows
 };
-// The codec alone (reference TbFastArgs, src/kvq_fast.hpp:16-37): rows row0 .. row0 + nrow - 1 of yin with their own group and position,
-// any profile; results indexed by row.
+// The codec alone (reference TbFastArgs, src/kvq_fast.hpp:16-37): rows row0 .. row0 + nrow - 1 of yin with their own group
+// and position, any profile; results indexed by row.
 struct TbProbeArgs {
   const uint8_t* blob; int nm; int has_trellis;
   // what the host looked up in the blob (see tb_descriptors in abi.hip): [ngrp][8] words
@@ -165,8 +170,9 @@ __host__ __device__ inline TbJobs tb_jobs(const TbEncArgs& A) { return TbJobs{A.
 // attention over trellis-coded rows (attend_tb.hip).  pairs [groups][2^(8 + kb)]: entry i = the table's integers, as two
 // fp16 values, of the states (i >> kb) & 255 and i & 255 (two consecutive elements from 8 + kb stream bits); gfac [groups]:
 // gain / 256; mu [groups][256] fp32 mean rows (zero rows where a group has none) or nullptr if no group has one
-// At a multiple of 64 bytes among a kernel's arguments: what a decode workgroup asks of it first does not straddle two cache lines, whatever stands in
-// front (4 layers of one token of 4 bits at 16,000 tokens 65.2 us with the rows' pointers across two lines, 64.3 so).
+// At a multiple of 64 bytes among a kernel's arguments: what a decode workgroup asks of it first does not straddle two
+// cache lines, whatever stands in front (4 layers of one token of 4 bits at 16,000 tokens 65.2 us with the rows' pointers
+// across two lines, 64.3 so).
 struct alignas(64) TbAttnArgs {
   const uint8_t* kpay; const uint8_t* vpay; const float* kscl; const float* vscl; int max_ctx, n_kv, stride;
   const uint32_t* pairs; const float* gfac; const float* mu; int layer;
@@ -190,15 +196,21 @@ __device__ __forceinline__ void tb_split_of(const TbAttnArgs& A, int b, int& spl
 void launch_tb_encode(const TbEncArgs&, hipStream_t);
 void launch_tb_search(const TbEncArgs&, hipStream_t);     // the searches alone: TbAttnArgs::jobs has their results stored
 void launch_tb_probe(const TbProbeArgs&, hipStream_t);
-// one or two tokens: searches of the encoder and attention over the keys in front of *d_pos; the combiner has to store the new rows and add them
+// one or two tokens: searches of the encoder and attention over the keys in front of *d_pos; the combiner has to store the
+// new rows and add them
 void launch_tb_encode_attend(const TbEncArgs&, const TbAttnArgs&, int kb, hipStream_t);
 void launch_tb_unpack(const uint8_t* blob, const int* grp, const int* pos, const uint8_t* pay, const uint32_t* side, int stride, const float* yin,
                       float* y, int rows, hipStream_t);
 
-// Trellis windows of at most so many rows are coded and stored by the attention launch, the others by a launch of their own: the workgroup that
-// holds the window codes 2 rows per token, 8 at a time, which costs about two tiles of its share (its range is shorter by so much) and saves
-// the launch between.  us per 16 layers, launch / here: 16 rows of 5 bits at 16,384 tokens 743 / 687; per 4 layers at 500 tokens 3 rows 87.9 /
-// 81.8, 10 rows 107.9 / 103.8, 16 rows 138.2 / 138.9 (nothing hides the coding there), 16 rows of 4 bits at 3,000 156.2 / 145.3.
+// Trellis windows of at most so many rows are coded and stored by the attention launch, the others by a launch of their
+// own: the workgroup that holds the window codes 2 rows per token, 8 at a time, which costs about two tiles of its share
+// (its range is shorter by so much) and saves the launch between.  us per 16 layers, launch / here: 16 rows of 5 bits at
+// 16,384 tokens 743 / 687; per 4 layers at 500 tokens 3 rows 87.9 / 81.8, 10 rows 107.9 / 103.8, 16 rows 138.2 / 138.9, 16
+// rows of 4 bits at 3,000 156.2 / 145.3.  16 is the widest window that loses nothing on short contexts, where nothing hides
+// the coding.  Of wider ones (4 layers, 5 bits; 6 rows a wave for 17 and 21 rows, 12 for 32 and 48) 17, 21, 32 and 48 rows
+// take 143 / 147, 158 / 162, 175 / 185 and 223 / 236 at 500 tokens, 152 / 142, 167 / 156, 193 / 183 and 244 / 234 at 3,000,
+// and 184 / 169, 193 / 181, 256 / 242 and 346 / 336 at 16,000: what long contexts would gain short ones would pay, and the
+// host does not know which it has.
 constexpr int kTbFuseRows = 16;
 
 // launchers (each checks nothing: the C layer validates shapes first)
@@ -280,20 +292,22 @@ __device__ __forceinline__ uint4 pack_out8(const float* y, int bf16) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// 16 bytes of a partial row, written through the XCD's L2 (agent scope) as it leaves the workgroup.  The combiner runs on other XCDs, so
-// what lies dirty in an L2 when the launch ends is written back then, with nothing else running: 9.6 MB of partials of 24
-// rows in 32 splits kept the combiner waiting 5 us behind the last workgroup, where 1.4 us are usual.  Written through, the
-// rows of the workgroups that end early are out before the last one ends.  us per 16 layers, ordinary / nontemporal / written through: 24
-// rows of 256 channels at 9,001 tokens 396 / 370 / 363, 64 rows of 128 at 32,768 741 / 733 / 730, 8 rows at 12,037 229 / 225 /
-// 225.  Decode and the smallest windows leave little, which nobody waits for, and such stores are in the way of their end: one token at
-// 32,741 tokens 173 / 173 / 176, 16 streams 27.2 / 27.8 / 28.0 a pass, 4 rows at 32,768 259 ordinary and 263; they keep ordinary stores.
+// 16 bytes of a partial row, written through the XCD's L2 (agent scope) as it leaves the workgroup.  The combiner runs on
+// other XCDs, so what lies dirty in an L2 when the launch ends is written back then, with nothing else running: 9.6 MB of
+// partials of 24 rows in 32 splits kept the combiner waiting 5 us behind the last workgroup, where 1.4 us are usual.
+// Written through, the rows of the workgroups that end early are out before the last one ends.  us per 16 layers, ordinary
+// / nontemporal / written through: 24 rows of 256 channels at 9,001 tokens 396 / 370 / 363, 64 rows of 128 at 32,768 741 /
+// 733 / 730, 8 rows at 12,037 229 / 225 / 225.  Decode and the smallest windows leave little, which nobody waits for, and
+// such stores are in the way of their end: one token at 32,741 tokens 173 / 173 / 176, 16 streams 27.2 / 27.8 / 28.0 a
+// pass, 4 rows at 32,768 259 ordinary and 263; they keep ordinary stores.
 __device__ __forceinline__ void store_partial16(uint16_t* p, uint4 v) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)p, u32x4{v.x, v.y, v.z, v.w}, "agent");
 }
 
-// least and greatest depth of tokens tok_lo .. tok_hi - 1 (at most 64), a token per lane: one trip to memory (a loop over them was one each:
-// 4 layers of 16 rows with a depth table at 9,000 tokens 68.9 us, 63.7 so, of 24 rows of 256 channels 88.8 and 85.8, of 16 trellis rows 177 and 172)
+// least and greatest depth of tokens tok_lo .. tok_hi - 1 (at most 64), a token per lane: one trip to memory (a loop over
+// them was one each: 4 layers of 16 rows with a depth table at 9,000 tokens 68.9 us, 63.7 so, of 24 rows of 256
+// channels 88.8 and 85.8, of 16 trellis rows 177 and 172)
 __device__ __forceinline__ void depth_range(const uint8_t* depth, int tok_lo, int tok_hi, int& least, int& most) {
   const int t = tok_lo + (int)(threadIdx.x & 63), last = max(tok_lo, tok_hi - 1);
   const int dp = depth[min(t, last)];
@@ -301,9 +315,9 @@ __device__ __forceinline__ void depth_range(const uint8_t* depth, int tok_lo, in
   most = __builtin_amdgcn_readfirstlane(lane_rows(lane_row16(dp, LaneMax{}), LaneMax{}));
 }
 
-// Sums and maxima of the plans below run through lane-crossing moves (a shift inside rows of 16 lanes, then two row broadcasts),
-// not through LDS: a plan stands in front of everything else a workgroup does (multi-stream passes, 5 trellis streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128
-// channels 14.9 and 13.9).
+// Sums and maxima of the plans below run through lane-crossing moves (a shift inside rows of 16 lanes, then two row
+// broadcasts), not through LDS: a plan stands in front of everything else a workgroup does (multi-stream passes, 5 trellis
+// streams of up to 3,000 tokens: 28.4 us a pass before, 27.5 since; 30 int4 streams of 128 channels 14.9 and 13.9).
 template <class Op>
 __device__ __forceinline__ int wave_scan(int v, Op op) {            // inclusive over the lanes; 0 is the neutral value
   v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));        // row_shr:1, 2, 4, 8
@@ -316,19 +330,21 @@ __device__ __forceinline__ int wave_scan(int v, Op op) {            // inclusive
 __device__ __forceinline__ int wave_scan_add(int v) { return wave_scan(v, [](int a, int b) { return a + b; }); }
 
 // Splits a slice of a prefill chunk uses, of the `S` its launch provides for.  The host sizes the grid without knowing the
-// position, so the choice is made on the device, by every wave of the attention launch and again by the combiner: lane s - 1
-// prices s splits, the cheapest wins (ties: the fewest).  Whole numbers only, so that two compilations cannot disagree.
+// position, so the choice is made on the device, by every wave of the attention launch and again by the combiner: lane s -
+// 1 prices s splits, the cheapest wins (ties: the fewest).  Whole numbers only, so that two compilations cannot disagree.
 // Times are in sixteenths of the time a workgroup takes for one 32-key tile (0.56 us): a workgroup costs kChunkOverhead
 // tiles before and after its loop (about 10 us: launch, query, first tile, merge, stores), one workgroup runs per CU, the
 // longest start first, and more than one split costs a combiner pass over M * s partial rows.
 // 1,500 rows on an empty cache in containers of 8,192 tokens, us per layer call: 105 with slices of 1,024 tokens in 4 and 8
 // splits (39 + 39 in the attention, 23 in the combiners), 46 with one split (42 in the attention, which then waits for its
-// longest workgroup: 47 tiles; 48 and 44 while the choice went through LDS).  2,048 rows behind 131,072: the same with 2 splits of one slice as with 4 of two.
+// longest workgroup: 47 tiles; 48 and 44 while the choice went through LDS).  2,048 rows behind 131,072: the same with 2
+// splits of one slice as with 4 of two.
 constexpr int kChunkOverhead = 18, kChunkMaxSplits = 64;
-// Price of s splits in those units, for a slice whose first and last row blocks walk so many tiles.  Workgroups times tiles would pass 2^31
-// with 2,048 rows on 4 KV heads at 11 M tokens, and the two readers of a choice have to agree on it: the caller cuts the tiles at
-// chunk_tile_cap (which changes no choice: beyond it the overhead is nothing).  That limit comes from the host, in `adapt`; 64-bit
-// products or a unit chosen here cost 1 % of a prompt's first slice, as instructions fetched cold in front of everything else.
+// Price of s splits in those units, for a slice whose first and last row blocks walk so many tiles.  Workgroups times tiles
+// would pass 2^31 with 2,048 rows on 4 KV heads at 11 M tokens, and the two readers of a choice have to agree on it: the
+// caller cuts the tiles at chunk_tile_cap (which changes no choice: beyond it the overhead is nothing).  That limit comes
+// from the host, in `adapt`; 64-bit products or a unit chosen here cost 1 % of a prompt's first slice, as instructions
+// fetched cold in front of everything else.
 __host__ __device__ constexpr unsigned chunk_price(int first, int last, int base, int M, int s) {
   const unsigned lo = first * 16 / s + 16 * kChunkOverhead, hi = last * 16 / s + 16 * kChunkOverhead;
   const unsigned n = (unsigned)base * s, idle = (256 - (n & 255)) & 255;        // workgroups, and CUs without one in the last round
@@ -360,13 +376,15 @@ __device__ __forceinline__ int splits_at(int S, int s_short, int pos) { return s
 
 // Multi-stream pass: how the W workgroups of one kv head are shared out over the pass's M <= 64 rows.  Streams differ in
 // length, and with the same number of splits for each the workgroups of the longest set the pace: every split is given
-// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 4 (one per wave) and no row more than 256.  c =
-// (tiles of all rows) / (W - M) always fits, since every row may round up by one; four halvings look for a smaller one.
+// about the same number of 32-key tiles instead: row t gets ceil(tiles / c) splits, c >= 4 (one per wave) and no row more
+// than 256.  c = (tiles of all rows) / (W - M) always fits, since every row may round up by one; four halvings look for a
+// smaller one.
 // 16 streams of 2,000 to 32,000 tokens: 36.7 us a pass with 16 splits each (the longest stream's workgroups walk 62 tiles,
-// the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.  Row t's splits are
-// workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by every wave from the
-// row map (lane t looks at row t); the first wave of the launch leaves the shares in memory for the combiner, whose
-// workgroups have nothing to hide the computation under (48 streams of 300 tokens, 5 bits: its launch 6.0 us when it computed the shares, 4.6 since).
+// the shortest's 4), 32.5 shared out over two workgroups per CU (four: 34.5), 30.6 with the new rows stored here as well.
+// Row t's splits are workgroups base .. base + n - 1 of the kv head, which is also where its partials lie.  Computed by
+// every wave from the row map (lane t looks at row t); the first wave of the launch leaves the shares in memory for the
+// combiner, whose workgroups have nothing to hide the computation under (48 streams of 300 tokens, 5 bits: its launch 6.0
+// us when it computed the shares, 4.6 since).
 struct MsShare { int row, split, n, pos, slot; size_t base; };
 // ceil(a / b) for quotients up to 2^16 and a below 2^27: the float quotient is off by one at most
 __device__ __forceinline__ int ms_tiles_per(int a, int b) {
