@@ -427,8 +427,9 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(AttnArgs A) {
   // With a barrier behind either phase the waves waited 130 cycles behind the matrix phase and 250 behind the vector phase
   // of a step of 2,780.  us, two barriers / one: 16 layers of 1,500 rows on an empty cache 742 / 704, of 64 rows at 32,768
   // tokens 731 / 716.
-  // 2,048 rows at 131,072 tokens, 2 layers 8,131 / 8,111: 1,420 / 1,332 cycles a tile, but the chip lowers its clock from
-  // 2.24 to 2.15 GHz - a long slice is bound by power, and only work left out shortens it.
+  // 2,048 rows at 131,072 tokens, 2 layers 8,043 / 8,027: the waves wait in 27 % of their cycles instead of 32, but are in
+  // line for an issue slot in 27 instead of 24 (1,401 / 1,384 cycles a tile, at 2.1 GHz) - a long slice is bound by what
+  // its two waves a SIMD have to issue.
   // The loads of a group live inside its own branch from the request to the last wait (a join would copy their registers).
   const int nstep = max((ntl + 1) >> 1, (ntl >> 1) + 1);
   auto requests = [&]() __attribute__((always_inline)) { if (nu > 0) { load_tile_raw(tile_of(1), raw1); load_tile_raw(tile_of(2), raw0); } };
