@@ -129,9 +129,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(WindowHead head_args
 #pragma unroll
   for (int rt = 0; rt < NRT; ++rt) {
     const h8 c = __builtin_bit_cast(h8, qraw[rt]);
-    // the element order of the K operand; the odd nibble of a code byte enters as 16 n (see the decode kernel)
-    const _Float16 se = (_Float16)4.f, so = (_Float16)0.25f;
-    const h8 f = h8{c[0] * se, c[4] * se, c[1] * so, c[5] * so, c[2] * se, c[6] * se, c[3] * so, c[7] * so};
+    const h8 f = h8{c[0], c[4], c[1], c[5], c[2], c[6], c[3], c[7]};       // the element order of the K operand
     s_q[(rt * 4 + wave) * 64 + lane] = __builtin_bit_cast(uint4, f);
   }
   int lenr[NRT];
@@ -202,7 +200,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(WindowHead head_args
     __syncthreads();                             // the query fragments are in LDS
   }
 
-  const float sc_log2 = 0.25f * kLog2e / sqrtf((float)kD);         // 1/4: the query fragments carry a factor 4
+  const float sc_log2 = kLog2e / sqrtf((float)kD);
   float m_run[NRT], l_run[NRT];
   f4 o[NRT][8];
 #pragma unroll

@@ -132,15 +132,16 @@ __device__ __forceinline__ uint32_t nib(uint32_t w, uint32_t mask, uint32_t magi
 template <int U>
 __device__ __forceinline__ void dequant_to_lds(uint8_t* buf, int t, const Raw<U>& R, uint32_t magic, float sc_log2) {
   const h2 c1032 = {(_Float16)1032.f, (_Float16)1032.f}, c1152 = {(_Float16)1152.f, (_Float16)1152.f};
+  const h2 c16 = {(_Float16)0.0625f, (_Float16)0.0625f}, c72 = {(_Float16)-72.f, (_Float16)-72.f};
 #pragma unroll
   for (int n = 0; n < 2 * U; ++n) {
     const int idx = t + 64 * (n >> 1) + (n & 1) * NTG, key = idx >> 4, p = idx & 15;      // physical dword p = 4g+m of the key row
     const uint32_t w = R.kw[n >> 1][n & 1], w8 = w >> 8;
     uint4 o;
     o.x = as_u32(as_h2(nib(w, 0x000f000fu, magic)) - c1032);
-    o.y = as_u32(as_h2(nib(w, 0x00f000f0u, magic)) - c1152);
+    o.y = as_u32(__builtin_elementwise_fma(as_h2(nib(w, 0x00f000f0u, magic)), c16, c72));      // (1024 + 16 n) / 16 - 72 = n - 8, exactly
     o.z = as_u32(as_h2(nib(w8, 0x000f000fu, magic)) - c1032);
-    o.w = as_u32(as_h2(nib(w8, 0x00f000f0u, magic)) - c1152);
+    o.w = as_u32(__builtin_elementwise_fma(as_h2(nib(w8, 0x00f000f0u, magic)), c16, c72));
     *reinterpret_cast<uint4*>(buf + kLdsK + key * kKPitch + (4 * (p & 3) + (p >> 2)) * 16) = o;
   }
 #pragma unroll
@@ -278,15 +279,12 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
   const size_t pidx = ((size_t)tl * A.S + split) * A.n_heads + head;
   {
     if constexpr (BF) rows16_to_f16(qraw);
-    // the odd nibble of a byte is 16 (n - 8) in the K image: its query channels carry 1/4 and the others 4 (products 4 q n
-    // either way; a plain 1/16 would push small queries into the fp16 subnormals), the 4 leaves with the softmax scale
-    const _Float16 se = (_Float16)4.f, so = (_Float16)0.25f;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int r = 32 * u + (tid >> 4);
       const bool some = r < RPB && rb * RPB + r < nrows;
       const h8 c = __builtin_bit_cast(h8, some ? qraw[u] : make_uint4(0, 0, 0, 0));
-      *reinterpret_cast<h8*>(s_q + r * kKPitch + 16 * (tid & 15)) = h8{c[0] * se, c[4] * se, c[1] * so, c[5] * so, c[2] * se, c[6] * se, c[3] * so, c[7] * so};
+      *reinterpret_cast<h8*>(s_q + r * kKPitch + 16 * (tid & 15)) = h8{c[0], c[4], c[1], c[5], c[2], c[6], c[3], c[7]};
     }
   }
   __syncthreads();
@@ -350,7 +348,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
 
-  const float sc_log2 = 0.25f * kLog2e / sqrtf((float)kD);      // 1/4: the query fragments carry a factor 4
+  const float sc_log2 = kLog2e / sqrtf((float)kD);
   uint32_t magic = kMagic;
   asm volatile("" : "+v"(magic));
   auto load_tile_raw = [&](int T, const LaneOffs& offs, auto& r) __attribute__((always_inline)) { load_raw(kv_page_uniform(A.kv, kvh, T << 5), (T << 5) % kPageTok, offs, r); };

@@ -18,18 +18,18 @@ __device__ __forceinline__ uint32_t as_u32(h2 h) { return __builtin_bit_cast(uin
 constexpr uint32_t kMagic = 0x64006400u;  // two fp16 1024.0
 constexpr float kLog2e = 1.4426950408889634f;
 
-// 8 codes of one dword -> 4 half2 in element order [n0,n4 | n1,n5 | n2,n6 | n3,n7] holding n-8 for even nibbles and
-// 16(n-8) for odd ones, all exact.  The factor 16 is undone by the query fragment.
+// 8 codes of one dword -> 4 half2 in element order [n0,n4 | n1,n5 | n2,n6 | n3,n7] holding n-8, exactly: 1024 + n less 1032 for
+// even nibbles, (1024 + 16 n) / 16 less 72 for odd ones.
 // (w & mask) | magic written as a bit-field insert; `magic` (0x64006400, no bit inside either nibble mask) is kept opaque
 // to the optimizer so that the pair is selected as one and-or instruction
 __device__ __forceinline__ uint32_t nib(uint32_t w, uint32_t mask, uint32_t magic) { return (w & mask) | (magic & ~mask); }
 __device__ __forceinline__ void dq_dword_int(uint32_t w, h2* out, uint32_t magic) {
-  const h2 c1032 = {(_Float16)1032.f, (_Float16)1032.f}, c1152 = {(_Float16)1152.f, (_Float16)1152.f};
+  const h2 c1032 = {(_Float16)1032.f, (_Float16)1032.f}, c16 = {(_Float16)0.0625f, (_Float16)0.0625f}, c72 = {(_Float16)-72.f, (_Float16)-72.f};
   const uint32_t t = w >> 8;
   out[0] = as_h2(nib(w, 0x000f000fu, magic)) - c1032;
-  out[1] = as_h2(nib(w, 0x00f000f0u, magic)) - c1152;
+  out[1] = __builtin_elementwise_fma(as_h2(nib(w, 0x00f000f0u, magic)), c16, c72);
   out[2] = as_h2(nib(t, 0x000f000fu, magic)) - c1032;
-  out[3] = as_h2(nib(t, 0x00f000f0u, magic)) - c1152;
+  out[3] = __builtin_elementwise_fma(as_h2(nib(t, 0x00f000f0u, magic)), c16, c72);
 }
 
 // K codes for the score MFMA need no arithmetic at all: a nibble left in place in an otherwise zero fp16 is the
