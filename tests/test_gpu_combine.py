@@ -76,3 +76,26 @@ def test_stream_whose_share_spans_sets(native, oracle):
         for t, n in enumerate(lens):
             refs[t].append(k[t:t + 1], v[t:t + 1], n)
             assert_attn_close(out[t:t + 1], refs[t].attend_f32(q[t:t + 1], n, want_f32=True)[1], f"stream of {n}")
+
+
+@pytest.mark.parametrize("M", [1, 2, 5])
+@pytest.mark.parametrize("unrot", [0, 1])
+def test_row_without_a_softmax_is_zero(native, oracle, M, unrot):
+    """A cached key whose scale is infinite leaves query heads that score it above everything without a softmax: their rows are zeros,
+    with and without the inverse rotation, and the other KV heads' rows keep their bits."""
+    ctx = 3000
+    q, k, v, _, _, _ = oracle.make_inputs(9400 + M, ctx, M)
+    q[:, :6] = 1.0
+    k[77, 0] = 1.0                                              # codes 7 in every channel: the score of key 77 is +inf below
+    oc = oracle.Cache(3072)
+    oc.append(k, v, 0)
+    outs = []
+    for bits in (oc.ks[0, 77, 0], 0x7c00):
+        ks = oc.ks.copy()
+        ks[0, 77, 0] = bits
+        with native.KvCache(max_ctx=3072) as kv:
+            kv.set_opt(4, unrot)
+            kv.import_rows(0, 0, oc.kc[:, :ctx], ks[:, :ctx], oc.vc[:, :ctx], oc.vs[:, :ctx])
+            outs.append(kv.layer_call(0, q, None, None, ctx - M).view(np.uint16))
+    assert np.array_equal(outs[0][:, 6:], outs[1][:, 6:])
+    assert outs[0][:, :6].any() and not (outs[1][:, :6] & 0x7fff).any()

@@ -576,7 +576,6 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
     L += wl[j];
   }
   L = lane_rows(lane_row16(L, LaneAdd{}), LaneAdd{});
-  const float inv = L > 0.f ? 1.f / L : 0.f;       // a row that saw no key at all (a rejected row of a multi-stream pass)
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   auto add = [&](const uint4& row, float w) __attribute__((always_inline)) {
     const uint4 r = w != 0.f ? row : make_uint4(0, 0, 0, 0);
@@ -599,8 +598,8 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
   // The four split lanes of a wave: each fold halves what a lane holds, channels 8 i + 4 (g / 2) + 2 (g % 2) are left
   *reinterpret_cast<float2*>(&s_o[wave][c8 + 4 * (g >> 1) + 2 * (g & 1)]) = fold_rows(acc);
   __syncthreads();
-  float y = 0.f;
-  if (tid < kD) y = (s_o[0][tid] + s_o[1][tid] + s_o[2][tid] + s_o[3][tid]) * inv;
+  float y = 0.f;                                   // stays for a row that saw no key (a rejected row of a multi-stream pass) and one without a softmax (scores that are not finite)
+  if (tid < kD && L > 0.f) y = (s_o[0][tid] + s_o[1][tid] + s_o[2][tid] + s_o[3][tid]) * (1.f / L);
   if (A.unrot) {                                   // uniform over the grid
     // inverse signed Hadamard rotation over the row's 128 channels (threads 0..127 = two waves)
     y = wave_hadamard(y, tid);
