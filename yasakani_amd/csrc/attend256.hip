@@ -444,7 +444,10 @@ __global__ void __launch_bounds__(256, 2) attend256_kernel(Attend256Head H, Attn
 // split it is the last one once more: a branch a request was 8 to 12 changes of the lane mask and jumps) and the requests of the new
 // keys in front, whose answers take two more barriers: one token at 20,011 246.2 / 241.0, at 2,000 150.3 / 145.2, 24 rows at 9,001
 // 329.0 / 326.3; 5-bit rows, one token at 16,001 266.0 / 256.4 (259.5 with the rows of the partials in front of what is picked
-// from), at 300 201 / 192, two at 3,000 212.5 / 204.3, 16 at 16,384 670 / 667.3.
+// from), at 300 201 / 192, two at 3,000 212.5 / 204.3, 16 at 16,384 670 / 667.3.  With two sets the compiler then spread the requests over
+// several trips until it was held to one (all_requested; two KV heads, one token at 20,000 164.2 / 162.3).  One set with K = 4 is one trip by
+// itself; with K = 8 two rows of eight are asked for behind the first answers, which measures the same, and four sets take longer in one
+// trip than in the compiler's several (one KV head at 20,000 171.0 / 173.1).
 // KB != 0: partials of launch_tb_encode_attend, which leave out the rows of the pass; token t also sees the keys *d_pos +
 // u, u <= t, which join the sum as splits of one key each, in fp32 (thread = channel; N names the rows).  The searches have
 // left what the rows may be coded with: wave 2 u + v of a workgroup picks the code of the K (v = 0) or V row of token u,
@@ -482,8 +485,8 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
   // Half h of wave w takes splits 8 K j + 4 K h + K w + k, k < K, of set j, 8 channels a lane.  A stream may hold any number of
   // sets: its weights go through LDS, thread t looking at split t.  Otherwise both rows of 16 lanes of a half look at the
   // (m, l) of the half's 4 K splits, the wave's own first: every wave finds the maximum and the sum of the weights by itself
-  // and has the weight of its k-th split in lane k of either row.  Rows and (m, l) are requested together: one memory round
-  // trip.  A row of weight 0 may be one that no workgroup wrote: it is zeroed before use.
+  // and has the weight of its k-th split in lane k of either row.  No request needs another's answer.  A row of weight 0 may be one that
+  // no workgroup wrote: it is zeroed before use.
   const int first = 4 * K * half + K * wave, last = MS ? max(A.S - 1, 0) : A.S - 1;    // a split past the last asks for the last once more
   const uint16_t* src = A.pacc16 + p0 * kD2 + c8;
   const uint32_t stride = (uint32_t)A.n_heads * kD2 * 2;
@@ -498,15 +501,26 @@ __global__ void __launch_bounds__(256) combine256_kernel(CombineArgs A, NewKeyAr
       }
   };
   constexpr int LOOK = MS ? 1 : SETS * K / 4;
+  constexpr bool HOLD = KB == 0 && SETS == 2;      // to one trip, see above
   float pmv[LOOK], plv[LOOK];
+  auto split_of = [&](int n) __attribute__((always_inline)) {
+    return MS ? tid : 8 * K * (n / (K / 4)) + 4 * K * half + ((16 * (n % (K / 4)) + (lane & 15) + K * wave) & (4 * K - 1));
+  };
 #pragma unroll
   for (int n = 0; n < LOOK; ++n) {
-    const int sp = MS ? tid : 8 * K * (n / (K / 4)) + 4 * K * half + ((16 * (n % (K / 4)) + (lane & 15) + K * wave) & (4 * K - 1));
+    const int sp = split_of(n);
     const uint32_t e = (uint32_t)min(sp, last) * A.n_heads;
     const float m1 = A.pm[p0 + e], l1 = A.pl[p0 + e];
-    pmv[n] = sp < A.S ? m1 : -1e30f; plv[n] = sp < A.S ? l1 : 0.f;
+    pmv[n] = HOLD || sp < A.S ? m1 : -1e30f; plv[n] = HOLD || sp < A.S ? l1 : 0.f;
   }
+  if constexpr (HOLD) all_requested();
   request(0);
+  if constexpr (HOLD) {
+    all_requested();
+#pragma unroll
+    for (int n = 0; n < LOOK; ++n)
+      if (split_of(n) >= A.S) { pmv[n] = -1e30f; plv[n] = 0.f; }
+  }
   float new_s[2] = {-1e30f, -1e30f}, new_v[2] = {0.f, 0.f};       // score in log2 units and V value (channel tid) of the new keys
   bool seen[2] = {false, false};               // uniform over the workgroup
   float ksc[2] = {0.f, 0.f};

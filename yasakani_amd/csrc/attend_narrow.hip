@@ -506,14 +506,17 @@ void launch_attend_narrow(const AttnArgs& A, hipStream_t st) {
 
 // combiner (reference: src/attention_kv4q.cu:325-332): M2 = max pm; w_s = pm_s > -1e29 ? 2^(pm_s - M2) * pl_s : 0;
 // y = sum w_s * (acc_s / l_s) / sum w_s.  grid (n_heads, M), block 256: 16 lanes x 8 channels cover a row, 16 split lanes
-// run in parallel.  S <= 64 * SETS; SETS sets of 64 splits are requested in one memory round trip.
+// run in parallel.  S <= 64 * SETS.
 // What it costs is a launch, that trip and a serial chain of a few hundred instructions, so the chain is what counts: every
 // wave finds maximum and weights by itself (a row's weights are in its own 16 lanes, read by row broadcasts), the four split lanes
 // of a wave are folded in registers (fold_rows), and one barrier is left where weights and sums through LDS took three.  us
 // per 16 layers, before / since: one token at 1,003 tokens 113.7 / 110.4, at 32,741 166.3 / 163.5, 8 rows at 12,037 tokens
 // 221.5 / 216.2; 4 layers of one token at 262,100 (128 splits, two sets) 135.0 / 134.7.  Requests without a branch of their own (a
 // split past the last asks for the last once more, weight 0), here and in the rows form below: 109.0 / 106.5, 158.4 / 156.3, 203.0 /
-// 201.7; 32 rows at 3,000 257.7 / 254.5.
+// 201.7; 32 rows at 3,000 257.7 / 254.5.  With four sets the compiler then asked for two to seven rows at a time, with waits in between,
+// until it was held to one trip (all_requested; 16 layers of one KV head at 20,000 tokens 119.2 / 116.7, 8 layers at 100,000 82.9 / 81.4).  With
+// one set it is one by itself; with two, two rows of eight are asked for behind the first answers, and held to one trip the kernel
+// takes longer (two KV heads at 20,000 tokens 123.7 / 125.0).
 // MS: a stream's share of the splits may exceed what is in flight at once (a loop over sets; 256 splits at most).
 // ADAPT: rows of a prefill slice that the rows form below does not take (inverse rotation, or more than 32 splits); as many
 // workgroups as the chip holds at once, each walks its share of the tokens, so that the choice of the splits is made 8
@@ -540,8 +543,8 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
   const size_t p0 = pair0 * A.n_heads + head;                  // split s lives at p0 + s * n_heads
   // Lane (g, i) of wave w takes channels 8 i .. 8 i + 7 of splits 64 j + 16 g + 4 w + k, k = 0 .. 3, and looks at the (m, l)
   // of split 64 j + 16 g + (i + 4 w) % 16: every wave finds the maximum and the sum of the weights by itself, and the weight
-  // of its k-th split is the one lane k of its row of 16 holds.  Rows and (m, l) are requested together: one memory round
-  // trip.  A row of weight 0 may be one that no workgroup wrote: it is zeroed before use.
+  // of its k-th split is the one lane k of its row of 16 holds.  No request needs another's answer.  A row of weight 0 may be one that no
+  // workgroup wrote: it is zeroed before use.
   const int first = 16 * g + 4 * wave, look = 16 * g + ((i + 4 * wave) & 15), last = MS ? max(A.S - 1, 0) : A.S - 1;
   const uint16_t* src = A.pacc16 + p0 * kD + c8;
   const uint32_t stride = (uint32_t)A.n_heads * kD * 2;
@@ -556,15 +559,23 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
         u[j][k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(src) + (uint32_t)min(sp, last) * stride);
       }
   };
+  constexpr bool HOLD = SETS == 4;                 // to one trip, see above
   float m[LOOK], wl[LOOK];
 #pragma unroll
   for (int j = 0; j < LOOK; ++j) {
     const int sp = 64 * j + look;
     const uint32_t e = (uint32_t)min(sp, last) * A.n_heads;
     const float m1 = A.pm[p0 + e], l1 = A.pl[p0 + e];
-    m[j] = sp < A.S ? m1 : -1e30f; wl[j] = sp < A.S ? l1 : 0.f;
+    m[j] = HOLD || sp < A.S ? m1 : -1e30f; wl[j] = HOLD || sp < A.S ? l1 : 0.f;
   }
+  if constexpr (HOLD) all_requested();
   request(0);
+  if constexpr (HOLD) {
+    all_requested();
+#pragma unroll
+    for (int j = 0; j < LOOK; ++j)
+      if (64 * j + look >= A.S) { m[j] = -1e30f; wl[j] = 0.f; }
+  }
   float M2 = m[0];
 #pragma unroll
   for (int j = 1; j < LOOK; ++j) M2 = fmaxf(M2, m[j]);
@@ -618,8 +629,9 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
 }
 // The combiner for wide passes (many rows, at most 32 splits, no un-rotation): one wave per (token, head) row, four
 // waves per workgroup, no LDS and no barrier.  Lane = (split lane 0..3, 8 channels); a split lane takes splits sl, sl + 4,
-// ... (at most 8), requests their rows together with the (m, l) pairs, and the four split lanes are summed by two
-// cross-lane exchanges.  Same arithmetic as combine_kernel up to the order of the sums.
+// ... (at most 8), requests their rows together with the (m, l) pairs - one trip, to which all_requested holds the compiler: it had
+// asked for l behind the answers (16 layers of 32 rows at 12,000 tokens 305.3 / 300.6 us, of 64 at 32,768 675.3 / 673.0, 8 layers of 1,000
+// at 9,000 1,366.6 / 1,361.7) - and the four split lanes are summed by two cross-lane exchanges.  Same arithmetic as combine_kernel up to the order of the sums.
 // ADAPT: rows of a prefill slice; 4 workgroups per CU, each walks its share - most slices on short contexts find nothing to do
 // here and should not pay for dispatching thousands of workgroups to find out.  A trip to memory stands in front of every
 // step, so with few splits a wave takes 2, 4 or 8 rows in one.  us, 16 layers, 8 workgroups per CU and one row a step / 4 and up to 8
@@ -651,6 +663,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args
         for (int k = 0; k < KN; ++k)
           u[r][k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(A.pacc16 + p0 * kD + c8) + (uint32_t)min(sl + 4 * k, A.S - 1) * stride);
       }
+      all_requested();
 #pragma unroll
       for (int r = 0; r < RB; ++r) {
         const float M2 = lane_rows(lane_row16(pmv[r], LaneMax{}), LaneMax{});

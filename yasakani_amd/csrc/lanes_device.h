@@ -49,6 +49,12 @@ struct LaneMin { __device__ __forceinline__ int operator()(int a, int b) const {
 struct LaneAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
 // over the four lanes l, l ^ 16, l ^ 32, l ^ 48
 template <class T, class Op> __device__ __forceinline__ T lane_rows(T v, Op op) { return lane_op32(lane_op16(v, op), op); }
+// Stands between the last request of a step and the first use of an answer: left to itself the compiler moves requests behind uses of
+// earlier ones to save registers, which makes one trip to memory two or more.
+__device__ __forceinline__ void all_requested() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 // Sums of eight values over lanes l and l ^ 32, shared out: a swap of a register's half with another's leaves in either half what
 // the other needs, so that a fold halves the registers.  The lower half ends with the sums of v[0 .. 3], the upper with v[4 .. 7].
 __device__ __forceinline__ float4 fold_halves(const float (&v)[8]) {

@@ -29,7 +29,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-featu
          "-S", "--cuda-device-only"]
 # as in the library's Makefile
 PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
-EXTRA = {"attend_mid.hip": PRELOAD + ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "attend_narrow.hip": PRELOAD}
+EXTRA = {"attend_mid.hip": PRELOAD + ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "attend_narrow.hip": PRELOAD, "attend256.hip": PRELOAD + ["-ffp-contract=off"]}
 
 VMEM = re.compile(r"^(global|buffer|scratch|flat)_(load|store|atomic)")
 REG = re.compile(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b")
