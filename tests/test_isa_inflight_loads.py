@@ -2,7 +2,9 @@
 them is in flight, results of hand-written matrix instructions touched before their passes are through: the checker itself
 on small hand-made listings, then the library's sources."""
 import os
+import re
 import shutil
+import subprocess
 
 import pytest
 
@@ -84,3 +86,14 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
     seen, problems = isa_check.check_sources(str(tmp_path))
     assert seen >= 5 * 2 * 14, "the hand-written loads were not found: the check looked at nothing"
     assert not problems, "\n".join(problems[:40])
+
+
+@pytest.mark.skipif(shutil.which(isa_check.HIPCC) is None and not os.path.exists(isa_check.HIPCC), reason="hipcc not found")
+@pytest.mark.parametrize("src,kernels", [("attend_mid.hip", 5), ("attend_tb_wide.hip", 4)])
+def test_kernels_short_of_registers_spill_none(tmp_path, src, kernels):
+    """a spilled register is copied where the compiler likes, beside loads in flight"""
+    out = str(tmp_path / "a.s")
+    subprocess.run([isa_check.HIPCC, *isa_check.FLAGS, *isa_check.EXTRA.get(src, []), src, "-o", out], cwd=isa_check.CSRC, check=True)
+    with open(out) as f:
+        spilled = re.findall(r"\.vgpr_spill_count: +(\d+)", f.read())
+    assert spilled == ["0"] * kernels

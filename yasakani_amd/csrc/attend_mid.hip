@@ -73,6 +73,10 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(WindowHead head_args
   constexpr int kStage = NRT <= 4 ? NRT : 2;
   __shared__ __align__(16) float s_acc[kStage][4][kAccWave];
   __shared__ float s_m[NRT][4][16], s_l[NRT][4][16];
+  // six row tiles leave no register for the rows' lengths: spilled, they are copied beside tile loads in flight.  From LDS they cost the
+  // narrower windows 1 % (16 layers of 3 rows at 2,000 tokens 142.1 us, 143.6 so)
+  constexpr bool kLenLds = NRT > 5;
+  __shared__ int s_len[kLenLds ? NRT : 1][16];
   const int split = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -141,6 +145,9 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(WindowHead head_args
     maxlen = max(maxlen, lenr[rt]);
     if (v) minlen = min(minlen, lenr[rt]);
   }
+  if (kLenLds && wave == 0 && g == 0)
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt) s_len[kLenLds ? rt : 0][i] = lenr[rt];
   maxlen = lane_row16(maxlen, LaneMax{}); minlen = lane_row16(minlen, LaneMin{});
   maxlen = __builtin_amdgcn_readfirstlane(maxlen); minlen = __builtin_amdgcn_readfirstlane(minlen);
 
@@ -314,7 +321,7 @@ __global__ void __launch_bounds__(256, 1) attend_mid_kernel(WindowHead head_args
         }
       if (need_mask) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) { const int key = t0 + tau(g, k); e[k] = key < lenr[rt] ? e[k] : -INFINITY; }
+        for (int k = 0; k < 8; ++k) { const int key = t0 + tau(g, k); e[k] = key < (kLenLds ? s_len[rt][i] : lenr[rt]) ? e[k] : -INFINITY; }
       }
       // online softmax with a lazily raised maximum: the row's offset only moves when a score exceeds it by more than
       // 2^kRaiseMid (or on the row's first keys), so the accumulators are rescaled on almost no tile
