@@ -36,22 +36,39 @@ def test_decode_splits_around_a_set(native, oracle, M, ctx, S):
     assert np.linalg.norm(back - want) <= (1e-3 + 2.0 ** -11) * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("M,ctx,splits", [(301, 200, 3), (65, 500, 7), (65, 1000, 10), (65, 8000, 27)])
-def test_slice_splits_of_every_size(native, oracle, M, ctx, splits):
-    """One KV head: 3 splits are merged 8 rows at a time (1,806 rows: 6 at the end), 7 four at a time (390: 2 at the end), 10 and 27."""
-    def price(s):                                               # chunk_price of the device, in Python
-        base = (6 * M + 127) // 128
+def _slice_plan(kvh, M, ctx, capacity):
+    """Splits the device uses for a slice (chunk_splits of the host, chunk_price of the device, in Python) and rows its combiner takes a step."""
+    base = kvh * ((6 * M + 127) // 128)
+
+    def launched(m):
+        b = kvh * ((6 * m + 127) // 128)
+        fill = lambda s: b * s / (256.0 * ((b * s + 255) // 256)) - 0.005 * s
+        return max(range(1, max(1, min(32, 12288 // m, capacity // 256, 2048 // b)) + 1), key=lambda s: (fill(s), -s))
+
+    def price(s):
         lo, hi = ((ctx + min(M, 22) + 31) // 32 * 16 // s + 288), ((ctx + M + 31) // 32 * 16 // s + 288)
         n = base * s
         idle = (256 - (n & 255)) & 255
         t = max(hi, (n >> 1) * (lo + hi) // 256 + lo * idle // 256)
         return t + 96 + M * s // 13 if s > 1 else t
-    launched = 32 if M == 65 else 17
-    assert min(range(1, launched + 1), key=lambda s: (price(s), s)) == splits
-    q, k, v, kn, vn, _ = oracle.make_inputs(9300 + splits, ctx, M, 6, 1)
-    oc = oracle.Cache(8192, 6, 1)
+
+    splits = min(range(1, launched(M) + 1), key=lambda s: (price(s), s))
+    rows = 6 * kvh * M
+    most = (rows - 1) // (2 * min((rows + 3) // 4, 1024))
+    return splits, 8 if splits <= 4 and most >= 8 else 4 if splits <= 8 and most >= 4 else 2 if splits <= 16 and most >= 2 else 1
+
+
+@pytest.mark.parametrize("kvh,M,ctx,splits,step", [(1, 301, 200, 3, 1), (1, 65, 500, 7, 1), (1, 65, 1000, 10, 1), (1, 65, 8000, 27, 1),
+                                                   (1, 682, 1000, 4, 1), (1, 683, 1000, 4, 2), (3, 229, 1000, 6, 2), (1, 1365, 1000, 3, 2),
+                                                   (1, 1371, 1000, 3, 4), (2, 1365, 1300, 2, 4), (2, 1371, 1300, 3, 8)])
+def test_slice_splits_of_every_size(native, oracle, kvh, M, ctx, splits, step):
+    """Slices of 2 to 27 splits; the combiner takes 1, 2, 4 or 8 rows a step, by splits and number of rows, both sides of every line (8,226
+    rows in fours and 16,452 in eights leave 2 and 4 at the end)."""
+    assert _slice_plan(kvh, M, ctx, 8192) == (splits, step)
+    q, k, v, kn, vn, _ = oracle.make_inputs(9300 + splits, ctx, M, 6 * kvh, kvh)
+    oc = oracle.Cache(8192, 6 * kvh, kvh)
     oc.append(k, v, 0)
-    with native.KvCache(max_ctx=8192, n_heads=6, n_kv_heads=1, max_rows=M) as kv:
+    with native.KvCache(max_ctx=8192, n_heads=6 * kvh, n_kv_heads=kvh, max_rows=M) as kv:
         kv.import_rows(0, 0, oc.kc[:, :ctx], oc.ks[:, :ctx], oc.vc[:, :ctx], oc.vs[:, :ctx])
         kv.poison_workspace()
         out = kv.layer_call(0, q, kn, vn, ctx)

@@ -636,7 +636,10 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
 // here and should not pay for dispatching thousands of workgroups to find out.  A trip to memory stands in front of every
 // step, so with few splits a wave takes 2, 4 or 8 rows in one.  us, 16 layers, 8 workgroups per CU and one row a step / 4 and up to 8
 // rows: 1,500 rows on an empty cache 660 / 653.8, 1,000 at 9,000 tokens 2,778 / 2,724; 2 layers of 2,048 at 131,072 7,610 / 7,575.  2
-// per CU: 651.8, 2,767, 7,590; one row a step with 4 per CU: 654, 2,815.
+// per CU: 651.8, 2,767, 7,590; one row a step with 4 per CU: 654, 2,815.  No more rows a step than leave at most half of the waves
+// without any: where the rows are few, fewer a step on more waves are faster.  4 layers, as many rows a step as eight pieces hold / so: one
+// KV head, 400 rows at 500 tokens 86.8 / 75.0 us, 1,500 on an empty cache 120.0 / 112.9; four, 400 at 500 109.7 / 102.6 (2 a step), 700 at
+// 500 131.2 / 130.7 (8 either way).
 template <bool ADAPT>
 __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args, CombineTail tail_args) {
   CombineArgs A = combine_args(head_args, tail_args);
@@ -692,9 +695,10 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args
       }
     }
   };
-  if (ADAPT && A.S <= 4) walk(std::integral_constant<int, 1>{});
-  else if (ADAPT && A.S <= 8) walk(std::integral_constant<int, 2>{});
-  else if (ADAPT && A.S <= 16) walk(std::integral_constant<int, 4>{});
+  const int most = ADAPT ? (total - 1) / (2 * (int)gridDim.x) : 1;         // rows a step, see above
+  if (ADAPT && A.S <= 4 && most >= 8) walk(std::integral_constant<int, 1>{});
+  else if (ADAPT && A.S <= 8 && most >= 4) walk(std::integral_constant<int, 2>{});
+  else if (ADAPT && A.S <= 16 && most >= 2) walk(std::integral_constant<int, 4>{});
   else walk(std::integral_constant<int, 8>{});
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
