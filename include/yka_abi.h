@@ -25,7 +25,9 @@
  *        page table / append / attend / append_attend / layer_call_host / append_host / replicate / captured passes /
  *        attn_bench work on it; its canonical image goes through yka_kv_export_rows256 / yka_kv_import_rows256; the
  *        other entry points return an error.
- * Q, new K/V and outputs are fp16 bit patterns, [rows][heads][head_dim].
+ * Q, new K/V and outputs are fp16 bit patterns, [rows][heads][head_dim].  All of them are finite.  Over 128-channel rows, decode passes (at
+ * most 2 rows, multi-stream passes, option key 3) take query channels up to 16,376 (they are multiplied by 4 or 1/4 in fp16, so odd
+ * channels also lose what lies below 2^-22); every other pass takes the whole fp16 range.
  */
 #ifndef YKA_ABI_H
 #define YKA_ABI_H

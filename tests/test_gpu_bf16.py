@@ -90,11 +90,13 @@ def test_post_step_writes_gate_rows(native, oracle, head_dim, bf):
         assert np.array_equal(a, b)
 
 
-@pytest.mark.parametrize("form,M", [("128", 2), ("128", 3), ("128", 10), ("128", 11), ("128", 65), ("128 streams", 5), ("256", 2), ("256", 3), ("256", 16), ("256", 17), ("256", 32),
+@pytest.mark.parametrize("form,M", [("128", 2), ("128", 3), ("128", 8), ("128", 9), ("128", 10), ("128", 11), ("128", 16), ("128", 17),
+                                    ("128", 21), ("128", 22), ("128", 64), ("128", 65), ("128 streams", 5), ("256", 2), ("256", 3), ("256", 16), ("256", 17), ("256", 32),
                                     ("256", 33), ("256 streams", 5), ("kv5", 1), ("kv5", 3), ("kv4", 2), ("kv4", 16), ("kv5", 16), ("kv5", 17), ("kv4", 64),
                                     ("kv5 streams", 3)])
 def test_bf16_rows_are_read_as_their_fp16_rounding(native, form, M):
-    """Every kernel that reads 16-bit rows (one case per kernel and at the row counts where the dispatch changes): bf16 rows
+    """Every kernel that reads 16-bit rows (one case per kernel and at the row counts where the dispatch changes; 128 channels: mid
+    kernel from 3 rows, wide kernel from 9, in blocks of four waves of rows at 17 .. 21 and 64, slices from 65): bf16 rows
     give what their values rounded to fp16 give - the cache bit for bit, fp16 subnormals and roundings included - and the
     same fp32 outputs rounded to bf16 instead of fp16."""
     from yasakani_amd import kvqp

@@ -71,8 +71,8 @@ def test_seeded_randomized_sweep(native, oracle):
 @pytest.mark.parametrize("M", [1, 2, 8, 16, 64, 130])
 def test_large_magnitudes(native, oracle, M):
     """Every kernel at the far end of the fp16 range: K rows of magnitude up to 6e4 (group scales up to 9e3), V rows of
-    magnitude up to 3e4, small queries so that the scores still discriminate.  The scaled K images of the mid kernel, the
-    exact codes x fp32 scales of the other two and the scaled V images all have to stay finite and exact."""
+    magnitude up to 3e4, small queries so that the scores still discriminate.  The exact K codes x fp32 scales and the scaled
+    V images all have to stay finite and exact."""
     rng = np.random.default_rng(8800 + M)
     ctx = 600
     k = np.clip(rng.standard_normal((ctx + M, 4, 128)) * 9000.0, -60000, 60000).astype(np.float16)
