@@ -135,8 +135,8 @@ int narrow_splits(const yka_kv* kv, int M, size_t ws_pairs = kWsPairs) {
 // tiles of the split and merge on chip), one workgroup per compute unit.  Splits: one workgroup per CU (256 of them), at
 // least four 32-key tiles (two steps of either group) per workgroup, sized like the decode grid by the expected context.
 // At 64 rows (three row blocks) that is 21 splits: 64 x 21 x 24 partial rows of 264 bytes, 8.5 MB.
-// The blocks of a window get the same number of waves of 32 rows: 144 rows are 96 + 48 and not 128 + 16 (figures at the roles in
-// attend_wide.hip).
+// The blocks of a window are cut at the even share of its rows rounded up to whole waves of 32: no block has more waves of rows than that, the last
+// may have fewer (144 rows are 96 + 48 and not 128 + 16, 132 are 96 + 36; figures at the roles in attend_wide.hip).
 int wide_rows_per_block(int M) {
   const int rows = kG * M, rb = (rows + 127) / 128;
   return M > kMaxSlice ? 128 : ((rows + rb - 1) / rb + 31) / 32 * 32;

@@ -216,7 +216,7 @@ typedef uint32_t Attend256Head __attribute__((ext_vector_type(8)));   // positio
 // TPT = 2 for a single-stream pass; MS (multi-stream pass, reference: src/q35_atxpk_ms.cu:13-33): one token per row tile,
 // which reads the container and the position its row map names.
 // In front of the first score stand three trips to memory (kernel arguments, position, tile): the head brings what the first loads
-// need with the wave, the query rows are asked for beside the position (stage_q256), the first tile behind them.  16 layers of one
+// need with the wave, the query rows are asked for beside the position (stage_q256), the first tile behind their answers.  16 layers of one
 // token at 32,745 tokens 252.1 -> 244.0 us, at 2,000 150.3 -> 149.2; two tokens at 5,000 177.5 -> 175.7; 4 layers at 100,000 114.0 -> 108.9.
 template <bool MS>
 __global__ void __launch_bounds__(256, 2) attend256_kernel(Attend256Head H, AttnArgs A) {
@@ -648,8 +648,8 @@ void launch_attend256(const AttnArgs& A, hipStream_t st) {
   else hipLaunchKernelGGL(attend256_kernel<false>, dim3(A.S, A.kv.n_kv, (A.M + 1) / 2), dim3(256), 0, st, H, A);
 }
 void launch_combine256(const CombineArgs& A, hipStream_t st) {
-  // a stream may hold any share of the splits (256 at most, in batches of 8 * kInFlight).  5 streams of up to 3,000 tokens, us a
-  // pass: 15.2 with 16 in flight (and 198 registers), 12.4 with 4 and splits of 4 tiles.
+  // Streams walk sets of 8 K splits, whatever share of them a stream holds (256 at most); other passes need S <= 8 * K * SETS.  5 streams
+  // of up to 3,000 tokens, us a pass: 15.2 with K = 16 (and 198 registers), 12.4 with 4 and splits of 4 tiles.
   if (A.plan) {
     if (A.M < 4) hipLaunchKernelGGL((combine256_kernel<8, 1, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});
     else hipLaunchKernelGGL((combine256_kernel<4, 1, true, 0>), dim3(A.n_heads, A.M), dim3(256), 0, st, A, NewKeyArgs<0>{});

@@ -116,7 +116,6 @@ __device__ __forceinline__ void attend_tb_body(TbAttnArgs A, const int bx, const
   }
   const int tl = TPT * rt + i / kG;
   const bool vrow = i < TPT * kG && tl < A.M && row_ok;
-  const int head = kvh * kG + i % kG;
   if constexpr (MS) request_q(min(rt, A.M - 1), 1);
   int dep = A.tok0 + tl;
   if (!MS && !cached && A.depth) {                   // uniform over the grid

@@ -9,9 +9,9 @@
 //     split of the keys.  The waves form two groups of four; group g walks the tiles tile0 + g, tile0 + g + 2, ... of
 //     the split, each with its own softmax state, and the two states are merged through LDS at the end: one partial
 //     row per (row, split), half as many splits as workgroups of four waves would need to fill the chip;
-//   * a group dequantizes each of its 32-key tiles ONCE into LDS - K as exact integer codes in fp16 (n-8, odd nibbles
-//     16(n-8)), V scaled and transposed (channel-major, the operand shape of the token-contracting MFMA) - and every
-//     wave of the group reads its MFMA fragments from there;
+//   * a group dequantizes each of its 32-key tiles ONCE into LDS - K as exact integer codes n-8 in fp16, V scaled
+//     and transposed (channel-major, the operand shape of the token-contracting MFMA) - and every wave of the group reads
+//     its MFMA fragments from there;
 //   * a wave owns one tile of 32 rows (MFMA 32x32x16: one K or V fragment read from LDS serves 32 rows) and stays
 //     under 256 registers, so the two waves of a SIMD (one of each group) fit and all MFMA results live in ordinary
 //     VGPRs (no accumulator-file copies);
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
   };
   // Who decodes: a quarter each, or, in a window whose blocks have rows for at most three waves of a group, the waves without rows:
   // all four quarters by one of them or two by each of two; the waves with rows then only compute.  us per 16 layers, a quarter
-  // by every wave in blocks of 128 rows / so, in blocks of the same number of waves: 24 rows (128 + 16, 96 + 48) at 30,000 tokens
+  // by every wave in blocks of 128 rows / so, in blocks cut at the even share rounded up to whole waves: 24 rows (128 + 16, 96 + 48) at 30,000 tokens
   // 454.5 / 427, with a tree at 9,000 283.6 / 268, 48 (128 + 128 + 32, three of 96) at 9,000 337.5 / 326.3, 16 at 30,000 338 / 328, 11 at
   // 5,000 203.5 / 200.5, 32 at 12,000 312 / 306.  One kernel for both was 1.5 % slower on blocks of four waves.
   const int computing = (min(nrows, (rb + 1) * RPB) - rb * RPB + 31) >> 5, feeder = wave - computing;

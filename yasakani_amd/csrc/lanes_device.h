@@ -109,7 +109,8 @@ __device__ __forceinline__ float wave_hadamard(float a, int lane) {
   a = lane_hadamard<1>(a, lane); a = lane_hadamard<2>(a, lane); a = lane_hadamard<4>(a, lane);
   a = lane_hadamard<8>(a, lane); a = lane_hadamard<16>(a, lane); return lane_hadamard<32>(a, lane);
 }
-// over a row of 16 lanes; op is a maximum or minimum (after two steps a quad holds one value, so the mirrored octet is lane ^ 4)
+// over a row of 16 lanes (after two steps a quad holds one value, so the mirrored octet is lane ^ 4); the lanes of a row end with one
+// value, sums included: every step adds the same two partial sums in either lane
 template <class T, class Op>
 __device__ __forceinline__ T lane_row16(T v, Op op) {
   v = op(v, lane_xor1(v));

@@ -94,8 +94,8 @@ struct CombineArgs { const float* pm; const float* pl; const uint16_t* pacc16; i
 // and are compiled with -amdgpu-kernarg-preload-count: those arrive in scalar registers with the wave, and the position
 // (the combiner's partials) is asked for at once instead of 0.3 us later, behind the load of the argument block.  us per 16
 // layers without / with: one token at 32,741 tokens 172.5 / 166.5, one 5-bit trellis row at 16,001 382 / 371, 8 rows at
-// 12,037 (the combiner alone) 226 / 220, one token at 1,003 115.4 / 113.8, 16 streams 27.1 / 26.7 a pass.  Not where it
-// measured nothing: the combiner of 256-channel rows.
+// 12,037 (the combiner alone) 226 / 220, one token at 1,003 115.4 / 113.8, 16 streams 27.1 / 26.7 a pass.  The combiner
+// of 256-channel rows takes its arguments as one block: split, it measured the same.
 // In the int4 decode kernel and the combiners such a pointer travels as an integer, and the combiners' arguments are split
 // into head and tail, not repeated: a pointer among a launch's arguments costs the host 0.2 us, and the 136 bytes of a
 // repeated block 0.45 us more than these 96.  A call issued outside a graph is as long as the host takes; 16 layers of one
