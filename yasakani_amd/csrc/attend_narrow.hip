@@ -633,13 +633,12 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
 // asked for l behind the answers (16 layers of 32 rows at 12,000 tokens 305.3 / 300.6 us, of 64 at 32,768 675.3 / 673.0, 8 layers of 1,000
 // at 9,000 1,366.6 / 1,361.7) - and the four split lanes are summed by two cross-lane exchanges.  Same arithmetic as combine_kernel up to the order of the sums.
 // ADAPT: rows of a prefill slice; 4 workgroups per CU, each walks its share - most slices on short contexts find nothing to do
-// here and should not pay for dispatching thousands of workgroups to find out.  A trip to memory stands in front of every
-// step, so with few splits a wave takes 2, 4 or 8 rows in one.  us, 16 layers, 8 workgroups per CU and one row a step / 4 and up to 8
-// rows: 1,500 rows on an empty cache 660 / 653.8, 1,000 at 9,000 tokens 2,778 / 2,724; 2 layers of 2,048 at 131,072 7,610 / 7,575.  2
-// per CU: 651.8, 2,767, 7,590; one row a step with 4 per CU: 654, 2,815.  No more rows a step than leave at most half of the waves
-// without any: where the rows are few, fewer a step on more waves are faster.  4 layers, as many rows a step as eight pieces hold / so: one
-// KV head, 400 rows at 500 tokens 86.8 / 75.0 us, 1,500 on an empty cache 120.0 / 112.9; four, 400 at 500 109.7 / 102.6 (2 a step), 700 at
-// 500 131.2 / 130.7 (8 either way).
+// here and should not pay for dispatching thousands of workgroups to find out (16 layers of 1,500 rows on an empty cache 637 us, with
+// 8 per CU 644).  A split lane asks for as many partials as there are splits for it, 1, 2, 4 or 8: eight whatever
+// their number cost as much as the row's own (4 layers of 300 rows at 2,000 tokens, one KV head, 7 splits 89.8 / 87.2 us; with eight KV heads 100 rows
+// there 101.5 / 98.3; 8 layers of 200 rows at 9,000, four heads, 364 / 355).  With few splits several rows a step, 8 / KN of them, measured
+// the same or took longer (4 layers, four KV heads, 800 rows at 2,000 tokens in 3 splits 231.0 / 221.6, 200 at 500 78.3 / 77.7; 2 splits of eight heads
+// alone gained, 800 rows at 2,000 409.5 / 411.7).
 template <bool ADAPT>
 __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args, CombineTail tail_args) {
   CombineArgs A = combine_args(head_args, tail_args);
@@ -649,56 +648,47 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args
   }
   const int lane = threadIdx.x & 63, sl = lane >> 4, c8 = (lane & 15) * 8, total = A.M * A.n_heads;
   const uint32_t stride = (uint32_t)A.n_heads * kD * 2;
-  // RB rows with KN partials a split lane, 8 pieces in flight: row = tok * n_heads + head
+  // KN partials a split lane: row = tok * n_heads + head
   auto walk = [&](auto kn_tag) __attribute__((always_inline)) {
-    constexpr int KN = decltype(kn_tag)::value, RB = 8 / KN;
-    for (int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RB; row0 < total; row0 += ADAPT ? 4 * (int)gridDim.x * RB : total) {
-      float pmv[RB], plv[RB];
-      uint4 u[RB][KN];
+    constexpr int KN = decltype(kn_tag)::value;
+    for (int row = blockIdx.x * 4 + (threadIdx.x >> 6); row < total; row += ADAPT ? 4 * (int)gridDim.x : total) {
+      uint4 u[KN];
       // lane t < S looks at split t; the maximum and every weight then come from cross-lane reads
+      const size_t p0 = (size_t)(row / A.n_heads) * A.S * A.n_heads + row % A.n_heads;
+      const uint32_t e = (uint32_t)min(lane, A.S - 1) * A.n_heads;
+      const float pmv = A.pm[p0 + e], plv = A.pl[p0 + e];
 #pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        const int row = min(row0 + r, total - 1);
-        const size_t p0 = (size_t)(row / A.n_heads) * A.S * A.n_heads + row % A.n_heads;
-        const uint32_t e = (uint32_t)min(lane, A.S - 1) * A.n_heads;
-        pmv[r] = A.pm[p0 + e]; plv[r] = A.pl[p0 + e];
-#pragma unroll
-        for (int k = 0; k < KN; ++k)
-          u[r][k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(A.pacc16 + p0 * kD + c8) + (uint32_t)min(sl + 4 * k, A.S - 1) * stride);
-      }
+      for (int k = 0; k < KN; ++k)
+        u[k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(A.pacc16 + p0 * kD + c8) + (uint32_t)min(sl + 4 * k, A.S - 1) * stride);
       all_requested();
+      const float M2 = lane_rows(lane_row16(pmv, LaneMax{}), LaneMax{});
+      const float wl = (lane < A.S && pmv > -1e29f) ? exp2f(pmv - M2) * plv : 0.f;     // weight of split `lane`
+      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      float wsum = 0.f;
 #pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        const float M2 = lane_rows(lane_row16(pmv[r], LaneMax{}), LaneMax{});
-        const float wl = (lane < A.S && pmv[r] > -1e29f) ? exp2f(pmv[r] - M2) * plv[r] : 0.f;     // weight of split `lane`
-        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        float wsum = 0.f;
+      for (int k = 0; k < KN; ++k) {
+        const float w = __shfl(wl, sl + 4 * k, 64);                        // < 32: a lane of this wave
+        const uint4 x = w != 0.f ? u[k] : make_uint4(0, 0, 0, 0);           // a row of weight 0 may be one that no workgroup wrote
+        const h8 v = __builtin_bit_cast(h8, x);
 #pragma unroll
-        for (int k = 0; k < KN; ++k) {
-          const float w = __shfl(wl, sl + 4 * k, 64);                        // < 32: a lane of this wave
-          const uint4 x = w != 0.f ? u[r][k] : make_uint4(0, 0, 0, 0);        // a row of weight 0 may be one that no workgroup wrote
-          const h8 v = __builtin_bit_cast(h8, x);
+        for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
+        wsum += w;
+      }
 #pragma unroll
-          for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
-          wsum += w;
-        }
+      for (int c = 0; c < 8; ++c) acc[c] = lane_rows(acc[c], LaneAdd{});
+      wsum = lane_rows(wsum, LaneAdd{});
+      if (sl == 0) {
+        const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+        float yv[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c] = lane_rows(acc[c], LaneAdd{});
-        wsum = lane_rows(wsum, LaneAdd{});
-        if (sl == 0 && row0 + r < total) {
-          const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-          float yv[8];
-#pragma unroll
-          for (int c = 0; c < 8; ++c) yv[c] = acc[c] * inv;
-          *reinterpret_cast<uint4*>(A.out16 + (size_t)(row0 + r) * kD + c8) = pack_out8(yv, A.out_bf16);
-        }
+        for (int c = 0; c < 8; ++c) yv[c] = acc[c] * inv;
+        *reinterpret_cast<uint4*>(A.out16 + (size_t)row * kD + c8) = pack_out8(yv, A.out_bf16);
       }
     }
   };
-  const int most = ADAPT ? (total - 1) / (2 * (int)gridDim.x) : 1;         // rows a step, see above
-  if (ADAPT && A.S <= 4 && most >= 8) walk(std::integral_constant<int, 1>{});
-  else if (ADAPT && A.S <= 8 && most >= 4) walk(std::integral_constant<int, 2>{});
-  else if (ADAPT && A.S <= 16 && most >= 2) walk(std::integral_constant<int, 4>{});
+  if (ADAPT && A.S <= 4) walk(std::integral_constant<int, 1>{});
+  else if (ADAPT && A.S <= 8) walk(std::integral_constant<int, 2>{});
+  else if (ADAPT && A.S <= 16) walk(std::integral_constant<int, 4>{});
   else walk(std::integral_constant<int, 8>{});
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
