@@ -33,9 +33,11 @@ def test_against_the_oracle(native, oracle, M, ctx, max_ctx, paged):
 
 
 # 2,049 and 2,100 rows: a second slice of 1 and 52 rows.  Option 4 (inverse rotation) and forced split counts keep the combiner.
+# 661 and 662 rows: one split gives 124 and 128 workgroups, both sides of the two forms of the kernel, with one split in use and with several.
 # Both sides round V and P to fp16 and sum in fp32 in another order: 1e-3 between them, two bf16 roundings (2^-8 each) on top.
 @pytest.mark.parametrize("M,ctx,opts", [(2049, 0, []), (2100, 4000, []), (1500, 0, [(4, 1)]), (1500, 2000, [(4, 1)]), (700, 9000, [(2, 5)]),
-                                        (333, 0, [(11, 1)]), (1500, 7000, [(11, 1)]), (90, 12000, [(10, 128)])])
+                                        (333, 0, [(11, 1)]), (1500, 7000, [(11, 1)]), (90, 12000, [(10, 128)]),
+                                        (661, 0, []), (662, 0, []), (661, 6000, [(11, 1)]), (662, 6000, [(11, 1)]), (661, 6000, []), (662, 6000, [])])
 def test_against_the_decode_kernel(native, M, ctx, opts):
     rng = np.random.default_rng(M + ctx)
     bf16 = (11, 1) in opts

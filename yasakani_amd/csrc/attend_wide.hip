@@ -200,6 +200,11 @@ __device__ __forceinline__ void scale_scores(float (&s)[16], const f16v& part, f
 // into the number of splits the length found on the device justifies (chunk_splits_used), the other workgroups exit.  A
 // slice that uses one split writes its output rows instead of partials.  While the keys of all kv heads fit one XCD's L2
 // the longest row blocks start first, spread over the XCDs (on a short context a block's length is its place in the slice).
+// FEW: a window whose blocks have three waves of rows at most (the roles below); a slice that one split would give less than half of the
+// CUs a workgroup: it mostly uses several, and what the early request of the query adds is instructions fetched cold in front of everything
+// else.  us per 4 layers, with the early request / without: one KV head (15 workgroups), 300 rows at 2,000 tokens 86.0 / 80.6, four
+// (20), 100 rows there 87 / 84.2, four (40), 200 rows at 500 78.6 / 77.2, four (96), 500 first rows 81.4 / 81.0; per 8 layers, four (132), 700 first rows
+// 199.7 / 201.2, four (188), 1,000 first rows 242.2 / 245.5.
 template <bool BF, bool CHUNK, bool FEW>
 __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, WindowSizes size_args, WindowTail tail_args) {
   AttnArgs A = window_args(head_args, size_args, tail_args);
@@ -212,7 +217,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
   // once and goes through LDS.  us per 16 layers, before / since (loops aligned, see the Makefile): 64 rows at 32,768 tokens 700 / 682,
   // 1,500 rows on an empty cache 686 / 661, 24 tree rows at 9,000 305 / 286, 32 rows at 3,000 253.5 / 242.5, 12 at 3,000 233.2 / 229.
   // A slice asks for the rows this workgroup takes if the slice uses one split, which is known before the position (1,500 rows 656 / 643.7;
-  // 1,000 rows at 9,000 tokens, where it asks twice, 2,685 / 2,693).
+  // 1,000 rows at 9,000 tokens, where it asks twice, 2,685 / 2,693), unless it is FEW.
   uint4 qraw[4];
   auto request_q = [&](int b, int kvh_q) __attribute__((always_inline)) {
 #pragma unroll
@@ -222,7 +227,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
     }
   };
   const int rb_q = n_rb - 1 - min((int)blockIdx.x / A.kv.n_kv, n_rb - 1), kvh_one = (int)blockIdx.x % A.kv.n_kv;
-  if constexpr (CHUNK) request_q(rb_q, kvh_one);
+  if constexpr (CHUNK && !FEW) request_q(rb_q, kvh_one);
   const int pos = *A.d_pos;
   if constexpr (CHUNK) { if (A.adapt) A.S = chunk_splits_used(pos, A.tok0, A.M, A.kv.n_kv, A.kv.max_ctx, A.S, A.adapt); }
   const int total = CHUNK ? A.S * A.kv.n_kv * n_rb : (int)gridDim.x;
@@ -241,7 +246,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
     }
   }
   const int split = pair % A.S, kvh = pair / A.S;
-  if constexpr (CHUNK) { if (rb != rb_q || kvh != kvh_one) request_q(rb, kvh); } else request_q(rb, kvh);
+  if constexpr (CHUNK && !FEW) { if (rb != rb_q || kvh != kvh_one) request_q(rb, kvh); } else request_q(rb, kvh);
   const int gt = tid & (NTG - 1);                  // gt: thread index inside the group
   const int grp = __builtin_amdgcn_readfirstlane(tid >> 8);           // wave uniform
   // waves w and w + 4 share a SIMD: group 1 counts its rows from the third wave, so that in a block of up to 64 rows no SIMD has two
@@ -534,7 +539,7 @@ __global__ void __launch_bounds__(NT) attend_wide_kernel(WindowHead head_args, W
   // 5,000 203.5 / 200.5, 32 at 12,000 312 / 306.  One kernel for both was 1.5 % slower on blocks of four waves.
   const int computing = (min(nrows, (rb + 1) * RPB) - rb * RPB + 31) >> 5, feeder = wave - computing;
   auto play = [&](auto group) __attribute__((always_inline)) {
-    if constexpr (!FEW) {
+    if constexpr (CHUNK || !FEW) {
       if (has_rows) run(std::integral_constant<int, kComputeFeed>{}, group, gt);
       else run(std::integral_constant<int, kFeed1>{}, group, gt);
     } else {
@@ -639,6 +644,9 @@ void launch_attend_wide(const AttnArgs& A, hipStream_t st) {
   if (A.rows_per_block <= 96) launch_wide<false, true>(A, st);       // three waves of rows at most in every block
   else launch_wide<false, false>(A, st);
 }
-void launch_attend_chunk(const AttnArgs& A, hipStream_t st) { launch_wide<true, false>(A, st); }
+void launch_attend_chunk(const AttnArgs& A, hipStream_t st) {
+  if (A.kv.n_kv * ((kG * A.M + A.rows_per_block - 1) / A.rows_per_block) < 128) launch_wide<true, true>(A, st);
+  else launch_wide<true, false>(A, st);
+}
 
 }  // namespace yka
