@@ -57,10 +57,12 @@ def _slice_splits(kvh, M, ctx, capacity):
 
 @pytest.mark.parametrize("kvh,M,ctx,splits", [(1, 301, 200, 3), (1, 200, 300, 4), (1, 100, 300, 5), (1, 65, 500, 7), (1, 65, 600, 8), (1, 65, 700, 9),
                                               (1, 65, 1000, 10), (1, 129, 5200, 16), (1, 65, 2700, 17), (1, 65, 8000, 27),
-                                              (2, 1000, 100, 2), (1, 682, 1000, 4), (1, 683, 600, 4), (1, 683, 1400, 5)])
+                                              (2, 1000, 100, 2), (1, 682, 1000, 4), (1, 683, 600, 4), (1, 683, 1400, 5),
+                                              (3, 1820, 2700, 2), (3, 1821, 2700, 2)])
 def test_slice_splits_of_every_size(native, oracle, kvh, M, ctx, splits):
-    """Slices of 2 to 27 splits: a split lane of the combiner takes 1, 2, 4 or 8 partials, both sides of every line.  Of the last four one has
-    rows for almost all of the 4,096 waves launched (4,092), the others for more (4,098 and 12,000)."""
+    """Slices of 2 to 27 splits: a split lane of the combiner takes 1, 2, 4 or 8 partials, both sides of every line.  Then rows
+    for less and more than the 4,096 waves launched (4,092, 4,098, 12,000), and for one and for eight rows a step (32,760 and 32,778, 2 at
+    the end)."""
     assert _slice_splits(kvh, M, ctx, 8192) == splits
     q, k, v, kn, vn, _ = oracle.make_inputs(9300 + splits, ctx, M, 6 * kvh, kvh)
     oc = oracle.Cache(8192, 6 * kvh, kvh)

@@ -11,7 +11,7 @@ from yasakani_amd import isa_check
 
 # kernel name, 16-byte requests of a step, 4-byte requests of a step: one entry per step
 FORMS = [("attend_narrow.hip", "combine_rows_kernelILb0E", [(8, 2)]),
-         ("attend_narrow.hip", "combine_rows_kernelILb1E", [(1, 2), (2, 2), (4, 2), (8, 2)]),
+         ("attend_narrow.hip", "combine_rows_kernelILb1E", [(1, 2), (2, 2), (4, 2), (8, 2), (8, 16)]),
          ("attend_narrow.hip", "combine_kernelILi1ELb0ELb0E", [(4, 2)]),
          ("attend_narrow.hip", "combine_kernelILi4ELb0ELb0E", [(16, 8)]),
          ("attend256.hip", "combine256_kernelILi4ELi1ELb0ELi0E", [(4, 2)]),

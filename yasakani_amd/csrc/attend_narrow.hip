@@ -636,9 +636,10 @@ __global__ void __launch_bounds__(256) combine_kernel(CombineHead head_args, Com
 // here and should not pay for dispatching thousands of workgroups to find out (16 layers of 1,500 rows on an empty cache 637 us, with
 // 8 per CU 644).  A split lane asks for as many partials as there are splits for it, 1, 2, 4 or 8: eight whatever
 // their number cost as much as the row's own (4 layers of 300 rows at 2,000 tokens, one KV head, 7 splits 89.8 / 87.2 us; with eight KV heads 100 rows
-// there 101.5 / 98.3; 8 layers of 200 rows at 9,000, four heads, 364 / 355).  With few splits several rows a step, 8 / KN of them, measured
-// the same or took longer (4 layers, four KV heads, 800 rows at 2,000 tokens in 3 splits 231.0 / 221.6, 200 at 500 78.3 / 77.7; 2 splits of eight heads
-// alone gained, 800 rows at 2,000 409.5 / 411.7).
+// there 101.5 / 98.3; 8 layers of 200 rows at 9,000, four heads, 364 / 355).  Several rows a step, so that
+// eight pieces are in flight, are slower while waves have few steps (4 layers, four KV heads, 800 rows at 2,000 tokens in 3 splits, 1 / 8 rows
+// a step, 221.6 / 231.0, 200 at 500 77.7 / 78.3) and faster where every wave has eight rows of a partial a lane each (4 layers of 2,048 rows at
+// 3,000 tokens, 2 splits, 636 / 625, eight KV heads, 800 rows at 2,000 411.5 / 407).
 template <bool ADAPT>
 __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args, CombineTail tail_args) {
   CombineArgs A = combine_args(head_args, tail_args);
@@ -648,48 +649,59 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(CombineHead head_args
   }
   const int lane = threadIdx.x & 63, sl = lane >> 4, c8 = (lane & 15) * 8, total = A.M * A.n_heads;
   const uint32_t stride = (uint32_t)A.n_heads * kD * 2;
-  // KN partials a split lane: row = tok * n_heads + head
-  auto walk = [&](auto kn_tag) __attribute__((always_inline)) {
-    constexpr int KN = decltype(kn_tag)::value;
-    for (int row = blockIdx.x * 4 + (threadIdx.x >> 6); row < total; row += ADAPT ? 4 * (int)gridDim.x : total) {
-      uint4 u[KN];
+  // RB rows a step, KN partials a split lane: row = tok * n_heads + head
+  auto walk = [&](auto kn_tag, auto rb_tag) __attribute__((always_inline)) {
+    constexpr int KN = decltype(kn_tag)::value, RB = decltype(rb_tag)::value;
+    for (int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RB; row0 < total; row0 += ADAPT ? 4 * (int)gridDim.x * RB : total) {
+      float pmv[RB], plv[RB];
+      uint4 u[RB][KN];
       // lane t < S looks at split t; the maximum and every weight then come from cross-lane reads
-      const size_t p0 = (size_t)(row / A.n_heads) * A.S * A.n_heads + row % A.n_heads;
-      const uint32_t e = (uint32_t)min(lane, A.S - 1) * A.n_heads;
-      const float pmv = A.pm[p0 + e], plv = A.pl[p0 + e];
 #pragma unroll
-      for (int k = 0; k < KN; ++k)
-        u[k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(A.pacc16 + p0 * kD + c8) + (uint32_t)min(sl + 4 * k, A.S - 1) * stride);
-      all_requested();
-      const float M2 = lane_rows(lane_row16(pmv, LaneMax{}), LaneMax{});
-      const float wl = (lane < A.S && pmv > -1e29f) ? exp2f(pmv - M2) * plv : 0.f;     // weight of split `lane`
-      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      float wsum = 0.f;
+      for (int r = 0; r < RB; ++r) {
+        const int row = min(row0 + r, total - 1);
+        const size_t p0 = (size_t)(row / A.n_heads) * A.S * A.n_heads + row % A.n_heads;
+        const uint32_t e = (uint32_t)min(lane, A.S - 1) * A.n_heads;
+        pmv[r] = A.pm[p0 + e]; plv[r] = A.pl[p0 + e];
 #pragma unroll
-      for (int k = 0; k < KN; ++k) {
-        const float w = __shfl(wl, sl + 4 * k, 64);                        // < 32: a lane of this wave
-        const uint4 x = w != 0.f ? u[k] : make_uint4(0, 0, 0, 0);           // a row of weight 0 may be one that no workgroup wrote
-        const h8 v = __builtin_bit_cast(h8, x);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
-        wsum += w;
+        for (int k = 0; k < KN; ++k)
+          u[r][k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(A.pacc16 + p0 * kD + c8) + (uint32_t)min(sl + 4 * k, A.S - 1) * stride);
       }
+      all_requested();
 #pragma unroll
-      for (int c = 0; c < 8; ++c) acc[c] = lane_rows(acc[c], LaneAdd{});
-      wsum = lane_rows(wsum, LaneAdd{});
-      if (sl == 0) {
-        const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-        float yv[8];
+      for (int r = 0; r < RB; ++r) {
+        const float M2 = lane_rows(lane_row16(pmv[r], LaneMax{}), LaneMax{});
+        const float wl = (lane < A.S && pmv[r] > -1e29f) ? exp2f(pmv[r] - M2) * plv[r] : 0.f;     // weight of split `lane`
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float wsum = 0.f;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) yv[c] = acc[c] * inv;
-        *reinterpret_cast<uint4*>(A.out16 + (size_t)row * kD + c8) = pack_out8(yv, A.out_bf16);
+        for (int k = 0; k < KN; ++k) {
+          const float w = __shfl(wl, sl + 4 * k, 64);                        // < 32: a lane of this wave
+          const uint4 x = w != 0.f ? u[r][k] : make_uint4(0, 0, 0, 0);        // a row of weight 0 may be one that no workgroup wrote
+          const h8 v = __builtin_bit_cast(h8, x);
+#pragma unroll
+          for (int c = 0; c < 8; ++c) acc[c] += w * (float)v[c];
+          wsum += w;
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[c] = lane_rows(acc[c], LaneAdd{});
+        wsum = lane_rows(wsum, LaneAdd{});
+        if (sl == 0 && row0 + r < total) {
+          const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+          float yv[8];
+#pragma unroll
+          for (int c = 0; c < 8; ++c) yv[c] = acc[c] * inv;
+          *reinterpret_cast<uint4*>(A.out16 + (size_t)(row0 + r) * kD + c8) = pack_out8(yv, A.out_bf16);
+        }
       }
     }
   };
-  if (ADAPT && A.S <= 4) walk(std::integral_constant<int, 1>{});
-  else if (ADAPT && A.S <= 8) walk(std::integral_constant<int, 2>{});
-  else if (ADAPT && A.S <= 16) walk(std::integral_constant<int, 4>{});
-  else walk(std::integral_constant<int, 8>{});
+  const std::integral_constant<int, 1> c1{};
+  const std::integral_constant<int, 8> c8_rows{};
+  if (ADAPT && A.S <= 4 && total >= 32 * (int)gridDim.x) walk(c1, c8_rows);
+  else if (ADAPT && A.S <= 4) walk(c1, c1);
+  else if (ADAPT && A.S <= 8) walk(std::integral_constant<int, 2>{}, c1);
+  else if (ADAPT && A.S <= 16) walk(std::integral_constant<int, 4>{}, c1);
+  else walk(std::integral_constant<int, 8>{}, c1);
 }
 void launch_combine(const CombineArgs& A, hipStream_t st) {
   if (A.plan) {                                    // a stream may hold any share of the splits (256 at most)
