@@ -67,7 +67,8 @@ def test_against_the_decode_kernel(native, M, ctx, opts):
 
 # the 256-channel formats: slices of 1,024 tokens on the wide kernels, row blocks of equal height; the same comparison
 @pytest.mark.parametrize("kk", [0, 4, 5])
-@pytest.mark.parametrize("M,ctx,opts", [(65, 0, []), (22, 500, []), (43, 100, []), (1025, 0, []), (1100, 700, [(4, 1)]), (200, 3000, [(2, 3)])])
+# 107 and 140 rows: six row blocks and seven, the last of six and five waves of rows, on either of the int4 kernels
+@pytest.mark.parametrize("M,ctx,opts", [(65, 0, []), (22, 500, []), (43, 100, []), (107, 300, []), (140, 300, []), (1025, 0, []), (1100, 700, [(4, 1)]), (200, 3000, [(2, 3)])])
 def test_256_channel_rows(native, kk, M, ctx, opts):
     from yasakani_amd import kvqp
     rng = np.random.default_rng(M + ctx + kk)

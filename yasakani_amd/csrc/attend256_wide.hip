@@ -176,8 +176,8 @@ __device__ __forceinline__ void quant_store_word256(const KvView& kv, int kvh, i
 }  // namespace
 
 // grid (S, n_kv, row blocks), block 512; wave w owns rows [16 w, 16 (w+1)) of the block, waves beyond the block's rows only
-// help with the dequantization; BF: bf16 rows come in
-template <bool BF>
+// help with the dequantization; BF: bf16 rows come in; FULL: every wave decodes an eighth (the roles below)
+template <bool BF, bool FULL>
 __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(WindowHead head_args, WindowSizes size_args, WindowTail tail_args) {
   const AttnArgs A = window_args(head_args, size_args, tail_args);
   __shared__ __align__(16) uint8_t lds[2][kLdsBuf];
@@ -415,15 +415,25 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(WindowHead head_a
   // share a SIMD with one of those, take one.  us per 16 layers, an eighth by every wave / so: 8 rows (3 waves) at 20,000 tokens
   // 308 / 297, 12 (5) at 9,000 287 / 267.5, 13 (5) at 20,000 358.6 (three eighths to each of the three waves) / 341, 16 (6) at 9,000
   // 310.7 / 294, 32 (6) at 8,000 357.7 / 343.6, 15 (6) at 20,000 387 / 367.
-  const int computing = (row_end - rb * RPB + 15) >> 4, feeder = wave - computing;
-  if (has_rows && (computing >= 7 ? wave < 4 : computing >= 5 && (wave & 2) != 0))
-    run(std::integral_constant<int, kFeedFirst>{}, computing >= 7 ? tid : tid - 128);
-  else if (has_rows && computing >= 7) run(std::integral_constant<int, kComputeFirst>{}, tid);
-  else if (has_rows) run(std::integral_constant<int, kComputeOnly>{}, lane);
-  else if (computing >= 7) run(std::integral_constant<int, kFeed1>{}, tid);
-  else if (computing == 6) run(std::integral_constant<int, kFeed3>{}, 64 * (2 + 3 * feeder) + lane);
-  else if (feeder < 4) run(std::integral_constant<int, kFeed2>{}, 64 * ((computing == 5 ? 2 : 0) + 2 * feeder) + lane);
-  else run(std::integral_constant<int, kIdle>{}, lane);
+  // A kernel of their own for launches of such blocks (FULL): beside the other roles the compiler's loops for them are slower.  us per 4
+  // layers, one kernel / so: 64 rows at 9,000 tokens 116.5 / 115.5, 200 at 30,000 770 / 751, 1,000 at 9,000 1,191 / 1,171, 1,500 at 30,000
+  // 5,152 / 5,046.  A last block of fewer rows is better off with the roles of its own (33 rows at 9,000, 112 + 86 in blocks, 93.0 / 96.8
+  // without, 53 at 2,000 83.7 / 86.2, 70 first rows 59.9 / 61.2) up to six blocks; in more it does not show (150 rows, 12 in the last, at 9,000 230.4 / 226.7).
+  if constexpr (FULL) {
+    if (!has_rows) run(std::integral_constant<int, kFeed1>{}, tid);
+    else if (wave < 4) run(std::integral_constant<int, kFeedFirst>{}, tid);
+    else run(std::integral_constant<int, kComputeFirst>{}, tid);
+  } else {
+    const int computing = (row_end - rb * RPB + 15) >> 4, feeder = wave - computing;
+    if (has_rows && (computing >= 7 ? wave < 4 : computing >= 5 && (wave & 2) != 0))
+      run(std::integral_constant<int, kFeedFirst>{}, computing >= 7 ? tid : tid - 128);
+    else if (has_rows && computing >= 7) run(std::integral_constant<int, kComputeFirst>{}, tid);
+    else if (has_rows) run(std::integral_constant<int, kComputeOnly>{}, lane);
+    else if (computing >= 7) run(std::integral_constant<int, kFeed1>{}, tid);
+    else if (computing == 6) run(std::integral_constant<int, kFeed3>{}, 64 * (2 + 3 * feeder) + lane);
+    else if (feeder < 4) run(std::integral_constant<int, kFeed2>{}, 64 * ((computing == 5 ? 2 : 0) + 2 * feeder) + lane);
+    else run(std::integral_constant<int, kIdle>{}, lane);
+  }
   if (!has_rows) return;                       // no barrier follows
   // ---- partials: normalised fp16.  o[b][r] of lane (row i, group g) is channel 16b + 4g + r.  Rows go through LDS (the
   //      tile buffers are free after the last barrier) so that every store instruction writes whole 512-byte rows ----
@@ -453,11 +463,17 @@ __global__ void __launch_bounds__(NT, 1) attend256_wide_kernel(WindowHead head_a
   }
 }
 
-void launch_attend256_wide(const AttnArgs& A, hipStream_t st) {
+template <bool FULL>
+static void launch(const AttnArgs& A, hipStream_t st) {
   const int rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block;
   const dim3 grid(A.S, A.kv.n_kv, rb);
-  if (A.in_bf16) hipLaunchKernelGGL(attend256_wide_kernel<true>, grid, dim3(NT), 0, st, window_head(A), window_sizes(A), window_tail(A));
-  else hipLaunchKernelGGL(attend256_wide_kernel<false>, grid, dim3(NT), 0, st, window_head(A), window_sizes(A), window_tail(A));
+  if (A.in_bf16) hipLaunchKernelGGL((attend256_wide_kernel<true, FULL>), grid, dim3(NT), 0, st, window_head(A), window_sizes(A), window_tail(A));
+  else hipLaunchKernelGGL((attend256_wide_kernel<false, FULL>), grid, dim3(NT), 0, st, window_head(A), window_sizes(A), window_tail(A));
+}
+void launch_attend256_wide(const AttnArgs& A, hipStream_t st) {
+  const int rb = (kG * A.M + A.rows_per_block - 1) / A.rows_per_block, last = kG * A.M - (rb - 1) * A.rows_per_block;
+  if (A.rows_per_block > 96 && (last > 96 || rb > 6)) launch<true>(A, st);
+  else launch<false>(A, st);
 }
 
 }  // namespace yka
